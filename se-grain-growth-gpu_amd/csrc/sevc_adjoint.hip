@@ -18,49 +18,206 @@
 namespace sevc {
 
 // Boundary energies for the window (compute_boundary_energies,
-// calculus.h:104-114) and their derivative e_b = d gamma_b / d GB_scaling.
-__global__ void k_win_prepare(Dev d, double* ebase) {
+// calculus.h:104-114).
+__global__ void k_win_prepare(Dev d) {
     TABLE_BLOCK(d.eblk, d.neb)
     if (i >= bd_.e || !d.benab[i]) return;
     const double e = (P.gb_eps == 0.0) ? 1.0 : boundary_compute_energy(d, i, P.gb_eps);
     d.ben[i] = e * P.gb_scaling;
-    ebase[i] = e;
 }
 
-// Grain areas at positions X (compute_grain_areas, calculus.h:224-234);
-// also into the state's area array when to_state is set.
-__global__ void k_win_area(Dev d, const double* X, double* A, int to_state) {
+// The window's topology is fixed, so what every step would look up again
+// (a vertex's edges, their far ends, its place in its three grains' lists,
+// the list neighbours there) is looked up once per window and kept in
+// vertex and grain order:
+//   nbr[v]  (w0, w1, w2, code): the far ends of the vertex's edges and, per
+//           grain slot j, which of them are the list's previous and next
+//           vertex (code bits 4j..4j+1 and 4j+2..4j+3) and whether the slot
+//           counts at all (bit 12 + j: the vertex is in the list and the
+//           list has 3 entries or more); kWinOn: an enabled vertex;
+//           kWinSearch: a list neighbour is not the end of one of the
+//           vertex's edges (the steps then search the lists)
+//   vse[3v + j]  stored energy of grain slot j
+//   veb[3v + j]  d gamma_b / d GB_scaling of edge j (null when every member
+//           has GB_eps = 0, where it is 1)
+//   wl[kq G + g]  entries 4 kq .. 4 kq + 3 of grain g's list, wn[g] its length
+//           (-1: disabled)
+// A step then takes two rounds of loads (these tables, then positions and
+// area signs) in place of six dependent ones.  Measured, 10,000 grains: the
+// step kernel 10.7 -> 4.6 us, the reverse step 11.4 -> 5.1, the areas 6.4 ->
+// 4.3 (an empty launch takes 4.5 in a busy stream: what is left is dispatch);
+// 16 members of 11,000 grains: 34.8 -> 12.4, 49.0 -> 18.5, 14.0 -> 8.5.
+constexpr int kWinOn = 1 << 16, kWinSearch = 1 << 15;
+constexpr int kWinList = 12;                 // list entries held in the table (longer lists are read on)
+
+__global__ void k_win_table_v(Dev d, int4* nbr, double* vse, double* veb) {
+    TABLE_BLOCK(d.vblk, d.nvb)
+    if (i >= bd_.e) return;
+    const int v = i;
+    if (!d.ven[v]) {
+        nbr[v] = make_int4(v, v, v, 0);
+        return;
+    }
+    int w[3], code = kWinOn;
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        const int b = d.vb[3 * v + j];
+        w[j] = other_end(d, b, v);
+        if (veb) veb[3 * (size_t)v + j] = (P.gb_eps == 0.0) ? 1.0 : boundary_compute_energy(d, b, P.gb_eps);
+    }
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        const int g = d.vg[3 * v + j];
+        const int n = d.glen[g];
+        const int k = grain_contains_vertex(d, g, v);
+        vse[3 * (size_t)v + j] = d.gse[g];
+        if (k < 0 || n < 3) continue;
+        const int* L = glist(d, g);
+        const int wp = L[(k + n - 1) % n], wn = L[(k + 1) % n];
+        const int ip = wp == w[0] ? 0 : (wp == w[1] ? 1 : (wp == w[2] ? 2 : 3));
+        const int in = wn == w[0] ? 0 : (wn == w[1] ? 1 : (wn == w[2] ? 2 : 3));
+        if (ip == 3 || in == 3) code |= kWinSearch;
+        code |= (ip << (4 * j)) | (in << (4 * j + 2)) | (1 << (12 + j));
+    }
+    nbr[v] = make_int4(w[0], w[1], w[2], code);
+}
+
+__global__ void k_win_table_g(Dev d, int4* wl, int* wn) {
     TABLE_BLOCK(d.gblk, d.ngb)
-    if (i >= bd_.e || !d.genab[i]) return;
-    const double a = grain_area_at(d, X, i, P.D);
-    A[i] = a;
-    if (to_state) d.garea[i] = a;
+    if (i >= bd_.e) return;
+    const int n = d.genab[i] ? d.glen[i] : -1;
+    const int* L = glist(d, i);
+    wn[i] = n;
+#pragma unroll
+    for (int q = 0; q < kWinList / 4; q++) {
+        int e[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) e[r] = 4 * q + r < n ? L[4 * q + r] : 0;
+        wl[(size_t)q * d.G + i] = make_int4(e[0], e[1], e[2], e[3]);
+    }
+}
+
+// Signs of the grain areas at positions X (compute_grain_areas,
+// calculus.h:224-234; the analytic force needs no more of them): neg[g] = 1
+// for a negative area.  The areas themselves go to `area` when given (the
+// last step of the window's forward leaves them in the state).
+__global__ void k_win_area(Dev d, const double* X, const int4* wl, const int* wn, uint8_t* neg, double* area) {
+    TABLE_BLOCK(d.gblk, d.ngb)
+    if (i >= bd_.e) return;
+    const int n = wn[i];
+    int L[kWinList];
+#pragma unroll
+    for (int q = 0; q < kWinList / 4; q++) {
+        const int4 t = wl[(size_t)q * d.G + i];
+        L[4 * q] = t.x; L[4 * q + 1] = t.y; L[4 * q + 2] = t.z; L[4 * q + 3] = t.w;
+    }
+    if (n < 0) return;
+    const double2* X2 = reinterpret_cast<const double2*>(X);
+    double2 p[kWinList];
+#pragma unroll
+    for (int k = 0; k < kWinList; k++) p[k] = k < n ? X2[L[k]] : make_double2(0.0, 0.0);
+    const double D = P.D;
+    double a = 0.0;
+    if (n > 0) {
+        AreaAcc acc;
+        acc.start(p[0].x, p[0].y);
+#pragma unroll
+        for (int k = 1; k < kWinList; k++)
+            if (k < n) acc.push(p[k].x, p[k].y, D);
+        if (n > kWinList) {
+            const int* Lg = glist(d, i);
+            for (int k = kWinList; k < n; k++) {
+                const double2 q = X2[Lg[k]];
+                acc.push(q.x, q.y, D);
+            }
+        }
+        a = acc.finish();
+    }
+    neg[i] = a < 0 ? 1 : 0;
+    if (area) area[i] = a;
+}
+
+// The list neighbours (previous, next) of v in its grain slot j, by search
+// (kWinSearch vertices only).
+__device__ __forceinline__ void win_search(const Dev& d, int v, int g, int* wp, int* wn) {
+    const int n = d.glen[g], k = grain_contains_vertex(d, g, v);
+    const int* L = glist(d, g);
+    *wp = L[(k + n - 1) % n];
+    *wn = L[(k + 1) % n];
+}
+
+// One of three values by a run-time index, by selects on values (indexing an
+// array would put it into LDS or scratch).
+__device__ __forceinline__ double2 pick3(double2 a, double2 b, double2 c, int k) {
+    const double x = k == 0 ? a.x : (k == 1 ? b.x : c.x), y = k == 0 ? a.y : (k == 1 ? b.y : c.y);
+    return make_double2(x, y);
 }
 
 // One window step x_n -> x_{n+1}: analytic velocity (calculus.h:143-154
-// with the analytic model) and update_vertices_positions
-// (calculus.h:391-404), written to a separate array so that neighbours
-// still read x_n.  Disabled slots are copied.
-__global__ void k_win_step(Dev d, const double* X, const double* A, double* Xn, int write_vel) {
+// with the analytic model, the sums of analytic_force_at) and
+// update_vertices_positions (calculus.h:391-404), written to a separate
+// array so that neighbours still read x_n.  Disabled slots are copied.
+__global__ void __launch_bounds__(kBlock) k_win_step(Dev d, const double* X, const uint8_t* neg, const int4* nbr,
+                                                     const double* vse, const double* veb, double* Xn, int write_vel) {
     TABLE_BLOCK(d.vblk, d.nvb)
     if (i >= bd_.e) return;
-    if (!d.ven[i]) {
-        Xn[2 * i] = X[2 * i];
-        Xn[2 * i + 1] = X[2 * i + 1];
+    const double2* X2 = reinterpret_cast<const double2*>(X);
+    const int4 t = nbr[i];
+    const double2 p = X2[i];
+    int g[3];
+    double se[3], eb[3];
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        g[j] = d.vg[3 * i + j];
+        se[j] = vse[3 * (size_t)i + j];
+        eb[j] = veb ? veb[3 * (size_t)i + j] : 1.0;
+    }
+    if (!(t.w & kWinOn)) {
+        reinterpret_cast<double2*>(Xn)[i] = p;
         return;
     }
-    double fx, fy;
-    analytic_force_at(d, X, A, P, i, &fx, &fy);
-    const double vx = fx * P.mobility, vy = fy * P.mobility;
-    if (write_vel) {
-        d.vel[2 * i] = vx;
-        d.vel[2 * i + 1] = vy;
+    const double2 q[3] = {X2[t.x], X2[t.y], X2[t.z]};
+    uint8_t ng[3];
+#pragma unroll
+    for (int j = 0; j < 3; j++) ng[j] = neg[g[j]];
+    const double D = P.D, x = p.x, y = p.y;
+    double ex = 0.0, ey = 0.0, gx = 0.0, gy = 0.0;
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        const double dx = wrapd(x, q[j].x, D), dy = wrapd(y, q[j].y, D);
+        const double L = mag(dx, dy);
+        const double gam = eb[j] * P.gb_scaling;
+        if (L > 0) {
+            ex += gam * (dx / L);
+            ey += gam * (dy / L);
+        }
     }
-    double x = X[2 * i], y = X[2 * i + 1];
-    x += vx * P.dt_max;
-    y += vy * P.dt_max;
-    Xn[2 * i] = dom_mod(x, P.D);
-    Xn[2 * i + 1] = dom_mod(y, P.D);
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        if (!((t.w >> (12 + j)) & 1)) continue;
+        double2 a, b;
+        if (t.w & kWinSearch) {
+            int wp, wn;
+            win_search(d, i, g[j], &wp, &wn);
+            a = X2[wp];
+            b = X2[wn];
+        } else {
+            a = pick3(q[0], q[1], q[2], (t.w >> (4 * j)) & 3);
+            b = pick3(q[0], q[1], q[2], (t.w >> (4 * j + 2)) & 3);
+        }
+        const double dpx = wrapd(x, a.x, D), dpy = wrapd(y, a.y, D);
+        const double dnx = wrapd(b.x, x, D), dny = wrapd(b.y, y, D);
+        const double sg = ng[j] ? -1.0 : 1.0;
+        const double c = se[j] * sg * 0.5;
+        gx += c * (dpy + dny);
+        gy += c * (-(dpx + dnx));
+    }
+    const double vx = -(ex + gx) * P.mobility, vy = -(ey + gy) * P.mobility;
+    if (write_vel) reinterpret_cast<double2*>(d.vel)[i] = make_double2(vx, vy);
+    double xn = x, yn = y;
+    xn += vx * P.dt_max;
+    yn += vy * P.dt_max;
+    reinterpret_cast<double2*>(Xn)[i] = make_double2(dom_mod(xn, D), dom_mod(yn, D));
 }
 
 // Window end: step counter and time as k_end advances them per step.
@@ -90,7 +247,7 @@ __global__ void k_win_init(Dev d, double* lam, double* acc_mu, double* acc_s, do
 }
 
 // One reverse step at vertex v, with lambda = dL/dx_{n+1} and the state
-// x_n (positions X, grain areas A):
+// x_n (positions X, area signs neg):
 //   lambda_n  = lambda - dt mu (H lambda)_v
 //   acc_mu   += dt (lambda . F_v)
 //   acc_s    += dt mu (lambda . dF_v/dGB_scaling),  dF_v/ds = -sum_b e_b u_b
@@ -99,66 +256,94 @@ __global__ void k_win_init(Dev d, double* lam, double* acc_mu, double* acc_s, do
 // (gamma_b / L)(I - u u^T)(lambda_v - lambda_w) to (H lambda)_v; a grain g
 // with list neighbours prev, next adds
 // SE_g sign(A_g)/2 (lambda_next.y - lambda_prev.y, lambda_prev.x - lambda_next.x).
-__global__ void k_win_adjoint(Dev d, const double* X, const double* A, const double* lam, double* lam2,
-                              double* acc_mu, double* acc_s, double* acc_se, const double* ebase) {
+__global__ void __launch_bounds__(kBlock) k_win_adjoint(Dev d, const double* X, const uint8_t* neg, const int4* nbr,
+                                                        const double* vse, const double* veb, const double* lam,
+                                                        double* lam2, double* acc_mu, double* acc_s, double* acc_se) {
     TABLE_BLOCK(d.vblk, d.nvb)
     if (i >= bd_.e) return;
     const int v = i;
-    if (!d.ven[v]) {
-        lam2[2 * v] = 0.0;
-        lam2[2 * v + 1] = 0.0;
+    const double2* X2 = reinterpret_cast<const double2*>(X);
+    const double2* M2 = reinterpret_cast<const double2*>(lam);
+    const int4 t = nbr[v];
+    const double2 p = X2[v], l = M2[v];
+    int g[3];
+    double se[3], ebs[3], ase[3];
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        g[j] = d.vg[3 * v + j];
+        se[j] = vse[3 * (size_t)v + j];
+        ebs[j] = veb ? veb[3 * (size_t)v + j] : 1.0;
+        ase[j] = acc_se[3 * (size_t)v + j];
+    }
+    const double am = acc_mu[v], as = acc_s[v];
+    if (!(t.w & kWinOn)) {
+        reinterpret_cast<double2*>(lam2)[v] = make_double2(0.0, 0.0);
         return;
     }
+    const double2 q[3] = {X2[t.x], X2[t.y], X2[t.z]};
+    const double2 m[3] = {M2[t.x], M2[t.y], M2[t.z]};
+    uint8_t ng[3];
+#pragma unroll
+    for (int j = 0; j < 3; j++) ng[j] = neg[g[j]];
     const double D = P.D, mu = P.mobility, dt = P.dt_max, dtm = dt * mu;
-    const double x = X[2 * v], y = X[2 * v + 1];
-    const double lx = lam[2 * v], ly = lam[2 * v + 1];
+    const double x = p.x, y = p.y;
+    const double lx = l.x, ly = l.y;
     double ex = 0.0, ey = 0.0, gx = 0.0, gy = 0.0;
     double hex = 0.0, hey = 0.0, hgx = 0.0, hgy = 0.0, sx = 0.0, sy = 0.0;
+#pragma unroll
     for (int j = 0; j < 3; j++) {
-        const int b = d.vb[3 * v + j];
-        const int w = other_end(d, b, v);
-        const double dx = wrapd(x, X[2 * w], D), dy = wrapd(y, X[2 * w + 1], D);
+        const double dx = wrapd(x, q[j].x, D), dy = wrapd(y, q[j].y, D);
         const double L = mag(dx, dy);
         if (L > 0) {
             const double ux = dx / L, uy = dy / L;
-            const double gam = d.ben[b];
+            const double eb = ebs[j];
+            const double gam = eb * P.gb_scaling;
             ex += gam * ux;
             ey += gam * uy;
-            const double wx = lx - lam[2 * w], wy = ly - lam[2 * w + 1];
+            const double wx = lx - m[j].x, wy = ly - m[j].y;
             const double uw = ux * wx + uy * wy;
             const double c = gam / L;
             hex += c * (wx - ux * uw);
             hey += c * (wy - uy * uw);
-            const double eb = ebase[b];
             sx += eb * ux;
             sy += eb * uy;
         }
     }
+#pragma unroll
     for (int j = 0; j < 3; j++) {
-        const int g = d.vg[3 * v + j];
-        const int n = d.glen[g];
-        const int k = grain_contains_vertex(d, g, v);
-        if (k < 0 || n < 3) continue;
-        const int* Lg = glist(d, g);
-        const int wp = Lg[(k + n - 1) % n], wn = Lg[(k + 1) % n];
-        const double dpx = wrapd(x, X[2 * wp], D), dpy = wrapd(y, X[2 * wp + 1], D);
-        const double dnx = wrapd(X[2 * wn], x, D), dny = wrapd(X[2 * wn + 1], y, D);
-        const double sg = A[g] < 0 ? -1.0 : 1.0;
-        const double c = d.gse[g] * sg * 0.5;
+        if (!((t.w >> (12 + j)) & 1)) continue;
+        double2 a, b, la, lb;
+        if (t.w & kWinSearch) {
+            int wp, wn;
+            win_search(d, v, g[j], &wp, &wn);
+            a = X2[wp];
+            b = X2[wn];
+            la = M2[wp];
+            lb = M2[wn];
+        } else {
+            const int ip = (t.w >> (4 * j)) & 3, in = (t.w >> (4 * j + 2)) & 3;
+            a = pick3(q[0], q[1], q[2], ip);
+            b = pick3(q[0], q[1], q[2], in);
+            la = pick3(m[0], m[1], m[2], ip);
+            lb = pick3(m[0], m[1], m[2], in);
+        }
+        const double dpx = wrapd(x, a.x, D), dpy = wrapd(y, a.y, D);
+        const double dnx = wrapd(b.x, x, D), dny = wrapd(b.y, y, D);
+        const double sg = ng[j] ? -1.0 : 1.0;
+        const double c = se[j] * sg * 0.5;
         gx += c * (dpy + dny);
         gy += c * (-(dpx + dnx));
-        hgx += c * (lam[2 * wn + 1] - lam[2 * wp + 1]);
-        hgy += c * (lam[2 * wp] - lam[2 * wn]);
-        const double q = sg * 0.5;
-        const double tse = -(lx * (q * (dpy + dny)) + ly * (q * (-(dpx + dnx))));
-        acc_se[3 * v + j] += dtm * tse;
+        hgx += c * (lb.y - la.y);
+        hgy += c * (la.x - lb.x);
+        const double h = sg * 0.5;
+        const double tse = -(lx * (h * (dpy + dny)) + ly * (h * (-(dpx + dnx))));
+        acc_se[3 * (size_t)v + j] = ase[j] + dtm * tse;
     }
     const double fx = -(ex + gx), fy = -(ey + gy);
     const double hx = hex + hgx, hy = hey + hgy;
-    acc_mu[v] += dt * (lx * fx + ly * fy);
-    acc_s[v] += dtm * (-(lx * sx + ly * sy));
-    lam2[2 * v] = lx - dtm * hx;
-    lam2[2 * v + 1] = ly - dtm * hy;
+    acc_mu[v] = am + dt * (lx * fx + ly * fy);
+    acc_s[v] = as + dtm * (-(lx * sx + ly * sy));
+    reinterpret_cast<double2*>(lam2)[v] = make_double2(lx - dtm * hx, ly - dtm * hy);
 }
 
 // Level 1 of the deterministic parameter sums: one lane per 256-vertex

@@ -54,13 +54,17 @@ __global__ void k_begin_rate(Dev d, int rescale_flipped);
 __global__ void k_nucl_manager(Dev d);
 __global__ void k_nucl_insert(Dev d);
 // kernels of sevc_adjoint.hip
-__global__ void k_win_prepare(Dev d, double* ebase);
-__global__ void k_win_area(Dev d, const double* X, double* A, int to_state);
-__global__ void k_win_step(Dev d, const double* X, const double* A, double* Xn, int write_vel);
+__global__ void k_win_prepare(Dev d);
+__global__ void k_win_table_v(Dev d, int4* nbr, double* vse, double* veb);
+__global__ void k_win_table_g(Dev d, int4* wl, int* wn);
+__global__ void k_win_area(Dev d, const double* X, const int4* wl, const int* wn, uint8_t* neg, double* area);
+__global__ void k_win_step(Dev d, const double* X, const uint8_t* neg, const int4* nbr, const double* vse,
+                           const double* veb, double* Xn, int write_vel);
 __global__ void k_win_end(Dev d, int steps);
 __global__ void k_win_init(Dev d, double* lam, double* acc_mu, double* acc_s, double* acc_se);
-__global__ void k_win_adjoint(Dev d, const double* X, const double* A, const double* lam, double* lam2,
-                              double* acc_mu, double* acc_s, double* acc_se, const double* ebase);
+__global__ void k_win_adjoint(Dev d, const double* X, const uint8_t* neg, const int4* nbr, const double* vse,
+                              const double* veb, const double* lam, double* lam2, double* acc_mu, double* acc_s,
+                              double* acc_se);
 __global__ void k_win_sum_l1(Dev d, const double* acc_mu, const double* acc_s, double* part);
 __global__ void k_win_sum_up(Dev d, double* part, double* out);
 __global__ void k_win_dse(Dev d, const double* acc_se, double* dse);
@@ -131,15 +135,20 @@ struct sevc_state {
     };
     std::vector<Ckpt> ckpts;
     // topology-fixed window: checkpoints of x every K steps (ck), the
-    // positions and areas of one segment (seg, segA; `holds` = its index),
-    // and the reverse-pass arrays
+    // positions and area signs of one segment (seg, segN; `holds` = its
+    // index), the topology tables of the steps (k_win_table_v / _g), and the
+    // reverse-pass arrays
     struct Window {
         int steps = 0, K = 0, nck = 0, holds = -1;
         bool ready = false;
-        double *ck = nullptr, *seg = nullptr, *segA = nullptr;
-        size_t ck_n = 0, seg_n = 0, segA_n = 0;
+        double *ck = nullptr, *seg = nullptr;
+        uint8_t* segN = nullptr;
+        size_t ck_n = 0, seg_n = 0, segN_n = 0;
+        int4 *nbr = nullptr, *wl = nullptr;
+        int* wn = nullptr;
+        double *vse = nullptr, *veb = nullptr;   // veb: only with a member of GB_eps != 0
         double *lamA = nullptr, *lamB = nullptr, *acc_mu = nullptr, *acc_s = nullptr, *acc_se = nullptr;
-        double *ebase = nullptr, *part = nullptr, *out = nullptr, *dse = nullptr;
+        double *part = nullptr, *out = nullptr, *dse = nullptr;
         bool seeded = false;              // lamA holds dL/dx from sevc_area_histogram
         // area histogram loss
         double *hA = nullptr, *hwg = nullptr, *hpart = nullptr, *hrange = nullptr, *htarget = nullptr;
@@ -1368,8 +1377,9 @@ int sevc_set_member_params(sevc_state* s, int32_t m, const double* pos, const do
 
 namespace {
 
-// (Re)allocate a window buffer of at least n doubles.
-int win_buffer(sevc_state* s, double** p, size_t* have, size_t n) {
+// (Re)allocate a window buffer of at least n values.
+template <typename T>
+int win_buffer(sevc_state* s, T** p, size_t* have, size_t n) {
     if (*p && *have >= n) return SEVC_OK;
     if (*p) {
         (void)hipStreamSynchronize(s->stream);
@@ -1386,12 +1396,14 @@ int win_buffer(sevc_state* s, double** p, size_t* have, size_t n) {
 // Reverse-pass arrays whose size depends only on the state.
 int win_fixed_buffers(sevc_state* s) {
     auto& w = s->win;
-    if (w.lamA) return SEVC_OK;
+    if (w.dse) return SEVC_OK;               // the last one allocated below
     const size_t V = s->V, n2 = 2 * V;
     int rc;
     if ((rc = dalloc(s, &w.lamA, n2)) || (rc = dalloc(s, &w.lamB, n2)) || (rc = dalloc(s, &w.acc_mu, V)) ||
         (rc = dalloc(s, &w.acc_s, V)) || (rc = dalloc(s, &w.acc_se, 3 * V)) ||
-        (rc = dalloc(s, &w.ebase, static_cast<size_t>(s->E))) ||
+        (rc = dalloc(s, &w.nbr, V)) || (rc = dalloc(s, &w.vse, 3 * V)) ||
+        (s->any_aniso && (rc = dalloc(s, &w.veb, 3 * V)) != SEVC_OK) ||
+        (rc = dalloc(s, &w.wl, 3 * static_cast<size_t>(s->G))) || (rc = dalloc(s, &w.wn, static_cast<size_t>(s->G))) ||
         (rc = dalloc(s, &w.part, 4 * static_cast<size_t>(s->d.nvb))) ||
         (rc = dalloc(s, &w.out, 2 * static_cast<size_t>(s->B))) ||
         (rc = dalloc(s, &w.dse, static_cast<size_t>(s->G))))
@@ -1399,19 +1411,22 @@ int win_fixed_buffers(sevc_state* s) {
     return SEVC_OK;
 }
 
-// Steps x_{c K} .. of segment c from the segment buffer's slot 0; areas of
-// each step into segA.  Forward of the window (state outputs on) or its
-// recomputation in the reverse pass (off).
-void win_run_segment(sevc_state* s, int len, bool forward) {
+// Steps x_{c K} .. of segment c from the segment buffer's slot 0; the area
+// signs of each step into segN.  `last`: the step (of this segment) that
+// leaves its velocities and areas in the state, the window's last one (-1:
+// none, as in the recomputation of the reverse pass).
+void win_run_segment(sevc_state* s, int len, int last) {
     const Dev& d = s->d;
     auto& w = s->win;
     const size_t n2 = 2 * static_cast<size_t>(s->V);
     for (int i = 0; i < len; ++i) {
         const double* X = w.seg + i * n2;
-        double* A = w.segA + static_cast<size_t>(i) * s->G;
-        launch(s, "win_area", k_win_area, d.ngb, kBlock, d, X, A, forward ? 1 : 0);
-        launch(s, "win_step", k_win_step, d.nvb, kBlock, d, X, static_cast<const double*>(A),
-               w.seg + (i + 1) * n2, forward ? 1 : 0);
+        uint8_t* neg = w.segN + static_cast<size_t>(i) * s->G;
+        launch(s, "win_area", k_win_area, d.ngb, kBlock, d, X, static_cast<const int4*>(w.wl),
+               static_cast<const int*>(w.wn), neg, i == last ? d.garea : static_cast<double*>(nullptr));
+        launch(s, "win_step", k_win_step, d.nvb, kBlock, d, X, static_cast<const uint8_t*>(neg),
+               static_cast<const int4*>(w.nbr), static_cast<const double*>(w.vse), static_cast<const double*>(w.veb),
+               w.seg + (i + 1) * n2, i == last ? 1 : 0);
     }
 }
 
@@ -1429,19 +1444,21 @@ int sevc_window_forward(sevc_state* s, int32_t steps, int32_t ckpt_every) {
     int rc;
     if ((rc = win_buffer(s, &w.ck, &w.ck_n, std::max<size_t>(1, nck) * n2)) != SEVC_OK ||
         (rc = win_buffer(s, &w.seg, &w.seg_n, (static_cast<size_t>(K) + 1) * n2)) != SEVC_OK ||
-        (rc = win_buffer(s, &w.segA, &w.segA_n, static_cast<size_t>(K) * s->G)) != SEVC_OK)
+        (rc = win_buffer(s, &w.segN, &w.segN_n, static_cast<size_t>(K) * s->G)) != SEVC_OK)
         return rc;
     if ((rc = win_fixed_buffers(s)) != SEVC_OK) return rc;
     w.ready = false;
     w.seeded = false;
-    launch(s, "win_prepare", k_win_prepare, d.neb, kBlock, d, w.ebase);
+    launch(s, "win_prepare", k_win_prepare, d.neb, kBlock, d);
+    launch(s, "win_table_v", k_win_table_v, d.nvb, kBlock, d, w.nbr, w.vse, w.veb);
+    launch(s, "win_table_g", k_win_table_g, d.ngb, kBlock, d, w.wl, w.wn);
     HIPCHK(hipMemcpyAsync(w.seg, d.pos, n2 * 8, hipMemcpyDeviceToDevice, s->stream));
     int last = 0;
     for (int c = 0; c < nck; ++c) {
         const int len = std::min(K, steps - c * K);
         if (c > 0) HIPCHK(hipMemcpyAsync(w.seg, w.seg + last * n2, n2 * 8, hipMemcpyDeviceToDevice, s->stream));
         HIPCHK(hipMemcpyAsync(w.ck + c * n2, w.seg, n2 * 8, hipMemcpyDeviceToDevice, s->stream));
-        win_run_segment(s, len, true);
+        win_run_segment(s, len, c == nck - 1 ? len - 1 : -1);
         last = len;
     }
     if (steps > 0) HIPCHK(hipMemcpyAsync(d.pos, w.seg + last * n2, n2 * 8, hipMemcpyDeviceToDevice, s->stream));
@@ -1479,14 +1496,15 @@ int sevc_adjoint_window(sevc_state* s, const double* const* dL_dpos, sevc_grads*
         const int len = std::min(w.K, w.steps - c * w.K);
         if (w.holds != c) {
             HIPCHK(hipMemcpyAsync(w.seg, w.ck + c * n2, n2 * 8, hipMemcpyDeviceToDevice, s->stream));
-            win_run_segment(s, len, false);
+            win_run_segment(s, len, -1);
             w.holds = c;
         }
         for (int i = len - 1; i >= 0; --i) {
             launch(s, "win_adjoint", k_win_adjoint, d.nvb, kBlock, d, static_cast<const double*>(w.seg + i * n2),
-                   static_cast<const double*>(w.segA + static_cast<size_t>(i) * s->G),
-                   static_cast<const double*>(cur), nxt, w.acc_mu, w.acc_s, w.acc_se,
-                   static_cast<const double*>(w.ebase));
+                   static_cast<const uint8_t*>(w.segN + static_cast<size_t>(i) * s->G),
+                   static_cast<const int4*>(w.nbr), static_cast<const double*>(w.vse),
+                   static_cast<const double*>(w.veb), static_cast<const double*>(cur), nxt, w.acc_mu, w.acc_s,
+                   w.acc_se);
             std::swap(cur, nxt);
         }
     }
