@@ -105,4 +105,20 @@ struct Dev {
     int free_rows;                        // blocks per kind of one free-slot search round (0: the default)
 };
 
+// One array of a mesh download (k_pack): n items of `src` go to byte `dst` of
+// the staging buffer.  PACK_RAW copies n 4-byte words, PACK_BYTE n bytes,
+// PACK_ID n ids (off taken from those >= 0); PACK_ROW takes the first `row`
+// ids of each `stride` of src, n ids in all.
+enum { PACK_RAW = 0, PACK_BYTE, PACK_ID, PACK_ROW };
+struct PackSeg {
+    const void* src;
+    unsigned long long dst, n;
+    int kind, off, row, stride;
+};
+constexpr int kPackSegs = 24;
+struct PackList {
+    PackSeg seg[kPackSegs];
+    int n;
+};
+
 }  // namespace sevc
