@@ -33,14 +33,13 @@ __global__ void k_velocity_analytic(Dev d);
 __global__ void k_grain_dadt(Dev d);
 __global__ void k_translate(Dev d);
 __global__ void k_text(Dev d);
-__global__ void k_label(Dev d);
+__global__ void k_label_disabled(Dev d);
 __global__ void k_poll_gather(Dev d);
 __global__ void k_poll(Dev d);
 __global__ void k_fix(Dev d, int stage);
 __global__ void k_fix_clear(Dev d, int stage, int with_area);
-__global__ void k_two_grain(Dev d);
-__global__ void k_label3(Dev d);
-__global__ void k_scan3(Dev d);
+__global__ void k_tri_all(Dev d);
+__global__ void k_t2_label(Dev d);
 __global__ void k_t2_par(Dev d);
 __global__ void k_t2_serial(Dev d);
 __global__ void k_st2(Dev d);
@@ -48,6 +47,7 @@ __global__ void k_st2_fix_clear(Dev d, int nclear);
 __global__ void k_translate_clear(Dev d, int nclear);
 __global__ void k_flip_par(Dev d);
 __global__ void k_flip_serial(Dev d);
+__global__ void k_events(Dev d);
 __global__ void k_nucl_area_l1(Dev d);
 __global__ void k_nucl_area_up(Dev d);
 __global__ void k_begin_rate(Dev d, int rescale_flipped);
@@ -99,6 +99,13 @@ struct sevc_state {
     bool any_aniso = false;                  // a member with GB_eps != 0 (energies change with the topology)
     bool any_debug = false;                  // a member with debug_lvl >= 1 (checks inside the step)
     bool ben_dirty = true;                   // boundary energies not computed since creation / a new scale
+    bool tri_dirty = true;                   // no grain listed for the two-triangle search yet (upload, restore)
+    // how the events run: 1 one launch per stage (a busy state), 0 one
+    // launch in all; -1: not known yet (the next step is a launch per stage,
+    // and its count of edited grains decides)
+    int busy = -1;
+    int* busy_h = nullptr;                   // pinned, written by the device when it changes
+    hipEvent_t lag[2] = {nullptr, nullptr};  // ends of earlier steps of the call (sevc_step)
     bool diag_next = false;
     bool any_stop = false;                   // a member with a stop rule (tmax, nmax, leave_percent)
     std::vector<MState> ms_host, ms_prev;
@@ -108,6 +115,7 @@ struct sevc_state {
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec1 = nullptr;
     hipGraph_t graph1 = nullptr;
+    int gbusy = -1;                      // how the captured steps run the events
     // kernel timing
     bool timing = false;
     bool timing_hot_only = false;
@@ -413,13 +421,17 @@ void launch_step(sevc_state* s, bool diag) {
     if (diag) launch(s, "grain_dadt", k_grain_dadt, d.ngb, kBlock, d);
     launch(s, "text", k_text, d.neb, kBlock, d);
     if (s->any_events) {
-        launch(s, "label", k_label, d.neb, kBlock, d);
+        if (s->tri_dirty) launch(s, "tri_all", k_tri_all, d.ngb, kBlock, d);
+        s->tri_dirty = false;
+    }
+    const bool one = s->any_events && !s->any_debug && s->busy == 0;
+    if (one) {
+        launch(s, "events", k_events, 1, 1024, d);
+    } else if (s->any_events) {
         launch(s, "poll_gather", k_poll_gather, kPollBig / 64, 64, d);
         launch(s, "poll", k_poll, 1, 1024, d);
-        launch(s, "scan3", k_scan3, d.ngb, kBlock, d);
-        launch(s, "two_grain", k_two_grain, 1, 64, d);
         if (s->any_debug) launch_check(s, CHK_TWO_GRAIN);
-        launch(s, "label3", k_label3, d.ngb, kBlock, d);     // only after a two-triangle event
+        launch(s, "t2_label", k_t2_label, kPollBig / 64, 64, d);
         launch(s, "t2_par", k_t2_par, kListGrid, 256, d);
         launch(s, "t2_serial", k_t2_serial, 1, 64, d);
         launch(s, "fix", k_fix, kFixGrid, 64, d, 1);
@@ -439,7 +451,7 @@ void launch_step(sevc_state* s, bool diag) {
             launch_check(s, CHK_FLIP);
         }
     }
-    if (s->any_events && !s->any_debug)
+    if (s->any_events && !s->any_debug && !one)
         launch(s, "translate", k_translate_clear, kClearGrid + d.nvb, kBlock, d, kClearGrid);
     else
         launch(s, "translate", k_translate, d.nvb, kBlock, d);
@@ -573,13 +585,14 @@ int sevc_batch_create(const sevc_options* opts, const sevc_mesh* meshes, int32_t
     DA(d.chk_bad, static_cast<size_t>(B));
     DA(d.gvx, G * S); DA(d.glen, G); DA(d.garea, G); DA(d.gdadt, G); DA(d.gori, G); DA(d.gse, G);
     DA(d.genab, G); DA(d.gtype, G); DA(d.gcand, G); DA(d.gfix, G);
-    DA(d.cnt, C_COUNT);
+    DA(d.cnt, C_TOTAL);
     DA(d.l_cand, E); DA(d.l_two, E); DA(d.l_t2, G); DA(d.l_t2c, G);
     DA(d.l_flipc, E);
     for (int k = 0; k < kFixStages; ++k) DA(d.l_fix[k], G);
     DA(d.l_dirty, G); DA(d.l_nucl, G); DA(d.l_conf, 4 * E + 16);
     DA(d.nscr, 12 * G + 16);
     DA(d.l_vfall, V + 16);
+    DA(d.l_tri, 6 * G); DA(d.busy, 1);
     DA(d.l_bigr, G + 16);
     DA(d.nrec, 4 * G + 16); DA(d.nal, G + 16); DA(d.l_nev, 8 * G + 16);
 
@@ -626,10 +639,17 @@ int sevc_batch_create(const sevc_options* opts, const sevc_mesh* meshes, int32_t
     DA(d.ms, static_cast<size_t>(B));
     d.prm = dprm;
 #undef DA
-    if (hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking) != hipSuccess) {
+    if (hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking) != hipSuccess ||
+        hipHostMalloc(&s->busy_h, sizeof(int)) != hipSuccess ||
+        hipEventCreateWithFlags(&s->lag[0], hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&s->lag[1], hipEventDisableTiming) != hipSuccess ||
+        hipMemset(d.busy, 0, sizeof(int)) != hipSuccess) {
         sevc_destroy(s);
         return SEVC_E_HIP;
     }
+    *s->busy_h = 0;
+    s->busy = s->any_events && !s->any_debug ? -1 : 0;
+    d.busy_host = s->busy_h;
 #define UP(dst, src, n) \
     do { if (hipMemcpy((dst), (src), (n), hipMemcpyHostToDevice) != hipSuccess) { sevc_destroy(s); return SEVC_E_HIP; } } while (0)
     UP(dvt, vt.data(), vt.size() * sizeof(Blk));
@@ -752,8 +772,8 @@ int sevc_batch_create(const sevc_options* opts, const sevc_mesh* meshes, int32_t
     if (hipMemcpy(d.mods, mods_none.data(), V * sizeof(ModRec), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(d.conf, minus1.data(), E * 4, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemset(d.gfix, 0, G * 4) != hipSuccess || hipMemset(d.gcand, 0, G) != hipSuccess ||
-        hipMemset(d.vnuc, 0, V) != hipSuccess || hipMemset(d.cnt, 0, C_COUNT * 4) != hipSuccess ||
-        hipMemset(d.n_flipped, 0, 4) != hipSuccess ||
+        hipMemset(d.vnuc, 0, V) != hipSuccess || hipMemset(d.cnt, 0, C_TOTAL * 4) != hipSuccess ||
+        hipMemset(d.n_flipped, 0, 4) != hipSuccess || hipMemset(d.blab, 2, E) != hipSuccess ||
         hipMemset(d.nucl_r, 0, V * 8) != hipSuccess || hipMemset(d.nucl_ori, 0, V * 8) != hipSuccess ||
         hipMemset(d.dE, 0, V * 8) != hipSuccess || hipMemset(d.nfac, 0, V * 8) != hipSuccess) {
         sevc_destroy(s);
@@ -780,6 +800,8 @@ void sevc_destroy(sevc_state* s) {
     for (auto& c : s->ckpts) (void)hipFree(c.buf);
     (void)hipFree(s->stage_d);
     (void)hipHostFree(s->stage_h);
+    (void)hipHostFree(s->busy_h);
+    for (hipEvent_t e : s->lag) if (e) (void)hipEventDestroy(e);
     for (void* p : s->allocs) (void)hipFree(p);
     for (auto e : s->pool) (void)hipEventDestroy(e);
     if (s->stream) (void)hipStreamDestroy(s->stream);
@@ -821,8 +843,11 @@ int sevc_kernel_times(sevc_state* s, int32_t max_entries, char (*names)[48], dou
     return k;
 }
 
-static int finish_call(sevc_state* s) {
+// The end of a call; `stepped`: it ran time steps (the labels of disabled
+// slots are left to its end).
+static int finish_call(sevc_state* s, bool stepped) {
     Dev d = s->d;
+    if (stepped && s->any_events) launch(s, "label_disabled", k_label_disabled, d.neb, kBlock, d);
     launch(s, "nucl_area_l1", k_nucl_area_l1, d.ngb, 64, d);
     launch(s, "nucl_area_up", k_nucl_area_up, s->B, 1024, d);
     s->ms_prev = s->ms_host;
@@ -871,16 +896,42 @@ static bool all_done(sevc_state* s) {
     return true;
 }
 
+// The device's word on how the events run, as of the last step it has ended
+// (any answer gives the same results; steps with checks inside, or without
+// events, have no choice).
+static int busy_now(const sevc_state* s) {
+    return s->any_events && !s->any_debug ? *static_cast<volatile int*>(s->busy_h) : 0;
+}
+
+// After the first step of a state: wait for it and take its word.
+static int busy_first(sevc_state* s) {
+    HIPCHK(hipStreamSynchronize(s->stream));
+    s->busy = busy_now(s);
+    return SEVC_OK;
+}
+
+// A call is at most 2 kLag steps ahead of the device, so that it hears of a
+// state that turns busy or calm.
+constexpr int kLag = 32;
+
 int sevc_step(sevc_state* s, int32_t n_steps, sevc_step_stats* st) {
     if (!s || n_steps < 0) return SEVC_E_INVALID_ARG;
     if (n_steps > 0) s->win.ready = false;       // the topology may change
     const int poll = stop_poll(s);
+    int rc;
     for (int k = 0; k < n_steps; ++k) {
         bool diag = s->diag_next;
         s->diag_next = false;
+        if (s->busy >= 0) s->busy = busy_now(s);
         s->timing_skip = s->timing && (s->timing_steps++ % s->timing_every) != 0;
         launch_step(s, diag);
         s->timing_skip = false;
+        if (s->busy < 0 && (rc = busy_first(s)) != SEVC_OK) return rc;
+        if ((k + 1) % kLag == 0) {
+            const int w = ((k + 1) / kLag) & 1;
+            if (k >= 2 * kLag) HIPCHK(hipEventSynchronize(s->lag[w]));
+            HIPCHK(hipEventRecord(s->lag[w], s->stream));
+        }
         if (s->timing && s->pending.size() > 4000) {
             (void)hipStreamSynchronize(s->stream);
             collect_timers(s);
@@ -889,52 +940,65 @@ int sevc_step(sevc_state* s, int32_t n_steps, sevc_step_stats* st) {
     }
     hipError_t le = hipGetLastError();
     if (le != hipSuccess) return fail(s, SEVC_E_HIP, std::string("launch: ") + hipGetErrorString(le));
-    int rc = finish_call(s);
+    rc = finish_call(s, n_steps > 0);
     fill_stats(s, 0, st);
     return rc;
+}
+
+// Captures kGraphSteps steps and one step as graphs, as the state stands
+// (busy or not).  They hold the steady step; one that must recompute the
+// energies or list the 3-sided grains runs outside them.
+static int capture(sevc_state* s) {
+    HIPCHK(hipStreamSynchronize(s->stream));
+    drop_graphs(s);
+    const bool timing = s->timing, dirty = s->ben_dirty, tri = s->tri_dirty;
+    const int busy = s->busy;
+    s->timing = s->ben_dirty = s->tri_dirty = false;
+    s->gbusy = s->busy = std::max(busy, 0);
+    HIPCHK(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
+    for (int k = 0; k < kGraphSteps; ++k) launch_step(s, false);
+    HIPCHK(hipStreamEndCapture(s->stream, &s->graph));
+    HIPCHK(hipGraphInstantiate(&s->gexec, s->graph, nullptr, nullptr, 0));
+    HIPCHK(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
+    launch_step(s, false);
+    HIPCHK(hipStreamEndCapture(s->stream, &s->graph1));
+    HIPCHK(hipGraphInstantiate(&s->gexec1, s->graph1, nullptr, nullptr, 0));
+    s->ben_dirty = dirty;
+    s->tri_dirty = tri;
+    s->timing = timing;
+    s->busy = busy;
+    return SEVC_OK;
 }
 
 int sevc_step_graph(sevc_state* s, int32_t n_steps, sevc_step_stats* st) {
     if (!s || n_steps < 0) return SEVC_E_INVALID_ARG;
     if (n_steps > 0) s->win.ready = false;
-    if (!s->gexec) {
-        bool timing = s->timing;
-        s->timing = false;
-        // the graphs hold the steady step (kGraphSteps of them, and one); a
-        // step that must recompute the energies runs outside them
-        const bool dirty = s->ben_dirty;
-        s->ben_dirty = false;
-        HIPCHK(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
-        for (int k = 0; k < kGraphSteps; ++k) launch_step(s, false);
-        HIPCHK(hipStreamEndCapture(s->stream, &s->graph));
-        HIPCHK(hipGraphInstantiate(&s->gexec, s->graph, nullptr, nullptr, 0));
-        HIPCHK(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
-        launch_step(s, false);
-        HIPCHK(hipStreamEndCapture(s->stream, &s->graph1));
-        HIPCHK(hipGraphInstantiate(&s->gexec1, s->graph1, nullptr, nullptr, 0));
-        s->ben_dirty = dirty;
-        s->timing = timing;
-    }
+    int rc;
     const int poll = stop_poll(s);
-    for (int k = 0, next_poll = poll; k < n_steps;) {
-        if (s->diag_next || s->ben_dirty) {
+    for (int k = 0, next_poll = poll; k < n_steps || !s->gexec;) {
+        if (k < n_steps && (s->diag_next || s->ben_dirty || s->busy < 0 || (s->tri_dirty && s->any_events))) {
             const bool diag = s->diag_next;
             s->diag_next = false;
             launch_step(s, diag);
+            if (s->busy < 0 && (rc = busy_first(s)) != SEVC_OK) return rc;
             k += 1;
+        } else if (!s->gexec || (s->gbusy != s->busy && s->busy >= 0)) {
+            if ((rc = capture(s)) != SEVC_OK) return rc;
         } else if (n_steps - k >= kGraphSteps) {
             HIPCHK(hipGraphLaunch(s->gexec, s->stream));
             k += kGraphSteps;
-        } else {
+        } else if (k < n_steps) {
             HIPCHK(hipGraphLaunch(s->gexec1, s->stream));
             k += 1;
         }
         if (k >= next_poll && k < n_steps) {
             next_poll = k + poll;
             if (all_done(s)) break;
+            s->busy = busy_now(s);               // the stream is idle: the device's word is up to date
         }
     }
-    int rc = finish_call(s);
+    rc = finish_call(s, n_steps > 0);
+    if (s->busy >= 0) s->busy = busy_now(s);
     fill_stats(s, 0, st);
     return rc;
 }
@@ -1293,7 +1357,7 @@ std::vector<std::pair<void*, size_t>> state_arrays(const sevc_state* s) {
             {d.conf, 4 * E}, {d.blab, E}, {d.l_flipped, 4 * (E + 16)}, {d.n_flipped, 4},
             {d.gvx, 4 * G * S}, {d.glen, 4 * G}, {d.garea, 8 * G}, {d.gdadt, 8 * G}, {d.gori, 8 * G},
             {d.gse, 8 * G}, {d.genab, G}, {d.gtype, G}, {d.gcand, G}, {d.gfix, 4 * G},
-            {d.cnt, 4 * static_cast<size_t>(C_COUNT)}, {d.bc_v, 8 * static_cast<size_t>(d.nvb)},
+            {d.cnt, 4 * static_cast<size_t>(C_TOTAL)}, {d.bc_v, 8 * static_cast<size_t>(d.nvb)},
             {d.bc_e, 8 * static_cast<size_t>(d.neb)}, {d.bc_g, 8 * static_cast<size_t>(d.ngb)},
             {d.ms, sizeof(MState) * static_cast<size_t>(s->B)}};
 }
@@ -1334,10 +1398,13 @@ int sevc_restore(sevc_state* s, int32_t slot) {
         HIPCHK(hipMemcpyAsync(a.first, c.buf + off, a.second, hipMemcpyDeviceToDevice, s->stream));
         off += (a.second + 255) / 256 * 256;
     }
+    // the grains listed for the two-triangle search are not kept: all are listed anew
+    HIPCHK(hipMemsetAsync(s->d.cnt + C_TRI, 0, sizeof(int), s->stream));
     HIPCHK(hipStreamSynchronize(s->stream));
     s->ms_host = c.ms;
     s->ms_prev = c.ms;
     s->ben_dirty = true;
+    s->tri_dirty = true;
     s->win.ready = false;
     return SEVC_OK;
 }
@@ -1417,7 +1484,9 @@ int sevc_set_member_mesh(sevc_state* s, int32_t m, const sevc_mesh* me) {
     up(d.gtype + go, gtype.data(), static_cast<size_t>(ng));
     ok = ok && hipMemset(d.gfix + go, 0, 4 * static_cast<size_t>(ng)) == hipSuccess &&
          hipMemset(d.gcand + go, 0, static_cast<size_t>(ng)) == hipSuccess &&
-         hipMemset(d.vnuc + vo, 0, static_cast<size_t>(nv)) == hipSuccess;
+         hipMemset(d.vnuc + vo, 0, static_cast<size_t>(nv)) == hipSuccess &&
+         hipMemset(d.blab + eo, 2, static_cast<size_t>(ne)) == hipSuccess &&
+         hipMemset(d.cnt + C_TRI, 0, sizeof(int)) == hipSuccess;
     if (!ok) return fail(s, SEVC_E_HIP, "upload of the member's mesh failed");
     // loop state: counts of the new mesh; the step counter and time go on
     MState M;
@@ -1431,6 +1500,8 @@ int sevc_set_member_mesh(sevc_state* s, int32_t m, const sevc_mesh* me) {
     HIPCHK(hipStreamSynchronize(s->stream));
     HIPCHK(hipGetLastError());
     s->ben_dirty = true;          // energies of the restored topology at the next step
+    if (s->any_events && !s->any_debug) s->busy = -1;
+    s->tri_dirty = true;
     s->win.ready = false;
     drop_graphs(s);
     return SEVC_OK;
@@ -1551,7 +1622,7 @@ int sevc_window_forward(sevc_state* s, int32_t steps, int32_t ckpt_every) {
     launch(s, "win_end", k_win_end, (s->B + 63) / 64, 64, d, static_cast<int>(steps));
     hipError_t le = hipGetLastError();
     if (le != hipSuccess) return fail(s, SEVC_E_HIP, std::string("launch: ") + hipGetErrorString(le));
-    if ((rc = finish_call(s)) != SEVC_OK) return rc;
+    if ((rc = finish_call(s, false)) != SEVC_OK) return rc;
     w.steps = steps;
     w.K = K;
     w.nck = nck;

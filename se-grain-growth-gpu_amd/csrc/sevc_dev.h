@@ -42,36 +42,62 @@ __device__ __forceinline__ int other_end(const Dev& d, int b, int v) {
     return d.bvx[2 * b] == v ? d.bvx[2 * b + 1] : d.bvx[2 * b];
 }
 
-// geometry.h:837-848
-__device__ __forceinline__ int grains_intersect(const Dev& d, int a, int b, int out[2]) {
+// The set operations on vertex-grain triples run on values already loaded and
+// keep their results in scalars: a result array filled at a run-time position
+// would live in scratch memory (or in LDS, where the compiler finds room).
+
+// geometry.h:837-848: the first two matches of (ga[i], gb[j]) in order of i,
+// then j (-1 where there are fewer); the number found, at most 2.
+__device__ __forceinline__ int triples_intersect(const int (&ga)[3], const int (&gb)[3], int& o0, int& o1) {
     int k = 0;
-    out[0] = out[1] = -1;
+    o0 = o1 = -1;
+#pragma unroll
     for (int i = 0; i < 3; i++)
-        for (int j = 0; j < 3; j++)
-            if (d.vg[3 * a + i] == d.vg[3 * b + j]) {
-                out[k++] = d.vg[3 * a + i];
-                if (k == 2) return 2;
-            }
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            const bool hit = ga[i] == gb[j];
+            o1 = hit && k == 1 ? ga[i] : o1;
+            o0 = hit && k == 0 ? ga[i] : o0;
+            k += hit && k < 2 ? 1 : 0;
+        }
     return k;
 }
 
-// geometry.h:886-898 (with grains_union, :863-875)
-__device__ __forceinline__ void grains_symdiff(const Dev& d, int a, int b, int out[2]) {
-    int gic[2], gun[4];
-    out[0] = out[1] = -1;
-    grains_intersect(d, a, b, gic);
-    gun[3] = -1;
-    for (int i = 0; i < 3; i++) gun[i] = d.vg[3 * a + i];
-    for (int i = 0; i < 3; i++) {
-        int g = d.vg[3 * b + i];
-        if (g != gun[0] && g != gun[1] && g != gun[2]) { gun[3] = g; break; }
+// geometry.h:886-898 (with grains_union, :863-875): the first two of the
+// union (ga, then the first of gb not among them, -1 if none) that are not
+// among the intersection (i0, i1).
+__device__ __forceinline__ void triples_symdiff(const int (&ga)[3], const int (&gb)[3], int i0, int i1, int& o0, int& o1) {
+    int fourth = -1;
+    bool have = false;
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        const int g = gb[j];
+        const bool other = !have && g != ga[0] && g != ga[1] && g != ga[2];
+        fourth = other ? g : fourth;
+        have = have || other;
     }
+    const int gun[4] = {ga[0], ga[1], ga[2], fourth};
     int k = 0;
-    for (int i = 0; i < 4; i++)
-        if (gun[i] != gic[0] && gun[i] != gic[1]) {
-            out[k++] = gun[i];
-            if (k == 2) return;
-        }
+    o0 = o1 = -1;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const bool out = gun[i] != i0 && gun[i] != i1;
+        o1 = out && k == 1 ? gun[i] : o1;
+        o0 = out && k == 0 ? gun[i] : o0;
+        k += out ? 1 : 0;
+    }
+}
+
+__device__ __forceinline__ void load_triple(const int* a, int v, int (&t)[3]) {
+#pragma unroll
+    for (int q = 0; q < 3; q++) t[q] = a[3 * v + q];
+}
+
+__device__ __forceinline__ int grains_intersect(const Dev& d, int a, int b, int& o0, int& o1) {
+    int ga[3], gb[3];
+    load_triple(d.vg, a, ga);
+    load_triple(d.vg, b, gb);
+    return triples_intersect(ga, gb, o0, o1);
 }
 
 __device__ __forceinline__ int* glist(const Dev& d, int g) { return d.gvx + (size_t)g * d.S; }
@@ -99,13 +125,22 @@ __device__ __forceinline__ int grain_contains_vertex(const Dev& d, int g, int v)
     return -1;
 }
 
-// geometry.h:724-734, reading the list eight entries (and the next one) at a
-// time: the first i (in order) with (L[i], L[(i+1) % n]) = (a, b) gives 1,
-// = (b, a) gives 2; -1 if none.
-__device__ __forceinline__ int grain_contains_consecutive(const Dev& d, int g, int a, int b) {
+// What a flip asks of a grain's list about its edge's ends a and b, from one
+// reading of the list (eight entries and the next one at a time, the searches
+// of all four grains around a flip in step): `ab` and `ba`, whether (a, b) /
+// (b, a) come one after the other round the list (grain_contains_consecutive,
+// geometry.h:724-734: 1 for the pair as asked, 2 for the other way round,
+// whichever comes first, -1 for neither), and the first place of a and of b
+// (-1: not in the list).
+struct GrainFind {
+    int ab, ba, a, b;
+};
+
+__device__ __forceinline__ GrainFind grain_find(const Dev& d, int g, int a, int b) {
     const int* L = glist(d, g);
     const int n = d.glen[g];
     const int l0 = n > 0 ? L[0] : -2;
+    GrainFind f = {-1, -1, -1, -1};
     for (int i0 = 0; i0 < n; i0 += 8) {
         int x[9];
 #pragma unroll
@@ -115,12 +150,16 @@ __device__ __forceinline__ int grain_contains_consecutive(const Dev& d, int g, i
         }
 #pragma unroll
         for (int q = 0; q < 8; q++) {
-            if (i0 + q >= n) break;
-            if (x[q] == a && x[q + 1] == b) return 1;
-            if (x[q] == b && x[q + 1] == a) return 2;
+            const bool in = i0 + q < n;
+            f.a = in && f.a < 0 && x[q] == a ? i0 + q : f.a;
+            f.b = in && f.b < 0 && x[q] == b ? i0 + q : f.b;
+            const int p = !in ? -1 : (x[q] == a && x[q + 1] == b) ? 1 : (x[q] == b && x[q + 1] == a) ? 2 : -1;
+            f.ab = f.ab < 0 ? p : f.ab;
         }
     }
-    return -1;
+    // asked the other way round, the same first pair answers
+    f.ba = f.ab < 0 ? -1 : 3 - f.ab;
+    return f;
 }
 
 // geometry.h:548-550, pow(c,3) as c*c*c
@@ -131,9 +170,9 @@ __device__ __forceinline__ double gb_energy_func(double d_alpha, double eps) {
 
 // geometry.h:559-564
 __device__ __forceinline__ double boundary_compute_energy(const Dev& d, int b, double eps) {
-    int gic[2];
-    if (grains_intersect(d, d.bvx[2 * b], d.bvx[2 * b + 1], gic) < 2) return 1.0;
-    return gb_energy_func(d.gori[gic[0]] - d.gori[gic[1]], eps);
+    int g0, g1;
+    if (grains_intersect(d, d.bvx[2 * b], d.bvx[2 * b + 1], g0, g1) < 2) return 1.0;
+    return gb_energy_func(d.gori[g0] - d.gori[g1], eps);
 }
 
 // geometry.h:513-517 plus the flip-threshold extension
@@ -144,9 +183,10 @@ __device__ __forceinline__ bool is_candidate(double te, double len, double dt, d
     return false;
 }
 
-__device__ __forceinline__ double member_dt(const Params& P, const MState& M) {
+// The step's dt for a minimum extinction time of the given bits (nondecreasing
+// in them).
+__device__ __forceinline__ double dt_from_tau(const Params& P, unsigned long long bits) {
     if (!P.adaptive) return P.dt_max;
-    unsigned long long bits = M.tau_bits;
     if (bits == 0x7FF0000000000000ull) return P.dt_max;
     double tau = __longlong_as_double((long long)bits);
     double dt = P.dt_safety * tau;
@@ -154,6 +194,8 @@ __device__ __forceinline__ double member_dt(const Params& P, const MState& M) {
     if (dt > P.dt_max) dt = P.dt_max;
     return dt;
 }
+
+__device__ __forceinline__ double member_dt(const Params& P, const MState& M) { return dt_from_tau(P, M.tau_bits); }
 
 // compute_area of grain g (geometry.h:757-765 after :908-931) with the
 // vertex positions X (2 doubles per vertex slot).
@@ -252,31 +294,86 @@ __device__ __forceinline__ int grain_block(const Dev& d, int g) {
 
 // Set an enable flag, counting a change of state.  No other thread writes
 // the same flag in the same launch (events that touch a slot are serial or
-// disjoint), so the read needs no atomic.
-__device__ __forceinline__ void set_vertex_enabled(const Dev& d, int v, bool on) {
-    if ((d.ven[v] != 0) != on) {
+// disjoint), so the read needs no atomic.  The forms with `was` take the
+// flag's value from the caller, who has loaded it with other data.
+__device__ __forceinline__ void set_vertex_enabled(const Dev& d, int v, bool was, bool on) {
+    if (was != on) {
         d.ven[v] = on ? 1 : 0;
         slot_count_add(d.bc_v, vertex_block(d, v), on);
     }
 }
-__device__ __forceinline__ void set_edge_enabled(const Dev& d, int e, bool on) {
-    if ((d.benab[e] != 0) != on) {
+__device__ __forceinline__ void set_edge_enabled(const Dev& d, int e, bool was, bool on) {
+    if (was != on) {
         d.benab[e] = on ? 1 : 0;
         slot_count_add(d.bc_e, edge_block(d, e), on);
     }
 }
-__device__ __forceinline__ void set_grain_enabled(const Dev& d, int g, bool on) {
-    if ((d.genab[g] != 0) != on) {
+__device__ __forceinline__ void set_grain_enabled(const Dev& d, int g, bool was, bool on) {
+    if (was != on) {
         d.genab[g] = on ? 1 : 0;
         slot_count_add(d.bc_g, grain_block(d, g), on);
     }
 }
+__device__ __forceinline__ void set_vertex_enabled(const Dev& d, int v, bool on) {
+    set_vertex_enabled(d, v, d.ven[v] != 0, on);
+}
+__device__ __forceinline__ void set_edge_enabled(const Dev& d, int e, bool on) {
+    set_edge_enabled(d, e, d.benab[e] != 0, on);
+}
+__device__ __forceinline__ void set_grain_enabled(const Dev& d, int g, bool on) {
+    set_grain_enabled(d, g, d.genab[g] != 0, on);
+}
 
-// Flag grain g for the fix stage `stage` (grain.fix = true) and list it once.
-__device__ __forceinline__ void flag_grain(const Dev& d, int g, int stage) {
-    const bool first = atomicExch(&d.gfix[g], 1) == 0;
-    const int i = wave_slot(&d.cnt[C_FIX0 + stage], first);
-    if (first) d.l_fix[stage][i] = g;
+// Flags the grains g[q] (where want[q]) for the fix stage `stage`
+// (grain.fix = true) and lists each once.  The exchanges of all N are issued
+// together, and one atomic per wave takes the list room of all its lanes, so
+// the chain is two atomics long whatever N (one grain at a time took two for
+// each: a flip's four took 8 us).
+template <int N>
+__device__ __forceinline__ void flag_grains(const Dev& d, const int (&g)[N], const bool (&want)[N], int stage) {
+    int old[N];
+#pragma unroll
+    for (int q = 0; q < N; q++) old[q] = want[q] ? atomicExch(&d.gfix[g[q]], 1) : 1;
+    unsigned long long m[N];
+    int total = 0;
+#pragma unroll
+    for (int q = 0; q < N; q++) {
+        m[q] = __ballot(old[q] == 0);
+        total += (int)__popcll(m[q]);
+    }
+    if (total == 0) return;
+    const int lane = (int)(threadIdx.x & 63);
+    const int leader = __ffsll((long long)__ballot(1)) - 1;
+    int base = 0;
+    if (lane == leader) base = atomicAdd(&d.cnt[C_FIX0 + stage], total);
+    base = __builtin_amdgcn_readlane(base, leader);
+#pragma unroll
+    for (int q = 0; q < N; q++) {
+        if (old[q] == 0) d.l_fix[stage][base + (int)__popcll(m[q] & ((1ull << lane) - 1ull))] = g[q];
+        base += (int)__popcll(m[q]);
+    }
+}
+
+// A list counter read in the launch that fills it (an atomic load: the
+// counters are only ever changed by atomics, which pass the vector cache).
+__device__ __forceinline__ int cnt_now(const Dev& d, int c) {
+    return __hip_atomic_load(&d.cnt[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Orders a wave's LDS accesses (its lanes run in step, so only the compiler
+// has to keep them in order).
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
+// An edit left grain g with three vertices: the next search for adjacent
+// 3-sided pairs looks at it (tri_items).  Each of a step's three edit stages
+// and its nucleations list a grain at most once, so 6 G entries hold them.
+__device__ __forceinline__ void list_tri(const Dev& d, int g, bool want) {
+    const int s = wave_slot(&d.cnt[C_TRI], want);
+    if (want && (unsigned)s < 6u * (unsigned)d.G) d.l_tri[s] = g;
 }
 
 // Inclusive prefix sum of v over the 64 lanes of a wave (every lane active),

@@ -24,6 +24,11 @@
 
 namespace sevc {
 
+// Every function here is inlined: one that is called with the state's Dev by
+// reference makes each lane of the kernel copy that structure to scratch
+// memory and read every field from there (the one-workgroup event stage: 153
+// us a step in place of 60).
+
 // ---------------------------------------------------------------------
 // step begin / end
 // ---------------------------------------------------------------------
@@ -135,8 +140,20 @@ __global__ void __launch_bounds__(64 * kCountWaves) k_count_all(Dev d) {
 __global__ void __launch_bounds__(1024) k_member_reduce(Dev d) {
     __shared__ int sa[16], sb[16];
     const int m = blockIdx.x;
-    // the step's work lists are done with: clear their counters for the next step
-    if (m == 0 && (int)threadIdx.x < C_COUNT) d.cnt[threadIdx.x] = 0;
+    // the step's work lists are done with: clear their counters for the next
+    // step; the numbers of edited grains say whether the state is busy
+    if (m == 0 && threadIdx.x < 64) {
+        const int c = (int)threadIdx.x < C_COUNT ? d.cnt[threadIdx.x] : 0;
+        const int edited = __builtin_amdgcn_readlane(c, C_FIX1) + __builtin_amdgcn_readlane(c, C_FIX2);
+        if ((int)threadIdx.x < C_COUNT) d.cnt[threadIdx.x] = 0;
+        if (threadIdx.x == 0) {
+            const int was = *d.busy, now = edited > kBusyOver ? 1 : (edited < kBusyUnder ? 0 : was);
+            if (now != was) {
+                *d.busy = now;
+                __hip_atomic_store(d.busy_host, now, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            }
+        }
+    }
     if (m >= d.B) return;
     MState& M = d.ms[m];
     const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wave = tid >> 6, nw = nt >> 6;
@@ -836,7 +853,7 @@ __global__ void __launch_bounds__(256) k_vel_vertex(Dev d, int tuning) {
 
 // The reference's two energy_diff passes for one vertex (also stores the
 // velocity parts exported by export_data, calculus.h:62-69).
-__device__ void velocity_generic(const Dev& d, const Params& P, int v, bool parts) {
+__device__ __forceinline__ void velocity_generic(const Dev& d, const Params& P, int v, bool parts) {
     double bx, gx, by, gy;
     double ex = energy_diff(d, P, 0, v, &bx, &gx);
     double ey = energy_diff(d, P, 1, v, &by, &gy);
@@ -1276,14 +1293,26 @@ __global__ void k_translate_clear(Dev d, int nclear) {
 // topological.h: extinction times, labels, votes
 // ---------------------------------------------------------------------
 
-// compute_t_ext, topological.h:303-334, fused with the adaptive-dt minimum:
-// the smallest positive t_ext of the member's enabled edges not shorter than
-// the flip threshold, reduced per block and then into the member's value by
-// one atomic minimum per block (skipped when the block's is not smaller).
-// The minimum does not depend on the order, so the result equals a serial
-// scan.
+// compute_t_ext, topological.h:303-334, fused with the adaptive-dt minimum
+// and with label_boundaries (:343-353).
+//
+// The minimum: the smallest positive t_ext of the member's enabled edges not
+// shorter than the flip threshold, reduced per block and then into the
+// member's value by one atomic minimum per block (skipped when the block's is
+// not smaller).  It does not depend on the order, so the result equals a
+// serial scan.
+//
+// The labels need the step's dt, which needs that minimum.  But the block's
+// own minimum already bounds dt from above (dt_from_tau does not decrease
+// with tau), so the edges that can be candidates are listed here, with this
+// bound, and the listed edges' labels are settled where the list is read
+// (k_poll_gather), with the final dt.  With dt_safety <= 1 the bound lists no
+// edge in vain.  A pass over all edges for the labels alone took 13.6 us at
+// 1M grains, 24 with the Monte Carlo workload's list atomics.  Disabled slots
+// (quirk A-6) are labelled at the end of the call (k_label_disabled).
 __global__ void k_text(Dev d) {
     __shared__ unsigned long long wmin[kBlock / 64];
+    __shared__ int wcnt[kBlock / 64], bbase;
     const int lb_ = xcd_remap((int)blockIdx.x, (int)gridDim.x);
     if (lb_ >= d.neb) return;
     const Blk bd_ = table_blk(d, d.eblk, lb_);
@@ -1302,14 +1331,16 @@ __global__ void k_text(Dev d) {
         va = reinterpret_cast<const double2*>(d.vel)[ab.x];
         vb = reinterpret_cast<const double2*>(d.vel)[ab.y];
     }
-    if (M.active && en) {
+    if (!M.active) return;                          // the same for the whole workgroup
+    double te = 0.0, norm = 0.0;
+    if (en) {
         const double D = P.D;
         d.bcand[i] = 0;
         // adjust_origin_for_points on (ini, end): U0 = 0, U1 = 0 + wrap(end - ini)
         double x1 = 0 + wrapd(pb.x, pa.x, D);
         double y1 = 0 + wrapd(pb.y, pa.y, D);
         double dx = x1 - 0, dy = y1 - 0;
-        double norm = mag(dx, dy);
+        norm = mag(dx, dy);
         // compute_boundary_arclengths (calculus.h:83-93): the same |wrap(end - ini)|
         d.blen[i] = norm;
         double tx, ty;
@@ -1321,45 +1352,28 @@ __global__ void k_text(Dev d) {
         double px = vb.x - va.x;
         double py = vb.y - va.y;
         double aux = tx * px + ty * py;
-        double te = (aux == 0) ? 100.0 : -norm / aux;
+        te = (aux == 0) ? 100.0 : -norm / aux;
         d.bt[i] = te;
         if (P.adaptive && te > 0 && !(norm < P.flip_thr)) v = (unsigned long long)__double_as_longlong(te);
     }
-    v = wave_min_u64(v);
-    if ((threadIdx.x & 63) == 0) wmin[threadIdx.x >> 6] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned long long r = wmin[0];
-        for (int w = 1; w < (int)(blockDim.x >> 6); w++) r = wmin[w] < r ? wmin[w] : r;
-        // the member's minimum (k_begin set it to +inf): the smallest value
-        // whatever the order, so the result equals a serial scan; a block
-        // whose minimum is not below the value already there skips the atomic
-        if (r < M.tau_bits) atomicMin(&M.tau_bits, r);
-    }
-}
-
-// label_boundaries, topological.h:343-353 (every slot, quirk A-6), and the
-// compaction of enabled candidates.
-__global__ void k_label(Dev d) {
-    __shared__ int wcnt[kBlock / 64], bbase;
-    TABLE_BLOCK(d.eblk, d.neb)
-    // the edge's data is loaded together with the member's state
-    const bool in = i < bd_.e;
-    const double te = in ? d.bt[i] : 0.0, len = in ? d.blen[i] : 0.0;
-    const uint8_t en = in ? d.benab[i] : 0;
-    if (!M.active || !P.events) return;             // the same for the whole workgroup
-    const double dt = member_dt(P, M);
-    const bool c = in && is_candidate(te, len, dt, P.flip_thr);
-    if (in) {
-        d.bcand[i] = c ? 1 : 0;
-        d.blab[i] = (uint8_t)((c && en ? 1 : 0) | (en ? 2 : 0));  // for k_scan3: one byte per edge (bit 2: k_poll)
-    }
-    // the workgroup's candidates take consecutive list positions with one
-    // atomic (a step with many candidates would otherwise queue one per wave
-    // on the counter)
-    const bool cand = c && en;
-    const unsigned long long bal = __ballot(cand);
     const int lane = (int)(threadIdx.x & 63), wave = (int)(threadIdx.x >> 6);
+    v = wave_min_u64(v);
+    if (lane == 0) wmin[wave] = v;
+    __syncthreads();
+    unsigned long long r = wmin[0];
+#pragma unroll
+    for (int w = 1; w < kBlock / 64; w++) r = wmin[w] < r ? wmin[w] : r;
+    // the member's minimum (k_begin set it to +inf): the smallest value
+    // whatever the order, so the result equals a serial scan; a block
+    // whose minimum is not below the value already there skips the atomic
+    const unsigned long long seen = M.tau_bits;
+    if (threadIdx.x == 0 && r < seen) atomicMin(&M.tau_bits, r);
+    if (!P.events) return;
+    // label_boundaries with the bound of dt; the workgroup's edges take
+    // consecutive list positions with one atomic
+    const bool cand = en && is_candidate(te, norm, dt_from_tau(P, r < seen ? r : seen), P.flip_thr);
+    if (in) d.blab[i] = (uint8_t)(en ? 2 : 0);
+    const unsigned long long bal = __ballot(cand);
     if (lane == 0) wcnt[wave] = (int)__popcll(bal);
     __syncthreads();
     int before = 0, total = 0;
@@ -1369,7 +1383,8 @@ __global__ void k_label(Dev d) {
         before += w < wave ? x : 0;
         total += x;
     }
-    if (threadIdx.x == 0 && total > 0) bbase = atomicAdd(&d.cnt[C_CAND], total);
+    if (total == 0) return;
+    if (threadIdx.x == 0) bbase = atomicAdd(&d.cnt[C_CAND], total);
     __syncthreads();
     if (cand) {
         const int k = bbase + before + (int)__popcll(bal & ((1ull << lane) - 1ull));
@@ -1378,29 +1393,43 @@ __global__ void k_label(Dev d) {
     }
 }
 
+// label_boundaries (topological.h:343-353) of the slots that were disabled
+// when their member was last labelled: the reference labels every slot (quirk
+// A-6) on every step, from values that a disabled slot keeps, so only the last
+// step's label is left.  Run at the end of a call.
+__global__ void k_label_disabled(Dev d) {
+    TABLE_BLOCK(d.eblk, d.neb)
+    if (i >= bd_.e || !P.events) return;
+    if (d.blab[i] & 2) return;
+    d.bcand[i] = is_candidate(d.bt[i], d.blen[i], M.lab_dt, P.flip_thr) ? 1 : 0;
+}
+
 // The boundaries polling and the conflict check look at, for each listed
-// candidate c at position k (nc <= kPollFast), mapped to list positions
-// through conf (k_label wrote conf[c] = k; -1 elsewhere), as columns of
+// candidate c at position k, mapped to list positions through conf (k_text
+// wrote conf[c] = k; -1 elsewhere), as columns of
 // d.pgat (column f at f * kPollFast):
 //   0..5    the boundaries of c's ends a0 (slots 0-2) and a1 (3-5), vb order;
 //   6..23   for slot j = 0..5 and r = 0..2 (column 6 + 3j + r): boundary r
 //           of the far end of the slot's edge x, -1 when x is c, x is
 //           disabled, or that boundary is x itself;
 //   24      bits 0-1: slot 0 of end a0 / a1 is c itself; bits 2-7: slot j
-//           holds an enabled edge other than c.
+//           holds an enabled edge other than c; bit 8: c is a candidate at
+//           the step's dt (k_text listed it with a bound of dt).
 // d.pgt[k] = t_ext of c.  Many workgroups issue these gathers, so that the
 // one-workgroup polling kernel reads contiguous columns only.
-__global__ void k_poll_gather(Dev d) {
-    const int nc = d.cnt[C_CAND];
+__device__ __forceinline__ void gather_items(const Dev& d, int nc, int k0, int stride) {
     if (nc > d.poll_fast && nc > d.poll_lds) return;
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nc; k += gridDim.x * blockDim.x) {
+    for (int k = k0; k < nc; k += stride) {
         const int c = d.l_cand[k];
         const int a[2] = {d.bvx[2 * c], d.bvx[2 * c + 1]};
-        d.pgt[k] = d.bt[c];
+        const double te = d.bt[c], len = d.blen[c];
+        const int m = member_of_edge(d, c);
+        d.pgt[k] = te;
         int eb[6];
 #pragma unroll
         for (int j = 0; j < 6; j++) eb[j] = d.vb[3 * a[j / 3] + j % 3];
         int bits = (eb[0] == c ? 1 : 0) | (eb[3] == c ? 2 : 0);
+        if (is_candidate(te, len, member_dt(d.prm[m], d.ms[m]), d.prm[m].flip_thr)) bits |= 256;
         int en[6], x0[6], x1[6];
 #pragma unroll
         for (int j = 0; j < 6; j++) {
@@ -1426,23 +1455,23 @@ __global__ void k_poll_gather(Dev d) {
     }
 }
 
+constexpr int kPollLds = 9 * kPollBig;      // LDS bytes of poll_list
+
 // polling_system (topological.h:549-578) as Jacobi rounds to a fixpoint,
 // then check_conflictive_boundaries (:83-121) and
 // unlabel_conflictive_boundaries (:129-155), over the compacted candidate
 // list.  Only vertices that touch a candidate can vote for one, so the
-// rounds are exact on the list.  One workgroup, in one of three ways by the
+// rounds are exact on the list.  A listed edge that is no candidate at the
+// step's dt takes part without a flag.  One workgroup, in one of three ways by the
 // list's length: up to 2,048 candidates with their mapped neighbours in
 // registers; up to 16,384 with flags and t_ext in LDS and the mapped
 // neighbours re-read from k_poll_gather's columns; longer lists by the
 // general rounds over global memory.
-__global__ void __launch_bounds__(1024) k_poll(Dev d) {
+// LDS (pbuf) of the first two ways: [cf int, cid int, ct double] x kPollFast,
+// or [ct double, cf byte] x kPollBig.
+__device__ __forceinline__ void poll_list(const Dev& d, int nc, unsigned char* pbuf) {
     __shared__ int changed;
-    // LDS of the first two ways: [cf int, cid int, ct double] x kPollFast,
-    // or [ct double, cf byte] x kPollBig
-    __shared__ __align__(16) unsigned char pbuf[9 * kPollBig];
-    static_assert(16 * kPollFast <= 9 * kPollBig, "the register way's arrays fit the buffer");
-    const int nc = d.cnt[C_CAND];
-    if (nc == 0) return;
+    static_assert(16 * kPollFast <= kPollLds, "the register way's arrays fit the buffer");
     const int tid = threadIdx.x, nt = blockDim.x;
     auto vote = [&](int v) {
         double min_t = 99999999;
@@ -1474,11 +1503,11 @@ __global__ void __launch_bounds__(1024) k_poll(Dev d) {
             if (on) {
                 cid[k] = d.l_cand[k];
                 ct[k] = d.pgt[k];
-                cf[k] = 1;
             }
 #pragma unroll
             for (int j = 0; j < 6; j++) ep[u][j] = on ? d.pgat[j * kPollBig + k] : -1;
             bits[u] = on ? d.pgat[24 * kPollBig + k] : 0;
+            if (on) cf[k] = (bits[u] >> 8) & 1;
         }
         __syncthreads();
         // vertices_vote (topological.h:362-386) at end e of the candidate at
@@ -1561,7 +1590,7 @@ __global__ void __launch_bounds__(1024) k_poll(Dev d) {
             if (k < nc) {
                 const int c = cid[k];
                 d.bcand[c] = keep[u] ? 1 : 0;
-                d.blab[c] = (uint8_t)(keep[u] ? 7 : 3);     // + the label after polling (bit 2)
+                d.blab[c] = (uint8_t)(2 | ((bits[u] >> 8) & 1) | (keep[u] ? 4 : 0));
                 d.conf[c] = -1;
             }
         }
@@ -1577,21 +1606,9 @@ __global__ void __launch_bounds__(1024) k_poll(Dev d) {
         const int* G = d.pgat;
         for (int k = tid; k < nc; k += nt) {
             ct[k] = d.pgt[k];
-            cf[k] = 1;
+            cf[k] = (uint8_t)((G[24 * kPollBig + k] >> 8) & 1);
         }
         __syncthreads();
-        // vertices_vote at end e of the candidate at position k (as in the
-        // register way above)
-        auto votes_self = [&](int e, int k, int bk) {
-            double min_t = 99999999;
-            int arg = -1;
-#pragma unroll
-            for (int r = 0; r < 3; r++) {
-                const int p = G[(3 * e + r) * kPollBig + k];
-                if (p >= 0 && cf[p] && ct[p] <= min_t) { min_t = ct[p]; arg = p; }
-            }
-            return arg >= 0 ? arg == k : ((bk >> e) & 1) != 0;
-        };
         for (;;) {
             if (tid == 0) changed = 0;
             unsigned two = 0;
@@ -1680,11 +1697,21 @@ __global__ void __launch_bounds__(1024) k_poll(Dev d) {
             const int c = d.l_cand[k];
             const bool kp = (keep >> u) & 1u;
             d.bcand[c] = kp ? 1 : 0;
-            d.blab[c] = (uint8_t)(kp ? 7 : 3);
+            d.blab[c] = (uint8_t)(2 | ((G[24 * kPollBig + k] >> 8) & 1) | (kp ? 4 : 0));
             d.conf[c] = -1;
         }
         return;
-    } else for (;;) {
+    }
+    // the list is longer than the gathered columns: its labels at the step's
+    // dt, then the general rounds
+    for (int k = tid; k < nc; k += nt) {
+        const int c = d.l_cand[k], m = member_of_edge(d, c);
+        const bool on = is_candidate(d.bt[c], d.blen[c], member_dt(d.prm[m], d.ms[m]), d.prm[m].flip_thr);
+        d.bcand[c] = on ? 1 : 0;
+        d.blab[c] = (uint8_t)(on ? 3 : 2);
+    }
+    __syncthreads();
+    for (;;) {
         if (tid == 0) changed = 0;
         // phase A: votes on the flags at the start of the round
         for (int k = tid; k < nc; k += nt) {
@@ -1763,12 +1790,12 @@ __global__ void __launch_bounds__(1024) k_poll(Dev d) {
         if (drop) d.bcand[c] = 0;
     }
     __syncthreads();
-    const int ncf = d.cnt[C_CONF];
+    const int ncf = cnt_now(d, C_CONF);
     for (int k = tid; k < ncf; k += nt) d.conf[d.l_conf[k]] = -1;
     // the label after polling of every listed candidate, bit 2 of its byte
     for (int k = tid; k < nc; k += nt) {
         const int c = d.l_cand[k];
-        d.blab[c] = (uint8_t)(d.bcand[c] ? 7 : 3);
+        d.blab[c] = (uint8_t)((d.blab[c] & 3) | (d.bcand[c] ? 4 : 0));
     }
 }
 
@@ -1809,7 +1836,7 @@ __device__ __forceinline__ void list_replace(const Dev& d, int g, int old_v, int
 }
 
 // perform_ADD_ops, perform_REMOVE_ops, perform_REPLACE_ops for one grain.
-__device__ void fix_one_grain(const Dev& d, int g) {
+__device__ __forceinline__ void fix_one_grain(const Dev& d, int g) {
     if (!d.genab[g]) return;
     int* L = glist(d, g);
     for (int i = 0; i < d.glen[g]; i++) {                       // :1040-1067
@@ -1824,19 +1851,24 @@ __device__ void fix_one_grain(const Dev& d, int g) {
         // entries leaves the same list in any order, so mark the doomed
         // positions first and compact once.
         const int n = d.glen[g];
-        uint64_t doomed[kMaxStride / 64] = {0, 0};
+        static_assert(kMaxStride <= 128, "two words mark a list's entries");
+        uint64_t doomed0 = 0, doomed1 = 0;
         for (int i = 0; i < n; i++) {
             int v = L[i];
             for (int j = 0; j < 4; j++) {
                 if (d.mods[v].fix[j] != FIX_REMOVE || d.mods[v].grn[j] != g) continue;
                 int w = d.mods[v].vrt[j];
                 for (int q = 0; q < n; q++)
-                    if (L[q] == w) { doomed[q >> 6] |= 1ull << (q & 63); break; }
+                    if (L[q] == w) {
+                        doomed0 |= q < 64 ? 1ull << q : 0;
+                        doomed1 |= q >= 64 ? 1ull << (q - 64) : 0;
+                        break;
+                    }
             }
         }
         int w = 0;
         for (int i = 0; i < n; i++)
-            if (!((doomed[i >> 6] >> (i & 63)) & 1ull)) L[w++] = L[i];
+            if (!(((i < 64 ? doomed0 : doomed1) >> (i & 63)) & 1ull)) L[w++] = L[i];
         for (int i = w; i < n; i++) L[i] = -1;
         d.glen[g] = w;
     }
@@ -1848,27 +1880,37 @@ __device__ void fix_one_grain(const Dev& d, int g) {
     }
 }
 
-// fix_grain_lists for the flagged grains of a stage, one wave (workgroup of
-// 64) per grain.  The wave stages the grain's list and the four deferred-edit
-// records of every listed vertex in LDS with one round of independent loads;
-// lane 0 then replays perform_ADD_ops, perform_REMOVE_ops and
-// perform_REPLACE_ops (topological.h:1035-1136) on the staged copy in exactly
-// the order fix_one_grain uses on global memory (an entry inserted or
+// fix_grain_lists for the flagged grains of a stage.
+//
+// fix_wave: one grain by one wave.  The wave stages the grain's list and the
+// four deferred-edit records of every listed vertex in LDS with one round of
+// independent loads; lane 0 then replays perform_ADD_ops, perform_REMOVE_ops
+// and perform_REPLACE_ops (topological.h:1035-1136) on the staged copy in
+// exactly the order fix_one_grain uses on global memory (an entry inserted or
 // replaced during the replay reads its vertex's records from global memory,
 // as fix_one_grain does), and the wave writes the list back, including the
 // -1 padding fix_one_grain leaves after the removals.  Records do not change
 // during this kernel, and each grain edits only its own list.
-__global__ void __launch_bounds__(64) k_fix(Dev d, int stage) {
-    __shared__ int Ls[kMaxStride];
-    __shared__ short src[kMaxStride];            // index of the staged records, -1: read globally
-    __shared__ unsigned char mf[4 * kMaxStride];
-    __shared__ int mg[4 * kMaxStride], mv[4 * kMaxStride], mp[4 * kMaxStride];
-    __shared__ unsigned short kinds[kMaxStride];   // per staged entry: 4 bits each for ADD, REMOVE, REPLACE records of this grain
-    __shared__ int n_add_s, n_fin_s;
-    const int n_items = d.cnt[C_FIX0 + stage];
-    const int lane = threadIdx.x;
-    for (int item = blockIdx.x; item < n_items; item += gridDim.x) {
-        const int g = d.l_fix[stage][item];
+constexpr int kQuick = 16;                // lanes, and most entries, of a grain edited by fix_items itself
+struct FixLds {
+    int Ls[kMaxStride];
+    short src[kMaxStride];                // index of the staged records, -1: read globally
+    unsigned char mf[4 * kMaxStride];
+    int mg[4 * kMaxStride], mv[4 * kMaxStride], mp[4 * kMaxStride];
+    unsigned short kinds[kMaxStride];     // per staged entry: 4 bits each for ADD, REMOVE, REPLACE records of this grain
+    int n_add, n_fin;
+    int nl[64];                           // fix_items: each group's list after its insertions
+    unsigned char from[64];               //            and the lane an entry came from (kQuick: inserted)
+};
+
+__device__ __forceinline__ void fix_wave(const Dev& d, int g, FixLds& f_) {
+    const int lane = (int)threadIdx.x & 63;
+    int* const Ls = f_.Ls;
+    short* const src = f_.src;
+    unsigned char* const mf = f_.mf;
+    int *const mg = f_.mg, *const mv = f_.mv, *const mp = f_.mp;
+    unsigned short* const kinds = f_.kinds;
+    {
         // the grain's flag, length and whole list row in one round of loads
         int* L = glist(d, g);
         const uint8_t en = d.genab[g];
@@ -1876,10 +1918,12 @@ __global__ void __launch_bounds__(64) k_fix(Dev d, int stage) {
         int row[kMaxStride / 64];
 #pragma unroll
         for (int q = 0; q < kMaxStride / 64; q++) row[q] = lane + 64 * q < d.S ? L[lane + 64 * q] : -1;
-        if (!en) continue;
+        if (!en) return;
         const int cap = d.prm[member_of_grain(d, g)].cap;
-        for (int i = lane; i < n0; i += 64) {
-            const int v = row[i >> 6];
+#pragma unroll
+        for (int r = 0; r < kMaxStride / 64; r++) {
+            const int i = lane + 64 * r, v = row[r];
+            if (i >= n0) continue;
             Ls[i] = v;
             src[i] = (short)i;
             unsigned kd = 0;
@@ -1897,7 +1941,7 @@ __global__ void __launch_bounds__(64) k_fix(Dev d, int stage) {
             }
             kinds[i] = (unsigned short)kd;
         }
-        __syncthreads();
+        wave_sync();
         if (lane == 0) {
             auto rec = [&](int es, int v, int j, int& f, int& gg, int& vv, int& pp) {
                 if (es >= 0) {
@@ -1929,7 +1973,7 @@ __global__ void __launch_bounds__(64) k_fix(Dev d, int stage) {
                 }
             }
             const int n_add = n;
-            uint64_t doomed[kMaxStride / 64] = {0, 0};               // REMOVE, :1086-1106
+            uint64_t doomed0 = 0, doomed1 = 0;                       // REMOVE, :1086-1106
             for (int i = 0; i < n; i++) {
                 const int es = src[i], v = Ls[i];
                 const unsigned km = es >= 0 ? ((kinds[es] >> 4) & 0xFu) : 0xFu;
@@ -1939,12 +1983,16 @@ __global__ void __launch_bounds__(64) k_fix(Dev d, int stage) {
                     rec(es, v, j, f, gg, vv, pp);
                     if (f != FIX_REMOVE || gg != g) continue;
                     for (int q = 0; q < n; q++)
-                        if (Ls[q] == vv) { doomed[q >> 6] |= 1ull << (q & 63); break; }
+                        if (Ls[q] == vv) {
+                            doomed0 |= q < 64 ? 1ull << q : 0;
+                            doomed1 |= q >= 64 ? 1ull << (q - 64) : 0;
+                            break;
+                        }
                 }
             }
             int w = 0;
             for (int i = 0; i < n; i++)
-                if (!((doomed[i >> 6] >> (i & 63)) & 1ull)) { Ls[w] = Ls[i]; src[w] = src[i]; w++; }
+                if (!(((i < 64 ? doomed0 : doomed1) >> (i & 63)) & 1ull)) { Ls[w] = Ls[i]; src[w] = src[i]; w++; }
             n = w;
             for (int i = 0; i < n; i++) {                            // REPLACE, :1124-1136
                 const int es = src[i], v = Ls[i];
@@ -1958,86 +2006,219 @@ __global__ void __launch_bounds__(64) k_fix(Dev d, int stage) {
                         if (Ls[q] == pp) { Ls[q] = vv; src[q] = -1; break; }
                 }
             }
-            n_add_s = n_add;
-            n_fin_s = n;
+            f_.n_add = n_add;
+            f_.n_fin = n;
         }
-        __syncthreads();
-        const int n_add = n_add_s, n_fin = n_fin_s;
+        wave_sync();
+        const int n_add = f_.n_add, n_fin = f_.n_fin;
         for (int i = lane; i < n_add; i += 64) L[i] = i < n_fin ? Ls[i] : -1;
-        if (lane == 0) d.glen[g] = n_fin;
-        __syncthreads();
+        if (lane == 0) {
+            d.glen[g] = n_fin;
+            if (n_fin == 3) list_tri(d, g, true);
+        }
+        wave_sync();
     }
+}
+
+// The flagged grains of a stage, four to a wave, sixteen lanes each (a list
+// has six entries on average).  A lane holds one entry and its vertex's
+// records; the insertions, removals and replacements that the records of this
+// grain ask for are placed by ballots over the group instead of being replayed
+// one by one, which gives the same list as long as no edit can see another's
+// result.  That is so for what flips and removals record (an insertion after
+// the recording vertex itself, a replacement of it), and is checked: a list of
+// more than 16 entries before or after its insertions, a second insertion or
+// replacement by one vertex, one that names another vertex, an inserted vertex
+// that itself records an edit of this grain, a repeated entry, or a list past
+// its capacity goes to fix_wave.  Wave w of nw takes items 4w .. 4w + 3, 4(w +
+// nw) ..  (One grain to a wave with the serial replay: 11.3 us at 1M grains
+// with 90 edited grains, 25 with the Monte Carlo workload's 12,000.)
+__device__ __forceinline__ void fix_items(const Dev& d, int stage, FixLds& f, int w, int nw) {
+    const int n_items = cnt_now(d, C_FIX0 + stage);
+    const int lane = (int)threadIdx.x & 63, l = lane & (kQuick - 1), g0 = lane & ~(kQuick - 1);
+    const unsigned below = (1u << l) - 1u;
+    // the group's part of a ballot
+    auto group = [&](bool x) { return (unsigned)(__ballot(x) >> g0) & 0xFFFFu; };
+    for (int base = 4 * w; base < n_items; base += 4 * nw) {
+        const int item = base + (lane >> 4);
+        const bool on = item < n_items;
+        const int g = on ? d.l_fix[stage][item] : 0;
+        int* L = glist(d, g);
+        const bool en = on && d.genab[g] != 0;
+        const int n0 = d.glen[g], v = l < d.S ? L[l] : -1;
+        const int mem = member_of_grain(d, g);
+        bool slow = en && n0 > kQuick;
+        const bool has = en && !slow && l < n0;
+        int4 rg = make_int4(-1, -1, -1, -1), rv = rg, rp = rg;
+        unsigned rf = 0x01010101u * (unsigned)FIX_NONE;
+        if (has) {
+            const int4* r = reinterpret_cast<const int4*>(&d.mods[v]);
+            rg = r[0];
+            rv = r[1];
+            rp = r[2];
+            rf = *reinterpret_cast<const unsigned*>(d.mods[v].fix);
+        }
+        const int cap = d.prm[mem].cap;
+        const int gq[4] = {rg.x, rg.y, rg.z, rg.w}, vq[4] = {rv.x, rv.y, rv.z, rv.w}, pq[4] = {rp.x, rp.y, rp.z, rp.w};
+        int adds = 0, reps = 0, vadd = -1, vrep = -1;
+        unsigned rem = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const unsigned k = (rf >> (8 * j)) & 255u;
+            const bool mine = gq[j] == g;
+            if (mine && k == FIX_ADD) { adds++; vadd = vq[j]; slow = slow || pq[j] != v; }
+            if (mine && k == FIX_REPLACE) { reps++; vrep = vq[j]; slow = slow || pq[j] != v; }
+            rem |= mine && k == FIX_REMOVE ? 1u << j : 0u;
+        }
+        slow = slow || adds > 1 || reps > 1;
+        if (adds > 0) {
+            // the inserted vertex's own records
+            const int4 tg = *reinterpret_cast<const int4*>(d.mods[vadd].grn);
+            const unsigned tf = *reinterpret_cast<const unsigned*>(d.mods[vadd].fix);
+            const int tq[4] = {tg.x, tg.y, tg.z, tg.w};
+#pragma unroll
+            for (int j = 0; j < 4; j++) slow = slow || (tq[j] == g && ((tf >> (8 * j)) & 255u) != FIX_NONE);
+        }
+        const unsigned am = group(adds > 0);
+        const int pre = __popc(am & below), n1 = n0 + __popc(am);
+        slow = slow || (en && (n1 > kQuick || n1 > cap));
+        bool slow_g = group(slow) != 0;
+        // insertions: the list after them, and where its entries came from
+        if (has && !slow_g) {
+            f.nl[g0 + l + pre] = v;
+            f.from[g0 + l + pre] = (unsigned char)l;
+            if (adds > 0) {
+                f.nl[g0 + l + pre + 1] = vadd;
+                f.from[g0 + l + pre + 1] = kQuick;
+            }
+        }
+        wave_sync();
+        const bool in1 = en && !slow_g && l < n1;
+        const int x = in1 ? f.nl[g0 + l] : -1, src = in1 ? f.from[g0 + l] : kQuick;
+        // an entry that inserts or is replaced is searched for by its value:
+        // it must be the first with it
+        const int back = g0 + (src & (kQuick - 1));
+        const int add_src = __shfl(adds, back), rep_src = __shfl(reps, back), vrep_src = __shfl(vrep, back);
+        unsigned pm = group(in1 && src < kQuick && (add_src > 0 || rep_src > 0));
+        bool dup = false;
+        while (__ballot(pm != 0)) {
+            const int o = pm ? __ffs((int)pm) - 1 : 0;
+            const int t = __shfl(x, g0 + o);
+            const unsigned m = group(in1 && x == t);
+            dup = dup || (pm && __ffs((int)m) - 1 != o);
+            pm &= pm - 1u;
+        }
+        slow_g = slow_g || dup;
+        // removals: the first entry with each value that a record names
+        bool gone = false;
+        const unsigned rm0 = group(has && rem != 0);
+        unsigned rm = slow_g ? 0u : rm0;
+        while (__ballot(rm != 0)) {
+            const int o = g0 + (rm ? __ffs((int)rm) - 1 : 0);
+            const unsigned rem_o = (unsigned)__shfl((int)rem, o);
+            const unsigned ro = rm ? rem_o : 0u;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int t = __shfl(vq[j], o);
+                const unsigned m = group(in1 && x == t);
+                if (((ro >> j) & 1u) && m && l == __ffs((int)m) - 1) gone = true;
+            }
+            rm &= rm - 1u;
+        }
+        const bool stay = in1 && !gone;
+        const unsigned sm = group(stay);
+        const int at = __popc(sm & below), n2 = __popc(sm);
+        // replacements, by entries that stay, of themselves
+        const bool rep = stay && src < kQuick && rep_src > 0;
+        if (en && !slow_g) {
+            if (stay) L[at] = rep ? vrep_src : x;
+            if (l >= n2 && l < n1) L[l] = -1;
+            if (l == 0) d.glen[g] = n2;
+        }
+        list_tri(d, g, en && !slow_g && l == 0 && n2 == 3);
+        wave_sync();
+        // the groups that need the replay, one after the other
+        for (unsigned long long todo = __ballot(en && slow_g && l == 0); todo; todo &= todo - 1ull) {
+            fix_wave(d, __builtin_amdgcn_readlane(g, __ffsll((long long)todo) - 1), f);
+            wave_sync();
+        }
+    }
+}
+
+__global__ void __launch_bounds__(64) k_fix(Dev d, int stage) {
+    __shared__ FixLds f;
+    fix_items(d, stage, f, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // clear_grains_fix_state (topological.h:1150-1163) for the flagged grains;
 // with with_area also the area update of main.cu:266 for them and for the
-// grains edited by the two-triangle stage (its dirty list).  One wave
-// (workgroup of 64) per grain: the lanes reset the listed vertices' records
-// and load the list's points in parallel, each forming the wrapped delta to
-// its predecessor; lane 0 then accumulates the shoelace sum over the deltas
-// in list order, the same arithmetic as grain_area.
-// Items of k_fix_clear's work for one 64-lane workgroup: workgroup `blk` of
-// `nblk` takes items blk, blk + nblk, ...
-__device__ __forceinline__ void fix_clear_items(const Dev& d, int stage, int with_area, int blk, int nblk) {
-    __shared__ double sdx[kMaxStride], sdy[kMaxStride];
-    const int n = d.cnt[C_FIX0 + stage];
-    const int nd = with_area ? min(d.cnt[C_DIRTY], d.G) : 0;
-    const int lane = threadIdx.x;
-    for (int item = blk; item < n + nd; item += nblk) {
-        int g;
-        if (item < n) {
-            g = d.l_fix[stage][item];
-            if (lane == 0) d.gfix[g] = 0;
-            if (!d.genab[g]) continue;
-            const int* L = glist(d, g);
-            const int m = d.glen[g];
-            for (int i = lane; i < m; i += 64) reset_mods(d, L[i]);
-            if (!with_area) continue;
-        } else {
-            g = d.l_dirty[item - n];
-            if (!d.genab[g]) continue;
-        }
-        const int m = d.glen[g];
+// grains edited by the two-triangle stage (its dirty list).  Four grains to a
+// wave, sixteen lanes each: the lanes reset the listed vertices' records and
+// load the list's points in parallel, each forming the wrapped delta to its
+// predecessor; the group's first lane then accumulates the shoelace sum over
+// the deltas in list order, the same arithmetic as grain_area.  Wave `blk` of
+// `nblk` takes items 4 blk .. 4 blk + 3, 4 (blk + nblk) ..; `c` is its room.
+struct ClearLds {
+    double2 dl[4][kMaxStride];
+};
+
+__device__ __forceinline__ void fix_clear_items(const Dev& d, int stage, int with_area, ClearLds& c, int blk, int nblk) {
+    const int n = cnt_now(d, C_FIX0 + stage);
+    const int nd = with_area ? min(cnt_now(d, C_DIRTY), d.G) : 0;
+    const int lane = (int)threadIdx.x & 63, l = lane & 15;
+    double2* const dl = c.dl[lane >> 4];
+    const double2* X = reinterpret_cast<const double2*>(d.pos);
+    for (int base = 4 * blk; base < n + nd; base += 4 * nblk) {
+        const int item = base + (lane >> 4);
+        const bool on = item < n + nd, flagged = item < n;
+        const int g = !on ? 0 : (flagged ? d.l_fix[stage][item] : d.l_dirty[item - n]);
         const int* L = glist(d, g);
+        const bool en = on && d.genab[g] != 0;
+        const int m = en ? d.glen[g] : 0;
         const double D = d.prm[member_of_grain(d, g)].D;
-        for (int i = 1 + lane; i < m; i += 64) {
-            const int w = L[i], wp = L[i - 1];
-            sdx[i] = wrapd(d.pos[2 * w], d.pos[2 * wp], D);
-            sdy[i] = wrapd(d.pos[2 * w + 1], d.pos[2 * wp + 1], D);
+        if (flagged && l == 0) d.gfix[g] = 0;
+        for (int i = l; i < m; i += 16) {
+            const int w = L[i], wp = i > 0 ? L[i - 1] : w;
+            if (with_area) {
+                const double2 p = X[w], q = X[wp];
+                dl[i] = make_double2(wrapd(p.x, q.x, D), wrapd(p.y, q.y, D));
+            }
+            if (flagged) reset_mods(d, w);
         }
-        __syncthreads();
-        if (lane == 0) {
+        wave_sync();
+        if (with_area && l == 0 && en) {
             double a = 0.0;
             if (m > 0) {
                 AreaAcc acc;
                 acc.start(0.0, 0.0);
-                for (int i = 1; i < m; i++) acc.push_delta(sdx[i], sdy[i]);
+                for (int i = 1; i < m; i++) acc.push_delta(dl[i].x, dl[i].y);
                 a = acc.finish();
             }
             d.garea[g] = a;
         }
-        __syncthreads();
+        wave_sync();
     }
 }
 
 __global__ void __launch_bounds__(64) k_fix_clear(Dev d, int stage, int with_area) {
-    fix_clear_items(d, stage, with_area, (int)blockIdx.x, (int)gridDim.x);
+    __shared__ ClearLds c;
+    fix_clear_items(d, stage, with_area, c, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // ---------------------------------------------------------------------
 // two adjacent 3-sided grains (topological.h:22-73, 840-985)
 // ---------------------------------------------------------------------
 
-__device__ bool two_qualifies(const Dev& d, int e) {
+__device__ __forceinline__ bool two_qualifies(const Dev& d, int e) {
     if (!d.benab[e]) return false;
-    int gic[2];
-    if (grains_intersect(d, d.bvx[2 * e], d.bvx[2 * e + 1], gic) < 2) return false;
-    return d.glen[gic[0]] == 3 && d.glen[gic[1]] == 3;
+    int g0, g1;
+    if (grains_intersect(d, d.bvx[2 * e], d.bvx[2 * e + 1], g0, g1) < 2) return false;
+    return d.glen[g0] == 3 && d.glen[g1] == 3;
 }
 
 // remove_two_grains, topological.h:840-955.  Returns CE (the edge whose
 // endpoint moved) or -1.
-__device__ int remove_two_grains(const Dev& d, int bnd, const int gnic[2]) {
+__device__ __forceinline__ int remove_two_grains(const Dev& d, int bnd, int gn0, int gn1) {
     int A = d.bvx[2 * bnd], B = d.bvx[2 * bnd + 1];
     int AC = -1, BD = -1, CE = -1, DF = -1;
     for (int i = 0; i < 3; i++) if (d.vb[3 * A + i] == bnd) { AC = d.vb[3 * A + (i + 1) % 3]; break; }
@@ -2053,14 +2234,19 @@ __device__ int remove_two_grains(const Dev& d, int bnd, const int gnic[2]) {
     else d.bvx[2 * CE + 1] = F;
     for (int p = 0; p < 3; p++) if (d.vb[3 * F + p] == DF) { d.vb[3 * F + p] = CE; break; }
     int G3, G4;
-    if (grain_contains_vertex(d, gnic[0], A) >= 0) { G3 = gnic[0]; G4 = gnic[1]; }
-    else { G3 = gnic[1]; G4 = gnic[0]; }
-    set_mod(d, A, 0, FIX_REMOVE, G3, A); flag_grain(d, G3, 0);
+    if (grain_contains_vertex(d, gn0, A) >= 0) { G3 = gn0; G4 = gn1; }
+    else { G3 = gn1; G4 = gn0; }
+    set_mod(d, A, 0, FIX_REMOVE, G3, A);
     set_mod(d, A, 1, FIX_REMOVE, G3, C);
     set_mod(d, A, 2, FIX_REMOVE, G3, Dv);
-    set_mod(d, B, 0, FIX_REMOVE, G4, B); flag_grain(d, G4, 0);
+    set_mod(d, B, 0, FIX_REMOVE, G4, B);
     set_mod(d, B, 1, FIX_REMOVE, G4, C);
     set_mod(d, B, 2, FIX_REMOVE, G4, Dv);
+    {
+        const int gg[2] = {G3, G4};
+        const bool all[2] = {true, true};
+        flag_grains(d, gg, all, 0);
+    }
     for (int i = 0; i < 3; i++) {
         set_edge_enabled(d, d.vb[3 * A + i], false);
         set_edge_enabled(d, d.vb[3 * B + i], false);
@@ -2072,7 +2258,7 @@ __device__ int remove_two_grains(const Dev& d, int bnd, const int gnic[2]) {
     return CE;
 }
 
-__device__ void sort_ints(int* a, int n) {
+__device__ __forceinline__ void sort_ints(int* a, int n) {
     for (int i = 1; i < n; i++) {
         int x = a[i], j = i - 1;
         while (j >= 0 && a[j] > x) { a[j + 1] = a[j]; j--; }
@@ -2086,10 +2272,8 @@ __device__ void sort_ints(int* a, int n) {
 // topological.h:965-985 sees them), each followed by the list fix-up of the
 // flagged grains.  The next pass's qualifying edges can only be edges of
 // grains whose list was just edited.
-__global__ void k_two_grain(Dev d) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    int n = d.cnt[C_TWO];
-    if (n == 0) return;
+__device__ __forceinline__ void two_grain_serial(const Dev& d) {
+    int n = cnt_now(d, C_TWO);
     int* lst = d.l_two;
     for (int it = 0; it < 20 && n > 0; it++) {
         sort_ints(lst, n);
@@ -2097,17 +2281,16 @@ __global__ void k_two_grain(Dev d) {
             int e = lst[k];
             if (!two_qualifies(d, e)) continue;
             if (!d.ms[member_of_edge(d, e)].active) continue;
-            int gic[2], gnic[2];
-            grains_intersect(d, d.bvx[2 * e], d.bvx[2 * e + 1], gic);
-            grains_symdiff(d, d.bvx[2 * e], d.bvx[2 * e + 1], gnic);
-            if (gnic[0] < 0 || gnic[1] < 0) { set_error(d, member_of_edge(d, e), SEVC_E_STATE); continue; }
-            int CE = remove_two_grains(d, e, gnic);
-            set_grain_enabled(d, gic[0], false);
-            set_grain_enabled(d, gic[1], false);
+            int ga[3], gb[3], g0, g1, gn0, gn1;
+            load_triple(d.vg, d.bvx[2 * e], ga);
+            load_triple(d.vg, d.bvx[2 * e + 1], gb);
+            triples_intersect(ga, gb, g0, g1);
+            triples_symdiff(ga, gb, g0, g1, gn0, gn1);
+            if (gn0 < 0 || gn1 < 0) { set_error(d, member_of_edge(d, e), SEVC_E_STATE); continue; }
+            int CE = remove_two_grains(d, e, gn0, gn1);
+            set_grain_enabled(d, g0, false);
+            set_grain_enabled(d, g1, false);
             d.ms[member_of_edge(d, e)].two += 1;
-            // the T2 labels k_scan3 took before this stage are redone
-            d.cnt[C_RELABEL] = 1;
-            d.cnt[C_T2] = 0;
             // an edge whose endpoint moved may qualify later in this pass
             if (CE > e && two_qualifies(d, CE)) {
                 bool have = false;
@@ -2120,7 +2303,7 @@ __global__ void k_two_grain(Dev d) {
             }
         }
         // fix_grain_lists for the flagged grains
-        const int nf = d.cnt[C_FIX0];
+        const int nf = cnt_now(d, C_FIX0);
         for (int q = 0; q < nf; q++) fix_one_grain(d, d.l_fix[0][q]);
         int nn = 0;
         for (int q = 0; q < nf; q++) {
@@ -2150,212 +2333,205 @@ __global__ void k_two_grain(Dev d) {
                     if (!have) lst[nn++] = e;
                 }
             }
+            // for the next step, should the passes end with this one
+            if (it == 19 && len == 3) list_tri(d, g, true);
         }
-        d.cnt[C_FIX0] = 0;
+        atomicExch(&d.cnt[C_FIX0], 0);
         n = nn;
     }
 }
 
-// Two-triangle candidates and T2 labels in one pass over the grains,
-// sharing the loads of a 3-sided grain's list, its vertices' edges and
-// grains and those edges' ends and flags.  Two-triangle candidates
-// (topological.h:22-73): edges whose two grains are both 3-sided, found
-// from the 3-sided grains; for edge (a, c) of 3-sided grain g the two grains
-// are vg(a) ∩ vg(c), the set grains_intersect forms from the edge's ends,
-// and the edge is listed once, by the lower of the two grains.  The T2
-// labels (as k_label3) are those before the two-triangle stage; k_label3
-// redoes them if that stage changes anything.
-__global__ void k_scan3(Dev d) {
-    __shared__ int q_s[kBlock];       // the block's enabled 3-sided grains
-    __shared__ int nq;
-    TABLE_BLOCK(d.gblk, d.ngb)
-    // the grain's data is loaded together with the member's state
-    const bool in = i < bd_.e;
-    const uint8_t en = in ? d.genab[i] : 0;
-    const int len = in ? d.glen[i] : 0;
-    if (threadIdx.x == 0) nq = 0;
-    __syncthreads();
-    const bool run = M.active && P.events;          // the same for the whole workgroup
-    if (run && en) {
-        if (len == 3) q_s[atomicAdd(&nq, 1)] = i;
-        else d.gcand[i] = 0;
-    }
-    __syncthreads();
-    // the 3-sided grains go to the first lanes, so that one wave carries
-    // their chains of loads and the others finish at once
-    if (!run || (int)threadIdx.x >= nq) return;
-    const int g = q_s[threadIdx.x];
-    uint8_t cand = 0;
-    {
+// Two-triangle candidates (topological.h:22-73): edges whose two grains are
+// both 3-sided.  The stage runs until none is left, and an edge can qualify
+// anew only when one of its grains was edited (a flip or a removal flags every
+// grain around the vertices it changes), so only the grains that an edit or a
+// nucleation left with three vertices since the last step (l_tri) are looked
+// at; k_tri_all lists them all for a state that was uploaded or restored.  For
+// edge (a, c) of 3-sided grain g the two grains are vg(a) and vg(c) in common,
+// the set grains_intersect forms from the edge's ends.  An edge that both of
+// its grains list comes twice; the second finds it gone.  (A pass over all
+// grains took 17.5 us at 1M grains, 8 at 2,000.)
+__device__ __forceinline__ void tri_items(const Dev& d, int n, int k0, int stride) {
+    for (int k = k0; k < n; k += stride) {
+        const int g = d.l_tri[k], m = member_of_grain(d, g);
+        if (!d.genab[g] || d.glen[g] != 3 || !d.ms[m].active || !d.prm[m].events) continue;
         const int* L = glist(d, g);
-        const int v0 = L[0], v1 = L[1], v2 = L[2];
-        const int vv[3] = {v0, v1, v2};
-        int bb[9], gv[9];
+        const int vv[3] = {L[0], L[1], L[2]};
+        int bb[9], gv[9], ini[9], end[9], be[9];
 #pragma unroll
         for (int e = 0; e < 9; e++) {
             bb[e] = d.vb[3 * vv[e / 3] + e % 3];
             gv[e] = d.vg[3 * vv[e / 3] + e % 3];
         }
-        // the edges' ends and the byte k_label and k_poll left: bit 0 the
-        // label before polling (is_candidate at this step's dt) of an enabled
-        // edge, bit 1 enabled, bit 2 the label after polling (an enabled
-        // edge's current label is set only if it was listed and kept); two
-        // loads per edge
-        int ini[9], end[9];
-        uint8_t bc[9], lab[9], be[9];
 #pragma unroll
         for (int e = 0; e < 9; e++) {
-            const int b = bb[e];
-            ini[e] = d.bvx[2 * b];
-            end[e] = d.bvx[2 * b + 1];
-            lab[e] = d.blab[b];
+            ini[e] = d.bvx[2 * bb[e]];
+            end[e] = d.bvx[2 * bb[e] + 1];
+            be[e] = d.benab[bb[e]];
         }
 #pragma unroll
-        for (int e = 0; e < 9; e++) {
-            be[e] = (lab[e] >> 1) & 1;
-            bc[e] = (lab[e] >> 2) & 1;
-        }
-        // label_3sided_grains (as k_label3)
-        auto in_g = [&](int x) { return x == v0 || x == v1 || x == v2; };
-        bool hit = false;
-        int ans = 0;
+        for (int q = 0; q < 3; q++) {
+            const int qc = (q + 1) % 3;
 #pragma unroll
-        for (int e = 0; e < 9; e++) {
-            const bool inn = in_g(ini[e]) && in_g(end[e]);
-            hit = hit || (inn && bc[e] && be[e]);
-            ans += (inn && (lab[e] & 1)) ? 1 : 0;
-        }
-        ans /= 2;
-        if (hit || ans == 3) cand = 1;
-        // two-triangle candidates: edge (a, c) of the grain with both of its
-        // grains 3-sided
-        for (int k = 0; k < 3; k++) {
-            const int kc = (k + 1) % 3;
-            const int c = vv[kc];
-            for (int q = 0; q < 3; q++) {
-                const int e = 3 * k + q;
-                const int oe = (ini[e] == vv[k]) ? end[e] : ini[e];
-                if (oe != c || !be[e]) continue;
-                int gic[2] = {-1, -1}, cnt = 0;
-                for (int x = 0; x < 3 && cnt < 2; x++)
-                    for (int y = 0; y < 3; y++)
-                        if (gv[3 * k + x] == gv[3 * kc + y]) { gic[cnt++] = gv[3 * k + x]; break; }
-                if (cnt < 2) continue;
-                if (d.glen[gic[0]] == 3 && d.glen[gic[1]] == 3) {
-                    const int lo = gic[0] < gic[1] ? gic[0] : gic[1];
-                    if (lo == g) {
-                        const int s = atomicAdd(&d.cnt[C_TWO], 1);     // rare: two adjacent 3-sided grains
-                        d.l_two[s] = bb[e];
+            for (int r = 0; r < 3; r++) {
+                const int e = 3 * q + r;
+                const int oe = (ini[e] == vv[q]) ? end[e] : ini[e];
+                if (oe != vv[qc] || !be[e]) continue;
+                int g0 = -1, g1 = -1;
+#pragma unroll
+                for (int x = 0; x < 3; x++) {
+                    const int h = gv[3 * q + x];
+                    if (h == gv[3 * qc] || h == gv[3 * qc + 1] || h == gv[3 * qc + 2]) {
+                        if (g0 < 0) g0 = h;
+                        else if (g1 < 0) g1 = h;
                     }
                 }
+                if (g1 < 0 || d.glen[g0] != 3 || d.glen[g1] != 3) continue;
+                const int s = atomicAdd(&d.cnt[C_TWO], 1);     // rare: two adjacent 3-sided grains
+                if (s < d.E) d.l_two[s] = bb[e];
             }
         }
     }
-    d.gcand[g] = cand;
-    const int s = wave_slot(&d.cnt[C_T2], cand != 0);
-    if (cand) d.l_t2[s] = g;
+}
+
+// Lists every enabled 3-sided grain next to another one (the first step
+// after an upload or a restore).
+__global__ void k_tri_all(Dev d) {
+    TABLE_BLOCK(d.gblk, d.ngb)
+    if (i >= bd_.e || !d.genab[i] || d.glen[i] != 3) return;
+    const int* L = glist(d, i);
+    bool near = false;
+    for (int e = 0; e < 9; e++) {
+        const int h = d.vg[3 * L[e / 3] + e % 3];
+        near = near || (h != i && h >= 0 && d.genab[h] && d.glen[h] == 3);
+    }
+    list_tri(d, i, near);
+}
+
+__device__ __forceinline__ int n_tri(const Dev& d) { return (int)min((unsigned)cnt_now(d, C_TRI), 6u * (unsigned)d.G); }
+
+// The polling gathers, and the two-triangle search beside them (it reads the
+// topology only) on the workgroups that a short candidate list leaves idle.
+__global__ void k_poll_gather(Dev d) {
+    const int n = (int)(gridDim.x * blockDim.x), k0 = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    gather_items(d, d.cnt[C_CAND], k0, n);
+    tri_items(d, n_tri(d), n - 1 - k0, n);
+}
+
+// After the gathers, by one workgroup: the vote rounds and the conflict check
+// on the step's candidate list, then (rarely) the passes of the two-triangle
+// stage.  The dt of the labels is noted for the slots that are labelled at the
+// end of the call (k_label_disabled).
+__device__ __forceinline__ void poll_stage(const Dev& d, int nc, unsigned char* pbuf) {
+    for (int m = (int)threadIdx.x; m < d.B; m += (int)blockDim.x)
+        if (d.ms[m].active && d.prm[m].events) d.ms[m].lab_dt = member_dt(d.prm[m], d.ms[m]);
+    if (nc > 0) poll_list(d, nc, pbuf);
+    if (threadIdx.x == 0) atomicExch(&d.cnt[C_TRI], 0);
+    if (cnt_now(d, C_TWO) > 0) {
+        __syncthreads();
+        if (threadIdx.x == 0) two_grain_serial(d);
+    }
+    __syncthreads();
+}
+
+__global__ void __launch_bounds__(1024) k_poll(Dev d) {
+    __shared__ __align__(16) unsigned char pbuf[kPollLds];
+    poll_stage(d, d.cnt[C_CAND], pbuf);
+}
+
+// label_3sided_grains after the two-triangle stage, from the candidate list: a
+// 3-sided grain is labelled when one of its own edges (both ends in the
+// grain's list) kept its label, or when all three are candidates, so it has
+// at least one listed candidate edge, and that edge's ends have the grain in
+// common.  Each labelled grain is listed by the lowest of its candidate edges.
+// (The pass over all grains that this replaces shared the 17.5 us above.)
+__device__ __forceinline__ void t2_label_items(const Dev& d, int k0, int stride) {
+    const int n = d.cnt[C_CAND];
+    for (int k = k0; k < n; k += stride) {
+        const int c = d.l_cand[k];
+        const int a = d.bvx[2 * c], b = d.bvx[2 * c + 1];
+        const uint8_t lab = d.blab[c], ce = d.benab[c];
+        if (!(lab & 1) || !ce || !d.ms[member_of_edge(d, c)].active) continue;
+        int ga[3], gb[3], gl[3];
+        uint8_t ge[3];
+#pragma unroll
+        for (int q = 0; q < 3; q++) { ga[q] = d.vg[3 * a + q]; gb[q] = d.vg[3 * b + q]; }
+#pragma unroll
+        for (int q = 0; q < 3; q++) { gl[q] = d.glen[ga[q]]; ge[q] = d.genab[ga[q]]; }
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+            const int g = ga[q];
+            if (gl[q] != 3 || !ge[q] || !(g == gb[0] || g == gb[1] || g == gb[2])) continue;
+            const int* L = glist(d, g);
+            const int v0 = L[0], v1 = L[1], v2 = L[2];
+            const int vv[3] = {v0, v1, v2};
+            int bb[9], ini[9], end[9];
+            uint8_t lb[9], be[9];
+#pragma unroll
+            for (int e = 0; e < 9; e++) bb[e] = d.vb[3 * vv[e / 3] + e % 3];
+#pragma unroll
+            for (int e = 0; e < 9; e++) {
+                ini[e] = d.bvx[2 * bb[e]];
+                end[e] = d.bvx[2 * bb[e] + 1];
+                lb[e] = d.blab[bb[e]];
+                be[e] = d.benab[bb[e]];
+            }
+            auto in_g = [&](int x) { return x == v0 || x == v1 || x == v2; };
+            // label_3sided_grains stops counting a vertex's edges at the first
+            // labelled one, but then the grain is a candidate whatever the
+            // count, so counting every visit gives the same label
+            bool hit = false;
+            int ans = 0, first = INT_MAX;
+#pragma unroll
+            for (int e = 0; e < 9; e++) {
+                const bool on = in_g(ini[e]) && in_g(end[e]) && be[e];
+                hit = hit || (on && (lb[e] & 4));
+                if (on && (lb[e] & 1)) {
+                    ans++;
+                    first = min(first, bb[e]);
+                }
+            }
+            if (!(hit || ans / 2 == 3) || first != c) continue;
+            d.gcand[g] = 1;
+            const int s = wave_slot(&d.cnt[C_T2], true);
+            d.l_t2[s] = g;
+        }
+    }
+}
+
+__global__ void k_t2_label(Dev d) {
+    t2_label_items(d, (int)(blockIdx.x * blockDim.x + threadIdx.x), (int)(gridDim.x * blockDim.x));
 }
 
 // ---------------------------------------------------------------------
 // T2: 3-sided grain removal (topological.h:614-668, 687-822, 994-1004)
 // ---------------------------------------------------------------------
 
-// clear_grains_state + label_3sided_grains; candidates are compacted.
-// k_scan3 takes these labels before the two-triangle stage; this kernel
-// redoes them when that stage removed a pair of grains (a step without such
-// an event leaves every datum the labels read unchanged).
-__global__ void k_label3(Dev d) {
-    if (d.cnt[C_RELABEL] == 0) return;
-    TABLE_BLOCK(d.gblk, d.ngb)
-    // the grain's data is loaded together with the member's state
-    const bool in = i < bd_.e;
-    const uint8_t en = in ? d.genab[i] : 0;
-    const int len = in ? d.glen[i] : 0;
-    if (!M.active || !P.events || !en) return;
-    const int g = i;
-    uint8_t cand = 0;
-    if (len == 3) {
-        // every datum of the 9 (vertex, edge) visits is loaded up front (three
-        // rounds of independent loads), then the visits run in the order of
-        // label_3sided_grains; "in g" is membership in the 3-entry list
-        // (grain_contains_vertex)
-        const double dt = member_dt(P, M);
-        const int* L = glist(d, g);
-        const int v0 = L[0], v1 = L[1], v2 = L[2];
-        const int vv[3] = {v0, v1, v2};
-        int bb[9];
-#pragma unroll
-        for (int e = 0; e < 9; e++) bb[e] = d.vb[3 * vv[e / 3] + e % 3];
-        int ini[9], end[9];
-        uint8_t bc[9], be[9];
-        double te[9], bl[9];
-#pragma unroll
-        for (int e = 0; e < 9; e++) {
-            const int b = bb[e];
-            ini[e] = d.bvx[2 * b];
-            end[e] = d.bvx[2 * b + 1];
-            bc[e] = d.bcand[b];
-            be[e] = d.benab[b];
-            te[e] = d.bt[b];
-            bl[e] = d.blen[b];
-        }
-        auto in_g = [&](int x) { return x == v0 || x == v1 || x == v2; };
-        // label_3sided_grains stops counting a vertex's edges at the first
-        // labelled one, but then the grain is a candidate whatever the count,
-        // so counting every visit gives the same label
-        bool hit = false;
-        int ans = 0;
-#pragma unroll
-        for (int e = 0; e < 9; e++) {
-            const bool inn = in_g(ini[e]) && in_g(end[e]);
-            hit = hit || (inn && bc[e] && be[e]);
-            ans += (inn && is_candidate(te[e], bl[e], dt, P.flip_thr) && be[e]) ? 1 : 0;
-        }
-        ans /= 2;
-        if (hit || ans == 3) cand = 1;
-    }
-    d.gcand[g] = cand;
-    const int s = wave_slot(&d.cnt[C_T2], cand != 0);
-    if (cand) d.l_t2[s] = g;
-}
-
-// remove_grain, topological.h:687-822
-// grains_intersect on vertex-grain triples already in registers.
-__device__ __forceinline__ int rg_intersect(const int* ga, const int* gb, int out[2]) {
-    int k = 0;
-    out[0] = out[1] = -1;
-    for (int i = 0; i < 3; i++)
-        for (int j = 0; j < 3; j++)
-            if (ga[i] == gb[j]) {
-                out[k++] = ga[i];
-                if (k == 2) return 2;
-            }
-    return k;
-}
-
-// remove_3sided_grain.  Everything the removal reads is loaded first (the
-// grain's vertices; their edges, grains and positions; those edges' ends),
-// then the reference's sequence of tests and writes runs on local copies
-// in the same order -- a later test sees an earlier write exactly as it
-// would in memory -- and the writes go out.
-__device__ void remove_grain(const Dev& d, int g, double D) {
+// remove_grain, topological.h:687-822.  Everything the removal reads is loaded
+// first (the grain's vertices; their edges, grains, positions and flags; those
+// edges' ends and flags), then the reference's sequence of tests and writes
+// runs on local copies in the same order -- a later test sees an earlier write
+// exactly as it would in memory -- and the writes go out.
+__device__ __forceinline__ void remove_grain(const Dev& d, int g, double D) {
     const int* Lg = glist(d, g);
     const int A = Lg[0], B = Lg[1], C = Lg[2];
     int vA[3], vB[3], vC[3], gA[3], gB[3], gC[3];
+    load_triple(d.vb, A, vA); load_triple(d.vb, B, vB); load_triple(d.vb, C, vC);
+    load_triple(d.vg, A, gA); load_triple(d.vg, B, gB); load_triple(d.vg, C, gC);
+    const double2* X = reinterpret_cast<const double2*>(d.pos);
+    const double2 pA = X[A], pB = X[B], pC = X[C];
+    const bool onB = d.ven[B] != 0, onC = d.ven[C] != 0, onG = d.genab[g] != 0;
+    int2 xA[3], xB[3], xC[3];                      // ends of the vertices' edges
+    bool onA_[3], onC_[3];                         // flags of A's and C's edges
 #pragma unroll
     for (int i = 0; i < 3; i++) {
-        vA[i] = d.vb[3 * A + i]; vB[i] = d.vb[3 * B + i]; vC[i] = d.vb[3 * C + i];
-        gA[i] = d.vg[3 * A + i]; gB[i] = d.vg[3 * B + i]; gC[i] = d.vg[3 * C + i];
+        xA[i] = reinterpret_cast<const int2*>(d.bvx)[vA[i]];
+        xB[i] = reinterpret_cast<const int2*>(d.bvx)[vB[i]];
+        xC[i] = reinterpret_cast<const int2*>(d.bvx)[vC[i]];
+        onA_[i] = d.benab[vA[i]] != 0;
+        onC_[i] = d.benab[vC[i]] != 0;
     }
-    const double xp0 = d.pos[2 * A], xp1 = d.pos[2 * B], xp2 = d.pos[2 * C];
-    const double yp0 = d.pos[2 * A + 1], yp1 = d.pos[2 * B + 1], yp2 = d.pos[2 * C + 1];
-    int xA[3][2], xB[3][2], xC[3][2];              // ends of the vertices' edges
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-        xA[i][0] = d.bvx[2 * vA[i]]; xA[i][1] = d.bvx[2 * vA[i] + 1];
-        xB[i][0] = d.bvx[2 * vB[i]]; xB[i][1] = d.bvx[2 * vB[i] + 1];
-        xC[i][0] = d.bvx[2 * vC[i]]; xC[i][1] = d.bvx[2 * vC[i] + 1];
-    }
+    const double xp0 = pA.x, xp1 = pB.x, xp2 = pC.x, yp0 = pA.y, yp1 = pB.y, yp2 = pC.y;
     double nAB = arclen(xp0, yp0, xp1, yp1, D);
     double nBC = arclen(xp1, yp1, xp2, yp2, D);
     double nCA = arclen(xp2, yp2, xp0, yp0, D);
@@ -2366,32 +2542,36 @@ __device__ void remove_grain(const Dev& d, int g, double D) {
     double ux0 = 0, uy0 = 0;
     double ax = xp0 + (nBC * ux0 + nCA * ux1 + nAB * ux2) / denom;
     double ay = yp0 + (nBC * uy0 + nCA * uy1 + nAB * uy2) / denom;
-    d.pos[2 * A] = dom_mod(ax, D);
-    d.pos[2 * A + 1] = dom_mod(ay, D);
-    int gic[2], G1, G2, G3;
-    rg_intersect(gB, gC, gic); G3 = (gic[0] == g) ? gic[1] : gic[0];
-    rg_intersect(gA, gB, gic); G2 = (gic[0] == g) ? gic[1] : gic[0];
-    rg_intersect(gA, gC, gic); G1 = (gic[0] == g) ? gic[1] : gic[0];
+    reinterpret_cast<double2*>(d.pos)[A] = make_double2(dom_mod(ax, D), dom_mod(ay, D));
+    int c0, c1, G1, G2, G3;
+    triples_intersect(gB, gC, c0, c1); G3 = (c0 == g) ? c1 : c0;
+    triples_intersect(gA, gB, c0, c1); G2 = (c0 == g) ? c1 : c0;
+    triples_intersect(gA, gC, c0, c1); G1 = (c0 == g) ? c1 : c0;
     if (G1 < 0 || G2 < 0 || G3 < 0) { set_error(d, member_of_grain(d, g), SEVC_E_STATE); return; }
-    d.vel[2 * A] = 0.0;
-    d.vel[2 * A + 1] = 0.0;
+    reinterpret_cast<double2*>(d.vel)[A] = make_double2(0.0, 0.0);
     // The searches below take the first match in index order, written as
     // unrolled loops (constant indices keep the small arrays in registers).
+    // Edges disabled twice (never in a valid mesh) count once.
     bool found = false;
+    int offBC = -1;
 #pragma unroll
     for (int i = 0; i < 3; i++) {
-        const int ei = xC[i][0], ee = xC[i][1];
-        if (!found && ((ei == B && ee == C) || (ee == B && ei == C))) { set_edge_enabled(d, vC[i], false); found = true; }
+        const int ei = xC[i].x, ee = xC[i].y;
+        if (!found && ((ei == B && ee == C) || (ee == B && ei == C))) {
+            set_edge_enabled(d, vC[i], onC_[i], false);
+            offBC = vC[i];
+            found = true;
+        }
     }
     int BEb = -1, CF = -1, be0 = -1, be1 = -1, cf0 = -1, cf1 = -1;
 #pragma unroll
     for (int i = 2; i >= 0; i--) {
-        const int ei = xB[i][0], ee = xB[i][1];
+        const int ei = xB[i].x, ee = xB[i].y;
         if (!(ei == A || ee == A) && !(ei == C || ee == C)) { BEb = vB[i]; be0 = ei; be1 = ee; }
     }
 #pragma unroll
     for (int i = 2; i >= 0; i--) {
-        const int ei = xC[i][0], ee = xC[i][1];
+        const int ei = xC[i].x, ee = xC[i].y;
         if (!(ei == A || ee == A) && !(ei == B || ee == B)) { CF = vC[i]; cf0 = ei; cf1 = ee; }
     }
     if (BEb < 0 || CF < 0) { set_error(d, member_of_grain(d, g), SEVC_E_STATE); return; }
@@ -2409,16 +2589,19 @@ __device__ void remove_grain(const Dev& d, int g, double D) {
     auto ends = [&](int e, int i, int& e0, int& e1) {
         if (e == CF) { e0 = cf0; e1 = cf1; }
         else if (e == BEb) { e0 = be0; e1 = be1; }
-        else { e0 = xA[i][0]; e1 = xA[i][1]; }
+        else { e0 = xA[i].x; e1 = xA[i].y; }
     };
     int curA[3] = {vA[0], vA[1], vA[2]};
     found = false;
+    int offAB = -1;
 #pragma unroll
     for (int i = 0; i < 3; i++) {
         int e0, e1;
         ends(curA[i], i, e0, e1);
         if (!found && (e0 == B || e1 == B)) {
-            set_edge_enabled(d, curA[i], false); curA[i] = BEb; d.vb[3 * A + i] = BEb; found = true;
+            set_edge_enabled(d, curA[i], onA_[i] && curA[i] != offBC, false);
+            offAB = curA[i];
+            curA[i] = BEb; d.vb[3 * A + i] = BEb; found = true;
         }
     }
     found = false;
@@ -2427,17 +2610,26 @@ __device__ void remove_grain(const Dev& d, int g, double D) {
         int e0, e1;
         if (curA[i] == BEb) { e0 = be0; e1 = be1; }
         else ends(curA[i], i, e0, e1);
-        if (!found && (e0 == C || e1 == C)) { set_edge_enabled(d, curA[i], false); d.vb[3 * A + i] = CF; found = true; }
+        if (!found && (e0 == C || e1 == C)) {
+            // (an entry replaced above is read again)
+            const bool was = curA[i] == vA[i] ? onA_[i] && curA[i] != offBC && curA[i] != offAB : d.benab[curA[i]] != 0;
+            set_edge_enabled(d, curA[i], was, false);
+            d.vb[3 * A + i] = CF; found = true;
+        }
     }
-    set_vertex_enabled(d, B, false);
-    set_vertex_enabled(d, C, false);
-    set_grain_enabled(d, g, false);
-    set_mod(d, B, 0, FIX_REMOVE, G2, B); flag_grain(d, G2, 1);
-    set_mod(d, C, 0, FIX_REMOVE, G1, C); flag_grain(d, G1, 1);
-    set_mod(d, B, 1, FIX_REMOVE, G3, B); flag_grain(d, G3, 1);
+    set_vertex_enabled(d, B, onB, false);
+    set_vertex_enabled(d, C, onC && C != B, false);
+    set_grain_enabled(d, g, onG, false);
+    set_mod(d, B, 0, FIX_REMOVE, G2, B);
+    set_mod(d, C, 0, FIX_REMOVE, G1, C);
+    set_mod(d, B, 1, FIX_REMOVE, G3, B);
     set_mod(d, C, 1, FIX_REPLACE, G3, A);
     d.mods[C].prev[1] = C;
+#pragma unroll
     for (int i = 0; i < 3; i++) if (gA[i] == g) d.vg[3 * A + i] = G3;
+    const int gg[3] = {G2, G1, G3};
+    const bool all[3] = {true, true, true};
+    flag_grains(d, gg, all, 1);
 }
 
 
@@ -2448,9 +2640,9 @@ __device__ void remove_grain(const Dev& d, int g, double D) {
 // until its own check passes), and a removal writes only data that no
 // non-adjacent candidate's check reads, so the outcome does not depend on
 // the schedule.
-__global__ void k_t2_par(Dev d) {
-    const int n = d.cnt[C_T2];
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
+__device__ __forceinline__ void t2_items(const Dev& d, int k0, int stride) {
+    const int n = cnt_now(d, C_T2);
+    for (int k = k0; k < n; k += stride) {
         int g = d.l_t2[k];
         if (!d.ms[member_of_grain(d, g)].active) continue;   // stopped by a failed check or an error
         // the grains of the three vertices and their flags, in three rounds
@@ -2482,10 +2674,12 @@ __global__ void k_t2_par(Dev d) {
     }
 }
 
-__global__ void k_t2_serial(Dev d) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    int n = d.cnt[C_T2C];
-    if (n == 0) return;
+__global__ void k_t2_par(Dev d) {
+    t2_items(d, (int)(blockIdx.x * blockDim.x + threadIdx.x), (int)(gridDim.x * blockDim.x));
+}
+
+__device__ __forceinline__ void t2_serial(const Dev& d) {
+    const int n = cnt_now(d, C_T2C);
     sort_ints(d.l_t2c, n);
     for (int k = 0; k < n; k++) {
         int g = d.l_t2c[k];
@@ -2493,20 +2687,27 @@ __global__ void k_t2_serial(Dev d) {
         int m = member_of_grain(d, g);
         if (!d.ms[m].active) continue;
         remove_grain(d, g, d.prm[m].D);
-        d.ms[m].removals += 1;
+        atomicAdd(reinterpret_cast<unsigned long long*>(&d.ms[m].removals), 1ull);
     }
 }
 
-// unlabel_boundaries_st2, topological.h:588-606
+__global__ void k_t2_serial(Dev d) {
+    if (threadIdx.x == 0 && blockIdx.x == 0) t2_serial(d);
+}
+
+// unlabel_boundaries_st2, topological.h:588-606; the T2 stage is over, so
+// its labels are taken back (t2_label_items sets labels only)
 __device__ __forceinline__ void st2_items(const Dev& d, int k0, int stride) {
+    const int nt2 = cnt_now(d, C_T2);
+    for (int k = k0; k < nt2; k += stride) d.gcand[d.l_t2[k]] = 0;
     const int n = d.cnt[C_CAND];
     for (int k = k0; k < n; k += stride) {
         int b = d.l_cand[k];
         if (!(d.benab[b] && d.bcand[b])) continue;
         if (!d.ms[member_of_edge(d, b)].active) continue;
-        int gic[2];
-        if (grains_intersect(d, d.bvx[2 * b], d.bvx[2 * b + 1], gic) < 2) { d.bcand[b] = 0; continue; }
-        if (d.glen[gic[0]] == 3 || d.glen[gic[1]] == 3) d.bcand[b] = 0;
+        int g0, g1;
+        if (grains_intersect(d, d.bvx[2 * b], d.bvx[2 * b + 1], g0, g1) < 2) { d.bcand[b] = 0; continue; }
+        if (d.glen[g0] == 3 || d.glen[g1] == 3) d.bcand[b] = 0;
     }
 }
 
@@ -2522,8 +2723,9 @@ __global__ void k_st2(Dev d) {
 // and writes fix flags, vertex edit records and areas.
 __global__ void __launch_bounds__(64) k_st2_fix_clear(Dev d, int nclear) {
     const int b = (int)blockIdx.x;
+    __shared__ ClearLds c;
     if (b < nclear) {
-        fix_clear_items(d, 1, 1, b, nclear);
+        fix_clear_items(d, 1, 1, c, b, nclear);
         return;
     }
     st2_items(d, (b - nclear) * 64 + (int)threadIdx.x, ((int)gridDim.x - nclear) * 64);
@@ -2571,76 +2773,57 @@ __device__ __forceinline__ void flip(const Dev& d, int bnd, const Params& P, con
         gA[k] = in.gA[k]; gB[k] = in.gB[k];
     }
     const double pax = in.pax, pay = in.pay, pbx = in.pbx, pby = in.pby;
-    int gic[2], gnic[2];
-    rg_intersect(gA, gB, gic);
-    {
-        // grains_symdiff (geometry.h:886-898) on the triples
-        int gun[4];
-        gnic[0] = gnic[1] = -1;
-        gun[3] = -1;
-        for (int k = 0; k < 3; k++) gun[k] = gA[k];
-        for (int k = 0; k < 3; k++) {
-            const int g = gB[k];
-            if (g != gun[0] && g != gun[1] && g != gun[2]) { gun[3] = g; break; }
-        }
-        int c = 0;
-        for (int k = 0; k < 4; k++)
-            if (gun[k] != gic[0] && gun[k] != gic[1]) {
-                gnic[c++] = gun[k];
-                if (c == 2) break;
-            }
-    }
-    int i = -1, j = -1, AC = -1, BEb = -1;
-    for (int k = 0; k < 3; k++) if (vA[k] == bnd) { i = (k + 1) % 3; AC = vA[i]; break; }
-    for (int k = 0; k < 3; k++) if (vB[k] == bnd) { j = (k + 1) % 3; BEb = vB[j]; break; }
-    if (i < 0 || j < 0 || gic[1] < 0 || gnic[1] < 0) { set_error(d, member_of_edge(d, bnd), SEVC_E_STATE); return; }
+    int gi0, gi1, gn0, gn1;
+    triples_intersect(gA, gB, gi0, gi1);
+    triples_symdiff(gA, gB, gi0, gi1, gn0, gn1);
+    // the first slot holding the edge at each end, and the slot after it
+    const int i = vA[0] == bnd ? 1 : (vA[1] == bnd ? 2 : (vA[2] == bnd ? 0 : -1));
+    const int j = vB[0] == bnd ? 1 : (vB[1] == bnd ? 2 : (vB[2] == bnd ? 0 : -1));
+    const int AC = i == 0 ? vA[0] : (i == 1 ? vA[1] : vA[2]);
+    const int BEb = j == 0 ? vB[0] : (j == 1 ? vB[1] : vB[2]);
+    if (i < 0 || j < 0 || gi1 < 0 || gn1 < 0) { set_error(d, member_of_edge(d, bnd), SEVC_E_STATE); return; }
     // reads that do not depend on the writes below, issued together
     const int ac0 = d.bvx[2 * AC];
     const int be0 = d.bvx[2 * BEb];
-    const int c2[2] = {grain_contains_consecutive(d, gic[0], A, B), grain_contains_consecutive(d, gic[1], A, B)};
-    const int c4[2] = {grain_contains_consecutive(d, gic[0], B, A), grain_contains_consecutive(d, gic[1], B, A)};
-    const int h3[2] = {grain_contains_vertex(d, gnic[0], A), grain_contains_vertex(d, gnic[1], A)};
-    const int h1[2] = {grain_contains_vertex(d, gnic[0], B), grain_contains_vertex(d, gnic[1], B)};
-    const double oi0 = d.gori[gic[0]], oi1 = d.gori[gic[1]], on0 = d.gori[gnic[0]], on1 = d.gori[gnic[1]];
-    d.vb[3 * A + i] = BEb; vA[i] = BEb;
-    d.vb[3 * B + j] = AC; vB[j] = AC;
+    const GrainFind f0 = grain_find(d, gi0, A, B), f1 = grain_find(d, gi1, A, B), fn0 = grain_find(d, gn0, A, B),
+                    fn1 = grain_find(d, gn1, A, B);
+    const double oi0 = d.gori[gi0], oi1 = d.gori[gi1], on0 = d.gori[gn0], on1 = d.gori[gn1];
+    d.vb[3 * A + i] = BEb;
+    d.vb[3 * B + j] = AC;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        vA[k] = k == i ? BEb : vA[k];
+        vB[k] = k == j ? AC : vB[k];
+    }
     if (ac0 == A) d.bvx[2 * AC] = B; else d.bvx[2 * AC + 1] = B;
     // BEb's ends as they are now (AC and BEb are distinct edges of a valid
     // mesh; if they coincide, the write above is seen)
     int nb0 = be0;
     if (BEb == AC) nb0 = (ac0 == A) ? B : ac0;
     if (nb0 == B) d.bvx[2 * BEb] = A; else d.bvx[2 * BEb + 1] = A;
-    int g1, g2, g3, g4;
-    for (g2 = 0; g2 < 2; g2++)
-        if (c2[g2] == 1) {
-            set_mod(d, A, 0, FIX_REMOVE, gic[g2], A);
-            flag_grain(d, gic[g2], 2);
-            break;
-        }
-    for (g4 = 0; g4 < 2; g4++)
-        if (c4[g4] == 1) {
-            set_mod(d, B, 0, FIX_REMOVE, gic[g4], B);
-            flag_grain(d, gic[g4], 2);
-            break;
-        }
-    for (g3 = 0; g3 < 2; g3++)
-        if (h3[g3] >= 0) {
-            set_mod(d, A, 1, FIX_ADD, gnic[g3], B);
-            d.mods[A].prev[1] = A;
-            flag_grain(d, gnic[g3], 2);
-            break;
-        }
-    for (g1 = 0; g1 < 2; g1++)
-        if (h1[g1] >= 0) {
-            set_mod(d, B, 1, FIX_ADD, gnic[g1], A);
-            d.mods[B].prev[1] = B;
-            flag_grain(d, gnic[g1], 2);
-            break;
-        }
+    // the grains around: g2 and g4 of the two that share the edge, g1 and g3 of
+    // the other two (the first that holds, else 2)
+    const int g2 = f0.ab == 1 ? 0 : (f1.ab == 1 ? 1 : 2), g4 = f0.ba == 1 ? 0 : (f1.ba == 1 ? 1 : 2);
+    const int g3 = fn0.a >= 0 ? 0 : (fn1.a >= 0 ? 1 : 2), g1 = fn0.b >= 0 ? 0 : (fn1.b >= 0 ? 1 : 2);
+    const int G2 = g2 == 0 ? gi0 : gi1, G4 = g4 == 0 ? gi0 : gi1, G3 = g3 == 0 ? gn0 : gn1, G1 = g1 == 0 ? gn0 : gn1;
+    if (g2 < 2) set_mod(d, A, 0, FIX_REMOVE, G2, A);
+    if (g4 < 2) set_mod(d, B, 0, FIX_REMOVE, G4, B);
+    if (g3 < 2) {
+        set_mod(d, A, 1, FIX_ADD, G3, B);
+        d.mods[A].prev[1] = A;
+    }
+    if (g1 < 2) {
+        set_mod(d, B, 1, FIX_ADD, G1, A);
+        d.mods[B].prev[1] = B;
+    }
+    const int gg[4] = {G2, G4, G3, G1};
+    const bool want[4] = {g2 < 2, g4 < 2, g3 < 2, g1 < 2};
+    flag_grains(d, gg, want, 2);
     if (g1 > 1 || g2 > 1 || g3 > 1 || g4 > 1) { set_error(d, member_of_edge(d, bnd), SEVC_E_STATE); return; }
+#pragma unroll
     for (int k = 0; k < 3; k++) {
-        if (gA[k] == gic[g2]) { gA[k] = gnic[g1]; d.vg[3 * A + k] = gnic[g1]; }
-        if (gB[k] == gic[g4]) { gB[k] = gnic[g3]; d.vg[3 * B + k] = gnic[g3]; }
+        if (gA[k] == G2) { gA[k] = G1; d.vg[3 * A + k] = G1; }
+        if (gB[k] == G4) { gB[k] = G3; d.vg[3 * B + k] = G3; }
     }
     // vector2_mean, geometry.h:311-317
     double dx = wrapd(pbx, pax, D);
@@ -2655,18 +2838,18 @@ __device__ __forceinline__ void flip(const Dev& d, int bnd, const Params& P, con
     // boundary_compute_energy on the rewired grains (no GB_scaling, topological.h:286)
     double e = 1.0;
     {
-        int gn[2];
-        if (rg_intersect(gA, gB, gn) == 2) {
+        int s0, s1;
+        if (triples_intersect(gA, gB, s0, s1) == 2) {
             auto ori = [&](int g) {
-                return g == gic[0] ? oi0 : g == gic[1] ? oi1 : g == gnic[0] ? on0 : g == gnic[1] ? on1 : d.gori[g];
+                return g == gi0 ? oi0 : g == gi1 ? oi1 : g == gn0 ? on0 : g == gn1 ? on1 : d.gori[g];
             };
-            e = gb_energy_func(ori(gn[0]) - ori(gn[1]), P.gb_eps);
+            e = gb_energy_func(ori(s0) - ori(s1), P.gb_eps);
         }
     }
     d.ben[bnd] = e;
     {
         // rescaled at the next step's start (k_begin) when no full pass runs
-        const int k = atomicAdd(d.n_flipped, 1);
+        const int k = wave_slot(d.n_flipped, true);
         if (k < d.E) d.l_flipped[k] = bnd;
     }
     d.vel[2 * A] = 0; d.vel[2 * A + 1] = 0;
@@ -2679,9 +2862,9 @@ __device__ __forceinline__ void flip(const Dev& d, int bnd, const Params& P, con
 // ends of two edges; a candidate reads those only if it shares a vertex, and
 // then both are in the serial list, so the outcome does not depend on the
 // schedule.
-__global__ void k_flip_par(Dev d) {
+__device__ __forceinline__ void flip_items(const Dev& d, int k0, int stride) {
     const int n = d.cnt[C_CAND];
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
+    for (int k = k0; k < n; k += stride) {
         int c = d.l_cand[k];
         // the candidate's flags and ends; its ends' edges, grains and
         // positions (what the flip reads first); those edges' flags: three
@@ -2714,10 +2897,12 @@ __global__ void k_flip_par(Dev d) {
     }
 }
 
-__global__ void k_flip_serial(Dev d) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    int n = d.cnt[C_FLIPC];
-    if (n == 0) return;
+__global__ void k_flip_par(Dev d) {
+    flip_items(d, (int)(blockIdx.x * blockDim.x + threadIdx.x), (int)(gridDim.x * blockDim.x));
+}
+
+__device__ __forceinline__ void flip_serial(const Dev& d) {
+    const int n = cnt_now(d, C_FLIPC);
     sort_ints(d.l_flipc, n);
     for (int k = 0; k < n; k++) {
         int c = d.l_flipc[k];
@@ -2725,8 +2910,64 @@ __global__ void k_flip_serial(Dev d) {
         int m = member_of_edge(d, c);
         if (!d.ms[m].active) continue;
         flip(d, c, d.prm[m], flip_in(d, d.bvx[2 * c], d.bvx[2 * c + 1]));
-        d.ms[m].flips += 1;
+        atomicAdd(reinterpret_cast<unsigned long long*>(&d.ms[m].flips), 1ull);
     }
+}
+
+__global__ void k_flip_serial(Dev d) {
+    if (threadIdx.x == 0 && blockIdx.x == 0) flip_serial(d);
+}
+
+// Every event stage of a step (main.cu:202-310) in one launch of one
+// workgroup, for states whose steps edit few grains: the stages of the
+// launches above, one after the other, with barriers between them in place
+// of launches.  A launch costs 3 to 4.5 us even when its list is empty and
+// starts with cold caches, so that each dependent load of the next stage goes
+// to memory; here the later stages find what the earlier ones read in the
+// workgroup's own L1 and L2.  2,000 grains, three events a step: 28 us where
+// the launches took 63; a batch of 45 events a step 66 us where they took 105;
+// 1M grains, 27 events a step, 82 us where they took 130.  Its time grows with
+// the number of edited grains (64 at a time), so busy states take the launches.
+__global__ void __launch_bounds__(1024) k_events(Dev d) {
+    __shared__ __align__(16) unsigned char buf[kPollLds];
+    const int tid = (int)threadIdx.x, nt = (int)blockDim.x, wave = tid >> 6;
+    constexpr int kWaves = 16;
+    static_assert(kWaves * sizeof(FixLds) <= kPollLds && kWaves * sizeof(ClearLds) <= kPollLds, "staging rooms fit");
+    FixLds* const fl = reinterpret_cast<FixLds*>(buf) + wave;
+    ClearLds* const cl = reinterpret_cast<ClearLds*>(buf) + wave;
+    const int nc = d.cnt[C_CAND];
+    gather_items(d, nc, tid, nt);
+    tri_items(d, n_tri(d), nt - 1 - tid, nt);
+    __syncthreads();
+    poll_stage(d, nc, buf);
+    const bool two = cnt_now(d, C_TWO) > 0;
+    if (nc == 0 && !two) return;
+    t2_label_items(d, tid, nt);
+    __syncthreads();
+    const bool t2 = cnt_now(d, C_T2) > 0;
+    if (t2) {
+        t2_items(d, tid, nt);
+        __syncthreads();
+        if (cnt_now(d, C_T2C) > 0) {
+            if (tid == 0) t2_serial(d);
+            __syncthreads();
+        }
+        fix_items(d, 1, *fl, wave, kWaves);
+        __syncthreads();
+    }
+    if (t2 || two) fix_clear_items(d, 1, 1, *cl, wave, kWaves);
+    st2_items(d, tid, nt);
+    __syncthreads();
+    flip_items(d, tid, nt);
+    __syncthreads();
+    if (cnt_now(d, C_FLIPC) > 0) {
+        if (tid == 0) flip_serial(d);
+        __syncthreads();
+    }
+    if (cnt_now(d, C_FIX2) == 0) return;
+    fix_items(d, 2, *fl, wave, kWaves);
+    __syncthreads();
+    fix_clear_items(d, 2, 0, *cl, wave, kWaves);
 }
 
 // ---------------------------------------------------------------------
@@ -2838,15 +3079,14 @@ __device__ __forceinline__ int generate_grain(const Dev& d, const Params& P, int
     r->D = other_end(d, r->AD, A);
     r->E = other_end(d, r->AE, A);
     r->F = other_end(d, r->AF, A);
-    int gAD[2], gAE[2], gAF[2];
-    grains_intersect(d, A, r->D, gAD);
-    grains_intersect(d, A, r->E, gAE);
-    grains_intersect(d, A, r->F, gAF);
-    if (gAD[0] == gAE[0] || gAD[0] == gAE[1]) { r->g2 = gAD[0]; r->g1 = gAD[1]; }
-    else if (gAD[1] == gAE[0] || gAD[1] == gAE[1]) { r->g2 = gAD[1]; r->g1 = gAD[0]; }
+    int ad0, ad1, ae0, ae1;
+    grains_intersect(d, A, r->D, ad0, ad1);
+    grains_intersect(d, A, r->E, ae0, ae1);
+    if (ad0 == ae0 || ad0 == ae1) { r->g2 = ad0; r->g1 = ad1; }
+    else if (ad1 == ae0 || ad1 == ae1) { r->g2 = ad1; r->g1 = ad0; }
     else return -1;
-    if (gAE[0] == r->g2) r->g3 = gAE[1];
-    else if (gAE[1] == r->g2) r->g3 = gAE[0];
+    if (ae0 == r->g2) r->g3 = ae1;
+    else if (ae1 == r->g2) r->g3 = ae0;
     else return -1;
     if (r->g1 < 0 || r->g2 < 0 || r->g3 < 0) return -1;
     const double ax = d.pos[2 * A], ay = d.pos[2 * A + 1], rr = d.nucl_r[A];
@@ -2894,7 +3134,7 @@ __device__ __forceinline__ int generate_grain(const Dev& d, const Params& P, int
 // Monte Carlo member: the nucleus radius and orientation from the vertex's
 // own Philox pair, dE and the factor dE - dE'.  The manager needs it only
 // for the vertex it picks, so it runs there, for that vertex alone.
-__device__ void nucl_factor_at(const Dev& d, const Params& P, const MState& M, int v) {
+__device__ __forceinline__ void nucl_factor_at(const Dev& d, const Params& P, const MState& M, int v) {
     d.dE[v] = 0;
     d.nfac[v] = 0;
     double ALs[3];
@@ -2973,7 +3213,7 @@ __global__ void __launch_bounds__(kBlock) k_begin_rate(Dev d, int rescale_flippe
 // in-wave scan, the wave totals scanned by wave 0, two barriers.
 // Returns the prefix; *total receives the sum.  All threads must call it;
 // blockDim.x is a multiple of 64 (at most 1024) and `sh` holds >= 65 ints.
-__device__ int wg_exclusive_scan(int x, int* sh, int* total) {
+__device__ __forceinline__ int wg_exclusive_scan(int x, int* sh, int* total) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = (int)(blockDim.x >> 6);
     const int inc = wave_inclusive_scan(x);
     if (lane == 63) sh[wave] = inc;
@@ -3006,7 +3246,7 @@ struct RunScan {
     int total;      // wanted slots of the member
 };
 
-__device__ RunScan run_scan(int first, int nblk, const int2* bc, int want, int* sh) {
+__device__ __forceinline__ RunScan run_scan(int first, int nblk, const int2* bc, int want, int* sh) {
     const int tid = threadIdx.x, nt = blockDim.x;
     const int C = (nblk + nt - 1) / nt;
     RunScan r;
@@ -3217,7 +3457,7 @@ __device__ __forceinline__ void collect_free3(const SlotKind K0, const SlotKind 
 // The k-th (0-based) slot of a member whose enable flag equals `want`,
 // given the member's run scan; -1 if there is none.  The lane whose run
 // holds rank k finds the block, wave 0 sweeps that block.
-__device__ int find_kth(const Blk* tbl, const RunScan& rs, const int2* bc, const uint8_t* en, int want, int k) {
+__device__ __forceinline__ int find_kth(const Blk* tbl, const RunScan& rs, const int2* bc, const uint8_t* en, int want, int k) {
     __shared__ int fb, fr, found;
     const int tid = threadIdx.x;
     if (tid == 0) { fb = -1; fr = 0; found = -1; }
@@ -3658,8 +3898,12 @@ __global__ void __launch_bounds__(64) k_nucl_insert(Dev d) {
             const int n_new = n_s[t];
             int* L = glist(d, gl[t]);
             for (int i = lane; i < max(n_old[t], n_new); i += 64) L[i] = i < n_new ? Ls[t][i] : -1;
-            if (lane == 0) d.glen[gl[t]] = n_new;
+            if (lane == 0) {
+                d.glen[gl[t]] = n_new;
+                if (n_new == 3) list_tri(d, gl[t], true);
+            }
         }
+        if (lane == 0) list_tri(d, g, true);
         {
             int* Lg = glist(d, g);
             for (int i = lane; i < d.S; i += 64) Lg[i] = i == 0 ? A : (i == 1 ? B : (i == 2 ? C : -1));

@@ -18,6 +18,11 @@ constexpr int kMaxHistBins = 64;     // bins of the device area histogram
 constexpr int kNuclThreads = 1024;   // workgroup of the nucleation manager (one per member)
 constexpr int kPollFast = 2048;      // candidate lists up to this length poll with registers and LDS (two per lane)
 constexpr int kPollBig = 16384;      // lists up to this length poll with flags and t_ext in LDS
+// A step that edits more grains than kBusyOver makes the state busy, one that
+// edits fewer than kBusyUnder makes it calm (member_reduce): a calm state's
+// events run in one workgroup (k_events), a busy one's in a launch per stage.
+// The line is where both cost the same (see k_events).
+constexpr int kBusyOver = 320, kBusyUnder = 160;
 constexpr int kCountWaves = 4;       // table blocks per workgroup of k_count_all (one wave each)
 
 // Per-member run parameters (from sevc_options).
@@ -40,6 +45,7 @@ struct MState {
     unsigned long long tau_bits;     // min positive t_ext (as ordered bits)
     long long flips, removals, two, nucl, vsteps, steps;
     double nucl_area_pct;
+    double lab_dt;                   // dt of the last step that labelled this member's edges
 };
 
 // A workgroup's range of one member's entities: [b, e).
@@ -47,7 +53,10 @@ struct Blk { int m, b, e; };
 
 enum Counter {
     C_CAND = 0, C_TWO, C_T2, C_T2C, C_FLIPC,
-    C_FIX0, C_FIX1, C_FIX2, C_DIRTY, C_NUCL, C_CONF, C_NEV, C_VFALL, C_RELABEL, C_BIGR, C_COUNT
+    C_FIX0, C_FIX1, C_FIX2, C_DIRTY, C_NUCL, C_CONF, C_NEV, C_VFALL, C_BIGR,
+    C_COUNT,                          // the counters above are cleared at the end of each step
+    C_TRI = C_COUNT,                  // l_tri: emptied when it is read
+    C_TOTAL
 };
 
 enum { FIX_ADD = 0, FIX_REMOVE = 1, FIX_REPLACE = 2, FIX_NONE = 3 };   // geometry.h:17
@@ -69,7 +78,7 @@ struct Dev {
     // boundaries
     int* bvx; double* ben; double* blen; double* bt; uint8_t* benab; uint8_t* bcand; int* conf;
     int* pgat; double* pgt;          // polling gathers: 25 columns of kPollBig, t_ext
-    uint8_t* blab;                  // per edge, from k_label: bit 0 candidate and enabled, bit 1 enabled
+    uint8_t* blab;                  // per edge: bit 0 candidate (enabled), bit 1 enabled when labelled, bit 2 label after polling
     int* l_flipped; int* n_flipped;  // edges flipped since the last step start (energies to rescale)
     int* vmem; int* emem; int* gmem;  // owning member of each vertex / edge / grain slot (batches)
     // grains
@@ -91,6 +100,7 @@ struct Dev {
     int* cnt;
     int* l_cand; int* l_two; int* l_t2; int* l_t2c; int* l_flipc;
     int* l_fix[kFixStages]; int* l_dirty; int* l_nucl; int* l_conf; int* l_vfall;
+    int* l_tri;                           // grains that an edit left with three vertices (next two-triangle search)
     int* l_bigr;                          // grains longer than the lane-per-grain velocity pass holds
     int* nrec; double* nal;               // rate-mode candidate sites: (site or -1, its 3 grains), shortest edge
     int* l_nev;                           // nucleation events of the step: (member, A, B, C, AB, BC, CA, g)
@@ -102,6 +112,8 @@ struct Dev {
     int* chk_bad;                         // violations per member found by the last check
     int poll_fast;                        // longest candidate list polled from registers (<= kPollFast)
     int poll_lds;                         // longest candidate list polled from LDS (<= kPollBig)
+    int* busy;                            // 1: many grains edited per step (device copy of *busy_host)
+    int* busy_host;                       // the same in pinned host memory, written when it changes
     int free_rows;                        // blocks per kind of one free-slot search round (0: the default)
 };
 
