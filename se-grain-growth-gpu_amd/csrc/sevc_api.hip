@@ -17,13 +17,13 @@
 namespace sevc {
 // kernels of sevc_kernels.hip
 __global__ void k_begin(Dev d, int rescale_flipped);
+__global__ void k_end(Dev d);
 __global__ void k_count_all(Dev d);
-__global__ void k_member_reduce(Dev d);
 __global__ void k_edge_len_energy(Dev d, int only_nucl);
 __global__ void k_grain_area(Dev d, int only_nucl);
 __global__ void k_vertex_energy(Dev d);
 __global__ void k_vel_grain(Dev d, int tuning);
-__global__ void k_vel_vertex(Dev d, int tuning);
+__global__ void k_vel_vertex(Dev d, int tuning, int listed);
 template <int VT> __global__ void k_vel_vtile(Dev d, int tuning);
 __global__ void k_vel_glane(Dev d, int tuning);
 __global__ void k_vel_bigrain(Dev d, int tuning);
@@ -50,8 +50,8 @@ __global__ void k_flip_serial(Dev d);
 __global__ void k_events(Dev d);
 __global__ void k_nucl_area_l1(Dev d);
 __global__ void k_nucl_area_up(Dev d);
-__global__ void k_begin_rate(Dev d, int rescale_flipped);
-__global__ void k_nucl_manager(Dev d);
+__global__ void k_rate_draw(Dev d);
+__global__ void k_head(Dev d, int what);
 __global__ void k_nucl_insert(Dev d);
 __global__ void k_pack(PackList L, char* out);
 // kernels of sevc_adjoint.hip
@@ -96,6 +96,10 @@ struct sevc_state {
     std::string err;
     bool any_nucl = false, any_events = false, any_adaptive = false, any_analytic = false;
     bool any_mc = false, any_rate = false;   // nucleation modes present
+    // the rate members' candidates are drawn, and the events applied, by
+    // k_head (head_rule)
+    bool head_draw = false, head_insert = false;
+    std::vector<double> ev_rate;             // events a step that each member may expect (at most)
     bool any_aniso = false;                  // a member with GB_eps != 0 (energies change with the topology)
     bool any_debug = false;                  // a member with debug_lvl >= 1 (checks inside the step)
     bool ben_dirty = true;                   // boundary energies not computed since creation / a new scale
@@ -170,6 +174,27 @@ struct sevc_state {
 };
 
 namespace {
+
+// Who draws the rate members' candidates and who applies the events.
+void head_rule(sevc_state* s) {
+    s->head_draw = s->head_insert = true;
+    for (int m = 0; m < s->B; ++m) {
+        const sevc_options& o = s->opts[m];
+        if (!(o.events && o.do_nucleation) || o.nucleation_mode != SEVC_NUCL_RATE) continue;
+        if (s->ng[m] > kHeadGrains) s->head_draw = false;
+        if (!(s->ev_rate[m] <= kHeadEvents)) s->head_insert = false;
+    }
+}
+
+// Events that member m may expect in a step with the stored energies SE (the
+// most so far: earlier ones can come back with a checkpoint).
+void expect_events(sevc_state* s, int m, const double* SE) {
+    const sevc_options& o = s->opts[m];
+    if (!(o.events && o.do_nucleation) || o.nucleation_mode != SEVC_NUCL_RATE) return;
+    double e = 0.0;
+    for (int g = 0; g < s->ng[m]; ++g) e += std::min(1.0, std::max(0.0, o.nucleation_rate * SE[g]));
+    if (e > s->ev_rate[m]) s->ev_rate[m] = e;
+}
 
 // Captured steps hold table sizes and parameters: dropped when they change.
 void drop_graphs(sevc_state* s) {
@@ -353,13 +378,14 @@ void launch_velocity(sevc_state* s, const Dev& d) {
     if (s->vel_path == 2) {
         launch(s, "vel_glane", k_vel_glane, d.ngb, kBlock, d, 0);
         launch(s, "vel_bigrain", k_vel_bigrain, kBigGrid, 64, d, 0);
-        launch(s, "velocity", k_vel_vertex, d.nvb, kBlock, d, 0);
+        launch(s, "velocity", k_vel_vertex, d.nvb, kBlock, d, 0, 1);
     } else if (s->vel_path == 1) {
         if (s->vtile_size == 32) launch(s, "vel_fused", k_vel_vtile<32>, d.nvtile, 128, d, 0);
         else launch(s, "vel_fused", k_vel_vtile<64>, d.nvtile, 256, d, 0);
     } else {
         launch(s, "vel_grain", k_vel_grain, d.ntile, 256, d, 0);
-        launch(s, "velocity", k_vel_vertex, d.nvb, kBlock, d, 0);
+        launch(s, "velocity", k_vel_vertex, d.nvb, kBlock, d, 0, 0);
+        return;                              // k_vel_grain leaves no vertex out
     }
     launch(s, "velocity_fallback", k_velocity_fallback, 64, 256, d);
 }
@@ -397,18 +423,20 @@ void launch_step(sevc_state* s, bool diag) {
     // step after creation or after a new scale (for the members active then,
     // as the reference's per-step pass would).
     const bool all_energies = diag || s->any_aniso || s->ben_dirty;
-    // the rate mode's candidate draw runs in the begin's launch
-    if (s->any_nucl && s->any_rate)
-        launch(s, "begin", k_begin_rate, 1 + d.ngb, kBlock, d, all_energies ? 0 : 1);
-    else
-        launch(s, "begin", k_begin, 1, 1024, d, all_energies ? 0 : 1);
-    if (all_energies) launch(s, "edge_len_energy", k_edge_len_energy, d.neb, kBlock, d, 0);
-    s->ben_dirty = false;
-    if (diag || s->any_analytic) launch(s, "grain_area", k_grain_area, d.ngb, kBlock, d, 0);
-    if (diag) launch(s, "vertex_energy", k_vertex_energy, d.nvb, kBlock, d);
+    const int nucl = HEAD_SELECT | (s->head_draw ? HEAD_DRAW : 0) | (s->head_insert ? HEAD_INSERT : 0);
+    if (s->any_rate && !s->head_draw) launch(s, "rate_draw", k_rate_draw, d.ngb, kBlock, d);
+    if (all_energies || !s->any_nucl) {
+        launch(s, "begin", k_begin, s->B, 256, d, all_energies ? 0 : 1);
+        if (all_energies) launch(s, "edge_len_energy", k_edge_len_energy, d.neb, kBlock, d, 0);
+        s->ben_dirty = false;
+        if (diag || s->any_analytic) launch(s, "grain_area", k_grain_area, d.ngb, kBlock, d, 0);
+        if (diag) launch(s, "vertex_energy", k_vertex_energy, d.nvb, kBlock, d);
+        if (s->any_nucl) launch(s, "head", k_head, s->B, kNuclThreads, d, nucl);
+    } else {
+        launch(s, "head", k_head, s->B, kNuclThreads, d, nucl | HEAD_BEGIN | HEAD_RESCALE);
+    }
     if (s->any_nucl) {
-        launch(s, "nucl_manager", k_nucl_manager, s->B, kNuclThreads, d);
-        launch(s, "nucl_insert", k_nucl_insert, kNuclInsGrid, 64, d);
+        if (!s->head_insert) launch(s, "nucl_insert", k_nucl_insert, kNuclInsGrid, 64, d);
         if (diag) launch(s, "vertex_energy", k_vertex_energy, d.nvb, kBlock, d);
     }
     if (s->any_debug) launch_check(s, CHK_NUCLEATION);
@@ -455,8 +483,7 @@ void launch_step(sevc_state* s, bool diag) {
         launch(s, "translate", k_translate_clear, kClearGrid + d.nvb, kBlock, d, kClearGrid);
     else
         launch(s, "translate", k_translate, d.nvb, kBlock, d);
-    // the per-block slot counts are kept by the events themselves
-    launch(s, "member_reduce", k_member_reduce, s->B, 1024, d);
+    // the next step's begin sums this one up (k_end after a call's last)
 }
 
 void build_table(std::vector<Blk>& tbl, std::vector<int>& first, const std::vector<int>& off,
@@ -732,6 +759,9 @@ int sevc_batch_create(const sevc_options* opts, const sevc_mesh* meshes, int32_t
         M.tau_bits = 0x7FF0000000000000ull;
     }
     s->ms_prev = s->ms_host;
+    s->ev_rate.assign(static_cast<size_t>(B), 0.0);
+    for (int m = 0; m < B; ++m) expect_events(s, m, meshes[m].g_SE);
+    head_rule(s);
     {
         // the two-pass velocity (measured the faster at 1M grains); the
         // one-pass tiling that fits the vertex order is prepared for
@@ -847,6 +877,7 @@ int sevc_kernel_times(sevc_state* s, int32_t max_entries, char (*names)[48], dou
 // slots are left to its end).
 static int finish_call(sevc_state* s, bool stepped) {
     Dev d = s->d;
+    if (stepped) launch(s, "end", k_end, s->B, 256, d);
     if (stepped && s->any_events) launch(s, "label_disabled", k_label_disabled, d.neb, kBlock, d);
     launch(s, "nucl_area_l1", k_nucl_area_l1, d.ngb, 64, d);
     launch(s, "nucl_area_up", k_nucl_area_up, s->B, 1024, d);
@@ -887,6 +918,7 @@ static int stop_poll(const sevc_state* s) { return s->any_stop ? 64 : 512; }
 
 static bool all_done(sevc_state* s) {
     if (s->ms_poll.size() != static_cast<size_t>(s->B)) s->ms_poll.resize(static_cast<size_t>(s->B));
+    launch(s, "end", k_end, s->B, 256, s->d);
     if (hipMemcpyAsync(s->ms_poll.data(), s->d.ms, sizeof(MState) * s->ms_poll.size(), hipMemcpyDeviceToHost,
                        s->stream) != hipSuccess ||
         hipStreamSynchronize(s->stream) != hipSuccess)
@@ -1196,10 +1228,10 @@ int sevc_autotune(sevc_state* s, int32_t* tile_grains) {
                 (void)hipMemsetAsync(d.cnt + C_BIGR, 0, sizeof(int), s->stream);
                 hipLaunchKernelGGL(k_vel_glane, dim3(d.ngb), dim3(kBlock), 0, s->stream, d, 1);
                 hipLaunchKernelGGL(k_vel_bigrain, dim3(kBigGrid), dim3(64), 0, s->stream, d, 1);
-                hipLaunchKernelGGL(k_vel_vertex, dim3(d.nvb), dim3(kBlock), 0, s->stream, d, 1);
+                hipLaunchKernelGGL(k_vel_vertex, dim3(d.nvb), dim3(kBlock), 0, s->stream, d, 1, 1);
             } else {
                 hipLaunchKernelGGL(k_vel_grain, dim3(d.ntile), dim3(256), 0, s->stream, d, 1);
-                hipLaunchKernelGGL(k_vel_vertex, dim3(d.nvb), dim3(kBlock), 0, s->stream, d, 1);
+                hipLaunchKernelGGL(k_vel_vertex, dim3(d.nvb), dim3(kBlock), 0, s->stream, d, 1, 0);
             }
         };
         once();   // warm-up
@@ -1499,6 +1531,8 @@ int sevc_set_member_mesh(sevc_state* s, int32_t m, const sevc_mesh* me) {
     hipLaunchKernelGGL(k_count_all, dim3(count_grid(d)), dim3(64 * kCountWaves), 0, s->stream, d);
     HIPCHK(hipStreamSynchronize(s->stream));
     HIPCHK(hipGetLastError());
+    expect_events(s, m, me->g_SE);
+    head_rule(s);
     s->ben_dirty = true;          // energies of the restored topology at the next step
     if (s->any_events && !s->any_debug) s->busy = -1;
     s->tri_dirty = true;
@@ -1514,7 +1548,11 @@ int sevc_set_member_params(sevc_state* s, int32_t m, const double* pos, const do
     const Dev& d = s->d;
     if (pos) HIPCHK(hipMemcpy(d.pos + 2 * static_cast<size_t>(s->voff[m]), pos, 16 * static_cast<size_t>(s->nv[m]),
                               hipMemcpyHostToDevice));
-    if (g_SE) HIPCHK(hipMemcpy(d.gse + s->goff[m], g_SE, 8 * static_cast<size_t>(s->ng[m]), hipMemcpyHostToDevice));
+    if (g_SE) {
+        HIPCHK(hipMemcpy(d.gse + s->goff[m], g_SE, 8 * static_cast<size_t>(s->ng[m]), hipMemcpyHostToDevice));
+        expect_events(s, m, g_SE);
+        head_rule(s);
+    }
     Params P;
     HIPCHK(hipMemcpy(&P, d.prm + m, sizeof(Params), hipMemcpyDeviceToHost));
     if (gb_scaling > 0) { P.gb_scaling = gb_scaling; s->opts[m].GB_scaling = gb_scaling; }

@@ -42,60 +42,55 @@ __device__ __forceinline__ bool member_runs(const Params& P, const MState& M) {
     return tok && gok;
 }
 
-// Whether a rate-mode member nucleates in the coming step (every gap-th).
-__device__ __forceinline__ bool rate_nucleates(const Params& P, const MState& M) {
+// Whether a rate-mode member nucleates in step n (every gap-th).
+__device__ __forceinline__ bool rate_nucleates(const Params& P, int n) {
     if (!(P.events && P.do_nucl) || P.nucl_mode != SEVC_NUCL_RATE) return false;
     const int gap = P.gap > 0 ? P.gap : 1;
-    return (M.n % gap) == 0;
+    return (n % gap) == 0;
 }
 
-// Loop condition of main.cu:120 (time rule), grain rule, nucleation gate
-// main.cu:137-141, for every member, by one workgroup.  The per-step
-// counters were cleared at the end of the previous step (k_member_reduce)
-// or at set-up.
-__device__ __forceinline__ void begin_members(const Dev& d, int rescale_flipped) {
-    const int tid = threadIdx.x, nt = blockDim.x;
-    for (int m = tid; m < d.B; m += nt) {
-        const Params& P = d.prm[m];
-        MState& M = d.ms[m];
+// Begins a step for member m (one workgroup): loop condition of main.cu:120
+// (time rule), grain rule, nucleation gate main.cu:137-141.
+__device__ __forceinline__ void begin_member(const Dev& d, int m, bool rescale_flipped) {
+    const Params& P = d.prm[m];
+    MState& M = d.ms[m];
+    if (threadIdx.x == 0) {
         M.tau_bits = 0x7FF0000000000000ull;
-        M.nucl_now = 0;
-        if (M.done) { M.active = 0; continue; }
-        if (!member_runs(P, M)) { M.active = 0; M.done = 1; continue; }
-        M.active = 1;
-        M.vsteps += M.n_venabled;
-        if (P.events && P.do_nucl) {
-            int gap = P.gap > 0 ? P.gap : 1;
-            if (P.nucl_mode == SEVC_NUCL_MC) {
-                if (M.curr_grains <= P.gate_grains) M.allow_nucl = 1;   // main.cu:137-139
-                M.nucl_now = ((M.n % gap) == 0 && M.allow_nucl) ? 1 : 0;
-            } else {
-                M.nucl_now = rate_nucleates(P, M) ? 1 : 0;
+        int nucl_now = 0;
+        const bool runs = !M.done && member_runs(P, M);
+        if (runs) {
+            M.vsteps += M.n_venabled;
+            if (P.events && P.do_nucl) {
+                const int gap = P.gap > 0 ? P.gap : 1;
+                if (P.nucl_mode == SEVC_NUCL_MC) {
+                    if (M.curr_grains <= P.gate_grains) M.allow_nucl = 1;   // main.cu:137-139
+                    nucl_now = ((M.n % gap) == 0 && M.allow_nucl) ? 1 : 0;
+                } else {
+                    nucl_now = rate_nucleates(P, M.n) ? 1 : 0;
+                }
             }
+        } else {
+            M.done = 1;
         }
+        M.nucl_now = nucl_now;
+        M.open = runs ? 1 : 0;
+        M.active = runs ? 1 : 0;
     }
+    __syncthreads();
     // flip (topological.h:286) leaves the flipped edge's energy without the
     // GB_scaling factor until compute_boundary_energies (calculus.h:104-114)
     // runs at the next step's start.  Steps that skip that pass (GB_eps = 0,
     // where every other energy is the scale itself) recompute only the
     // edges flipped since, for the members active in this step (steps that
-    // run k_edge_len_energy recompute every energy there).
-    __syncthreads();
-    const int nf = rescale_flipped ? min(*d.n_flipped, d.E) : 0;
-    for (int k = tid; k < nf; k += nt) {
+    // run k_edge_len_energy recompute every energy there).  k_text empties
+    // the list.
+    const int nf = rescale_flipped && M.active ? min(*d.n_flipped, d.E) : 0;
+    for (int k = (int)threadIdx.x; k < nf; k += (int)blockDim.x) {
         const int b = d.l_flipped[k];
-        const int m = member_of_edge(d, b);
-        const Params& P = d.prm[m];
-        if (!d.ms[m].active || !d.benab[b]) continue;
+        if (member_of_edge(d, b) != m || !d.benab[b]) continue;
         const double e = (P.gb_eps == 0.0) ? 1.0 : boundary_compute_energy(d, b, P.gb_eps);
         d.ben[b] = e * P.gb_scaling;
     }
-    __syncthreads();
-    if (tid == 0) *d.n_flipped = 0;
-}
-
-__global__ void __launch_bounds__(1024) k_begin(Dev d, int rescale_flipped) {
-    begin_members(d, rescale_flipped);
 }
 
 // Per table block, for grains, edges and vertices in one launch: the
@@ -103,7 +98,7 @@ __global__ void __launch_bounds__(1024) k_begin(Dev d, int rescale_flipped) {
 // The steps keep them from then on (each event that enables or disables a
 // slot adds to its block's pair: set_*_enabled).  The enabled counts feed
 // the grain / vertex totals of main.cu:317 (one partial per table block,
-// summed per member by k_member_reduce); the pairs also serve the
+// summed per member by end_member); the pairs also serve the
 // nucleation (free-slot search, alive-vertex draw), which reads them before
 // the step's insertions.  One wave
 // per table block: each lane reads four flags 64 bytes apart (four
@@ -135,18 +130,18 @@ __global__ void __launch_bounds__(64 * kCountWaves) k_count_all(Dev d) {
     if (lane == 0) out[lb] = make_int2(r, (bd.e - bd.b) - r);
 }
 
-// One workgroup per member: sums the per-block partials of the enabled
-// grain and vertex counts.
-__global__ void __launch_bounds__(1024) k_member_reduce(Dev d) {
+// Sums up member m's last step, if one is open (one workgroup): the per-block
+// partials of the enabled grain and vertex counts, then the step counter,
+// time and stop rules.  Workgroup 0 also clears the step's list counters and
+// says whether the state is busy.
+__device__ __forceinline__ void end_member(const Dev& d, int m) {
     __shared__ int sa[16], sb[16];
-    const int m = blockIdx.x;
-    // the step's work lists are done with: clear their counters for the next
-    // step; the numbers of edited grains say whether the state is busy
     if (m == 0 && threadIdx.x < 64) {
         const int c = (int)threadIdx.x < C_COUNT ? d.cnt[threadIdx.x] : 0;
         const int edited = __builtin_amdgcn_readlane(c, C_FIX1) + __builtin_amdgcn_readlane(c, C_FIX2);
+        const int ran = __builtin_amdgcn_readlane(c, C_RAN);
         if ((int)threadIdx.x < C_COUNT) d.cnt[threadIdx.x] = 0;
-        if (threadIdx.x == 0) {
+        if (threadIdx.x == 0 && ran) {
             const int was = *d.busy, now = edited > kBusyOver ? 1 : (edited < kBusyUnder ? 0 : was);
             if (now != was) {
                 *d.busy = now;
@@ -154,7 +149,6 @@ __global__ void __launch_bounds__(1024) k_member_reduce(Dev d) {
             }
         }
     }
-    if (m >= d.B) return;
     MState& M = d.ms[m];
     const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wave = tid >> 6, nw = nt >> 6;
     // each lane reads its share of the grain and vertex partials, up to 16
@@ -178,30 +172,40 @@ __global__ void __launch_bounds__(1024) k_member_reduce(Dev d) {
 #pragma unroll
         for (int q = 0; q < kBatch; q++) { a += tg[q]; b2 += tv[q]; }
     }
-    if (!M.active) return;
-    {
-        a = wave_sum(a);
-        b2 = wave_sum(b2);
-        if (lane == 0) { sa[wave] = a; sb[wave] = b2; }
-        __syncthreads();
-        if (tid == 0) {
-            int ra = 0, rb = 0;
-            for (int w = 0; w < nw; w++) { ra += sa[w]; rb += sb[w]; }
-            M.curr_grains = (int)ra;
-            M.n_venabled = (int)rb;
-            // main.cu:388-393: step counter, time and stop rules
-            const Params& P = d.prm[m];
-            M.dt = member_dt(P, M);
-            M.n += 1;
-            M.steps += 1;
-            if (P.adaptive) M.t += M.dt;
-            else M.t = M.n * P.dt_max;
-            if (M.status != 0) M.done = 1;
-            if (M.curr_grains <= P.min_grains && P.min_grains > 0) M.done = 1;
-        }
+    if (!M.active || !M.open) return;                // the same for the whole workgroup
+    a = wave_sum(a);
+    b2 = wave_sum(b2);
+    if (lane == 0) { sa[wave] = a; sb[wave] = b2; }
+    __syncthreads();
+    if (tid == 0) {
+        int ra = 0, rb = 0;
+        for (int w = 0; w < nw; w++) { ra += sa[w]; rb += sb[w]; }
+        M.curr_grains = (int)ra;
+        M.n_venabled = (int)rb;
+        // main.cu:388-393: step counter, time and stop rules
+        const Params& P = d.prm[m];
+        M.dt = member_dt(P, M);
+        M.n += 1;
+        M.steps += 1;
+        if (P.adaptive) M.t += M.dt;
+        else M.t = M.n * P.dt_max;
+        if (M.status != 0) M.done = 1;
+        if (M.curr_grains <= P.min_grains && P.min_grains > 0) M.done = 1;
+        M.open = 0;
     }
+    __syncthreads();
 }
 
+// Sums up the last step of every member (the end of a call, and where the
+// host asks whether all have finished), one workgroup each.
+__global__ void __launch_bounds__(256) k_end(Dev d) { end_member(d, (int)blockIdx.x); }
+
+// The same, and begins the next step: the steps without nucleation, and those
+// whose energies are recomputed before it.
+__global__ void __launch_bounds__(256) k_begin(Dev d, int rescale_flipped) {
+    end_member(d, (int)blockIdx.x);
+    begin_member(d, (int)blockIdx.x, rescale_flipped != 0);
+}
 
 // ---------------------------------------------------------------------
 // calculus.h: lengths, energies, areas, velocities, translation
@@ -322,8 +326,9 @@ __device__ __forceinline__ void analytic_force(const Dev& d, const Params& P, in
 // the two list neighbours and every other delta is shared.  Each track is
 // still the reference's sequential sum U_i = U_{i-1} + delta_i, and each
 // area the reference's left-to-right shoelace sum, so the results are
-// bit-identical.  Pass 2 sends vertices with dom_mod(x) != x or
-// dom_mod(y) != y to the two-pass path, which this form does not cover.
+// bit-identical.  A vertex with dom_mod(x) != x or dom_mod(y) != y (a
+// coordinate equal to D), where the other coordinate moves too, has its two
+// areas formed from the points themselves.
 //
 // The (grain, slot) pairs of the shifted areas are dealt to the lanes in
 // order of their loop length after slot k, n - k (then grain), so that the
@@ -332,7 +337,7 @@ __device__ __forceinline__ void analytic_force(const Dev& d, const Params& P, in
 // the tile's grains with at least n - k entries).
 constexpr int kTilePts = 448;   // with the per-slot and per-grain arrays: 8 workgroups of 256 per CU
 static_assert(kTilePts >= kMaxStride, "a tile must hold the longest grain list");
-__global__ void __launch_bounds__(256) k_vel_grain(Dev d, int tuning) {
+__global__ void __launch_bounds__(256, 8) k_vel_grain(Dev d, int tuning) {
     __shared__ double2 Ps[kTilePts];
     __shared__ double2 Ds[kTilePts];        // wrap(P_k - P_{k-1}) of list slot k > 0
     __shared__ int Ls[kTilePts];
@@ -474,51 +479,73 @@ __global__ void __launch_bounds__(256) k_vel_grain(Dev d, int tuning) {
             const int v = Ls[p];
             const double x = Ps[p].x, y = Ps[p].y;
             const double px = dom_mod(x + SEVC_GRAD_EPS, D), qy = dom_mod(y + SEVC_GRAD_EPS, D);
-            // the unshifted track up to U_{k-1}, with the sum a of
-            // U_i x U_{i+1} for i <= k - 2 (both shifted polygons share it)
-            double ux = 0, uy = 0, a = 0;
-            for (int i = 1; i < k; i++) {
-                const double2 di = Ds[b0 + i];
-                const double nx = ux + di.x, ny = uy + di.y;
-                a += ux * ny - uy * nx;
-                ux = nx;
-                uy = ny;
-            }
-            // index k: the x-shifted polygon's point (xX, Y_k), the
-            // y-shifted one's (X_k, yY); index k + 1: deltas from the shifted
-            // point; later the shared deltas
-            double sx = a, sy = a, xX = 0, yY = 0;
-            if (k > 0) {
-                const double ex = wrapd(px, Ps[p - 1].x, D), ey = wrapd(qy, Ps[p - 1].y, D);
-                const double2 dk = Ds[p];
-                const double nx = ux + dk.x, ny = uy + dk.y;
-                xX = ux + ex;
-                yY = uy + ey;
-                sx += ux * ny - uy * xX;
-                sy += ux * yY - uy * nx;
-                ux = nx;
-                uy = ny;
-            }
-            if (k + 1 < n) {
-                const double ex1 = wrapd(Ps[p + 1].x, px, D), ey1 = wrapd(Ps[p + 1].y, qy, D);
-                const double2 d1 = Ds[p + 1];
-                const double nx = ux + d1.x, ny = uy + d1.y;
-                const double nxX = xX + ex1, nyY = yY + ey1;
-                sx += xX * ny - uy * nxX;
-                sy += ux * nyY - yY * nx;
-                ux = nx; uy = ny; xX = nxX; yY = nyY;
-                for (int i = k + 2; i < n; i++) {
-                    const double2 di = Ds[b0 + i];
-                    const double nx2 = ux + di.x, ny2 = uy + di.y;
-                    const double nxX2 = xX + di.x, nyY2 = yY + di.y;
-                    sx += xX * ny2 - uy * nxX2;
-                    sy += ux * nyY2 - yY * nx2;
-                    ux = nx2; uy = ny2; xX = nxX2; yY = nyY2;
+            const double pyy = dom_mod(y, D), qx = dom_mod(x, D);
+            double sx, sy;
+            if (!(pyy == y && qx == x)) {
+                // a coordinate that dom_mod moves (equal to D: rare): the two
+                // shifted polygons from their points, one after the other
+                sx = sy = 0.0;
+#pragma unroll 1
+                for (int c = 0; c < 2; c++) {
+                    const double vx = c == 0 ? px : qx, vy = c == 0 ? pyy : qy;
+                    AreaAcc acc;
+                    acc.start(k == 0 ? vx : Ps[b0].x, k == 0 ? vy : Ps[b0].y);
+#pragma unroll 1
+                    for (int i = 1; i < n; i++) acc.push(i == k ? vx : Ps[b0 + i].x, i == k ? vy : Ps[b0 + i].y, D);
+                    const double z = 0;
+                    acc.area += acc.ux * z - acc.uy * z;
+                    if (c == 0) sx = acc.area;
+                    else sy = acc.area;
                 }
+            } else {
+                // the unshifted track up to U_{k-1}, with the sum a of
+                // U_i x U_{i+1} for i <= k - 2 (both shifted polygons share it)
+                double ux = 0, uy = 0, a = 0;
+                for (int i = 1; i < k; i++) {
+                    const double2 di = Ds[b0 + i];
+                    const double nx = ux + di.x, ny = uy + di.y;
+                    a += ux * ny - uy * nx;
+                    ux = nx;
+                    uy = ny;
+                }
+                // index k: the x-shifted polygon's point (xX, Y_k), the
+                // y-shifted one's (X_k, yY); index k + 1: deltas from the shifted
+                // point; later the shared deltas
+                double xX = 0, yY = 0;
+                sx = a;
+                sy = a;
+                if (k > 0) {
+                    const double ex = wrapd(px, Ps[p - 1].x, D), ey = wrapd(qy, Ps[p - 1].y, D);
+                    const double2 dk = Ds[p];
+                    const double nx = ux + dk.x, ny = uy + dk.y;
+                    xX = ux + ex;
+                    yY = uy + ey;
+                    sx += ux * ny - uy * xX;
+                    sy += ux * yY - uy * nx;
+                    ux = nx;
+                    uy = ny;
+                }
+                if (k + 1 < n) {
+                    const double ex1 = wrapd(Ps[p + 1].x, px, D), ey1 = wrapd(Ps[p + 1].y, qy, D);
+                    const double2 d1 = Ds[p + 1];
+                    const double nx = ux + d1.x, ny = uy + d1.y;
+                    const double nxX = xX + ex1, nyY = yY + ey1;
+                    sx += xX * ny - uy * nxX;
+                    sy += ux * nyY - yY * nx;
+                    ux = nx; uy = ny; xX = nxX; yY = nyY;
+                    for (int i = k + 2; i < n; i++) {
+                        const double2 di = Ds[b0 + i];
+                        const double nx2 = ux + di.x, ny2 = uy + di.y;
+                        const double nxX2 = xX + di.x, nyY2 = yY + di.y;
+                        sx += xX * ny2 - uy * nxX2;
+                        sy += ux * nyY2 - yY * nx2;
+                        ux = nx2; uy = ny2; xX = nxX2; yY = nyY2;
+                    }
+                }
+                const double z = 0;
+                sx += xX * z - uy * z;
+                sy += ux * z - yY * z;
             }
-            const double z = 0;
-            sx += xX * z - uy * z;
-            sy += ux * z - yY * z;
             const double ax = sx * 0.5, ay = sy * 0.5;
             const double a0 = fabs(area_s[g]), se = se_s[g];
             const double tx = se * (fabs(ax) - a0), ty = se * (fabs(ay) - a0);
@@ -785,7 +812,7 @@ __global__ void __launch_bounds__(64) k_vel_bigrain(Dev d, int tuning) {
 
 // A vertex for the two-pass velocity (k_velocity_fallback).  Each vertex is
 // listed at most once per step (the list holds V entries; the counter is
-// cleared by k_begin); timing launches of the autotuner list nothing.
+// cleared when the next step begins); timing launches of the autotuner list nothing.
 __device__ __forceinline__ void push_vfall(const Dev& d, int v) {
     const int s = atomicAdd(&d.cnt[C_VFALL], 1);
     if (s < d.V) d.l_vfall[s] = v;
@@ -794,10 +821,11 @@ __device__ __forceinline__ void push_vfall(const Dev& d, int v) {
 // Velocity, pass 2 of 2: the line-tension part of energy_diff
 // (calculus.h:28-37,57-60) -- six shifted lengths -- plus the three
 // stored-energy terms of pass 1 summed in vertex.grains order, then
-// v = -dE/grad_eps * mobility (calculus.h:149-150).  Vertices whose
-// unshifted coordinate dom_mod would move (a coordinate equal to D) are
-// listed for the two-pass path.
-__global__ void __launch_bounds__(256) k_vel_vertex(Dev d, int tuning) {
+// v = -dE/grad_eps * mobility (calculus.h:149-150).  With `listed` set (the
+// lane-per-grain pass 1), vertices whose unshifted coordinate dom_mod would
+// move (a coordinate equal to D) are listed for the two-pass path, which that
+// pass 1 leaves them to; k_vel_grain covers them.
+__global__ void __launch_bounds__(256) k_vel_vertex(Dev d, int tuning, int listed) {
     TABLE_BLOCK(d.vblk, d.nvb)
     const int v = i;
     const bool in = i < bd_.e;
@@ -825,7 +853,7 @@ __global__ void __launch_bounds__(256) k_vel_vertex(Dev d, int tuning) {
     const double x = p.x, y = p.y;
     const double px = dom_mod(x + SEVC_GRAD_EPS, D), pyy = dom_mod(y, D);
     const double qx = dom_mod(x, D), qy = dom_mod(y + SEVC_GRAD_EPS, D);
-    if (!((pyy == y) && (qx == x))) {
+    if (listed && !((pyy == y) && (qx == x))) {
         if (!tuning) push_vfall(d, v);
         return;
     }
@@ -1315,6 +1343,7 @@ __global__ void k_text(Dev d) {
     __shared__ int wcnt[kBlock / 64], bbase;
     const int lb_ = xcd_remap((int)blockIdx.x, (int)gridDim.x);
     if (lb_ >= d.neb) return;
+    if (lb_ == 0 && threadIdx.x == 0) *d.n_flipped = 0;   // read by begin_member, filled by the flips
     const Blk bd_ = table_blk(d, d.eblk, lb_);
     const Params& P = d.prm[bd_.m];
     MState& M = d.ms[bd_.m];
@@ -1363,7 +1392,7 @@ __global__ void k_text(Dev d) {
     unsigned long long r = wmin[0];
 #pragma unroll
     for (int w = 1; w < kBlock / 64; w++) r = wmin[w] < r ? wmin[w] : r;
-    // the member's minimum (k_begin set it to +inf): the smallest value
+    // the member's minimum (begin_member set it to +inf): the smallest value
     // whatever the order, so the result equals a serial scan; a block
     // whose minimum is not below the value already there skips the atomic
     const unsigned long long seen = M.tau_bits;
@@ -2426,7 +2455,12 @@ __device__ __forceinline__ void poll_stage(const Dev& d, int nc, unsigned char* 
     for (int m = (int)threadIdx.x; m < d.B; m += (int)blockDim.x)
         if (d.ms[m].active && d.prm[m].events) d.ms[m].lab_dt = member_dt(d.prm[m], d.ms[m]);
     if (nc > 0) poll_list(d, nc, pbuf);
-    if (threadIdx.x == 0) atomicExch(&d.cnt[C_TRI], 0);
+    if (threadIdx.x == 0) {
+        atomicExch(&d.cnt[C_TRI], 0);
+        d.cnt[C_NEV] = 0;
+        d.cnt[C_NUCL] = 0;
+        d.cnt[C_RAN] = 1;
+    }
     if (cnt_now(d, C_TWO) > 0) {
         __syncthreads();
         if (threadIdx.x == 0) two_grain_serial(d);
@@ -2848,7 +2882,7 @@ __device__ __forceinline__ void flip(const Dev& d, int bnd, const Params& P, con
     }
     d.ben[bnd] = e;
     {
-        // rescaled at the next step's start (k_begin) when no full pass runs
+        // rescaled at the next step's start (begin_member) when no full pass runs
         const int k = wave_slot(d.n_flipped, true);
         if (k < d.E) d.l_flipped[k] = bnd;
     }
@@ -3072,6 +3106,8 @@ struct NuclGeom {
 };
 
 // generate_grain_for_nucleation, nucleation2.cu:116-212
+// (kEnergy: with dE, which the insertion does not use)
+template <bool kEnergy>
 __device__ __forceinline__ int generate_grain(const Dev& d, const Params& P, int A, double eps, double scaling, int do_scale,
                               NuclGeom* r) {
     const double Dm = P.D;
@@ -3104,6 +3140,7 @@ __device__ __forceinline__ int generate_grain(const Dev& d, const Params& P, int
         out[k][0] = dom_mod(px, Dm);
         out[k][1] = dom_mod(py, Dm);
     }
+    if (!kEnergy) return 0;
     double LAB = arclen(r->Apos[0], r->Apos[1], r->Bpos[0], r->Bpos[1], Dm);
     double LBC = arclen(r->Bpos[0], r->Bpos[1], r->Cpos[0], r->Cpos[1], Dm);
     double LCA = arclen(r->Cpos[0], r->Cpos[1], r->Apos[0], r->Apos[1], Dm);
@@ -3147,9 +3184,9 @@ __device__ __forceinline__ void nucl_factor_at(const Dev& d, const Params& P, co
     d.nucl_ori[v] = 2 * SEVC_PI * u1;
     NuclGeom g0, g1;
     double de = 0.0, de_ = 0.0;
-    if (generate_grain(d, P, v, P.gb_eps, P.gb_scaling, 0, &g0) == 0) de = g0.dE;
+    if (generate_grain<true>(d, P, v, P.gb_eps, P.gb_scaling, 0, &g0) == 0) de = g0.dE;
     d.dE[v] = de;
-    if (generate_grain(d, P, v, P.gb_eps, P.gb_scaling, 1, &g1) == 0) de_ = g1.dE;
+    if (generate_grain<true>(d, P, v, P.gb_eps, P.gb_scaling, 1, &g1) == 0) de_ = g1.dE;
     d.nfac[v] = de - de_;
 }
 
@@ -3159,26 +3196,18 @@ __device__ __forceinline__ void nucl_factor_at(const Dev& d, const Params& P, co
 // list entry floor(u1 * n) of the grain; the candidate's record holds the
 // site (-1 when its shortest boundary has zero length: no candidate), the
 // site's three grains and that shortest length.
-// One grain table block of the rate mode's candidate draw.  It runs in the
-// launch of the step's begin (k_begin_rate), so it decides whether its
-// member runs and nucleates from the loop state itself, by the same rules
-// (member_runs, rate_nucleates) that the begin workgroup writes into it.
-__device__ __forceinline__ void rate_cand_block(const Dev& d, int lb) {
-    const Blk bd_ = table_blk(d, d.gblk, lb);
-    const Params& P = d.prm[bd_.m];
-    const MState& M = d.ms[bd_.m];
-    const int i = bd_.b + (int)threadIdx.x;
-    // the grain's data is loaded together with the member's state
-    const bool in = i < bd_.e;
-    const uint8_t en = in ? d.genab[i] : 0;
-    const int len = in ? d.glen[i] : 0;
-    const double se = in ? d.gse[i] : 0.0;
-    if (!member_runs(P, M) || !rate_nucleates(P, M)) return;
-    if (!en || len < 1) return;
+// rate_cand draws for grain i (its flag, list length and SE given) in step n.
+struct RateCand {
+    int site, g[3];
+    double al;
+};
+__device__ __forceinline__ bool rate_cand(const Dev& d, const Params& P, int n, int i, uint8_t en, int len, double se,
+                                          RateCand* c) {
+    if (!en || len < 1) return false;
     double p = P.nucl_rate * se;
     double u0, u1;
-    sevc_uniform2(P.seed, (uint32_t)M.n, (uint32_t)(i - P.goff), kStreamRate, 0u, &u0, &u1);
-    if (!(u0 < p)) return;
+    sevc_uniform2(P.seed, (uint32_t)n, (uint32_t)(i - P.goff), kStreamRate, 0u, &u0, &u1);
+    if (!(u0 < p)) return false;
     int k = (int)(u1 * (double)len);
     if (k >= len) k = len - 1;
     const int A = glist(d, i)[k];
@@ -3189,24 +3218,37 @@ __device__ __forceinline__ void rate_cand_block(const Dev& d, int lb) {
 #pragma unroll
     for (int q = 0; q < 3; q++) al[q] = edge_len_from(d, vb[q], A, P.D);
     double minAL = al[0];
-    for (int q = 0; q < 3; q++) if (minAL > al[q]) minAL = al[q];
-    const int s = wave_slot(&d.cnt[C_NUCL], true);
-    d.l_nucl[s] = i;
-    d.nrec[4 * s] = (minAL > 0) ? A : -1;
 #pragma unroll
-    for (int q = 0; q < 3; q++) d.nrec[4 * s + 1 + q] = vg[q];
-    d.nal[s] = minAL;
+    for (int q = 0; q < 3; q++) if (minAL > al[q]) minAL = al[q];
+    c->site = (minAL > 0) ? A : -1;
+#pragma unroll
+    for (int q = 0; q < 3; q++) c->g[q] = vg[q];
+    c->al = minAL;
+    return true;
 }
 
-// The step's begin (workgroup 0, dispatched first) and the rate mode's
-// candidate draw (one workgroup per grain table block) in one launch.
-__global__ void __launch_bounds__(kBlock) k_begin_rate(Dev d, int rescale_flipped) {
-    if (blockIdx.x == 0) {
-        begin_members(d, rescale_flipped);
-        return;
-    }
-    const int lb = xcd_remap((int)blockIdx.x - 1, (int)gridDim.x - 1);
-    if (lb < d.ngb) rate_cand_block(d, lb);
+__device__ __forceinline__ void put_cand(const Dev& d, int s, int i, const RateCand& c) {
+    d.l_nucl[s] = i;
+    *reinterpret_cast<int4*>(d.nrec + 4 * (size_t)s) = make_int4(c.site, c.g[0], c.g[1], c.g[2]);
+    d.nal[s] = c.al;
+}
+
+// The draw over all grains for the states whose members are too large for
+// k_head to draw itself.  It runs before the step begins, while the last one
+// may still be open, so the step's number is worked out here, and whether the
+// member runs at all is left to k_head, which then drops the candidates.
+__global__ void __launch_bounds__(kBlock) k_rate_draw(Dev d) {
+    TABLE_BLOCK(d.gblk, d.ngb)
+    // the grain's data is loaded together with the member's state
+    const bool in = i < bd_.e;
+    const uint8_t en = in ? d.genab[i] : 0;
+    const int len = in ? d.glen[i] : 0;
+    const double se = in ? d.gse[i] : 0.0;
+    const int n = M.n + (M.open && M.active ? 1 : 0);
+    if (M.done || !rate_nucleates(P, n)) return;
+    RateCand c;
+    if (!rate_cand(d, P, n, i, en, len, se, &c)) return;
+    put_cand(d, wave_slot(&d.cnt[C_NUCL], true), i, c);
 }
 
 // Exclusive prefix sum of one int per thread over the workgroup: an
@@ -3497,15 +3539,27 @@ __device__ __forceinline__ int find_kth(const Blk* tbl, const RunScan& rs, const
     return f;
 }
 
-// One workgroup per member: picks the nucleation events of this step and
-// assigns their free slots; k_nucl_insert applies them.
-//  MC mode (nucleation2.cu:292-443, 33-72, 474): one uniformly chosen alive
-//  vertex, Metropolis acceptance, first free grain / 3 boundaries / 2
-//  vertices.
-//  RATE mode: candidates in grain order; a candidate is dropped when an
-//  earlier candidate's site shares a grain with it; kept events take the
-//  free slots in rank order.  Kept events are grain-disjoint, so they can
-//  be applied in parallel.
+// The head of a step, one workgroup per member, as `what` asks:
+//  HEAD_BEGIN   sums up the last step and begins this one (end_member,
+//               begin_member; HEAD_RESCALE: with the flipped edges' energies);
+//  HEAD_SELECT  picks the nucleation events of this step and assigns their
+//               free slots:
+//   MC mode (nucleation2.cu:292-443, 33-72, 474): one uniformly chosen alive
+//   vertex, Metropolis acceptance, first free grain / 3 boundaries / 2
+//   vertices.
+//   RATE mode: candidates in grain order; a candidate is dropped when an
+//   earlier candidate's site shares a grain with it; kept events take the
+//   free slots in rank order.  Kept events are grain-disjoint, so they can
+//   be applied in parallel.
+//  HEAD_DRAW    draws the rate mode's candidates itself (else k_rate_draw has
+//               listed them);
+//  HEAD_INSERT  applies the events, a wave each (else they are listed for
+//               k_nucl_insert).
+// Each part was a launch of its own (3 to 4.5 us, with cold caches).  A
+// member's draw by its one workgroup costs 0.6 us per 1,024 grains, so
+// members above kHeadGrains leave it to k_rate_draw; six events are applied at
+// a time in about 8 us, so states that expect more than kHeadEvents in a member
+// leave them to k_nucl_insert.
 // Scratch: 12 ints per grain slot of the member, at 12*goff in d.nscr:
 //  [0,ng) candidates, [ng,4ng) their site grains, [4ng,5ng) kept sites,
 //  [5ng,6ng) free grains, [6ng,9ng) free boundaries, [9ng,11ng) free
@@ -3518,18 +3572,271 @@ constexpr int kSlotLds = 1024;       // listed blocks of the free-slot search he
 
 __device__ __forceinline__ int nucl_hash(int g) { return (int)(((unsigned)g * 2654435761u) >> 20); }
 
-__global__ void __launch_bounds__(kNuclThreads) k_nucl_manager(Dev d) {
+// The selection's arrays, and in their place (they are read no more by then)
+// the staging rooms of the insertions.
+struct SelectLds {
+    int c[kNuclLds], site[kNuclLds], sg[3 * kNuclLds], k[kNuclLds], q[kNuclLds];
+    double al[kNuclLds];                      // shortest edge at each candidate's site
+    int hk[kNuclHash], hv[kNuclHash];
+};
+
+// nucleate (nucleation2.cu:474-676, after its checks) for one event, by one
+// wave, followed by the recomputation of main.cu:171-177 restricted to what an
+// event changes: the lengths and energies (calculus.h:83-114) of its six
+// boundaries and the areas (:224-234) of its four grains.  Events are
+// grain-disjoint: no event reads a vertex, boundary or grain list another one
+// writes, so they run concurrently, and each event's refresh reads only its
+// own writes.  The lists of the three grains at the site are staged in LDS
+// with one round of loads; the edits of grain_add_vertex and
+// grain_remove_vertex (geometry.h:629-666) are applied to the staged copies in
+// the reference's order (a grain named twice keeps one copy, so the edits
+// compose), each by the whole wave, and written back.  The new slots were
+// found free, so their flags are not read.
+struct InsertLds {
+    int Ls[3][kMaxStride];
+    int n_s[3];
+    double sdx[4][kMaxStride], sdy[4][kMaxStride];
+};
+
+__device__ __forceinline__ void insert_event(const Dev& d, int m, int A, int B, int C, int AB, int BC, int CA, int g,
+                                             InsertLds& lds) {
+    auto& Ls = lds.Ls;
+    auto& n_s = lds.n_s;
+    auto& sdx = lds.sdx;
+    auto& sdy = lds.sdy;
+    const int lane = (int)threadIdx.x & 63;
+    const Params& P = d.prm[m];
+    NuclGeom r;
+    // nucleation2.cu:526 passes (scaling, eps) swapped; only dE is affected
+    if (generate_grain<false>(d, P, A, P.gb_scaling, P.gb_eps, 1, &r) != 0) return;
+    const int gl[3] = {r.g1, r.g2, r.g3};
+    int sl[3];
+    sl[0] = 0;
+    sl[1] = gl[1] == gl[0] ? 0 : 1;
+    sl[2] = gl[2] == gl[0] ? 0 : (gl[2] == gl[1] ? sl[1] : 2);
+    int n_old[3];
+#pragma unroll
+    for (int t = 0; t < 3; t++) n_old[t] = sl[t] == t ? d.glen[gl[t]] : 0;
+#pragma unroll
+    for (int t = 0; t < 3; t++) {
+        if (sl[t] != t) continue;
+        const int* L = glist(d, gl[t]);
+        for (int i = lane; i < n_old[t]; i += 64) Ls[t][i] = L[i];
+    }
+    // what the serial edits below read, loaded with the lists (nothing
+    // writes these entries before they are read)
+    int vgA[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) vgA[k] = d.vg[3 * A + k];
+    const int ae0 = d.bvx[2 * r.AE], ae1 = d.bvx[2 * r.AE + 1], af0 = d.bvx[2 * r.AF];
+    if (lane == 0) { n_s[0] = n_old[0]; n_s[1] = n_old[1]; n_s[2] = n_old[2]; }
+    wave_sync();
+    const int S = P.cap;
+    auto find = [&](int t, int n, int v) {                      // first place of v, -1 if none
+        for (int i0 = 0; i0 < n; i0 += 64) {
+            const unsigned long long hit = __ballot(i0 + lane < n && Ls[t][min(i0 + lane, kMaxStride - 1)] == v);
+            if (hit) return i0 + __ffsll((long long)hit) - 1;
+        }
+        return -1;
+    };
+    // moves the entries from place `lo` on by `by` places
+    auto shift = [&](int t, int lo, int n, int by) {
+        int x[kMaxStride / 64];
+#pragma unroll
+        for (int q = 0; q < kMaxStride / 64; q++) x[q] = lo + lane + 64 * q < n ? Ls[t][lo + lane + 64 * q] : -1;
+        wave_sync();
+#pragma unroll
+        for (int q = 0; q < kMaxStride / 64; q++)
+            if (lo + lane + 64 * q < n) Ls[t][lo + lane + 64 * q + by] = x[q];
+    };
+    auto ladd = [&](int t, int v, int prev) {                   // grain_add_vertex
+        const int n = n_s[t], pos = find(t, n, prev) + 1;
+        const int err = pos == 0 ? SEVC_E_STATE : (n >= S ? SEVC_E_GRAIN_FULL : 0);
+        if (err) {
+            if (lane == 0) set_error(d, m, err);
+            return;
+        }
+        shift(t, pos, n, 1);
+        if (lane == 0) {
+            Ls[t][pos] = v;
+            n_s[t] = n + 1;
+        }
+        wave_sync();
+    };
+    auto lremove = [&](int t, int v) {                          // grain_remove_vertex
+        const int n = n_s[t], pos = find(t, n, v);
+        if (pos < 0) return;
+        shift(t, pos + 1, n, -1);
+        if (lane == 0) n_s[t] = n - 1;
+        wave_sync();
+    };
+    ladd(sl[0], C, A);
+    if (ae0 == A) ladd(sl[1], B, ae1);
+    else if (ae1 == A) ladd(sl[1], B, ae0);
+    ladd(sl[2], C, A);
+    ladd(sl[2], B, C);
+    lremove(sl[2], A);
+    if (lane == 0) {
+        // init_vertex (geometry.h:346-361) for B and C
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            const int v = q == 0 ? B : C;
+            d.pos[2 * v] = q == 0 ? r.Bpos[0] : r.Cpos[0];
+            d.pos[2 * v + 1] = q == 0 ? r.Bpos[1] : r.Cpos[1];
+            d.vel[2 * v] = 0.0; d.vel[2 * v + 1] = 0.0;
+            d.venergy[v] = 0.0;
+            set_vertex_enabled(d, v, false, true);
+            d.vnuc[v] = 0;
+            reset_mods(d, v);
+        }
+        d.pos[2 * A] = r.Apos[0]; d.pos[2 * A + 1] = r.Apos[1];
+        // init_boundary (geometry.h:491-504) for AB, BC, CA and the
+        // boundary slots they and AD, AE, AF take at A, B, C: each
+        // vertex's table was cleared, so add_boundary fills it in order
+        // (vb[A] = AB, CA, AD; vb[B] = AB, BC; vb[C] = BC, CA), after
+        // which the reference swaps the first two slots of B and C and
+        // puts AE, AF third
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+            const int b = q == 0 ? AB : (q == 1 ? BC : CA);
+            d.bvx[2 * b] = q == 0 ? A : (q == 1 ? B : C);
+            d.bvx[2 * b + 1] = q == 0 ? B : (q == 1 ? C : A);
+            d.blen[b] = 0;
+            d.bt[b] = SEVC_MAX_T_EXT;
+            set_edge_enabled(d, b, false, true);
+            d.bcand[b] = 0;
+            d.conf[b] = -1;
+        }
+        d.vb[3 * A] = AB; d.vb[3 * A + 1] = CA; d.vb[3 * A + 2] = r.AD;
+        d.vb[3 * B] = BC; d.vb[3 * B + 1] = AB; d.vb[3 * B + 2] = r.AE;
+        d.vb[3 * C] = CA; d.vb[3 * C + 1] = BC; d.vb[3 * C + 2] = r.AF;
+        // nucleate_grain (geometry.h:596-606); its list is written below
+        d.glen[g] = 3;
+        d.garea[g] = 0;
+        d.gse[g] = 0;
+        set_grain_enabled(d, g, false, true);
+        d.gcand[g] = 0;
+        d.gfix[g] = 0;
+        d.gtype[g] = T_NUCLEATED;
+        d.gori[g] = d.nucl_ori[A];
+        {
+            const int k = vgA[0] == r.g3 ? 0 : (vgA[1] == r.g3 ? 1 : (vgA[2] == r.g3 ? 2 : -1));
+            if (k >= 0) d.vg[3 * A + k] = g;
+        }
+        d.vg[3 * B] = g; d.vg[3 * B + 1] = r.g2; d.vg[3 * B + 2] = r.g3;
+        d.vg[3 * C] = g; d.vg[3 * C + 1] = r.g3; d.vg[3 * C + 2] = r.g1;
+        if (ae0 == A) d.bvx[2 * r.AE] = B;
+        else if (ae1 == A) d.bvx[2 * r.AE + 1] = B;
+        if (af0 == A) d.bvx[2 * r.AF] = C;
+        else d.bvx[2 * r.AF + 1] = C;
+        atomicAdd((unsigned long long*)&d.ms[m].nucl, 1ull);
+    }
+    wave_sync();
+    // write the edited lists back (-1 after the end, as the reference's
+    // removal leaves) and the new grain's list
+#pragma unroll
+    for (int t = 0; t < 3; t++) {
+        if (sl[t] != t) continue;
+        const int n_new = n_s[t];
+        int* L = glist(d, gl[t]);
+        for (int i = lane; i < max(n_old[t], n_new); i += 64) L[i] = i < n_new ? Ls[t][i] : -1;
+        if (lane == 0) {
+            d.glen[gl[t]] = n_new;
+            if (n_new == 3) list_tri(d, gl[t], true);
+        }
+    }
+    if (lane == 0) list_tri(d, g, true);
+    {
+        int* Lg = glist(d, g);
+        for (int i = lane; i < d.S; i += 64) Lg[i] = i == 0 ? A : (i == 1 ? B : (i == 2 ? C : -1));
+    }
+    wave_sync();
+    // refresh: the six boundaries (lanes 0-5), then the areas of g1, g2,
+    // g3 and g from the wrapped deltas of their lists, summed in list
+    // order by lanes 0-3 as grain_area does
+    const double Dm = P.D;
+    if (lane < 6) {
+        // the six edges and their ends' positions after the event: AB, BC,
+        // CA between the new vertices, AD at A, AE rewired to B, AF to C
+        // (arclen gives the same bits in either end order)
+        const int b = lane == 0 ? AB : lane == 1 ? BC : lane == 2 ? CA : lane == 3 ? r.AD : lane == 4 ? r.AE : r.AF;
+        // by selection (no pointer into r, which would put it in scratch)
+        const bool a0 = lane == 0 || lane == 3, b0 = lane == 1 || lane == 4;
+        const double x0 = a0 ? r.Apos[0] : (b0 ? r.Bpos[0] : r.Cpos[0]);
+        const double y0 = a0 ? r.Apos[1] : (b0 ? r.Bpos[1] : r.Cpos[1]);
+        const double x1 = lane == 0 ? r.Bpos[0] : lane == 1 ? r.Cpos[0] : lane == 2 ? r.Apos[0]
+                        : lane == 3 ? r.Dpos[0] : lane == 4 ? r.Epos[0] : r.Fpos[0];
+        const double y1 = lane == 0 ? r.Bpos[1] : lane == 1 ? r.Cpos[1] : lane == 2 ? r.Apos[1]
+                        : lane == 3 ? r.Dpos[1] : lane == 4 ? r.Epos[1] : r.Fpos[1];
+        d.blen[b] = arclen(x0, y0, x1, y1, Dm);
+        const double e = (P.gb_eps == 0.0) ? 1.0 : boundary_compute_energy(d, b, P.gb_eps);
+        d.ben[b] = e * P.gb_scaling;
+    }
+#pragma unroll
+    for (int t = 0; t < 3; t++) {
+        const int n = n_s[sl[t]];
+        for (int i = 1 + lane; i < n; i += 64) {
+            const int w = Ls[sl[t]][i], wp = Ls[sl[t]][i - 1];
+            sdx[t][i] = wrapd(d.pos[2 * w], d.pos[2 * wp], Dm);
+            sdy[t][i] = wrapd(d.pos[2 * w + 1], d.pos[2 * wp + 1], Dm);
+        }
+    }
+    if (lane < 2) {                                  // g: A, B, C
+        const int w = lane == 0 ? B : C, wp = lane == 0 ? A : B;
+        sdx[3][1 + lane] = wrapd(d.pos[2 * w], d.pos[2 * wp], Dm);
+        sdy[3][1 + lane] = wrapd(d.pos[2 * w + 1], d.pos[2 * wp + 1], Dm);
+    }
+    wave_sync();
+    if (lane < 4) {
+        const int t = lane;
+        const int gg = t == 0 ? gl[0] : (t == 1 ? gl[1] : (t == 2 ? gl[2] : g));
+        const int st = t == 0 ? sl[0] : (t == 1 ? sl[1] : sl[2]);
+        const int n = t < 3 ? n_s[st] : 3;
+        if (d.genab[gg]) {
+            double a = 0.0;
+            if (n > 0) {
+                AreaAcc acc;
+                acc.start(0.0, 0.0);
+                for (int i = 1; i < n; i++) acc.push_delta(sdx[t][i], sdy[t][i]);
+                a = acc.finish();
+            }
+            d.garea[gg] = a;
+        }
+    }
+}
+
+// The events that the heads listed, one wave (workgroup of 64) each.
+__global__ void __launch_bounds__(64) k_nucl_insert(Dev d) {
+    __shared__ InsertLds lds;
+    const int n_ev = min(d.cnt[C_NEV], d.G);
+    for (int item = blockIdx.x; item < n_ev; item += gridDim.x) {
+        const int4 a = *reinterpret_cast<const int4*>(d.l_nev + 8 * (size_t)item);
+        const int4 b = *reinterpret_cast<const int4*>(d.l_nev + 8 * (size_t)item + 4);
+        insert_event(d, a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, lds);
+        wave_sync();
+    }
+}
+
+__global__ void __launch_bounds__(kNuclThreads) k_head(Dev d, int what) {
     __shared__ int sh[kNuclThreads + 1];
     __shared__ int nkeep, ncand, ev0;
-    __shared__ int c_s[kNuclLds], site_s[kNuclLds], sg_s[3 * kNuclLds], k_s[kNuclLds], q_s[kNuclLds];
-    __shared__ double al_s[kNuclLds];         // shortest edge at each candidate's site
-    __shared__ int hk[kNuclHash], hv[kNuclHash];
+    constexpr int kInsWaves = 6;
+    __shared__ union {
+        SelectLds sel;
+        InsertLds ins[kInsWaves];
+    } u;
+    int *const c_s = u.sel.c, *const site_s = u.sel.site, *const sg_s = u.sel.sg, *const k_s = u.sel.k,
+        *const q_s = u.sel.q, *const hk = u.sel.hk, *const hv = u.sel.hv;
+    double* const al_s = u.sel.al;
     __shared__ int4 bl_s[kSlotLds];
     __shared__ int fo_s[kSlotLds];            // the free slots found (grains, boundaries, vertices)
     const int m = blockIdx.x;
-    if (m >= d.B) return;
     const Params& P = d.prm[m];
     MState& M = d.ms[m];
+    if (what & HEAD_BEGIN) {
+        end_member(d, m);
+        begin_member(d, m, (what & HEAD_RESCALE) != 0);
+    }
     // a single member's block ranges are the whole tables
     const int gb0 = d.B == 1 ? 0 : d.gblk_first[m], gb1 = d.B == 1 ? d.ngb : d.gblk_first[m + 1];
     const int eb0 = d.B == 1 ? 0 : d.eblk_first[m], eb1 = d.B == 1 ? d.neb : d.eblk_first[m + 1];
@@ -3575,13 +3882,43 @@ __global__ void __launch_bounds__(kNuclThreads) k_nucl_manager(Dev d) {
         }
     } else {
         // this member's candidates (grain, list index), then grain order
-        const int total = d.cnt[C_NUCL];
-        for (int q = tid; q < total; q += nt) {
-            const int g = d.l_nucl[q];
-            if (g >= P.goff && g < P.goff + ng) {
-                const int e = atomicAdd(&ncand, 1);
-                cand[e] = g;
-                if (e < kNuclLds) { k_s[e] = g; q_s[e] = q; }
+        if (what & HEAD_DRAW) {
+            const int n = M.n;
+            for (int i0 = tid; i0 < ng; i0 += 4 * nt) {
+                uint8_t en[4];
+                int len[4];
+                double se[4];
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int i = P.goff + i0 + r * nt;
+                    const bool in = i0 + r * nt < ng;
+                    en[r] = in ? d.genab[i] : 0;
+                    len[r] = in ? d.glen[i] : 0;
+                    se[r] = in ? d.gse[i] : 0.0;
+                }
+#pragma unroll 1
+                for (int r = 0; r < 4; r++) {
+                    const int i = P.goff + i0 + r * nt;
+                    const uint8_t e_ = r == 0 ? en[0] : r == 1 ? en[1] : r == 2 ? en[2] : en[3];
+                    const int l_ = r == 0 ? len[0] : r == 1 ? len[1] : r == 2 ? len[2] : len[3];
+                    const double s_ = r == 0 ? se[0] : r == 1 ? se[1] : r == 2 ? se[2] : se[3];
+                    RateCand c;
+                    if (!rate_cand(d, P, n, i, e_, l_, s_, &c)) continue;
+                    const int e = atomicAdd(&ncand, 1), q = P.goff + e;
+                    cand[e] = i;
+                    put_cand(d, q, i, c);
+                    if (e < kNuclLds) { k_s[e] = i; q_s[e] = q; }
+                }
+            }
+        } else {
+            const int total = d.cnt[C_NUCL];
+            for (int q = tid; q < total; q += nt) {
+                const int g = d.l_nucl[q];
+                if (g >= P.goff && g < P.goff + ng) {
+                    const int e = atomicAdd(&ncand, 1);
+                    cand[e] = g;
+                    if (e < kNuclLds) { k_s[e] = g; q_s[e] = q; }
+                }
             }
         }
         __syncthreads();
@@ -3749,6 +4086,15 @@ __global__ void __launch_bounds__(kNuclThreads) k_nucl_manager(Dev d) {
     const int* fv = kinds[2].out;
     // event r needs grain slot r, boundary slots 3r..3r+2, vertex slots 2r, 2r+1
     const int n_ev = min(K, min(got[0], min(got[1] / 3, got[2] / 2)));
+    if (what & HEAD_INSERT) {
+        __syncthreads();
+        const int wave = tid >> 6;
+        if (wave < kInsWaves)
+            for (int r = wave; r < n_ev; r += kInsWaves)
+                insert_event(d, m, kept[r], fv[2 * r], fv[2 * r + 1], fe[3 * r], fe[3 * r + 1], fe[3 * r + 2], fg[r],
+                             u.ins[wave]);
+        return;
+    }
     if (tid == 0) ev0 = n_ev > 0 ? atomicAdd(&d.cnt[C_NEV], n_ev) : 0;
     __syncthreads();
     for (int r = tid; r < n_ev; r += nt) {
@@ -3761,207 +4107,6 @@ __global__ void __launch_bounds__(kNuclThreads) k_nucl_manager(Dev d) {
         ev[5] = fe[3 * r + 1];
         ev[6] = fe[3 * r + 2];
         ev[7] = fg[r];
-    }
-}
-
-// nucleate (nucleation2.cu:474-676, after its checks) for the events the
-// managers listed, one wave (workgroup of 64) per event, followed by the
-// recomputation of main.cu:171-177 restricted to what an event changes:
-// the lengths and energies (calculus.h:83-114) of its six boundaries and the
-// areas (:224-234) of its four grains.  Events are grain-disjoint: no event
-// reads a vertex, boundary or grain list another one writes, so they run
-// concurrently, and each event's refresh reads only its own writes.
-// The lists of the three grains at the site are staged in LDS with one
-// round of loads; lane 0 applies the edits of grain_add_vertex and
-// grain_remove_vertex (geometry.h:629-666) to the staged copies in the
-// reference's order (a grain named twice keeps one copy, so the edits
-// compose), and the wave writes them back.
-__global__ void __launch_bounds__(64) k_nucl_insert(Dev d) {
-    __shared__ int Ls[3][kMaxStride];
-    __shared__ int n_s[3];
-    __shared__ double sdx[4][kMaxStride], sdy[4][kMaxStride];
-    const int lane = threadIdx.x;
-    const int n_ev = min(d.cnt[C_NEV], d.G);
-    for (int item = blockIdx.x; item < n_ev; item += gridDim.x) {
-        const int* ev = d.l_nev + 8 * (size_t)item;
-        const int m = ev[0], A = ev[1], B = ev[2], C = ev[3], AB = ev[4], BC = ev[5], CA = ev[6], g = ev[7];
-        const Params& P = d.prm[m];
-        NuclGeom r;
-        // nucleation2.cu:526 passes (scaling, eps) swapped; only dE is affected
-        if (generate_grain(d, P, A, P.gb_scaling, P.gb_eps, 1, &r) != 0) continue;
-        const int gl[3] = {r.g1, r.g2, r.g3};
-        int sl[3];
-        sl[0] = 0;
-        sl[1] = gl[1] == gl[0] ? 0 : 1;
-        sl[2] = gl[2] == gl[0] ? 0 : (gl[2] == gl[1] ? sl[1] : 2);
-        int n_old[3];
-#pragma unroll
-        for (int t = 0; t < 3; t++) n_old[t] = sl[t] == t ? d.glen[gl[t]] : 0;
-#pragma unroll
-        for (int t = 0; t < 3; t++) {
-            if (sl[t] != t) continue;
-            const int* L = glist(d, gl[t]);
-            for (int i = lane; i < n_old[t]; i += 64) Ls[t][i] = L[i];
-        }
-        // what the serial edits below read, loaded with the lists (nothing
-        // writes these entries before they are read)
-        int vgA[3];
-#pragma unroll
-        for (int k = 0; k < 3; k++) vgA[k] = d.vg[3 * A + k];
-        const int ae0 = d.bvx[2 * r.AE], ae1 = d.bvx[2 * r.AE + 1], af0 = d.bvx[2 * r.AF];
-        if (lane == 0) { n_s[0] = n_old[0]; n_s[1] = n_old[1]; n_s[2] = n_old[2]; }
-        __syncthreads();
-        if (lane == 0) {
-            const int S = P.cap;
-            auto ladd = [&](int t, int v, int prev) {               // grain_add_vertex
-                const int n = n_s[t];
-                int pos = -1;
-                for (int i = 0; i < n; i++) if (Ls[t][i] == prev) { pos = i + 1; break; }
-                if (pos < 0) { set_error(d, m, SEVC_E_STATE); return; }
-                if (n >= S) { set_error(d, m, SEVC_E_GRAIN_FULL); return; }
-                for (int q = n; q > pos; q--) Ls[t][q] = Ls[t][q - 1];
-                Ls[t][pos] = v;
-                n_s[t] = n + 1;
-            };
-            auto lremove = [&](int t, int v) {                      // grain_remove_vertex
-                const int n = n_s[t];
-                for (int i = 0; i < n; i++)
-                    if (Ls[t][i] == v) {
-                        for (int j = i; j < n - 1; j++) Ls[t][j] = Ls[t][j + 1];
-                        n_s[t] = n - 1;
-                        return;
-                    }
-            };
-            // init_vertex (geometry.h:346-361) for B and C
-#pragma unroll
-            for (int q = 0; q < 2; q++) {
-                const int v = q == 0 ? B : C;
-                d.pos[2 * v] = q == 0 ? r.Bpos[0] : r.Cpos[0];
-                d.pos[2 * v + 1] = q == 0 ? r.Bpos[1] : r.Cpos[1];
-                d.vel[2 * v] = 0.0; d.vel[2 * v + 1] = 0.0;
-                d.venergy[v] = 0.0;
-                set_vertex_enabled(d, v, true);
-                d.vnuc[v] = 0;
-                reset_mods(d, v);
-            }
-            d.pos[2 * A] = r.Apos[0]; d.pos[2 * A + 1] = r.Apos[1];
-            // init_boundary (geometry.h:491-504) for AB, BC, CA and the
-            // boundary slots they and AD, AE, AF take at A, B, C: each
-            // vertex's table was cleared, so add_boundary fills it in order
-            // (vb[A] = AB, CA, AD; vb[B] = AB, BC; vb[C] = BC, CA), after
-            // which the reference swaps the first two slots of B and C and
-            // puts AE, AF third
-#pragma unroll
-            for (int q = 0; q < 3; q++) {
-                const int b = q == 0 ? AB : (q == 1 ? BC : CA);
-                d.bvx[2 * b] = q == 0 ? A : (q == 1 ? B : C);
-                d.bvx[2 * b + 1] = q == 0 ? B : (q == 1 ? C : A);
-                d.blen[b] = 0;
-                d.bt[b] = SEVC_MAX_T_EXT;
-                set_edge_enabled(d, b, true);
-                d.bcand[b] = 0;
-                d.conf[b] = -1;
-            }
-            d.vb[3 * A] = AB; d.vb[3 * A + 1] = CA; d.vb[3 * A + 2] = r.AD;
-            d.vb[3 * B] = BC; d.vb[3 * B + 1] = AB; d.vb[3 * B + 2] = r.AE;
-            d.vb[3 * C] = CA; d.vb[3 * C + 1] = BC; d.vb[3 * C + 2] = r.AF;
-            // nucleate_grain (geometry.h:596-606); its list is written below
-            d.glen[g] = 3;
-            d.garea[g] = 0;
-            d.gse[g] = 0;
-            set_grain_enabled(d, g, true);
-            d.gcand[g] = 0;
-            d.gfix[g] = 0;
-            d.gtype[g] = T_NUCLEATED;
-            d.gori[g] = d.nucl_ori[A];
-            for (int k = 0; k < 3; k++) if (vgA[k] == r.g3) { d.vg[3 * A + k] = g; break; }
-            d.vg[3 * B] = g; d.vg[3 * B + 1] = r.g2; d.vg[3 * B + 2] = r.g3;
-            d.vg[3 * C] = g; d.vg[3 * C + 1] = r.g3; d.vg[3 * C + 2] = r.g1;
-            ladd(sl[0], C, A);
-            if (ae0 == A) ladd(sl[1], B, ae1);
-            else if (ae1 == A) ladd(sl[1], B, ae0);
-            ladd(sl[2], C, A);
-            ladd(sl[2], B, C);
-            lremove(sl[2], A);
-            if (ae0 == A) d.bvx[2 * r.AE] = B;
-            else if (ae1 == A) d.bvx[2 * r.AE + 1] = B;
-            if (af0 == A) d.bvx[2 * r.AF] = C;
-            else d.bvx[2 * r.AF + 1] = C;
-            atomicAdd((unsigned long long*)&d.ms[m].nucl, 1ull);
-        }
-        __syncthreads();
-        // write the edited lists back (-1 after the end, as the reference's
-        // removal leaves) and the new grain's list
-#pragma unroll
-        for (int t = 0; t < 3; t++) {
-            if (sl[t] != t) continue;
-            const int n_new = n_s[t];
-            int* L = glist(d, gl[t]);
-            for (int i = lane; i < max(n_old[t], n_new); i += 64) L[i] = i < n_new ? Ls[t][i] : -1;
-            if (lane == 0) {
-                d.glen[gl[t]] = n_new;
-                if (n_new == 3) list_tri(d, gl[t], true);
-            }
-        }
-        if (lane == 0) list_tri(d, g, true);
-        {
-            int* Lg = glist(d, g);
-            for (int i = lane; i < d.S; i += 64) Lg[i] = i == 0 ? A : (i == 1 ? B : (i == 2 ? C : -1));
-        }
-        __syncthreads();
-        // refresh: the six boundaries (lanes 0-5), then the areas of g1, g2,
-        // g3 and g from the wrapped deltas of their lists, summed in list
-        // order by lanes 0-3 as grain_area does
-        const double Dm = P.D;
-        if (lane < 6) {
-            // the six edges and their ends' positions after the event: AB, BC,
-            // CA between the new vertices, AD at A, AE rewired to B, AF to C
-            // (arclen gives the same bits in either end order)
-            const int b = lane == 0 ? AB : lane == 1 ? BC : lane == 2 ? CA : lane == 3 ? r.AD : lane == 4 ? r.AE : r.AF;
-            // by selection (no pointer into r, which would put it in scratch)
-            const bool a0 = lane == 0 || lane == 3, b0 = lane == 1 || lane == 4;
-            const double x0 = a0 ? r.Apos[0] : (b0 ? r.Bpos[0] : r.Cpos[0]);
-            const double y0 = a0 ? r.Apos[1] : (b0 ? r.Bpos[1] : r.Cpos[1]);
-            const double x1 = lane == 0 ? r.Bpos[0] : lane == 1 ? r.Cpos[0] : lane == 2 ? r.Apos[0]
-                            : lane == 3 ? r.Dpos[0] : lane == 4 ? r.Epos[0] : r.Fpos[0];
-            const double y1 = lane == 0 ? r.Bpos[1] : lane == 1 ? r.Cpos[1] : lane == 2 ? r.Apos[1]
-                            : lane == 3 ? r.Dpos[1] : lane == 4 ? r.Epos[1] : r.Fpos[1];
-            d.blen[b] = arclen(x0, y0, x1, y1, Dm);
-            const double e = (P.gb_eps == 0.0) ? 1.0 : boundary_compute_energy(d, b, P.gb_eps);
-            d.ben[b] = e * P.gb_scaling;
-        }
-#pragma unroll
-        for (int t = 0; t < 3; t++) {
-            const int n = n_s[sl[t]];
-            for (int i = 1 + lane; i < n; i += 64) {
-                const int w = Ls[sl[t]][i], wp = Ls[sl[t]][i - 1];
-                sdx[t][i] = wrapd(d.pos[2 * w], d.pos[2 * wp], Dm);
-                sdy[t][i] = wrapd(d.pos[2 * w + 1], d.pos[2 * wp + 1], Dm);
-            }
-        }
-        if (lane < 2) {                                  // g: A, B, C
-            const int w = lane == 0 ? B : C, wp = lane == 0 ? A : B;
-            sdx[3][1 + lane] = wrapd(d.pos[2 * w], d.pos[2 * wp], Dm);
-            sdy[3][1 + lane] = wrapd(d.pos[2 * w + 1], d.pos[2 * wp + 1], Dm);
-        }
-        __syncthreads();
-        if (lane < 4) {
-            const int t = lane;
-            const int gg = t == 0 ? gl[0] : (t == 1 ? gl[1] : (t == 2 ? gl[2] : g));
-            const int st = t == 0 ? sl[0] : (t == 1 ? sl[1] : sl[2]);
-            const int n = t < 3 ? n_s[st] : 3;
-            if (d.genab[gg]) {
-                double a = 0.0;
-                if (n > 0) {
-                    AreaAcc acc;
-                    acc.start(0.0, 0.0);
-                    for (int i = 1; i < n; i++) acc.push_delta(sdx[t][i], sdy[t][i]);
-                    a = acc.finish();
-                }
-                d.garea[gg] = a;
-            }
-        }
-        __syncthreads();
     }
 }
 

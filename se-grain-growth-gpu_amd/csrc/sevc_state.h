@@ -22,8 +22,13 @@ constexpr int kPollBig = 16384;      // lists up to this length poll with flags 
 // edits fewer than kBusyUnder makes it calm (member_reduce): a calm state's
 // events run in one workgroup (k_events), a busy one's in a launch per stage.
 // The line is where both cost the same (see k_events).
+constexpr int kHeadGrains = 8192;    // largest member whose candidates k_head draws itself
+constexpr int kHeadEvents = 8;       // most nucleations a member may expect for k_head to apply them itself
 constexpr int kBusyOver = 320, kBusyUnder = 160;
 constexpr int kCountWaves = 4;       // table blocks per workgroup of k_count_all (one wave each)
+
+// What k_head does besides the nucleation's selection.
+enum { HEAD_BEGIN = 1, HEAD_SELECT = 2, HEAD_DRAW = 4, HEAD_INSERT = 8, HEAD_RESCALE = 16 };
 
 // Per-member run parameters (from sevc_options).
 struct Params {
@@ -41,6 +46,7 @@ struct Params {
 struct MState {
     int n, active, done, curr_grains, allow_nucl, nucl_now, status, n_venabled;
     int chk_phase;                   // phase of a failed check (debug_lvl >= 1), else 0
+    int open;                        // a step has begun and is not yet summed up (end_member)
     double t, dt;
     unsigned long long tau_bits;     // min positive t_ext (as ordered bits)
     long long flips, removals, two, nucl, vsteps, steps;
@@ -53,9 +59,10 @@ struct Blk { int m, b, e; };
 
 enum Counter {
     C_CAND = 0, C_TWO, C_T2, C_T2C, C_FLIPC,
-    C_FIX0, C_FIX1, C_FIX2, C_DIRTY, C_NUCL, C_CONF, C_NEV, C_VFALL, C_BIGR,
-    C_COUNT,                          // the counters above are cleared at the end of each step
-    C_TRI = C_COUNT,                  // l_tri: emptied when it is read
+    C_FIX0, C_FIX1, C_FIX2, C_DIRTY, C_CONF, C_VFALL, C_BIGR, C_RAN,
+    C_COUNT,                          // the counters above are cleared when the next step begins
+    C_NUCL = C_COUNT,                 // these once they have been read:
+    C_NEV, C_TRI,
     C_TOTAL
 };
 
