@@ -139,15 +139,28 @@ struct GrainFind {
 __device__ __forceinline__ GrainFind grain_find(const Dev& d, int g, int a, int b) {
     const int* L = glist(d, g);
     const int n = d.glen[g];
-    const int l0 = n > 0 ? L[0] : -2;
+    // the first eight entries come with the length where the row has them
+    const bool wide = d.S % 4 == 0 && d.S >= 8;
+    int4 h0 = make_int4(-1, -1, -1, -1), h1 = h0;
+    if (wide) {
+        h0 = reinterpret_cast<const int4*>(L)[0];
+        h1 = reinterpret_cast<const int4*>(L)[1];
+    }
+    const int l0 = wide ? h0.x : (n > 0 ? L[0] : -2);
     GrainFind f = {-1, -1, -1, -1};
+#pragma unroll 1
     for (int i0 = 0; i0 < n; i0 += 8) {
         int x[9];
+        if (wide && i0 == 0) {
+            x[0] = h0.x; x[1] = h0.y; x[2] = h0.z; x[3] = h0.w;
+            x[4] = h1.x; x[5] = h1.y; x[6] = h1.z; x[7] = h1.w;
+            x[8] = n > 8 ? L[8] : -2;
+        } else {
 #pragma unroll
-        for (int q = 0; q < 9; q++) {
-            const int i = i0 + q;
-            x[q] = i < n ? L[i] : (i == n ? l0 : -2);
+            for (int q = 0; q < 9; q++) x[q] = i0 + q < n ? L[i0 + q] : -2;
         }
+#pragma unroll
+        for (int q = 0; q < 9; q++) x[q] = i0 + q == n ? l0 : (i0 + q > n ? -2 : x[q]);
 #pragma unroll
         for (int q = 0; q < 8; q++) {
             const bool in = i0 + q < n;
@@ -274,54 +287,39 @@ __device__ __forceinline__ void slot_count_add(int2* bc, int blk, bool enable) {
               enable ? 0xFFFFFFFF00000001ull : 0x00000000FFFFFFFFull);
 }
 
-// Table block of a slot: members own consecutive runs of kBlock slots from
-// their offsets.
-__device__ __forceinline__ int vertex_block(const Dev& d, int v) {
-    if (d.B == 1) return v / kBlock;
-    const int m = d.vmem[v];
-    return d.vblk_first[m] + (v - d.prm[m].voff) / kBlock;
-}
-__device__ __forceinline__ int edge_block(const Dev& d, int e) {
-    if (d.B == 1) return e / kBlock;
-    const int m = d.emem[e];
-    return d.eblk_first[m] + (e - d.prm[m].eoff) / kBlock;
-}
-__device__ __forceinline__ int grain_block(const Dev& d, int g) {
-    if (d.B == 1) return g / kBlock;
-    const int m = d.gmem[g];
-    return d.gblk_first[m] + (g - d.prm[m].goff) / kBlock;
+// Where a member's slots and table blocks start (members own consecutive runs
+// of kBlock slots from their offsets): loaded once per event, with its other
+// data, for all the flags it changes.
+struct SlotBase {
+    int voff, eoff, goff, vf, ef, gf;
+};
+__device__ __forceinline__ SlotBase slot_base(const Dev& d, int m) {
+    if (d.B == 1) return SlotBase{0, 0, 0, 0, 0, 0};
+    const Params& P = d.prm[m];
+    return SlotBase{P.voff, P.eoff, P.goff, d.vblk_first[m], d.eblk_first[m], d.gblk_first[m]};
 }
 
-// Set an enable flag, counting a change of state.  No other thread writes
+// Set an enable flag whose value is known to be `was` (loaded by the caller
+// with its other data), counting a change of state.  No other thread writes
 // the same flag in the same launch (events that touch a slot are serial or
-// disjoint), so the read needs no atomic.  The forms with `was` take the
-// flag's value from the caller, who has loaded it with other data.
-__device__ __forceinline__ void set_vertex_enabled(const Dev& d, int v, bool was, bool on) {
+// disjoint).
+__device__ __forceinline__ void set_vertex_enabled(const Dev& d, const SlotBase& S, int v, bool was, bool on) {
     if (was != on) {
         d.ven[v] = on ? 1 : 0;
-        slot_count_add(d.bc_v, vertex_block(d, v), on);
+        slot_count_add(d.bc_v, S.vf + (v - S.voff) / kBlock, on);
     }
 }
-__device__ __forceinline__ void set_edge_enabled(const Dev& d, int e, bool was, bool on) {
+__device__ __forceinline__ void set_edge_enabled(const Dev& d, const SlotBase& S, int e, bool was, bool on) {
     if (was != on) {
         d.benab[e] = on ? 1 : 0;
-        slot_count_add(d.bc_e, edge_block(d, e), on);
+        slot_count_add(d.bc_e, S.ef + (e - S.eoff) / kBlock, on);
     }
 }
-__device__ __forceinline__ void set_grain_enabled(const Dev& d, int g, bool was, bool on) {
+__device__ __forceinline__ void set_grain_enabled(const Dev& d, const SlotBase& S, int g, bool was, bool on) {
     if (was != on) {
         d.genab[g] = on ? 1 : 0;
-        slot_count_add(d.bc_g, grain_block(d, g), on);
+        slot_count_add(d.bc_g, S.gf + (g - S.goff) / kBlock, on);
     }
-}
-__device__ __forceinline__ void set_vertex_enabled(const Dev& d, int v, bool on) {
-    set_vertex_enabled(d, v, d.ven[v] != 0, on);
-}
-__device__ __forceinline__ void set_edge_enabled(const Dev& d, int e, bool on) {
-    set_edge_enabled(d, e, d.benab[e] != 0, on);
-}
-__device__ __forceinline__ void set_grain_enabled(const Dev& d, int g, bool on) {
-    set_grain_enabled(d, g, d.genab[g] != 0, on);
 }
 
 // Flags the grains g[q] (where want[q]) for the fix stage `stage`

@@ -1928,8 +1928,12 @@ struct FixLds {
     int mg[4 * kMaxStride], mv[4 * kMaxStride], mp[4 * kMaxStride];
     unsigned short kinds[kMaxStride];     // per staged entry: 4 bits each for ADD, REMOVE, REPLACE records of this grain
     int n_add, n_fin;
-    int nl[64];                           // fix_items: each group's list after its insertions
-    unsigned char from[64];               //            and the lane an entry came from (kQuick: inserted)
+};
+// Room of a wave in fix_items: each group's list after its insertions, and the
+// lane an entry came from (kQuick: inserted).
+struct QuickLds {
+    int nl[64];
+    unsigned char from[64];
 };
 
 __device__ __forceinline__ void fix_wave(const Dev& d, int g, FixLds& f_) {
@@ -2062,8 +2066,10 @@ __device__ __forceinline__ void fix_wave(const Dev& d, int g, FixLds& f_) {
 // its capacity goes to fix_wave.  Wave w of nw takes items 4w .. 4w + 3, 4(w +
 // nw) ..  (One grain to a wave with the serial replay: 11.3 us at 1M grains
 // with 90 edited grains, 25 with the Monte Carlo workload's 12,000.)
-__device__ __forceinline__ void fix_items(const Dev& d, int stage, FixLds& f, int w, int nw) {
-    const int n_items = cnt_now(d, C_FIX0 + stage);
+// `grain` gives the items' grains; `replay` takes a mask of lanes, the first of
+// each group that needs fix_wave, and its grain in those lanes.
+template <class Grain, class Replay>
+__device__ __forceinline__ void fix_items(const Dev& d, int n_items, Grain grain, QuickLds& f, int w, int nw, Replay replay) {
     const int lane = (int)threadIdx.x & 63, l = lane & (kQuick - 1), g0 = lane & ~(kQuick - 1);
     const unsigned below = (1u << l) - 1u;
     // the group's part of a ballot
@@ -2071,7 +2077,7 @@ __device__ __forceinline__ void fix_items(const Dev& d, int stage, FixLds& f, in
     for (int base = 4 * w; base < n_items; base += 4 * nw) {
         const int item = base + (lane >> 4);
         const bool on = item < n_items;
-        const int g = on ? d.l_fix[stage][item] : 0;
+        const int g = on ? grain(item) : 0;
         int* L = glist(d, g);
         const bool en = on && d.genab[g] != 0;
         const int n0 = d.glen[g], v = l < d.S ? L[l] : -1;
@@ -2166,17 +2172,20 @@ __device__ __forceinline__ void fix_items(const Dev& d, int stage, FixLds& f, in
         }
         list_tri(d, g, en && !slow_g && l == 0 && n2 == 3);
         wave_sync();
-        // the groups that need the replay, one after the other
-        for (unsigned long long todo = __ballot(en && slow_g && l == 0); todo; todo &= todo - 1ull) {
-            fix_wave(d, __builtin_amdgcn_readlane(g, __ffsll((long long)todo) - 1), f);
-            wave_sync();
-        }
+        replay(__ballot(en && slow_g && l == 0), g);
     }
 }
 
 __global__ void __launch_bounds__(64) k_fix(Dev d, int stage) {
     __shared__ FixLds f;
-    fix_items(d, stage, f, (int)blockIdx.x, (int)gridDim.x);
+    __shared__ QuickLds q;
+    fix_items(d, d.cnt[C_FIX0 + stage], [&](int k) { return d.l_fix[stage][k]; }, q, (int)blockIdx.x, (int)gridDim.x,
+              [&](unsigned long long todo, int g) {
+                  for (; todo; todo &= todo - 1ull) {
+                      fix_wave(d, __builtin_amdgcn_readlane(g, __ffsll((long long)todo) - 1), f);
+                      wave_sync();
+                  }
+              });
 }
 
 // clear_grains_fix_state (topological.h:1150-1163) for the flagged grains;
@@ -2186,21 +2195,24 @@ __global__ void __launch_bounds__(64) k_fix(Dev d, int stage) {
 // load the list's points in parallel, each forming the wrapped delta to its
 // predecessor; the group's first lane then accumulates the shoelace sum over
 // the deltas in list order, the same arithmetic as grain_area.  Wave `blk` of
-// `nblk` takes items 4 blk .. 4 blk + 3, 4 (blk + nblk) ..; `c` is its room.
+// `nblk` takes items 4 blk .. 4 blk + 3, 4 (blk + nblk) ..; `c` is its room (a
+// longer list is summed from memory).  The first n items are flagged grains,
+// the nd that follow only have their areas formed.
+constexpr int kClearList = 32;
 struct ClearLds {
-    double2 dl[4][kMaxStride];
+    double2 dl[4][kClearList];
 };
 
-__device__ __forceinline__ void fix_clear_items(const Dev& d, int stage, int with_area, ClearLds& c, int blk, int nblk) {
-    const int n = cnt_now(d, C_FIX0 + stage);
-    const int nd = with_area ? min(cnt_now(d, C_DIRTY), d.G) : 0;
+template <class Grain>
+__device__ __forceinline__ void fix_clear_items(const Dev& d, int n, int nd, Grain grain, int with_area, ClearLds& c,
+                                                int blk, int nblk) {
     const int lane = (int)threadIdx.x & 63, l = lane & 15;
     double2* const dl = c.dl[lane >> 4];
     const double2* X = reinterpret_cast<const double2*>(d.pos);
     for (int base = 4 * blk; base < n + nd; base += 4 * nblk) {
         const int item = base + (lane >> 4);
         const bool on = item < n + nd, flagged = item < n;
-        const int g = !on ? 0 : (flagged ? d.l_fix[stage][item] : d.l_dirty[item - n]);
+        const int g = on ? grain(item) : 0;
         const int* L = glist(d, g);
         const bool en = on && d.genab[g] != 0;
         const int m = en ? d.glen[g] : 0;
@@ -2208,7 +2220,7 @@ __device__ __forceinline__ void fix_clear_items(const Dev& d, int stage, int wit
         if (flagged && l == 0) d.gfix[g] = 0;
         for (int i = l; i < m; i += 16) {
             const int w = L[i], wp = i > 0 ? L[i - 1] : w;
-            if (with_area) {
+            if (with_area && i < kClearList) {
                 const double2 p = X[w], q = X[wp];
                 dl[i] = make_double2(wrapd(p.x, q.x, D), wrapd(p.y, q.y, D));
             }
@@ -2217,7 +2229,9 @@ __device__ __forceinline__ void fix_clear_items(const Dev& d, int stage, int wit
         wave_sync();
         if (with_area && l == 0 && en) {
             double a = 0.0;
-            if (m > 0) {
+            if (m > kClearList) {
+                a = grain_area(d, g, D);
+            } else if (m > 0) {
                 AreaAcc acc;
                 acc.start(0.0, 0.0);
                 for (int i = 1; i < m; i++) acc.push_delta(dl[i].x, dl[i].y);
@@ -2229,9 +2243,16 @@ __device__ __forceinline__ void fix_clear_items(const Dev& d, int stage, int wit
     }
 }
 
+// The grains that a stage's launches flagged, from the global lists.
+__device__ __forceinline__ void clear_stage(const Dev& d, int stage, int with_area, ClearLds& c, int blk, int nblk) {
+    const int n = cnt_now(d, C_FIX0 + stage), nd = with_area ? min(cnt_now(d, C_DIRTY), d.G) : 0;
+    fix_clear_items(d, n, nd, [&](int k) { return k < n ? d.l_fix[stage][k] : d.l_dirty[k - n]; }, with_area, c, blk,
+                    nblk);
+}
+
 __global__ void __launch_bounds__(64) k_fix_clear(Dev d, int stage, int with_area) {
     __shared__ ClearLds c;
-    fix_clear_items(d, stage, with_area, c, (int)blockIdx.x, (int)gridDim.x);
+    clear_stage(d, stage, with_area, c, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // ---------------------------------------------------------------------
@@ -2276,14 +2297,17 @@ __device__ __forceinline__ int remove_two_grains(const Dev& d, int bnd, int gn0,
         const bool all[2] = {true, true};
         flag_grains(d, gg, all, 0);
     }
+    const SlotBase S = slot_base(d, member_of_edge(d, bnd));
+    auto edge_off = [&](int e) { set_edge_enabled(d, S, e, d.benab[e] != 0, false); };
+    auto vertex_off = [&](int v) { set_vertex_enabled(d, S, v, d.ven[v] != 0, false); };
     for (int i = 0; i < 3; i++) {
-        set_edge_enabled(d, d.vb[3 * A + i], false);
-        set_edge_enabled(d, d.vb[3 * B + i], false);
+        edge_off(d.vb[3 * A + i]);
+        edge_off(d.vb[3 * B + i]);
     }
-    set_edge_enabled(d, DF, false);
-    set_edge_enabled(d, bnd, false);
-    set_vertex_enabled(d, A, false); set_vertex_enabled(d, Dv, false);
-    set_vertex_enabled(d, C, false); set_vertex_enabled(d, B, false);
+    edge_off(DF);
+    edge_off(bnd);
+    vertex_off(A); vertex_off(Dv);
+    vertex_off(C); vertex_off(B);
     return CE;
 }
 
@@ -2317,8 +2341,11 @@ __device__ __forceinline__ void two_grain_serial(const Dev& d) {
             triples_symdiff(ga, gb, g0, g1, gn0, gn1);
             if (gn0 < 0 || gn1 < 0) { set_error(d, member_of_edge(d, e), SEVC_E_STATE); continue; }
             int CE = remove_two_grains(d, e, gn0, gn1);
-            set_grain_enabled(d, g0, false);
-            set_grain_enabled(d, g1, false);
+            {
+                const SlotBase S = slot_base(d, member_of_edge(d, e));
+                set_grain_enabled(d, S, g0, d.genab[g0] != 0, false);
+                set_grain_enabled(d, S, g1, d.genab[g1] != 0, false);
+            }
             d.ms[member_of_edge(d, e)].two += 1;
             // an edge whose endpoint moved may qualify later in this pass
             if (CE > e && two_qualifies(d, CE)) {
@@ -2380,7 +2407,8 @@ __device__ __forceinline__ void two_grain_serial(const Dev& d) {
 // the set grains_intersect forms from the edge's ends.  An edge that both of
 // its grains list comes twice; the second finds it gone.  (A pass over all
 // grains took 17.5 us at 1M grains, 8 at 2,000.)
-__device__ __forceinline__ void tri_items(const Dev& d, int n, int k0, int stride) {
+__device__ __forceinline__ bool tri_items(const Dev& d, int n, int k0, int stride) {
+    bool found = false;
     for (int k = k0; k < n; k += stride) {
         const int g = d.l_tri[k], m = member_of_grain(d, g);
         if (!d.genab[g] || d.glen[g] != 3 || !d.ms[m].active || !d.prm[m].events) continue;
@@ -2418,9 +2446,11 @@ __device__ __forceinline__ void tri_items(const Dev& d, int n, int k0, int strid
                 if (g1 < 0 || d.glen[g0] != 3 || d.glen[g1] != 3) continue;
                 const int s = atomicAdd(&d.cnt[C_TWO], 1);     // rare: two adjacent 3-sided grains
                 if (s < d.E) d.l_two[s] = bb[e];
+                found = true;
             }
         }
     }
+    return found;
 }
 
 // Lists every enabled 3-sided grain next to another one (the first step
@@ -2447,30 +2477,37 @@ __global__ void k_poll_gather(Dev d) {
     tri_items(d, n_tri(d), n - 1 - k0, n);
 }
 
-// After the gathers, by one workgroup: the vote rounds and the conflict check
-// on the step's candidate list, then (rarely) the passes of the two-triangle
-// stage.  The dt of the labels is noted for the slots that are labelled at the
-// end of the call (k_label_disabled).
-__device__ __forceinline__ void poll_stage(const Dev& d, int nc, unsigned char* pbuf) {
+// One workgroup per step notes the dt of its labels, for the slots that are
+// labelled at the end of the call (k_label_disabled), and empties the lists
+// that the step has read.
+__device__ __forceinline__ void note_step(const Dev& d) {
     for (int m = (int)threadIdx.x; m < d.B; m += (int)blockDim.x)
         if (d.ms[m].active && d.prm[m].events) d.ms[m].lab_dt = member_dt(d.prm[m], d.ms[m]);
-    if (nc > 0) poll_list(d, nc, pbuf);
     if (threadIdx.x == 0) {
-        atomicExch(&d.cnt[C_TRI], 0);
         d.cnt[C_NEV] = 0;
         d.cnt[C_NUCL] = 0;
         d.cnt[C_RAN] = 1;
     }
-    if (cnt_now(d, C_TWO) > 0) {
-        __syncthreads();
-        if (threadIdx.x == 0) two_grain_serial(d);
+}
+
+// The passes of the two-triangle stage (rarely any), by one workgroup.
+__device__ __forceinline__ void two_stage(const Dev& d) {
+    if (threadIdx.x == 0) {
+        atomicExch(&d.cnt[C_TRI], 0);
+        if (cnt_now(d, C_TWO) > 0) two_grain_serial(d);
     }
     __syncthreads();
 }
 
+// After the gathers: the vote rounds and the conflict check on the step's
+// candidate list, then the two-triangle stage.
 __global__ void __launch_bounds__(1024) k_poll(Dev d) {
     __shared__ __align__(16) unsigned char pbuf[kPollLds];
-    poll_stage(d, d.cnt[C_CAND], pbuf);
+    const int nc = d.cnt[C_CAND];
+    note_step(d);
+    if (nc > 0) poll_list(d, nc, pbuf);
+    __syncthreads();
+    two_stage(d);
 }
 
 // label_3sided_grains after the two-triangle stage, from the candidate list: a
@@ -2541,12 +2578,24 @@ __global__ void k_t2_label(Dev d) {
 // T2: 3-sided grain removal (topological.h:614-668, 687-822, 994-1004)
 // ---------------------------------------------------------------------
 
+// Flags grains for a fix stage in the global lists (flag_grains).
+struct FlagGlobal {
+    const Dev& d;
+    int stage;
+    template <int N>
+    __device__ __forceinline__ void operator()(const int (&g)[N], const bool (&want)[N]) const {
+        flag_grains(d, g, want, stage);
+    }
+};
+
 // remove_grain, topological.h:687-822.  Everything the removal reads is loaded
 // first (the grain's vertices; their edges, grains, positions and flags; those
 // edges' ends and flags), then the reference's sequence of tests and writes
 // runs on local copies in the same order -- a later test sees an earlier write
 // exactly as it would in memory -- and the writes go out.
-__device__ __forceinline__ void remove_grain(const Dev& d, int g, double D) {
+// `flag` flags the grains to be edited (flag_grains, or k_events' own list).
+template <class Flag>
+__device__ __forceinline__ void remove_grain(const Dev& d, int g, double D, const SlotBase& S, Flag flag) {
     const int* Lg = glist(d, g);
     const int A = Lg[0], B = Lg[1], C = Lg[2];
     int vA[3], vB[3], vC[3], gA[3], gB[3], gC[3];
@@ -2592,7 +2641,7 @@ __device__ __forceinline__ void remove_grain(const Dev& d, int g, double D) {
     for (int i = 0; i < 3; i++) {
         const int ei = xC[i].x, ee = xC[i].y;
         if (!found && ((ei == B && ee == C) || (ee == B && ei == C))) {
-            set_edge_enabled(d, vC[i], onC_[i], false);
+            set_edge_enabled(d, S, vC[i], onC_[i], false);
             offBC = vC[i];
             found = true;
         }
@@ -2633,7 +2682,7 @@ __device__ __forceinline__ void remove_grain(const Dev& d, int g, double D) {
         int e0, e1;
         ends(curA[i], i, e0, e1);
         if (!found && (e0 == B || e1 == B)) {
-            set_edge_enabled(d, curA[i], onA_[i] && curA[i] != offBC, false);
+            set_edge_enabled(d, S, curA[i], onA_[i] && curA[i] != offBC, false);
             offAB = curA[i];
             curA[i] = BEb; d.vb[3 * A + i] = BEb; found = true;
         }
@@ -2647,13 +2696,13 @@ __device__ __forceinline__ void remove_grain(const Dev& d, int g, double D) {
         if (!found && (e0 == C || e1 == C)) {
             // (an entry replaced above is read again)
             const bool was = curA[i] == vA[i] ? onA_[i] && curA[i] != offBC && curA[i] != offAB : d.benab[curA[i]] != 0;
-            set_edge_enabled(d, curA[i], was, false);
+            set_edge_enabled(d, S, curA[i], was, false);
             d.vb[3 * A + i] = CF; found = true;
         }
     }
-    set_vertex_enabled(d, B, onB, false);
-    set_vertex_enabled(d, C, onC && C != B, false);
-    set_grain_enabled(d, g, onG, false);
+    set_vertex_enabled(d, S, B, onB, false);
+    set_vertex_enabled(d, S, C, onC && C != B, false);
+    set_grain_enabled(d, S, g, onG, false);
     set_mod(d, B, 0, FIX_REMOVE, G2, B);
     set_mod(d, C, 0, FIX_REMOVE, G1, C);
     set_mod(d, B, 1, FIX_REMOVE, G3, B);
@@ -2663,7 +2712,7 @@ __device__ __forceinline__ void remove_grain(const Dev& d, int g, double D) {
     for (int i = 0; i < 3; i++) if (gA[i] == g) d.vg[3 * A + i] = G3;
     const int gg[3] = {G2, G1, G3};
     const bool all[3] = {true, true, true};
-    flag_grains(d, gg, all, 1);
+    flag(gg, all);
 }
 
 
@@ -2702,7 +2751,7 @@ __device__ __forceinline__ void t2_items(const Dev& d, int k0, int stride) {
             d.l_t2c[s] = g;
         } else {
             int m = member_of_grain(d, g);
-            remove_grain(d, g, d.prm[m].D);
+            remove_grain(d, g, d.prm[m].D, slot_base(d, m), FlagGlobal{d, 1});
         }
         wave_count(d, !clash, member_of_grain(d, g), &MState::removals);
     }
@@ -2712,21 +2761,23 @@ __global__ void k_t2_par(Dev d) {
     t2_items(d, (int)(blockIdx.x * blockDim.x + threadIdx.x), (int)(gridDim.x * blockDim.x));
 }
 
-__device__ __forceinline__ void t2_serial(const Dev& d) {
-    const int n = cnt_now(d, C_T2C);
-    sort_ints(d.l_t2c, n);
+// The conflicting candidates, all labelled, in index order by one lane.
+template <class Flag>
+__device__ __forceinline__ void t2_serial(const Dev& d, int* list, int n, Flag flag) {
+    sort_ints(list, n);
+#pragma unroll 1
     for (int k = 0; k < n; k++) {
-        int g = d.l_t2c[k];
-        if (!(d.genab[g] && d.gcand[g])) continue;
+        int g = list[k];
+        if (!d.genab[g]) continue;
         int m = member_of_grain(d, g);
         if (!d.ms[m].active) continue;
-        remove_grain(d, g, d.prm[m].D);
+        remove_grain(d, g, d.prm[m].D, slot_base(d, m), flag);
         atomicAdd(reinterpret_cast<unsigned long long*>(&d.ms[m].removals), 1ull);
     }
 }
 
 __global__ void k_t2_serial(Dev d) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) t2_serial(d);
+    if (threadIdx.x == 0 && blockIdx.x == 0) t2_serial(d, d.l_t2c, cnt_now(d, C_T2C), FlagGlobal{d, 1});
 }
 
 // unlabel_boundaries_st2, topological.h:588-606; the T2 stage is over, so
@@ -2759,7 +2810,7 @@ __global__ void __launch_bounds__(64) k_st2_fix_clear(Dev d, int nclear) {
     const int b = (int)blockIdx.x;
     __shared__ ClearLds c;
     if (b < nclear) {
-        fix_clear_items(d, 1, 1, c, b, nclear);
+        clear_stage(d, 1, 1, c, b, nclear);
         return;
     }
     st2_items(d, (b - nclear) * 64 + (int)threadIdx.x, ((int)gridDim.x - nclear) * 64);
@@ -2797,7 +2848,8 @@ __device__ __forceinline__ FlipIn flip_in(const Dev& d, int A, int B) {
 // ends of the rewired edges; the lists of the four grains around; their
 // orientations), then the reference's sequence of tests and writes runs on
 // local copies in the same order and the writes go out.
-__device__ __forceinline__ void flip(const Dev& d, int bnd, const Params& P, const FlipIn& in) {
+template <class Flag>
+__device__ __forceinline__ void flip(const Dev& d, int bnd, const Params& P, const FlipIn& in, Flag flag) {
     const double D = P.D;
     const int A = in.A, B = in.B;
     int vA[3], vB[3], gA[3], gB[3];
@@ -2852,7 +2904,7 @@ __device__ __forceinline__ void flip(const Dev& d, int bnd, const Params& P, con
     }
     const int gg[4] = {G2, G4, G3, G1};
     const bool want[4] = {g2 < 2, g4 < 2, g3 < 2, g1 < 2};
-    flag_grains(d, gg, want, 2);
+    flag(gg, want);
     if (g1 > 1 || g2 > 1 || g3 > 1 || g4 > 1) { set_error(d, member_of_edge(d, bnd), SEVC_E_STATE); return; }
 #pragma unroll
     for (int k = 0; k < 3; k++) {
@@ -2925,7 +2977,7 @@ __device__ __forceinline__ void flip_items(const Dev& d, int k0, int stride) {
             d.l_flipc[s] = c;
         } else {
             int m = member_of_edge(d, c);
-            flip(d, c, d.prm[m], fi);
+            flip(d, c, d.prm[m], fi, FlagGlobal{d, 2});
         }
         wave_count(d, !clash, member_of_edge(d, c), &MState::flips);
     }
@@ -2935,21 +2987,23 @@ __global__ void k_flip_par(Dev d) {
     flip_items(d, (int)(blockIdx.x * blockDim.x + threadIdx.x), (int)(gridDim.x * blockDim.x));
 }
 
-__device__ __forceinline__ void flip_serial(const Dev& d) {
-    const int n = cnt_now(d, C_FLIPC);
-    sort_ints(d.l_flipc, n);
+// The conflicting candidates, all labelled, in index order by one lane.
+template <class Flag>
+__device__ __forceinline__ void flip_serial(const Dev& d, int* list, int n, Flag flag) {
+    sort_ints(list, n);
+#pragma unroll 1
     for (int k = 0; k < n; k++) {
-        int c = d.l_flipc[k];
-        if (!(d.benab[c] && d.bcand[c])) continue;
+        int c = list[k];
+        if (!d.benab[c]) continue;
         int m = member_of_edge(d, c);
         if (!d.ms[m].active) continue;
-        flip(d, c, d.prm[m], flip_in(d, d.bvx[2 * c], d.bvx[2 * c + 1]));
+        flip(d, c, d.prm[m], flip_in(d, d.bvx[2 * c], d.bvx[2 * c + 1]), flag);
         atomicAdd(reinterpret_cast<unsigned long long*>(&d.ms[m].flips), 1ull);
     }
 }
 
 __global__ void k_flip_serial(Dev d) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) flip_serial(d);
+    if (threadIdx.x == 0 && blockIdx.x == 0) flip_serial(d, d.l_flipc, cnt_now(d, C_FLIPC), FlagGlobal{d, 2});
 }
 
 // Every event stage of a step (main.cu:202-310) in one launch of one
@@ -2962,46 +3016,438 @@ __global__ void k_flip_serial(Dev d) {
 // the launches took 63; a batch of 45 events a step 66 us where they took 105;
 // 1M grains, 27 events a step, 82 us where they took 130.  Its time grows with
 // the number of edited grains (64 at a time), so busy states take the launches.
+//
+// Up to kEvMax listed edges (one to a lane) a lane keeps its edge's
+// surroundings in registers, and everything the stages exchange goes through
+// LDS: the list position of an edge, the kept edge at a vertex, the labelled
+// grains and the flagged grains are small hash tables, so that no stage waits
+// for an atomic on memory or reads back what another one wrote there (the
+// stages as they are for the launches, one after the other: 28 us at 2,000
+// grains, 66 for the batch, 82 at 1M grains).  Longer lists, and steps with a
+// two-triangle candidate, run the launches' stages.
+// kEvMax: an edge has at most three grains in common with its ends, so at most
+// 3 kEvMax grains are labelled (a lane each), and three grains flagged by each.
+constexpr int kEvMax = 340;
+struct EvLds {
+    static constexpr int kEH = 2048, kVH = 2048, kTH = 2048, kFH = 4096, kT2 = 3 * kEvMax;
+    int ek[kEH], ep[kEH];             // listed edge -> list position
+    int vk[kVH], vp[kVH];             // vertex -> the kept edge at it, kMany if several
+    int tk[kTH];                      // labelled grains
+    int fk[kFH], fl[3 * kT2];         // flagged grains (hash) and their list
+    int t2[kT2], con[kT2];            // labelled grains, conflicting events
+    double ct[kEvMax];
+    int cid[kEvMax];
+    unsigned char cf[kEvMax];         // the edge's label
+    int nt2, ncon, nfl, changed, two, nslow;
+    int slow[3 * kT2];                // grains for fix_wave
+    QuickLds quick[16];
+    static constexpr int kSlow = 4;
+    union {
+        FixLds fix[kSlow];
+        ClearLds clear[16];
+    } room;
+};
+static_assert(sizeof(EvLds) <= kPollLds, "the event stages' tables fit");
+static_assert(EvLds::kT2 <= 1024 && 4 * kEvMax <= 3 * EvLds::kT2 && 3 * EvLds::kT2 < EvLds::kFH && EvLds::kT2 < EvLds::kTH &&
+                  2 * kEvMax < EvLds::kVH && kEvMax < EvLds::kEH,
+              "every list and table holds what a step can put in");
+constexpr int kFree = -1, kMany = -2;
+
+__device__ __forceinline__ int ev_hash(int x, int size) { return (int)(((unsigned)x * 2654435761u) >> 16) & (size - 1); }
+
+// The place of key x, or of the first free place after it.
+__device__ __forceinline__ int ev_find(const int* key, int size, int x) {
+    int h = ev_hash(x, size);
+    while (key[h] != x && key[h] != kFree) h = (h + 1) & (size - 1);
+    return h;
+}
+// Puts key x in; its place, and whether it is new.
+__device__ __forceinline__ int ev_put(int* key, int size, int x, bool* fresh) {
+    int h = ev_hash(x, size);
+    for (;;) {
+        const int was = atomicCAS(&key[h], kFree, x);
+        if (was == kFree || was == x) {
+            *fresh = was == kFree;
+            return h;
+        }
+        h = (h + 1) & (size - 1);
+    }
+}
+
+// Flags grains in LDS: each once in the list.
+struct FlagLds {
+    EvLds& s;
+    template <int N>
+    __device__ __forceinline__ void operator()(const int (&g)[N], const bool (&want)[N]) const {
+#pragma unroll 1
+        for (int q = 0; q < N; q++) {
+            int x = g[0];
+            bool w = want[0];
+#pragma unroll
+            for (int r = 1; r < N; r++) {
+                x = q == r ? g[r] : x;
+                w = q == r ? want[r] : w;
+            }
+            bool fresh;
+            if (!w) continue;
+            ev_put(s.fk, EvLds::kFH, x, &fresh);
+            if (fresh) s.fl[atomicAdd(&s.nfl, 1)] = x;
+        }
+    }
+};
+
+// The flagged grains' edits, then their clearing (with areas after the T2
+// stage); leaves the flag table empty.
+__device__ __forceinline__ void ev_edit(const Dev& d, EvLds& s, int with_area) {
+    const int tid = (int)threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int n = s.nfl;
+    fix_items(d, n, [&](int k) { return s.fl[k]; }, s.quick[wave], wave, 16, [&](unsigned long long todo, int g) {
+        if ((todo >> lane) & 1ull) s.slow[atomicAdd(&s.nslow, 1)] = g;
+    });
+    __syncthreads();
+    if (s.nslow > 0) {
+        if (wave < EvLds::kSlow)
+            for (int k = wave; k < s.nslow; k += EvLds::kSlow) {
+                fix_wave(d, s.slow[k], s.room.fix[wave]);
+                wave_sync();
+            }
+        __syncthreads();
+    }
+    for (int h = tid; h < EvLds::kFH; h += 1024) s.fk[h] = kFree;
+    fix_clear_items(d, n, 0, [&](int k) { return s.fl[k]; }, with_area, s.room.clear[wave], wave, 16);
+    __syncthreads();
+    if (tid == 0) s.nfl = s.nslow = 0;
+    __syncthreads();
+}
+
+// The event stages for a list of nc <= kEvMax edges; false (nothing done yet)
+// when a two-triangle candidate was found.
+__device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, EvLds& s) {
+    const int tid = (int)threadIdx.x;
+    const bool on = tid < nc;
+    // the edge and its ends
+    int c = -1, m = 0;
+    int2 ab = make_int2(0, 0);
+    double te = 0.0, len = 0.0;
+    if (on) c = d.l_cand[tid];
+    for (int h = tid; h < EvLds::kEH; h += 1024) s.ek[h] = kFree;
+    for (int h = tid; h < EvLds::kVH; h += 1024) { s.vk[h] = kFree; s.vp[h] = kFree; }
+    for (int h = tid; h < EvLds::kTH; h += 1024) s.tk[h] = kFree;
+    for (int h = tid; h < EvLds::kFH; h += 1024) s.fk[h] = kFree;
+    if (tid == 0) s.nt2 = s.ncon = s.nfl = s.two = s.nslow = 0;
+    if (on) {
+        ab = reinterpret_cast<const int2*>(d.bvx)[c];
+        te = d.bt[c];
+        len = d.blen[c];
+        m = member_of_edge(d, c);
+    }
+    __syncthreads();
+    if (on) {
+        bool fresh;
+        s.ep[ev_put(s.ek, EvLds::kEH, c, &fresh)] = tid;
+    }
+    if (tri_items(d, ntri, 1023 - tid, 1024)) s.two = 1;
+    // the ends' edges, grains and positions; the edges' other ends and flags;
+    // the lengths of the grains around
+    FlipIn fi{};
+    bool cand = false, en6[6], ge[3];
+    int w6[6], gl[3];
+    if (on) {
+        fi = flip_in(d, ab.x, ab.y);
+        cand = is_candidate(te, len, member_dt(d.prm[m], d.ms[m]), d.prm[m].flip_thr);
+    }
+#pragma unroll
+    for (int j = 0; j < 6; j++) {
+        const int x = j < 3 ? fi.vA[j] : fi.vB[j - 3];
+        const bool other = on && x != c;
+        const int2 e = other ? reinterpret_cast<const int2*>(d.bvx)[x] : make_int2(0, 0);
+        en6[j] = other && d.benab[x] != 0;
+        w6[j] = e.x == (j < 3 ? ab.x : ab.y) ? e.y : e.x;
+    }
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        gl[q] = on ? d.glen[fi.gA[q]] : 0;
+        ge[q] = on && d.genab[fi.gA[q]] != 0;
+    }
+    if (on) {
+        s.ct[tid] = te;
+        s.cid[tid] = c;
+        s.cf[tid] = cand ? 1 : 0;
+    }
+    __syncthreads();
+    if (s.two) return false;
+    if (tid == 0) atomicExch(&d.cnt[C_TRI], 0);         // searched; the edits below list anew
+    if (nc == 0) return true;
+    auto edge_pos = [&](int x) {
+        const int h = ev_find(s.ek, EvLds::kEH, x);
+        return s.ek[h] == x ? s.ep[h] : -1;
+    };
+    auto flagp = [&](int p) { return p >= 0 && s.cf[p] != 0; };
+    int ep[6];
+#pragma unroll
+    for (int j = 0; j < 6; j++) ep[j] = on ? edge_pos(j < 3 ? fi.vA[j] : fi.vB[j - 3]) : -1;
+
+    // polling (poll_list's rounds)
+    auto votes_self = [&](int e) {
+        double min_t = 99999999;
+        int arg = -1;
+#pragma unroll
+        for (int r = 0; r < 3; r++) {
+            const int p = e == 0 ? ep[r] : ep[3 + r];
+            if (flagp(p) && s.ct[p] <= min_t) { min_t = s.ct[p]; arg = p; }
+        }
+        return arg >= 0 ? arg == tid : (e == 0 ? fi.vA[0] : fi.vB[0]) == c;
+    };
+    for (;;) {
+        if (tid == 0) s.changed = 0;
+        const bool two = on && s.cf[tid] && votes_self(0) && votes_self(1);
+        __syncthreads();
+        if (two)
+#pragma unroll
+            for (int j = 0; j < 6; j++)
+                if (ep[j] >= 0 && ep[j] != tid && s.cf[ep[j]]) { s.cf[ep[j]] = 0; s.changed = 1; }
+        __syncthreads();
+        const int ch = s.changed;
+        __syncthreads();
+        if (!ch) break;
+    }
+    // the conflict check (poll_list's), the kept edge at the far end of a
+    // neighbour from the vertex table
+    bool keep = on && s.cf[tid] != 0;
+    if (keep) {
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            bool fresh;
+            const int h = ev_put(s.vk, EvLds::kVH, e == 0 ? ab.x : ab.y, &fresh);
+            const int was = atomicCAS(&s.vp[h], kFree, tid);
+            if (was != kFree && was != tid) atomicExch(&s.vp[h], kMany);
+        }
+    }
+    __syncthreads();
+    if (keep) {
+#pragma unroll 1
+        for (int j = 0; j < 6; j++) {
+            const bool e0 = j < 3;
+            bool en = en6[0];
+            int w = w6[0], own = ep[0], x = fi.vA[0];
+#pragma unroll
+            for (int r = 1; r < 6; r++) {
+                en = j == r ? en6[r] : en;
+                w = j == r ? w6[r] : w;
+                own = j == r ? ep[r] : own;
+                x = j == r ? (r < 3 ? fi.vA[r] : fi.vB[r - 3]) : x;
+            }
+            if (!en || flagp(own)) continue;
+            const int h = ev_find(s.vk, EvLds::kVH, w);
+            if (s.vk[h] != w) continue;
+            int pbe = s.vp[h], pbi = -1;
+            if (pbe == kMany) {
+                pbe = -1;
+                for (int r = 2; r >= 0; r--) {
+                    const int y = d.vb[3 * w + r], p = y == x ? -1 : edge_pos(y);
+                    if (flagp(p)) pbe = p;
+                }
+            }
+#pragma unroll
+            for (int r = 2; r >= 0; r--) {               // first in slot order
+                const int p = e0 ? ep[r] : ep[3 + r];
+                if (flagp(p)) pbi = p;
+            }
+            if (pbi < 0 || pbe < 0) continue;
+            const double ti = s.ct[pbi], tb = s.ct[pbe];
+            const int bi = s.cid[pbi], be = s.cid[pbe];
+            const int win = ti == tb ? (bi < be ? bi : be) : (ti < tb ? bi : be);
+            if (win != c) keep = false;
+        }
+    }
+    __syncthreads();                                     // every label read
+    if (on) {
+        s.cf[tid] = (unsigned char)((keep ? 1 : 0) | (cand ? 2 : 0));
+        d.conf[c] = -1;
+    }
+    __syncthreads();
+
+    // T2 labels (t2_label_items)
+    if (cand) {
+#pragma unroll 1
+        for (int q = 0; q < 3; q++) {
+            const int g = q == 0 ? fi.gA[0] : (q == 1 ? fi.gA[1] : fi.gA[2]);
+            const int n = q == 0 ? gl[0] : (q == 1 ? gl[1] : gl[2]);
+            const bool e_ = q == 0 ? ge[0] : (q == 1 ? ge[1] : ge[2]);
+            if (n != 3 || !e_ || !(g == fi.gB[0] || g == fi.gB[1] || g == fi.gB[2])) continue;
+            const int* L = glist(d, g);
+            const int vv[3] = {L[0], L[1], L[2]};
+            int bb[9];
+            int2 ends[9];
+            bool be[9];
+#pragma unroll
+            for (int e = 0; e < 9; e++) bb[e] = d.vb[3 * vv[e / 3] + e % 3];
+#pragma unroll
+            for (int e = 0; e < 9; e++) {
+                ends[e] = reinterpret_cast<const int2*>(d.bvx)[bb[e]];
+                be[e] = d.benab[bb[e]] != 0;
+            }
+            auto in_g = [&](int x) { return x == vv[0] || x == vv[1] || x == vv[2]; };
+            bool hit = false;
+            int ans = 0, first = INT_MAX;
+#pragma unroll
+            for (int e = 0; e < 9; e++) {
+                const bool in = in_g(ends[e].x) && in_g(ends[e].y) && be[e];
+                if (!in) continue;
+                const int p = edge_pos(bb[e]), lab = p >= 0 ? s.cf[p] : 0;
+                hit = hit || (lab & 1);
+                if (lab & 2) {
+                    ans++;
+                    first = min(first, bb[e]);
+                }
+            }
+            if (!(hit || ans / 2 == 3) || first != c) continue;
+            bool fresh;
+            ev_put(s.tk, EvLds::kTH, g, &fresh);
+            s.t2[atomicAdd(&s.nt2, 1)] = g;
+        }
+    }
+    __syncthreads();
+    const int nt2 = s.nt2;
+    const FlagLds flag{s};
+    if (nt2 > 0) {
+        // a candidate with no other one around is removed at once (t2_items)
+        bool go = false;
+        int g = 0, mg = 0;
+        if (tid < nt2) {
+            g = s.t2[tid];
+            mg = member_of_grain(d, g);
+            const int* L = glist(d, g);
+            int h[9];
+#pragma unroll
+            for (int e = 0; e < 9; e++) h[e] = d.vg[3 * L[e / 3] + e % 3];
+            bool clash = false;
+#pragma unroll 1
+            for (int e = 0; e < 9; e++) {
+                int x = h[0];
+#pragma unroll
+                for (int r = 1; r < 9; r++) x = e == r ? h[r] : x;
+                clash = clash || (x != g && x >= 0 && s.tk[ev_find(s.tk, EvLds::kTH, x)] == x);
+            }
+            if (clash) s.con[atomicAdd(&s.ncon, 1)] = g;
+            go = !clash;
+        }
+        __syncthreads();
+        if (go) remove_grain(d, g, d.prm[mg].D, slot_base(d, mg), flag);
+        wave_count(d, go, mg, &MState::removals);
+        __syncthreads();
+        if (s.ncon > 0) {
+            if (tid == 0) t2_serial(d, s.con, s.ncon, flag);
+            __syncthreads();
+            if (tid == 0) s.ncon = 0;
+        }
+        if (tid == 0) d.cnt[C_FIX1] = s.nfl;
+        ev_edit(d, s, 1);
+    }
+
+    // unlabel_boundaries_st2 (st2_items), then the flips (flip_items); after a
+    // removal the surroundings are read again
+    bool live = keep;
+    if (nt2 > 0 && keep) {
+        live = d.benab[c] != 0 && d.ms[m].active;
+        ab = reinterpret_cast<const int2*>(d.bvx)[c];
+        fi = flip_in(d, ab.x, ab.y);
+#pragma unroll
+        for (int q = 0; q < 3; q++) gl[q] = d.glen[fi.gA[q]];
+    }
+    bool label = keep;
+    if (live) {
+        int g0, g1;
+        const int k = triples_intersect(fi.gA, fi.gB, g0, g1);
+        int n0 = 0, n1 = 0;
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+            n0 = fi.gA[q] == g0 ? gl[q] : n0;
+            n1 = fi.gA[q] == g1 ? gl[q] : n1;
+        }
+        label = !(k < 2 || n0 == 3 || n1 == 3);
+    }
+    if (keep) d.bcand[c] = label ? 1 : 0;
+    live = live && label;
+    if (on) s.cf[tid] = live ? 1 : 0;
+    __syncthreads();
+    bool clash = false;
+    if (live) {
+#pragma unroll 1
+        for (int j = 0; j < 6; j++) {
+            int x = fi.vA[0];
+#pragma unroll
+            for (int r = 1; r < 6; r++) x = j == r ? (r < 3 ? fi.vA[r] : fi.vB[r - 3]) : x;
+            clash = clash || (x != c && flagp(edge_pos(x)));
+        }
+        if (clash) s.con[atomicAdd(&s.ncon, 1)] = c;
+        else flip(d, c, d.prm[m], fi, flag);
+    }
+    wave_count(d, live && !clash, m, &MState::flips);
+    __syncthreads();
+    if (s.ncon > 0) {
+        if (tid == 0) flip_serial(d, s.con, s.ncon, flag);
+        __syncthreads();
+    }
+    if (s.nfl == 0) return true;
+    if (tid == 0) d.cnt[C_FIX2] = s.nfl;
+    ev_edit(d, s, 0);
+    return true;
+}
+
 __global__ void __launch_bounds__(1024) k_events(Dev d) {
     __shared__ __align__(16) unsigned char buf[kPollLds];
     const int tid = (int)threadIdx.x, nt = (int)blockDim.x, wave = tid >> 6;
+    const int nc = d.cnt[C_CAND], ntri = n_tri(d);
+    note_step(d);
+    if (nc == 0 && ntri == 0) return;
+    if (nc <= kEvMax) {
+        if (events_in_lds(d, nc, ntri, *reinterpret_cast<EvLds*>(buf))) return;
+    } else {
+        tri_items(d, ntri, nt - 1 - tid, nt);
+    }
+    // the launches' stages
     constexpr int kWaves = 16;
-    static_assert(kWaves * sizeof(FixLds) <= kPollLds && kWaves * sizeof(ClearLds) <= kPollLds, "staging rooms fit");
-    FixLds* const fl = reinterpret_cast<FixLds*>(buf) + wave;
-    ClearLds* const cl = reinterpret_cast<ClearLds*>(buf) + wave;
-    const int nc = d.cnt[C_CAND];
-    gather_items(d, nc, tid, nt);
-    tri_items(d, n_tri(d), nt - 1 - tid, nt);
+    struct Room {
+        FixLds fix;
+        QuickLds quick;
+        ClearLds clear;
+    };
+    static_assert(8 * sizeof(Room) <= kPollLds, "staging rooms fit");
+    Room* const room = reinterpret_cast<Room*>(buf) + wave;
+    auto edits = [&](int stage) {
+        if (wave < 8)
+            fix_items(d, cnt_now(d, C_FIX0 + stage), [&](int k) { return d.l_fix[stage][k]; }, room->quick, wave, 8,
+                      [&](unsigned long long todo, int g) {
+                          for (; todo; todo &= todo - 1ull) {
+                              fix_wave(d, __builtin_amdgcn_readlane(g, __ffsll((long long)todo) - 1), room->fix);
+                              wave_sync();
+                          }
+                      });
+        __syncthreads();
+        if (wave < 8) clear_stage(d, stage, stage == 1 ? 1 : 0, room->clear, wave, 8);
+        __syncthreads();
+    };
     __syncthreads();
-    poll_stage(d, nc, buf);
-    const bool two = cnt_now(d, C_TWO) > 0;
-    if (nc == 0 && !two) return;
+    gather_items(d, nc, tid, nt);
+    __syncthreads();
+    if (nc > 0) poll_list(d, nc, buf);
+    __syncthreads();
+    two_stage(d);
     t2_label_items(d, tid, nt);
     __syncthreads();
-    const bool t2 = cnt_now(d, C_T2) > 0;
-    if (t2) {
-        t2_items(d, tid, nt);
-        __syncthreads();
-        if (cnt_now(d, C_T2C) > 0) {
-            if (tid == 0) t2_serial(d);
-            __syncthreads();
-        }
-        fix_items(d, 1, *fl, wave, kWaves);
-        __syncthreads();
-    }
-    if (t2 || two) fix_clear_items(d, 1, 1, *cl, wave, kWaves);
+    t2_items(d, tid, nt);
+    __syncthreads();
+    if (tid == 0) t2_serial(d, d.l_t2c, cnt_now(d, C_T2C), FlagGlobal{d, 1});
+    __syncthreads();
+    edits(1);
     st2_items(d, tid, nt);
     __syncthreads();
     flip_items(d, tid, nt);
     __syncthreads();
-    if (cnt_now(d, C_FLIPC) > 0) {
-        if (tid == 0) flip_serial(d);
-        __syncthreads();
-    }
-    if (cnt_now(d, C_FIX2) == 0) return;
-    fix_items(d, 2, *fl, wave, kWaves);
+    if (tid == 0) flip_serial(d, d.l_flipc, cnt_now(d, C_FLIPC), FlagGlobal{d, 2});
     __syncthreads();
-    fix_clear_items(d, 2, 0, *cl, wave, kWaves);
+    edits(2);
 }
 
 // ---------------------------------------------------------------------
@@ -3631,7 +4077,8 @@ __device__ __forceinline__ void insert_event(const Dev& d, int m, int A, int B, 
     const int ae0 = d.bvx[2 * r.AE], ae1 = d.bvx[2 * r.AE + 1], af0 = d.bvx[2 * r.AF];
     if (lane == 0) { n_s[0] = n_old[0]; n_s[1] = n_old[1]; n_s[2] = n_old[2]; }
     wave_sync();
-    const int S = P.cap;
+    const int cap = P.cap;
+    const SlotBase SB = slot_base(d, m);
     auto find = [&](int t, int n, int v) {                      // first place of v, -1 if none
         for (int i0 = 0; i0 < n; i0 += 64) {
             const unsigned long long hit = __ballot(i0 + lane < n && Ls[t][min(i0 + lane, kMaxStride - 1)] == v);
@@ -3651,7 +4098,7 @@ __device__ __forceinline__ void insert_event(const Dev& d, int m, int A, int B, 
     };
     auto ladd = [&](int t, int v, int prev) {                   // grain_add_vertex
         const int n = n_s[t], pos = find(t, n, prev) + 1;
-        const int err = pos == 0 ? SEVC_E_STATE : (n >= S ? SEVC_E_GRAIN_FULL : 0);
+        const int err = pos == 0 ? SEVC_E_STATE : (n >= cap ? SEVC_E_GRAIN_FULL : 0);
         if (err) {
             if (lane == 0) set_error(d, m, err);
             return;
@@ -3685,7 +4132,7 @@ __device__ __forceinline__ void insert_event(const Dev& d, int m, int A, int B, 
             d.pos[2 * v + 1] = q == 0 ? r.Bpos[1] : r.Cpos[1];
             d.vel[2 * v] = 0.0; d.vel[2 * v + 1] = 0.0;
             d.venergy[v] = 0.0;
-            set_vertex_enabled(d, v, false, true);
+            set_vertex_enabled(d, SB, v, false, true);
             d.vnuc[v] = 0;
             reset_mods(d, v);
         }
@@ -3703,7 +4150,7 @@ __device__ __forceinline__ void insert_event(const Dev& d, int m, int A, int B, 
             d.bvx[2 * b + 1] = q == 0 ? B : (q == 1 ? C : A);
             d.blen[b] = 0;
             d.bt[b] = SEVC_MAX_T_EXT;
-            set_edge_enabled(d, b, false, true);
+            set_edge_enabled(d, SB, b, false, true);
             d.bcand[b] = 0;
             d.conf[b] = -1;
         }
@@ -3714,7 +4161,7 @@ __device__ __forceinline__ void insert_event(const Dev& d, int m, int A, int B, 
         d.glen[g] = 3;
         d.garea[g] = 0;
         d.gse[g] = 0;
-        set_grain_enabled(d, g, false, true);
+        set_grain_enabled(d, SB, g, false, true);
         d.gcand[g] = 0;
         d.gfix[g] = 0;
         d.gtype[g] = T_NUCLEATED;
