@@ -619,7 +619,7 @@ int sevc_batch_create(const sevc_options* opts, const sevc_mesh* meshes, int32_t
     DA(d.l_dirty, G); DA(d.l_nucl, G); DA(d.l_conf, 4 * E + 16);
     DA(d.nscr, 12 * G + 16);
     DA(d.l_vfall, V + 16);
-    DA(d.l_tri, 6 * G); DA(d.busy, 1);
+    DA(d.l_tri, 6 * G); DA(d.busy, 1); DA(d.c_id, kEvMax); DA(d.c_te, kEvMax);
     DA(d.l_bigr, G + 16);
     DA(d.nrec, 4 * G + 16); DA(d.nal, G + 16); DA(d.l_nev, 8 * G + 16);
 

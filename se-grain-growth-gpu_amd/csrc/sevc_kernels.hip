@@ -1419,6 +1419,10 @@ __global__ void k_text(Dev d) {
         const int k = bbase + before + (int)__popcll(bal & ((1ull << lane) - 1ull));
         d.l_cand[k] = i;
         d.conf[i] = k;          // list position, for k_poll_gather
+        if (k < kEvMax) {       // for k_events
+            d.c_id[k] = make_int4(i, ab.x, ab.y, bd_.m);
+            d.c_te[k] = make_double2(te, norm);
+        }
     }
 }
 
@@ -2066,10 +2070,27 @@ __device__ __forceinline__ void fix_wave(const Dev& d, int g, FixLds& f_) {
 // its capacity goes to fix_wave.  Wave w of nw takes items 4w .. 4w + 3, 4(w +
 // nw) ..  (One grain to a wave with the serial replay: 11.3 us at 1M grains
 // with 90 edited grains, 25 with the Monte Carlo workload's 12,000.)
-// `grain` gives the items' grains; `replay` takes a mask of lanes, the first of
-// each group that needs fix_wave, and its grain in those lanes.
-template <class Grain, class Replay>
-__device__ __forceinline__ void fix_items(const Dev& d, int n_items, Grain grain, QuickLds& f, int w, int nw, Replay replay) {
+// `grain` gives the items' grains and `record` a vertex's record; `replay`
+// takes a mask of lanes, the first of each group that needs fix_wave, and its
+// grain in those lanes; `after` takes an edited list: each lane's group (its
+// first lane), place, entry and whether it has one, the grain and the length.
+struct EditRec {
+    int g[4], v[4], p[4];
+    unsigned fix;
+};
+__device__ __forceinline__ EditRec no_edits() {
+    return EditRec{{-1, -1, -1, -1}, {-1, -1, -1, -1}, {-1, -1, -1, -1}, 0x01010101u * (unsigned)FIX_NONE};
+}
+__device__ __forceinline__ EditRec record_global(const Dev& d, int v) {
+    const int4* r = reinterpret_cast<const int4*>(&d.mods[v]);
+    const int4 a = r[0], b = r[1], c = r[2];
+    return EditRec{{a.x, a.y, a.z, a.w}, {b.x, b.y, b.z, b.w}, {c.x, c.y, c.z, c.w},
+                   *reinterpret_cast<const unsigned*>(d.mods[v].fix)};
+}
+
+template <class Grain, class Record, class Replay, class After>
+__device__ __forceinline__ void fix_items(const Dev& d, int n_items, Grain grain, Record record, QuickLds& f, int w, int nw,
+                                          Replay replay, After after) {
     const int lane = (int)threadIdx.x & 63, l = lane & (kQuick - 1), g0 = lane & ~(kQuick - 1);
     const unsigned below = (1u << l) - 1u;
     // the group's part of a ballot
@@ -2084,35 +2105,25 @@ __device__ __forceinline__ void fix_items(const Dev& d, int n_items, Grain grain
         const int mem = member_of_grain(d, g);
         bool slow = en && n0 > kQuick;
         const bool has = en && !slow && l < n0;
-        int4 rg = make_int4(-1, -1, -1, -1), rv = rg, rp = rg;
-        unsigned rf = 0x01010101u * (unsigned)FIX_NONE;
-        if (has) {
-            const int4* r = reinterpret_cast<const int4*>(&d.mods[v]);
-            rg = r[0];
-            rv = r[1];
-            rp = r[2];
-            rf = *reinterpret_cast<const unsigned*>(d.mods[v].fix);
-        }
+        EditRec r = no_edits();
+        if (has) r = record(v);
         const int cap = d.prm[mem].cap;
-        const int gq[4] = {rg.x, rg.y, rg.z, rg.w}, vq[4] = {rv.x, rv.y, rv.z, rv.w}, pq[4] = {rp.x, rp.y, rp.z, rp.w};
         int adds = 0, reps = 0, vadd = -1, vrep = -1;
         unsigned rem = 0;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const unsigned k = (rf >> (8 * j)) & 255u;
-            const bool mine = gq[j] == g;
-            if (mine && k == FIX_ADD) { adds++; vadd = vq[j]; slow = slow || pq[j] != v; }
-            if (mine && k == FIX_REPLACE) { reps++; vrep = vq[j]; slow = slow || pq[j] != v; }
+            const unsigned k = (r.fix >> (8 * j)) & 255u;
+            const bool mine = r.g[j] == g;
+            if (mine && k == FIX_ADD) { adds++; vadd = r.v[j]; slow = slow || r.p[j] != v; }
+            if (mine && k == FIX_REPLACE) { reps++; vrep = r.v[j]; slow = slow || r.p[j] != v; }
             rem |= mine && k == FIX_REMOVE ? 1u << j : 0u;
         }
         slow = slow || adds > 1 || reps > 1;
         if (adds > 0) {
             // the inserted vertex's own records
-            const int4 tg = *reinterpret_cast<const int4*>(d.mods[vadd].grn);
-            const unsigned tf = *reinterpret_cast<const unsigned*>(d.mods[vadd].fix);
-            const int tq[4] = {tg.x, tg.y, tg.z, tg.w};
+            const EditRec t = record(vadd);
 #pragma unroll
-            for (int j = 0; j < 4; j++) slow = slow || (tq[j] == g && ((tf >> (8 * j)) & 255u) != FIX_NONE);
+            for (int j = 0; j < 4; j++) slow = slow || (t.g[j] == g && ((t.fix >> (8 * j)) & 255u) != FIX_NONE);
         }
         const unsigned am = group(adds > 0);
         const int pre = __popc(am & below), n1 = n0 + __popc(am);
@@ -2154,7 +2165,7 @@ __device__ __forceinline__ void fix_items(const Dev& d, int n_items, Grain grain
             const unsigned ro = rm ? rem_o : 0u;
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const int t = __shfl(vq[j], o);
+                const int t = __shfl(r.v[j], o);
                 const unsigned m = group(in1 && x == t);
                 if (((ro >> j) & 1u) && m && l == __ffs((int)m) - 1) gone = true;
             }
@@ -2170,22 +2181,31 @@ __device__ __forceinline__ void fix_items(const Dev& d, int n_items, Grain grain
             if (l >= n2 && l < n1) L[l] = -1;
             if (l == 0) d.glen[g] = n2;
         }
+        after(g0, at, rep ? vrep_src : x, stay && !slow_g, g, en && !slow_g ? n2 : -1);
         list_tri(d, g, en && !slow_g && l == 0 && n2 == 3);
         wave_sync();
         replay(__ballot(en && slow_g && l == 0), g);
     }
 }
 
+// The grains that a stage's launches flagged, from the global lists.
+__device__ __forceinline__ void fix_stage(const Dev& d, int stage, FixLds& f, QuickLds& q, int w, int nw) {
+    fix_items(
+        d, cnt_now(d, C_FIX0 + stage), [&](int k) { return d.l_fix[stage][k]; },
+        [&](int v) { return record_global(d, v); }, q, w, nw,
+        [&](unsigned long long todo, int g) {
+            for (; todo; todo &= todo - 1ull) {
+                fix_wave(d, __builtin_amdgcn_readlane(g, __ffsll((long long)todo) - 1), f);
+                wave_sync();
+            }
+        },
+        [](int, int, int, bool, int, int) {});
+}
+
 __global__ void __launch_bounds__(64) k_fix(Dev d, int stage) {
     __shared__ FixLds f;
     __shared__ QuickLds q;
-    fix_items(d, d.cnt[C_FIX0 + stage], [&](int k) { return d.l_fix[stage][k]; }, q, (int)blockIdx.x, (int)gridDim.x,
-              [&](unsigned long long todo, int g) {
-                  for (; todo; todo &= todo - 1ull) {
-                      fix_wave(d, __builtin_amdgcn_readlane(g, __ffsll((long long)todo) - 1), f);
-                      wave_sync();
-                  }
-              });
+    fix_stage(d, stage, f, q, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // clear_grains_fix_state (topological.h:1150-1163) for the flagged grains;
@@ -2578,10 +2598,14 @@ __global__ void k_t2_label(Dev d) {
 // T2: 3-sided grain removal (topological.h:614-668, 687-822, 994-1004)
 // ---------------------------------------------------------------------
 
-// Flags grains for a fix stage in the global lists (flag_grains).
-struct FlagGlobal {
+// Where an event's deferred list edits go: the vertices' records in memory and
+// the stage's list of flagged grains (k_events keeps both in LDS: EditLds).
+struct EditGlobal {
     const Dev& d;
     int stage;
+    __device__ __forceinline__ int open(int v) const { return v; }
+    __device__ __forceinline__ void put(int v, int slot, int fix, int grn, int vrt) const { set_mod(d, v, slot, fix, grn, vrt); }
+    __device__ __forceinline__ void put_prev(int v, int slot, int prev) const { d.mods[v].prev[slot] = prev; }
     template <int N>
     __device__ __forceinline__ void operator()(const int (&g)[N], const bool (&want)[N]) const {
         flag_grains(d, g, want, stage);
@@ -2593,9 +2617,9 @@ struct FlagGlobal {
 // edges' ends and flags), then the reference's sequence of tests and writes
 // runs on local copies in the same order -- a later test sees an earlier write
 // exactly as it would in memory -- and the writes go out.
-// `flag` flags the grains to be edited (flag_grains, or k_events' own list).
-template <class Flag>
-__device__ __forceinline__ void remove_grain(const Dev& d, int g, double D, const SlotBase& S, Flag flag) {
+// The list edits go to `ed`.
+template <class Edit>
+__device__ __forceinline__ void remove_grain(const Dev& d, int g, double D, const SlotBase& S, Edit ed) {
     const int* Lg = glist(d, g);
     const int A = Lg[0], B = Lg[1], C = Lg[2];
     int vA[3], vB[3], vC[3], gA[3], gB[3], gC[3];
@@ -2703,16 +2727,17 @@ __device__ __forceinline__ void remove_grain(const Dev& d, int g, double D, cons
     set_vertex_enabled(d, S, B, onB, false);
     set_vertex_enabled(d, S, C, onC && C != B, false);
     set_grain_enabled(d, S, g, onG, false);
-    set_mod(d, B, 0, FIX_REMOVE, G2, B);
-    set_mod(d, C, 0, FIX_REMOVE, G1, C);
-    set_mod(d, B, 1, FIX_REMOVE, G3, B);
-    set_mod(d, C, 1, FIX_REPLACE, G3, A);
-    d.mods[C].prev[1] = C;
+    const int rB = ed.open(B), rC = ed.open(C);
+    ed.put(rB, 0, FIX_REMOVE, G2, B);
+    ed.put(rC, 0, FIX_REMOVE, G1, C);
+    ed.put(rB, 1, FIX_REMOVE, G3, B);
+    ed.put(rC, 1, FIX_REPLACE, G3, A);
+    ed.put_prev(rC, 1, C);
 #pragma unroll
     for (int i = 0; i < 3; i++) if (gA[i] == g) d.vg[3 * A + i] = G3;
     const int gg[3] = {G2, G1, G3};
     const bool all[3] = {true, true, true};
-    flag(gg, all);
+    ed(gg, all);
 }
 
 
@@ -2751,7 +2776,7 @@ __device__ __forceinline__ void t2_items(const Dev& d, int k0, int stride) {
             d.l_t2c[s] = g;
         } else {
             int m = member_of_grain(d, g);
-            remove_grain(d, g, d.prm[m].D, slot_base(d, m), FlagGlobal{d, 1});
+            remove_grain(d, g, d.prm[m].D, slot_base(d, m), EditGlobal{d, 1});
         }
         wave_count(d, !clash, member_of_grain(d, g), &MState::removals);
     }
@@ -2762,8 +2787,8 @@ __global__ void k_t2_par(Dev d) {
 }
 
 // The conflicting candidates, all labelled, in index order by one lane.
-template <class Flag>
-__device__ __forceinline__ void t2_serial(const Dev& d, int* list, int n, Flag flag) {
+template <class Edit>
+__device__ __forceinline__ void t2_serial(const Dev& d, int* list, int n, Edit ed) {
     sort_ints(list, n);
 #pragma unroll 1
     for (int k = 0; k < n; k++) {
@@ -2771,13 +2796,13 @@ __device__ __forceinline__ void t2_serial(const Dev& d, int* list, int n, Flag f
         if (!d.genab[g]) continue;
         int m = member_of_grain(d, g);
         if (!d.ms[m].active) continue;
-        remove_grain(d, g, d.prm[m].D, slot_base(d, m), flag);
+        remove_grain(d, g, d.prm[m].D, slot_base(d, m), ed);
         atomicAdd(reinterpret_cast<unsigned long long*>(&d.ms[m].removals), 1ull);
     }
 }
 
 __global__ void k_t2_serial(Dev d) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) t2_serial(d, d.l_t2c, cnt_now(d, C_T2C), FlagGlobal{d, 1});
+    if (threadIdx.x == 0 && blockIdx.x == 0) t2_serial(d, d.l_t2c, cnt_now(d, C_T2C), EditGlobal{d, 1});
 }
 
 // unlabel_boundaries_st2, topological.h:588-606; the T2 stage is over, so
@@ -2848,8 +2873,8 @@ __device__ __forceinline__ FlipIn flip_in(const Dev& d, int A, int B) {
 // ends of the rewired edges; the lists of the four grains around; their
 // orientations), then the reference's sequence of tests and writes runs on
 // local copies in the same order and the writes go out.
-template <class Flag>
-__device__ __forceinline__ void flip(const Dev& d, int bnd, const Params& P, const FlipIn& in, Flag flag) {
+template <class Edit>
+__device__ __forceinline__ void flip(const Dev& d, int bnd, const Params& P, const FlipIn& in, Edit ed) {
     const double D = P.D;
     const int A = in.A, B = in.B;
     int vA[3], vB[3], gA[3], gB[3];
@@ -2892,19 +2917,20 @@ __device__ __forceinline__ void flip(const Dev& d, int bnd, const Params& P, con
     const int g2 = f0.ab == 1 ? 0 : (f1.ab == 1 ? 1 : 2), g4 = f0.ba == 1 ? 0 : (f1.ba == 1 ? 1 : 2);
     const int g3 = fn0.a >= 0 ? 0 : (fn1.a >= 0 ? 1 : 2), g1 = fn0.b >= 0 ? 0 : (fn1.b >= 0 ? 1 : 2);
     const int G2 = g2 == 0 ? gi0 : gi1, G4 = g4 == 0 ? gi0 : gi1, G3 = g3 == 0 ? gn0 : gn1, G1 = g1 == 0 ? gn0 : gn1;
-    if (g2 < 2) set_mod(d, A, 0, FIX_REMOVE, G2, A);
-    if (g4 < 2) set_mod(d, B, 0, FIX_REMOVE, G4, B);
+    const int rA = ed.open(A), rB = ed.open(B);
+    if (g2 < 2) ed.put(rA, 0, FIX_REMOVE, G2, A);
+    if (g4 < 2) ed.put(rB, 0, FIX_REMOVE, G4, B);
     if (g3 < 2) {
-        set_mod(d, A, 1, FIX_ADD, G3, B);
-        d.mods[A].prev[1] = A;
+        ed.put(rA, 1, FIX_ADD, G3, B);
+        ed.put_prev(rA, 1, A);
     }
     if (g1 < 2) {
-        set_mod(d, B, 1, FIX_ADD, G1, A);
-        d.mods[B].prev[1] = B;
+        ed.put(rB, 1, FIX_ADD, G1, A);
+        ed.put_prev(rB, 1, B);
     }
     const int gg[4] = {G2, G4, G3, G1};
     const bool want[4] = {g2 < 2, g4 < 2, g3 < 2, g1 < 2};
-    flag(gg, want);
+    ed(gg, want);
     if (g1 > 1 || g2 > 1 || g3 > 1 || g4 > 1) { set_error(d, member_of_edge(d, bnd), SEVC_E_STATE); return; }
 #pragma unroll
     for (int k = 0; k < 3; k++) {
@@ -2977,7 +3003,7 @@ __device__ __forceinline__ void flip_items(const Dev& d, int k0, int stride) {
             d.l_flipc[s] = c;
         } else {
             int m = member_of_edge(d, c);
-            flip(d, c, d.prm[m], fi, FlagGlobal{d, 2});
+            flip(d, c, d.prm[m], fi, EditGlobal{d, 2});
         }
         wave_count(d, !clash, member_of_edge(d, c), &MState::flips);
     }
@@ -2988,8 +3014,8 @@ __global__ void k_flip_par(Dev d) {
 }
 
 // The conflicting candidates, all labelled, in index order by one lane.
-template <class Flag>
-__device__ __forceinline__ void flip_serial(const Dev& d, int* list, int n, Flag flag) {
+template <class Edit>
+__device__ __forceinline__ void flip_serial(const Dev& d, int* list, int n, Edit ed) {
     sort_ints(list, n);
 #pragma unroll 1
     for (int k = 0; k < n; k++) {
@@ -2997,13 +3023,13 @@ __device__ __forceinline__ void flip_serial(const Dev& d, int* list, int n, Flag
         if (!d.benab[c]) continue;
         int m = member_of_edge(d, c);
         if (!d.ms[m].active) continue;
-        flip(d, c, d.prm[m], flip_in(d, d.bvx[2 * c], d.bvx[2 * c + 1]), flag);
+        flip(d, c, d.prm[m], flip_in(d, d.bvx[2 * c], d.bvx[2 * c + 1]), ed);
         atomicAdd(reinterpret_cast<unsigned long long*>(&d.ms[m].flips), 1ull);
     }
 }
 
 __global__ void k_flip_serial(Dev d) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) flip_serial(d, d.l_flipc, cnt_now(d, C_FLIPC), FlagGlobal{d, 2});
+    if (threadIdx.x == 0 && blockIdx.x == 0) flip_serial(d, d.l_flipc, cnt_now(d, C_FLIPC), EditGlobal{d, 2});
 }
 
 // Every event stage of a step (main.cu:202-310) in one launch of one
@@ -3012,46 +3038,58 @@ __global__ void k_flip_serial(Dev d) {
 // of launches.  A launch costs 3 to 4.5 us even when its list is empty and
 // starts with cold caches, so that each dependent load of the next stage goes
 // to memory; here the later stages find what the earlier ones read in the
-// workgroup's own L1 and L2.  2,000 grains, three events a step: 28 us where
-// the launches took 63; a batch of 45 events a step 66 us where they took 105;
-// 1M grains, 27 events a step, 82 us where they took 130.  Its time grows with
+// workgroup's own L1 and L2.  2,000 grains, three events a step: 25 us where
+// the launches took 63; a batch of 45 events a step 51 us where they took 105;
+// 1M grains, 27 events a step, 68 us where they took 130.  Its time grows with
 // the number of edited grains (64 at a time), so busy states take the launches.
 //
 // Up to kEvMax listed edges (one to a lane) a lane keeps its edge's
 // surroundings in registers, and everything the stages exchange goes through
 // LDS: the list position of an edge, the kept edge at a vertex, the labelled
-// grains and the flagged grains are small hash tables, so that no stage waits
-// for an atomic on memory or reads back what another one wrote there (the
-// stages as they are for the launches, one after the other: 28 us at 2,000
-// grains, 66 for the batch, 82 at 1M grains).  Longer lists, and steps with a
-// two-triangle candidate, run the launches' stages.
-// kEvMax: an edge has at most three grains in common with its ends, so at most
-// 3 kEvMax grains are labelled (a lane each), and three grains flagged by each.
-constexpr int kEvMax = 340;
+// and the flagged grains and the vertices' edit records are small hash tables,
+// so that no stage waits for an atomic on memory or reads back what another
+// one wrote there.  A dependent load takes 1.3 us (2,000 grains) to 2.6 us (1M)
+// in this kernel, so what a later stage reads is touched early, together with
+// other loads (ev_touch).  With the launches' stages one after the other in one
+// workgroup it took 28 us at 2,000 grains, 66 for the batch, 82 at 1M; the
+// edit records in LDS (instead of memory) and the early loads are 5 us of it.
+// Longer lists, and steps with a two-triangle candidate, run the launches'
+// stages.
+// Sizes: an edge has at most three grains in common with its ends, so at most
+// 3 kEvMax grains are labelled (a lane each); a removal flags three grains and
+// records edits at two vertices, a flip four and two.
 struct EvLds {
-    static constexpr int kEH = 2048, kVH = 2048, kTH = 2048, kFH = 4096, kT2 = 3 * kEvMax;
+    static constexpr int kEH = 1024, kVH = 1024, kTH = 2048, kFH = 4096, kRH = 2048;
+    static constexpr int kT2 = 3 * kEvMax, kFlag = 3 * kT2, kRec = 2 * kT2;
     int ek[kEH], ep[kEH];             // listed edge -> list position
     int vk[kVH], vp[kVH];             // vertex -> the kept edge at it, kMany if several
     int tk[kTH];                      // labelled grains
-    int fk[kFH], fl[3 * kT2];         // flagged grains (hash) and their list
+    int fk[kFH], fl[kFlag];           // flagged grains (hash) and their list
+    int rk[kRH];                      // vertex -> its edit record (two edits: an event records no more)
+    short ri[kRH];
+    int rv[kRec], rgrn[2][kRec], rvrt[2][kRec], rprev[kRec];
+    unsigned short rfix[kRec];
     int t2[kT2], con[kT2];            // labelled grains, conflicting events
     double ct[kEvMax];
     int cid[kEvMax];
     unsigned char cf[kEvMax];         // the edge's label
-    int nt2, ncon, nfl, changed, two, nslow;
-    int slow[3 * kT2];                // grains for fix_wave
+    int nt2, ncon, nfl, nrec, changed, two, nslow;
+    int slow[kFlag];                  // grains for fix_wave
     QuickLds quick[16];
-    static constexpr int kSlow = 4;
+    static constexpr int kSlow = 3;
     union {
         FixLds fix[kSlow];
-        ClearLds clear[16];
+        ClearLds clear[kSlow];
     } room;
 };
 static_assert(sizeof(EvLds) <= kPollLds, "the event stages' tables fit");
-static_assert(EvLds::kT2 <= 1024 && 4 * kEvMax <= 3 * EvLds::kT2 && 3 * EvLds::kT2 < EvLds::kFH && EvLds::kT2 < EvLds::kTH &&
-                  2 * kEvMax < EvLds::kVH && kEvMax < EvLds::kEH,
+static_assert(EvLds::kT2 <= 1024 && 4 * kEvMax <= EvLds::kFlag && EvLds::kFlag < EvLds::kFH && EvLds::kT2 < EvLds::kTH &&
+                  EvLds::kRec < EvLds::kRH && 2 * kEvMax < EvLds::kVH && kEvMax < EvLds::kEH,
               "every list and table holds what a step can put in");
 constexpr int kFree = -1, kMany = -2;
+
+// Loads x now, so that a later stage finds it in a cache.
+__device__ __forceinline__ void ev_touch(int x) { asm volatile("" ::"v"(x)); }
 
 __device__ __forceinline__ int ev_hash(int x, int size) { return (int)(((unsigned)x * 2654435761u) >> 16) & (size - 1); }
 
@@ -3074,9 +3112,30 @@ __device__ __forceinline__ int ev_put(int* key, int size, int x, bool* fresh) {
     }
 }
 
-// Flags grains in LDS: each once in the list.
-struct FlagLds {
+// An event's list edits in LDS (see EditGlobal).  A vertex's record is filled by
+// one lane: parallel events share no recording vertex.
+struct EditLds {
     EvLds& s;
+    __device__ __forceinline__ int open(int v) const {
+        bool fresh;
+        const int h = ev_put(s.rk, EvLds::kRH, v, &fresh);
+        if (!fresh) return s.ri[h];
+        const int r = atomicAdd(&s.nrec, 1);
+        s.ri[h] = (short)r;
+        s.rv[r] = v;
+        s.rgrn[0][r] = s.rgrn[1][r] = -1;
+        s.rvrt[0][r] = s.rvrt[1][r] = -1;
+        s.rprev[r] = -1;
+        s.rfix[r] = (unsigned short)(0x0101u * (unsigned)FIX_NONE);
+        return r;
+    }
+    __device__ __forceinline__ void put(int r, int slot, int fix, int grn, int vrt) const {
+        s.rgrn[slot][r] = grn;
+        s.rvrt[slot][r] = vrt;
+        const unsigned keep = slot == 0 ? 0xFF00u : 0x00FFu;
+        s.rfix[r] = (unsigned short)((s.rfix[r] & keep) | ((unsigned)fix << (8 * slot)));
+    }
+    __device__ __forceinline__ void put_prev(int r, int, int prev) const { s.rprev[r] = prev; }   // of slot 1
     template <int N>
     __device__ __forceinline__ void operator()(const int (&g)[N], const bool (&want)[N]) const {
 #pragma unroll 1
@@ -3096,27 +3155,77 @@ struct FlagLds {
     }
 };
 
-// The flagged grains' edits, then their clearing (with areas after the T2
-// stage); leaves the flag table empty.
-__device__ __forceinline__ void ev_edit(const Dev& d, EvLds& s, int with_area) {
-    const int tid = (int)threadIdx.x, wave = tid >> 6, lane = tid & 63;
+__device__ __forceinline__ EditRec record_lds(const EvLds& s, int v) {
+    EditRec r = no_edits();
+    const int h = ev_find(s.rk, EvLds::kRH, v);
+    if (s.rk[h] != v) return r;
+    const int k = s.ri[h];
+    r.g[0] = s.rgrn[0][k];
+    r.g[1] = s.rgrn[1][k];
+    r.v[0] = s.rvrt[0][k];
+    r.v[1] = s.rvrt[1][k];
+    r.p[1] = s.rprev[k];
+    r.fix = s.rfix[k] | (0x01010000u * (unsigned)FIX_NONE);
+    return r;
+}
+
+// The flagged grains' edits from the records in LDS, after the T2 stage with
+// the area update of main.cu:266 on the edited lists (the lanes of a list's
+// entries load their points together; the deltas are summed in list order).
+// The vertices' records in memory stay empty, so nothing is cleared there,
+// except for the grains that need fix_wave, which reads them from memory.
+// Leaves the tables of flagged grains and records empty.
+__device__ __forceinline__ void ev_edit(const Dev& d, EvLds& s, bool with_area) {
+    const int tid = (int)threadIdx.x, wave = tid >> 6, lane = tid & 63, l = lane & (kQuick - 1);
     const int n = s.nfl;
-    fix_items(d, n, [&](int k) { return s.fl[k]; }, s.quick[wave], wave, 16, [&](unsigned long long todo, int g) {
-        if ((todo >> lane) & 1ull) s.slow[atomicAdd(&s.nslow, 1)] = g;
-    });
+    QuickLds& q = s.quick[wave];
+    const double2* X = reinterpret_cast<const double2*>(d.pos);
+    fix_items(
+        d, n, [&](int k) { return s.fl[k]; }, [&](int v) { return record_lds(s, v); }, q, wave, 16,
+        [&](unsigned long long todo, int g) {
+            if ((todo >> lane) & 1ull) s.slow[atomicAdd(&s.nslow, 1)] = g;
+        },
+        [&](int g0, int at, int v, bool has, int g, int n2) {
+            if (!with_area) return;                      // the same for every lane
+            wave_sync();
+            if (has) q.nl[g0 + at] = v;
+            wave_sync();
+            const double2 p = l < n2 ? X[q.nl[g0 + l]] : make_double2(0.0, 0.0);
+            const double D = d.prm[n2 >= 0 ? member_of_grain(d, g) : 0].D;
+            const double px = __shfl_up(p.x, 1, kQuick), py = __shfl_up(p.y, 1, kQuick);
+            const double dx = wrapd(p.x, px, D), dy = wrapd(p.y, py, D);
+            AreaAcc acc;
+            acc.start(0.0, 0.0);
+#pragma unroll 1
+            for (int k = 1; __ballot(k < n2); k++) {
+                const double ex = __shfl(dx, k, kQuick), ey = __shfl(dy, k, kQuick);
+                if (k < n2) acc.push_delta(ex, ey);
+            }
+            if (n2 >= 0 && l == 0) d.garea[g] = n2 > 0 ? acc.finish() : 0.0;
+        });
     __syncthreads();
     if (s.nslow > 0) {
+        for (int r = tid; r < s.nrec; r += 1024) {
+            const int v = s.rv[r];
+            for (int j = 0; j < 2; j++) set_mod(d, v, j, (s.rfix[r] >> (8 * j)) & 255, s.rgrn[j][r], s.rvrt[j][r]);
+            d.mods[v].prev[1] = s.rprev[r];
+        }
+        __syncthreads();
         if (wave < EvLds::kSlow)
             for (int k = wave; k < s.nslow; k += EvLds::kSlow) {
                 fix_wave(d, s.slow[k], s.room.fix[wave]);
                 wave_sync();
             }
         __syncthreads();
+        if (wave < EvLds::kSlow)
+            fix_clear_items(d, s.nslow, 0, [&](int k) { return s.slow[k]; }, with_area ? 1 : 0, s.room.clear[wave], wave,
+                            EvLds::kSlow);
+        for (int r = tid; r < s.nrec; r += 1024) reset_mods(d, s.rv[r]);
     }
     for (int h = tid; h < EvLds::kFH; h += 1024) s.fk[h] = kFree;
-    fix_clear_items(d, n, 0, [&](int k) { return s.fl[k]; }, with_area, s.room.clear[wave], wave, 16);
+    for (int h = tid; h < EvLds::kRH; h += 1024) s.rk[h] = kFree;
     __syncthreads();
-    if (tid == 0) s.nfl = s.nslow = 0;
+    if (tid == 0) s.nfl = s.nslow = s.nrec = 0;
     __syncthreads();
 }
 
@@ -3126,21 +3235,21 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, Ev
     const int tid = (int)threadIdx.x;
     const bool on = tid < nc;
     // the edge and its ends
-    int c = -1, m = 0;
-    int2 ab = make_int2(0, 0);
-    double te = 0.0, len = 0.0;
-    if (on) c = d.l_cand[tid];
+    int4 id = make_int4(-1, 0, 0, 0);
+    double2 tl = make_double2(0.0, 0.0);
+    if (on) {
+        id = d.c_id[tid];
+        tl = d.c_te[tid];
+    }
     for (int h = tid; h < EvLds::kEH; h += 1024) s.ek[h] = kFree;
     for (int h = tid; h < EvLds::kVH; h += 1024) { s.vk[h] = kFree; s.vp[h] = kFree; }
     for (int h = tid; h < EvLds::kTH; h += 1024) s.tk[h] = kFree;
     for (int h = tid; h < EvLds::kFH; h += 1024) s.fk[h] = kFree;
-    if (tid == 0) s.nt2 = s.ncon = s.nfl = s.two = s.nslow = 0;
-    if (on) {
-        ab = reinterpret_cast<const int2*>(d.bvx)[c];
-        te = d.bt[c];
-        len = d.blen[c];
-        m = member_of_edge(d, c);
-    }
+    for (int h = tid; h < EvLds::kRH; h += 1024) s.rk[h] = kFree;
+    if (tid == 0) s.nt2 = s.ncon = s.nfl = s.nrec = s.two = s.nslow = 0;
+    const int c = id.x, m = id.w;
+    int2 ab = make_int2(id.y, id.z);
+    const double te = tl.x, len = tl.y;
     __syncthreads();
     if (on) {
         bool fresh;
@@ -3169,6 +3278,19 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, Ev
         gl[q] = on ? d.glen[fi.gA[q]] : 0;
         ge[q] = on && d.genab[fi.gA[q]] != 0;
     }
+    if (cand) {
+        // what a flip of the edge, and the edits after it, read
+        const bool ori = d.prm[m].gb_eps != 0.0;
+        int t[12];
+#pragma unroll
+        for (int q = 0; q < 6; q++) {
+            const int g = q < 3 ? fi.gA[q] : fi.gB[q - 3];
+            t[2 * q] = glist(d, g)[0];
+            t[2 * q + 1] = q < 3 ? (ori ? reinterpret_cast<const int*>(d.gori)[2 * g] : 0) : d.glen[g];
+        }
+#pragma unroll
+        for (int q = 0; q < 12; q++) ev_touch(t[q]);
+    }
     if (on) {
         s.ct[tid] = te;
         s.cid[tid] = c;
@@ -3183,9 +3305,23 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, Ev
         return s.ek[h] == x ? s.ep[h] : -1;
     };
     auto flagp = [&](int p) { return p >= 0 && s.cf[p] != 0; };
+    // (the first probes of the six searches are read together)
     int ep[6];
+    {
+        int hh[6], kk[6];
 #pragma unroll
-    for (int j = 0; j < 6; j++) ep[j] = on ? edge_pos(j < 3 ? fi.vA[j] : fi.vB[j - 3]) : -1;
+        for (int j = 0; j < 6; j++) {
+            hh[j] = ev_hash(j < 3 ? fi.vA[j] : fi.vB[j - 3], EvLds::kEH);
+            kk[j] = s.ek[hh[j]];
+            ep[j] = s.ep[hh[j]];
+        }
+#pragma unroll
+        for (int j = 0; j < 6; j++) {
+            const int x = j < 3 ? fi.vA[j] : fi.vB[j - 3];
+            if (!on || kk[j] == kFree) ep[j] = -1;
+            else if (kk[j] != x) ep[j] = edge_pos(x);
+        }
+    }
 
     // polling (poll_list's rounds)
     auto votes_self = [&](int e) {
@@ -3282,11 +3418,25 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, Ev
             bool be[9];
 #pragma unroll
             for (int e = 0; e < 9; e++) bb[e] = d.vb[3 * vv[e / 3] + e % 3];
+            int gv[9], on3[3];
+            double x3[3];
+            // what the removal reads is loaded with them
+#pragma unroll
+            for (int e = 0; e < 9; e++) gv[e] = d.vg[3 * vv[e / 3] + e % 3];
+#pragma unroll
+            for (int e = 0; e < 3; e++) {
+                x3[e] = d.pos[2 * (size_t)vv[e]];
+                on3[e] = d.ven[vv[e]];
+            }
 #pragma unroll
             for (int e = 0; e < 9; e++) {
                 ends[e] = reinterpret_cast<const int2*>(d.bvx)[bb[e]];
                 be[e] = d.benab[bb[e]] != 0;
             }
+#pragma unroll
+            for (int e = 0; e < 9; e++) ev_touch(gv[e]);
+#pragma unroll
+            for (int e = 0; e < 3; e++) { ev_touch((int)__double2loint(x3[e])); ev_touch(on3[e]); }
             auto in_g = [&](int x) { return x == vv[0] || x == vv[1] || x == vv[2]; };
             bool hit = false;
             int ans = 0, first = INT_MAX;
@@ -3309,7 +3459,7 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, Ev
     }
     __syncthreads();
     const int nt2 = s.nt2;
-    const FlagLds flag{s};
+    const EditLds ed{s};
     if (nt2 > 0) {
         // a candidate with no other one around is removed at once (t2_items)
         bool go = false;
@@ -3333,16 +3483,16 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, Ev
             go = !clash;
         }
         __syncthreads();
-        if (go) remove_grain(d, g, d.prm[mg].D, slot_base(d, mg), flag);
+        if (go) remove_grain(d, g, d.prm[mg].D, slot_base(d, mg), ed);
         wave_count(d, go, mg, &MState::removals);
         __syncthreads();
         if (s.ncon > 0) {
-            if (tid == 0) t2_serial(d, s.con, s.ncon, flag);
+            if (tid == 0) t2_serial(d, s.con, s.ncon, ed);
             __syncthreads();
             if (tid == 0) s.ncon = 0;
         }
         if (tid == 0) d.cnt[C_FIX1] = s.nfl;
-        ev_edit(d, s, 1);
+        ev_edit(d, s, true);
     }
 
     // unlabel_boundaries_st2 (st2_items), then the flips (flip_items); after a
@@ -3381,17 +3531,17 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, Ev
             clash = clash || (x != c && flagp(edge_pos(x)));
         }
         if (clash) s.con[atomicAdd(&s.ncon, 1)] = c;
-        else flip(d, c, d.prm[m], fi, flag);
+        else flip(d, c, d.prm[m], fi, ed);
     }
     wave_count(d, live && !clash, m, &MState::flips);
     __syncthreads();
     if (s.ncon > 0) {
-        if (tid == 0) flip_serial(d, s.con, s.ncon, flag);
+        if (tid == 0) flip_serial(d, s.con, s.ncon, ed);
         __syncthreads();
     }
     if (s.nfl == 0) return true;
     if (tid == 0) d.cnt[C_FIX2] = s.nfl;
-    ev_edit(d, s, 0);
+    ev_edit(d, s, false);
     return true;
 }
 
@@ -3416,14 +3566,7 @@ __global__ void __launch_bounds__(1024) k_events(Dev d) {
     static_assert(8 * sizeof(Room) <= kPollLds, "staging rooms fit");
     Room* const room = reinterpret_cast<Room*>(buf) + wave;
     auto edits = [&](int stage) {
-        if (wave < 8)
-            fix_items(d, cnt_now(d, C_FIX0 + stage), [&](int k) { return d.l_fix[stage][k]; }, room->quick, wave, 8,
-                      [&](unsigned long long todo, int g) {
-                          for (; todo; todo &= todo - 1ull) {
-                              fix_wave(d, __builtin_amdgcn_readlane(g, __ffsll((long long)todo) - 1), room->fix);
-                              wave_sync();
-                          }
-                      });
+        if (wave < 8) fix_stage(d, stage, room->fix, room->quick, wave, 8);
         __syncthreads();
         if (wave < 8) clear_stage(d, stage, stage == 1 ? 1 : 0, room->clear, wave, 8);
         __syncthreads();
@@ -3438,14 +3581,14 @@ __global__ void __launch_bounds__(1024) k_events(Dev d) {
     __syncthreads();
     t2_items(d, tid, nt);
     __syncthreads();
-    if (tid == 0) t2_serial(d, d.l_t2c, cnt_now(d, C_T2C), FlagGlobal{d, 1});
+    if (tid == 0) t2_serial(d, d.l_t2c, cnt_now(d, C_T2C), EditGlobal{d, 1});
     __syncthreads();
     edits(1);
     st2_items(d, tid, nt);
     __syncthreads();
     flip_items(d, tid, nt);
     __syncthreads();
-    if (tid == 0) flip_serial(d, d.l_flipc, cnt_now(d, C_FLIPC), FlagGlobal{d, 2});
+    if (tid == 0) flip_serial(d, d.l_flipc, cnt_now(d, C_FLIPC), EditGlobal{d, 2});
     __syncthreads();
     edits(2);
 }

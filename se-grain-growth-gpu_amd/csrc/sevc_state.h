@@ -22,6 +22,7 @@ constexpr int kPollBig = 16384;      // lists up to this length poll with flags 
 // edits fewer than kBusyUnder makes it calm (member_reduce): a calm state's
 // events run in one workgroup (k_events), a busy one's in a launch per stage.
 // The line is where both cost the same (see k_events).
+constexpr int kEvMax = 192;          // longest candidate list that k_events runs in LDS
 constexpr int kHeadGrains = 8192;    // largest member whose candidates k_head draws itself
 constexpr int kHeadEvents = 8;       // most nucleations a member may expect for k_head to apply them itself
 constexpr int kBusyOver = 320, kBusyUnder = 160;
@@ -107,6 +108,7 @@ struct Dev {
     int* cnt;
     int* l_cand; int* l_two; int* l_t2; int* l_t2c; int* l_flipc;
     int* l_fix[kFixStages]; int* l_dirty; int* l_nucl; int* l_conf; int* l_vfall;
+    int4* c_id; double2* c_te;            // the first kEvMax listed edges: (edge, its ends, member), (t_ext, length)
     int* l_tri;                           // grains that an edit left with three vertices (next two-triangle search)
     int* l_bigr;                          // grains longer than the lane-per-grain velocity pass holds
     int* nrec; double* nal;               // rate-mode candidate sites: (site or -1, its 3 grains), shortest edge
