@@ -172,7 +172,11 @@ __device__ __forceinline__ void end_member(const Dev& d, int m) {
 #pragma unroll
         for (int q = 0; q < kBatch; q++) { a += tg[q]; b2 += tv[q]; }
     }
-    if (!M.active || !M.open) return;                // the same for the whole workgroup
+    // thread 0 may go on to begin the next step, which opens the member: every
+    // wave has to have read the flags before that
+    const bool sum_up = M.active && M.open;
+    __syncthreads();
+    if (!sum_up) return;
     a = wave_sum(a);
     b2 = wave_sum(b2);
     if (lane == 0) { sa[wave] = a; sb[wave] = b2; }
