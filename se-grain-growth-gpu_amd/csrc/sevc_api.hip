@@ -425,7 +425,7 @@ void launch_step(sevc_state* s, bool diag) {
     const bool all_energies = diag || s->any_aniso || s->ben_dirty;
     const int nucl = HEAD_SELECT | (s->head_draw ? HEAD_DRAW : 0) | (s->head_insert ? HEAD_INSERT : 0);
     if (s->any_rate && !s->head_draw) launch(s, "rate_draw", k_rate_draw, d.ngb, kBlock, d);
-    if (all_energies || !s->any_nucl) {
+    if (all_energies || s->any_analytic || !s->any_nucl) {
         launch(s, "begin", k_begin, s->B, 256, d, all_energies ? 0 : 1);
         if (all_energies) launch(s, "edge_len_energy", k_edge_len_energy, d.neb, kBlock, d, 0);
         s->ben_dirty = false;
