@@ -1,6 +1,7 @@
 """The ways a step's launches can go, against the oracle bit for bit: the
 analytic velocity with nucleation (areas on every step, whatever computes the
-energies)."""""
+energies), and candidate lists on both sides of what the event stages hold in
+LDS, few and many edits a step, with removals and two-triangle pairs."""
 import numpy as np
 import pytest
 
@@ -51,3 +52,13 @@ def test_analytic_with_nucleation(nucl, gb_eps, graph):
         o, mesh = _start(n, 31, side=20.0, **kw)
         mesh["g_SE"][:] = 3.0 + 6.0 * mesh["g_SE"]
     assert _same(o, mesh, [1, 12, 17], graph)[3] > 0
+
+
+# candidates a step (192 fit the stages' LDS tables): below 80; below 140; 233
+# to 46; 278 to 47; 841 to 212, past what one workgroup is given at first
+@pytest.mark.parametrize("n,flip", [(90, 0.9), (180, 0.9), (500, 0.7), (2000, 0.5), (2000, 0.7)])
+@pytest.mark.parametrize("calls", [[1] * 14, [14]])
+def test_list_lengths(n, flip, calls):
+    o, mesh = _start(n, 5, adaptive_dt=0, dt=1e-5, do_nucleation=0, flip_threshold=flip / np.sqrt(n))
+    total = _same(o, mesh, calls)
+    assert total[0] > 20 and total[1] > 3
