@@ -29,7 +29,7 @@ __global__ void k_win_prepare(Dev d) {
 // The window's topology is fixed, so what every step would look up again
 // (a vertex's edges, their far ends, its place in its three grains' lists,
 // the list neighbours there) is looked up once per window and kept in
-// vertex and grain order:
+// vertex order:
 //   nbr[v]  (w0, w1, w2, code): the far ends of the vertex's edges and, per
 //           grain slot j, which of them are the list's previous and next
 //           vertex (code bits 4j..4j+1 and 4j+2..4j+3) and whether the slot
@@ -40,100 +40,157 @@ __global__ void k_win_prepare(Dev d) {
 //   vse[3v + j]  stored energy of grain slot j
 //   veb[3v + j]  d gamma_b / d GB_scaling of edge j (null when every member
 //           has GB_eps = 0, where it is 1)
-//   wl[kq G + g]  entries 4 kq .. 4 kq + 3 of grain g's list, wn[g] its length
-//           (-1: disabled)
-// A step then takes two rounds of loads (these tables, then positions and
-// area signs) in place of six dependent ones.  Measured, 10,000 grains: the
-// step kernel 10.7 -> 4.6 us, the reverse step 11.4 -> 5.1, the areas 6.4 ->
-// 4.3 (an empty launch takes 4.5 in a busy stream: what is left is dispatch);
-// 16 members of 11,000 grains: 34.8 -> 12.4, 49.0 -> 18.5, 14.0 -> 8.5.
+// and the grains' lists in one of two ways.  Where the vertices are ordered
+// along the mesh (win_own_rule), a table block's 256 vertices have about 160
+// grains between them, and the step's workgroup forms their area signs itself:
+//   wb.count[lb]  grains at the enabled vertices of block lb, at most kWinGrains
+//   wb.grain[lb kWinGrains + k]  the k-th one and its list's length (-1: disabled)
+//   wb.list[(kq nvb + lb) kWinGrains + k]  entries 4 kq .. 4 kq + 3 of its list
+//   wb.loc[v]  the block's numbers of the vertex's three grains, 10 bits each
+// Each grain's area is then formed by 1.3 workgroups on average, but a step is
+// one launch and its two chains of loads run side by side: 10,000 grains 6.2 us
+// a step (areas 4.3 and step 4.7 as two launches), 40,000 8.2 (11.3); 16 members
+// of 11,000 the same 20.  Otherwise
+//   wl[kq G + g], wn[g]  the same per grain, for a launch of k_win_area per step.
 constexpr int kWinOn = 1 << 16, kWinSearch = 1 << 15;
 constexpr int kWinList = 12;                 // list entries held in the table (longer lists are read on)
+constexpr int kWinGrains = kWinBlockGrains;
+static_assert(kWinGrains == 3 * kBlock && kWinGrains <= 1024, "three grains a vertex, numbered in 10 bits");
 
-__global__ void k_win_table_v(Dev d, int4* nbr, double* vse, double* veb) {
+__device__ __forceinline__ void win_list4(const Dev& d, int g, int n, int q, int (&e)[4]) {
+    const int* L = glist(d, g);
+#pragma unroll
+    for (int r = 0; r < 4; r++) e[r] = 4 * q + r < n ? L[4 * q + r] : 0;
+}
+
+__global__ void __launch_bounds__(kBlock) k_win_table_v(Dev d, int4* nbr, double* vse, double* veb, WinBlocks wb) {
     TABLE_BLOCK(d.vblk, d.nvb)
-    if (i >= bd_.e) return;
     const int v = i;
-    if (!d.ven[v]) {
-        nbr[v] = make_int4(v, v, v, 0);
-        return;
-    }
-    int w[3], code = kWinOn;
+    const bool in = i < bd_.e, on = in && d.ven[v] != 0;
+    int vg[3] = {0, 0, 0};
+    if (in && !on) nbr[v] = make_int4(v, v, v, 0);
+    if (on) {
+        int w[3], code = kWinOn;
 #pragma unroll
-    for (int j = 0; j < 3; j++) {
-        const int b = d.vb[3 * v + j];
-        w[j] = other_end(d, b, v);
-        if (veb) veb[3 * (size_t)v + j] = (P.gb_eps == 0.0) ? 1.0 : boundary_compute_energy(d, b, P.gb_eps);
-    }
+        for (int j = 0; j < 3; j++) {
+            const int b = d.vb[3 * v + j];
+            w[j] = other_end(d, b, v);
+            if (veb) veb[3 * (size_t)v + j] = (P.gb_eps == 0.0) ? 1.0 : boundary_compute_energy(d, b, P.gb_eps);
+        }
 #pragma unroll
-    for (int j = 0; j < 3; j++) {
-        const int g = d.vg[3 * v + j];
-        const int n = d.glen[g];
-        const int k = grain_contains_vertex(d, g, v);
-        vse[3 * (size_t)v + j] = d.gse[g];
-        if (k < 0 || n < 3) continue;
-        const int* L = glist(d, g);
-        const int wp = L[(k + n - 1) % n], wn = L[(k + 1) % n];
-        const int ip = wp == w[0] ? 0 : (wp == w[1] ? 1 : (wp == w[2] ? 2 : 3));
-        const int in = wn == w[0] ? 0 : (wn == w[1] ? 1 : (wn == w[2] ? 2 : 3));
-        if (ip == 3 || in == 3) code |= kWinSearch;
-        code |= (ip << (4 * j)) | (in << (4 * j + 2)) | (1 << (12 + j));
+        for (int j = 0; j < 3; j++) {
+            const int g = d.vg[3 * v + j];
+            const int n = d.glen[g];
+            const int k = grain_contains_vertex(d, g, v);
+            vg[j] = g;
+            vse[3 * (size_t)v + j] = d.gse[g];
+            if (k < 0 || n < 3) continue;
+            const int* L = glist(d, g);
+            const int wp = L[(k + n - 1) % n], wn = L[(k + 1) % n];
+            const int ip = wp == w[0] ? 0 : (wp == w[1] ? 1 : (wp == w[2] ? 2 : 3));
+            const int in = wn == w[0] ? 0 : (wn == w[1] ? 1 : (wn == w[2] ? 2 : 3));
+            if (ip == 3 || in == 3) code |= kWinSearch;
+            code |= (ip << (4 * j)) | (in << (4 * j + 2)) | (1 << (12 + j));
+        }
+        nbr[v] = make_int4(w[0], w[1], w[2], code);
     }
-    nbr[v] = make_int4(w[0], w[1], w[2], code);
+    if (!wb.loc) return;
+    // the block's grains, numbered by a table of the grains met so far
+    constexpr int kSlots = 2048;
+    __shared__ int key[kSlots], num[kSlots], met[kWinGrains], n_met;
+    for (int h = (int)threadIdx.x; h < kSlots; h += kBlock) key[h] = -1;
+    if (threadIdx.x == 0) n_met = 0;
+    __syncthreads();
+    int at[3] = {0, 0, 0};
+    if (on)
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            int h = (int)(((unsigned)vg[j] * 2654435761u) >> 16) & (kSlots - 1);
+            for (;; h = (h + 1) & (kSlots - 1)) {
+                const int was = atomicCAS(&key[h], -1, vg[j]);
+                if (was == -1) {
+                    num[h] = atomicAdd(&n_met, 1);
+                    met[num[h]] = vg[j];
+                }
+                if (was == -1 || was == vg[j]) break;
+            }
+            at[j] = h;
+        }
+    __syncthreads();
+    if (in) wb.loc[v] = on ? num[at[0]] | (num[at[1]] << 10) | (num[at[2]] << 20) : 0;
+    const int n = n_met;
+    if (threadIdx.x == 0) wb.count[lb_] = n;
+    for (int k = (int)threadIdx.x; k < n; k += kBlock) {
+        const int g = met[k], len = d.genab[g] ? d.glen[g] : -1;
+        wb.grain[(size_t)lb_ * kWinGrains + k] = make_int2(g, len);
+#pragma unroll
+        for (int q = 0; q < kWinList / 4; q++) {
+            int e[4];
+            win_list4(d, g, len, q, e);
+            wb.list[((size_t)q * d.nvb + lb_) * kWinGrains + k] = make_int4(e[0], e[1], e[2], e[3]);
+        }
+    }
 }
 
 __global__ void k_win_table_g(Dev d, int4* wl, int* wn) {
     TABLE_BLOCK(d.gblk, d.ngb)
     if (i >= bd_.e) return;
     const int n = d.genab[i] ? d.glen[i] : -1;
-    const int* L = glist(d, i);
     wn[i] = n;
 #pragma unroll
     for (int q = 0; q < kWinList / 4; q++) {
         int e[4];
-#pragma unroll
-        for (int r = 0; r < 4; r++) e[r] = 4 * q + r < n ? L[4 * q + r] : 0;
+        win_list4(d, i, n, q, e);
         wl[(size_t)q * d.G + i] = make_int4(e[0], e[1], e[2], e[3]);
     }
 }
 
-// Signs of the grain areas at positions X (compute_grain_areas,
-// calculus.h:224-234; the analytic force needs no more of them): neg[g] = 1
-// for a negative area.  The areas themselves go to `area` when given (the
-// last step of the window's forward leaves them in the state).
-__global__ void k_win_area(Dev d, const double* X, const int4* wl, const int* wn, uint8_t* neg, double* area) {
-    TABLE_BLOCK(d.gblk, d.ngb)
-    if (i >= bd_.e) return;
-    const int n = wn[i];
-    int L[kWinList];
-#pragma unroll
-    for (int q = 0; q < kWinList / 4; q++) {
-        const int4 t = wl[(size_t)q * d.G + i];
-        L[4 * q] = t.x; L[4 * q + 1] = t.y; L[4 * q + 2] = t.z; L[4 * q + 3] = t.w;
-    }
-    if (n < 0) return;
-    const double2* X2 = reinterpret_cast<const double2*>(X);
+// Area of grain g (list length n > 0, its first entries in L) at positions X
+// (compute_grain_areas, calculus.h:224-234).
+__device__ __forceinline__ double win_area(const Dev& d, const double2* X2, int g, int n, const int (&L)[kWinList], double D) {
     double2 p[kWinList];
 #pragma unroll
     for (int k = 0; k < kWinList; k++) p[k] = k < n ? X2[L[k]] : make_double2(0.0, 0.0);
-    const double D = P.D;
-    double a = 0.0;
-    if (n > 0) {
-        AreaAcc acc;
-        acc.start(p[0].x, p[0].y);
+    if (n <= 0) return 0.0;
+    AreaAcc acc;
+    acc.start(p[0].x, p[0].y);
 #pragma unroll
-        for (int k = 1; k < kWinList; k++)
-            if (k < n) acc.push(p[k].x, p[k].y, D);
-        if (n > kWinList) {
-            const int* Lg = glist(d, i);
-            for (int k = kWinList; k < n; k++) {
-                const double2 q = X2[Lg[k]];
-                acc.push(q.x, q.y, D);
-            }
+    for (int k = 1; k < kWinList; k++)
+        if (k < n) acc.push(p[k].x, p[k].y, D);
+    if (n > kWinList) {
+        const int* Lg = glist(d, g);
+        for (int k = kWinList; k < n; k++) {
+            const double2 q = X2[Lg[k]];
+            acc.push(q.x, q.y, D);
         }
-        a = acc.finish();
     }
-    neg[i] = a < 0 ? 1 : 0;
+    return acc.finish();
+}
+
+// Signs of the grain areas at positions X (the analytic force needs no more of
+// them): neg[g] = 1 for a negative area, where the steps' workgroups do not form
+// them themselves (wl given).  The areas go to `area` when given (the last step
+// of the window's forward leaves them in the state).
+__global__ void k_win_area(Dev d, const double* X, const int4* wl, const int* wn, uint8_t* neg, double* area) {
+    TABLE_BLOCK(d.gblk, d.ngb)
+    if (i >= bd_.e) return;
+    const int n = wl ? wn[i] : (d.genab[i] ? d.glen[i] : -1);
+    int L[kWinList];
+#pragma unroll
+    for (int q = 0; q < kWinList / 4; q++) {
+        int e[4];
+        if (wl) {
+            const int4 t = wl[(size_t)q * d.G + i];
+            e[0] = t.x; e[1] = t.y; e[2] = t.z; e[3] = t.w;
+        } else {
+            win_list4(d, i, n, q, e);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) L[4 * q + r] = e[r];
+    }
+    if (n < 0) return;
+    const double a = win_area(d, reinterpret_cast<const double2*>(X), i, n, L, P.D);
+    if (neg) neg[i] = a < 0 ? 1 : 0;
     if (area) area[i] = a;
 }
 
@@ -156,30 +213,71 @@ __device__ __forceinline__ double2 pick3(double2 a, double2 b, double2 c, int k)
 // One window step x_n -> x_{n+1}: analytic velocity (calculus.h:143-154
 // with the analytic model, the sums of analytic_force_at) and
 // update_vertices_positions (calculus.h:391-404), written to a separate
-// array so that neighbours still read x_n.  Disabled slots are copied.
-__global__ void __launch_bounds__(kBlock) k_win_step(Dev d, const double* X, const uint8_t* neg, const int4* nbr,
-                                                     const double* vse, const double* veb, double* Xn, int write_vel) {
+// array so that neighbours still read x_n.  Disabled slots are copied.  The
+// area signs of the vertex's three grains go to sgn, for the reverse step.
+// kOwn: the workgroup forms them itself from its block's lists (wb), else they
+// are in neg.  A step at 10,000 grains or fewer is bound by the latency of its
+// launches and loads (an empty launch takes 4.5 us in a busy stream), so the
+// areas' lists are read unconditionally, with the vertices' own data, and both
+// gathers of positions are in flight together.
+template <bool kOwn>
+__global__ void __launch_bounds__(kBlock) k_win_step(Dev d, const double* X, const uint8_t* neg, WinBlocks wb,
+                                                     const int4* nbr, const double* vse, const double* veb, double* Xn,
+                                                     uint8_t* sgn, int write_vel) {
     TABLE_BLOCK(d.vblk, d.nvb)
-    if (i >= bd_.e) return;
+    __shared__ uint8_t own[kOwn ? kWinGrains : 1];
+    const bool in = i < bd_.e;
     const double2* X2 = reinterpret_cast<const double2*>(X);
-    const int4 t = nbr[i];
-    const double2 p = X2[i];
-    int g[3];
+    const int iv = in ? i : bd_.b;
+    const int4 t = nbr[iv];
+    const double2 p = X2[iv];
     double se[3], eb[3];
+    uint8_t ng[3];
 #pragma unroll
     for (int j = 0; j < 3; j++) {
-        g[j] = d.vg[3 * i + j];
-        se[j] = vse[3 * (size_t)i + j];
-        eb[j] = veb ? veb[3 * (size_t)i + j] : 1.0;
+        se[j] = vse[3 * (size_t)iv + j];
+        eb[j] = veb ? veb[3 * (size_t)iv + j] : 1.0;
     }
+    double2 q[3];
+    if (kOwn) {
+        const int loc = wb.loc[iv], n_own = wb.count[lb_];
+        const size_t row = (size_t)lb_ * kWinGrains, qs = (size_t)d.nvb * kWinGrains;
+        int k = (int)threadIdx.x;
+        int2 gn = wb.grain[row + k];
+        int4 l[kWinList / 4];
+#pragma unroll
+        for (int r = 0; r < kWinList / 4; r++) l[r] = wb.list[r * qs + row + k];
+        q[0] = X2[t.x]; q[1] = X2[t.y]; q[2] = X2[t.z];
+        while (k < n_own) {
+            int L[kWinList];
+#pragma unroll
+            for (int r = 0; r < kWinList / 4; r++) {
+                L[4 * r] = l[r].x; L[4 * r + 1] = l[r].y; L[4 * r + 2] = l[r].z; L[4 * r + 3] = l[r].w;
+            }
+            own[k] = win_area(d, X2, gn.x, gn.y, L, P.D) < 0 ? 1 : 0;
+            k += kBlock;
+            if (k >= n_own) break;
+            gn = wb.grain[row + k];
+#pragma unroll
+            for (int r = 0; r < kWinList / 4; r++) l[r] = wb.list[r * qs + row + k];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 3; j++) ng[j] = own[(loc >> (10 * j)) & 1023];
+    } else {
+        int g[3];
+#pragma unroll
+        for (int j = 0; j < 3; j++) g[j] = d.vg[3 * iv + j];
+        q[0] = X2[t.x]; q[1] = X2[t.y]; q[2] = X2[t.z];
+#pragma unroll
+        for (int j = 0; j < 3; j++) ng[j] = (t.w & kWinOn) ? neg[g[j]] : 0;
+    }
+    if (!in) return;
     if (!(t.w & kWinOn)) {
         reinterpret_cast<double2*>(Xn)[i] = p;
         return;
     }
-    const double2 q[3] = {X2[t.x], X2[t.y], X2[t.z]};
-    uint8_t ng[3];
-#pragma unroll
-    for (int j = 0; j < 3; j++) ng[j] = neg[g[j]];
+    sgn[i] = (uint8_t)(ng[0] | (ng[1] << 1) | (ng[2] << 2));
     const double D = P.D, x = p.x, y = p.y;
     double ex = 0.0, ey = 0.0, gx = 0.0, gy = 0.0;
 #pragma unroll
@@ -198,7 +296,7 @@ __global__ void __launch_bounds__(kBlock) k_win_step(Dev d, const double* X, con
         double2 a, b;
         if (t.w & kWinSearch) {
             int wp, wn;
-            win_search(d, i, g[j], &wp, &wn);
+            win_search(d, i, d.vg[3 * i + j], &wp, &wn);
             a = X2[wp];
             b = X2[wn];
         } else {
@@ -247,7 +345,7 @@ __global__ void k_win_init(Dev d, double* lam, double* acc_mu, double* acc_s, do
 }
 
 // One reverse step at vertex v, with lambda = dL/dx_{n+1} and the state
-// x_n (positions X, area signs neg):
+// x_n (positions X, area signs of the vertex's grains sgn):
 //   lambda_n  = lambda - dt mu (H lambda)_v
 //   acc_mu   += dt (lambda . F_v)
 //   acc_s    += dt mu (lambda . dF_v/dGB_scaling),  dF_v/ds = -sum_b e_b u_b
@@ -256,7 +354,7 @@ __global__ void k_win_init(Dev d, double* lam, double* acc_mu, double* acc_s, do
 // (gamma_b / L)(I - u u^T)(lambda_v - lambda_w) to (H lambda)_v; a grain g
 // with list neighbours prev, next adds
 // SE_g sign(A_g)/2 (lambda_next.y - lambda_prev.y, lambda_prev.x - lambda_next.x).
-__global__ void __launch_bounds__(kBlock) k_win_adjoint(Dev d, const double* X, const uint8_t* neg, const int4* nbr,
+__global__ void __launch_bounds__(kBlock) k_win_adjoint(Dev d, const double* X, const uint8_t* sgn, const int4* nbr,
                                                         const double* vse, const double* veb, const double* lam,
                                                         double* lam2, double* acc_mu, double* acc_s, double* acc_se) {
     TABLE_BLOCK(d.vblk, d.nvb)
@@ -266,11 +364,10 @@ __global__ void __launch_bounds__(kBlock) k_win_adjoint(Dev d, const double* X, 
     const double2* M2 = reinterpret_cast<const double2*>(lam);
     const int4 t = nbr[v];
     const double2 p = X2[v], l = M2[v];
-    int g[3];
+    const int sb = sgn[v];
     double se[3], ebs[3], ase[3];
 #pragma unroll
     for (int j = 0; j < 3; j++) {
-        g[j] = d.vg[3 * v + j];
         se[j] = vse[3 * (size_t)v + j];
         ebs[j] = veb ? veb[3 * (size_t)v + j] : 1.0;
         ase[j] = acc_se[3 * (size_t)v + j];
@@ -282,9 +379,6 @@ __global__ void __launch_bounds__(kBlock) k_win_adjoint(Dev d, const double* X, 
     }
     const double2 q[3] = {X2[t.x], X2[t.y], X2[t.z]};
     const double2 m[3] = {M2[t.x], M2[t.y], M2[t.z]};
-    uint8_t ng[3];
-#pragma unroll
-    for (int j = 0; j < 3; j++) ng[j] = neg[g[j]];
     const double D = P.D, mu = P.mobility, dt = P.dt_max, dtm = dt * mu;
     const double x = p.x, y = p.y;
     const double lx = l.x, ly = l.y;
@@ -315,7 +409,7 @@ __global__ void __launch_bounds__(kBlock) k_win_adjoint(Dev d, const double* X, 
         double2 a, b, la, lb;
         if (t.w & kWinSearch) {
             int wp, wn;
-            win_search(d, v, g[j], &wp, &wn);
+            win_search(d, v, d.vg[3 * v + j], &wp, &wn);
             a = X2[wp];
             b = X2[wn];
             la = M2[wp];
@@ -329,7 +423,7 @@ __global__ void __launch_bounds__(kBlock) k_win_adjoint(Dev d, const double* X, 
         }
         const double dpx = wrapd(x, a.x, D), dpy = wrapd(y, a.y, D);
         const double dnx = wrapd(b.x, x, D), dny = wrapd(b.y, y, D);
-        const double sg = ng[j] ? -1.0 : 1.0;
+        const double sg = (sb >> j) & 1 ? -1.0 : 1.0;
         const double c = se[j] * sg * 0.5;
         gx += c * (dpy + dny);
         gy += c * (-(dpx + dnx));
@@ -345,6 +439,11 @@ __global__ void __launch_bounds__(kBlock) k_win_adjoint(Dev d, const double* X, 
     acc_s[v] = as + dtm * (-(lx * sx + ly * sy));
     reinterpret_cast<double2*>(lam2)[v] = make_double2(lx - dtm * hx, ly - dtm * hy);
 }
+
+template __global__ void k_win_step<false>(Dev, const double*, const uint8_t*, WinBlocks, const int4*, const double*,
+                                           const double*, double*, uint8_t*, int);
+template __global__ void k_win_step<true>(Dev, const double*, const uint8_t*, WinBlocks, const int4*, const double*,
+                                          const double*, double*, uint8_t*, int);
 
 // Level 1 of the deterministic parameter sums: one lane per 256-vertex
 // table block sums its enabled slots left to right (the chunks of the

@@ -56,14 +56,15 @@ __global__ void k_nucl_insert(Dev d);
 __global__ void k_pack(PackList L, char* out);
 // kernels of sevc_adjoint.hip
 __global__ void k_win_prepare(Dev d);
-__global__ void k_win_table_v(Dev d, int4* nbr, double* vse, double* veb);
+__global__ void k_win_table_v(Dev d, int4* nbr, double* vse, double* veb, WinBlocks wb);
 __global__ void k_win_table_g(Dev d, int4* wl, int* wn);
 __global__ void k_win_area(Dev d, const double* X, const int4* wl, const int* wn, uint8_t* neg, double* area);
-__global__ void k_win_step(Dev d, const double* X, const uint8_t* neg, const int4* nbr, const double* vse,
-                           const double* veb, double* Xn, int write_vel);
+template <bool kOwn>
+__global__ void k_win_step(Dev d, const double* X, const uint8_t* neg, WinBlocks wb, const int4* nbr, const double* vse,
+                           const double* veb, double* Xn, uint8_t* sgn, int write_vel);
 __global__ void k_win_end(Dev d, int steps);
 __global__ void k_win_init(Dev d, double* lam, double* acc_mu, double* acc_s, double* acc_se);
-__global__ void k_win_adjoint(Dev d, const double* X, const uint8_t* neg, const int4* nbr, const double* vse,
+__global__ void k_win_adjoint(Dev d, const double* X, const uint8_t* sgn, const int4* nbr, const double* vse,
                               const double* veb, const double* lam, double* lam2, double* acc_mu, double* acc_s,
                               double* acc_se);
 __global__ void k_win_sum_l1(Dev d, const double* acc_mu, const double* acc_s, double* part);
@@ -152,17 +153,19 @@ struct sevc_state {
     char *stage_d = nullptr, *stage_h = nullptr;
     size_t stage_n = 0;
     // topology-fixed window: checkpoints of x every K steps (ck), the
-    // positions and area signs of one segment (seg, segN; `holds` = its
-    // index), the topology tables of the steps (k_win_table_v / _g), and the
+    // positions and area signs at the vertices of one segment (seg, segN;
+    // `holds` = its index), the topology tables of the steps (k_win_table_v /
+    // _g: the lists by table block where `own`, else by grain), and the
     // reverse-pass arrays
     struct Window {
         int steps = 0, K = 0, nck = 0, holds = -1;
-        bool ready = false;
+        bool ready = false, own = true;
         double *ck = nullptr, *seg = nullptr;
-        uint8_t* segN = nullptr;
+        uint8_t *segN = nullptr, *neg = nullptr;
         size_t ck_n = 0, seg_n = 0, segN_n = 0;
         int4 *nbr = nullptr, *wl = nullptr;
         int* wn = nullptr;
+        WinBlocks wb{};
         double *vse = nullptr, *veb = nullptr;   // veb: only with a member of GB_eps != 0
         double *lamA = nullptr, *lamB = nullptr, *acc_mu = nullptr, *acc_s = nullptr, *acc_se = nullptr;
         double *part = nullptr, *out = nullptr, *dse = nullptr;
@@ -351,6 +354,28 @@ int pick_vtile(const sevc_state* s, const std::vector<int>& vg, const std::vecto
     for (int VT : {64, 32})
         if (100 * vtile_overflow(s, VT, vg, ven, glen) <= nen) return VT;
     return 0;
+}
+
+// Whether the steps of a topology-fixed window form the area signs in their own
+// workgroups: each block of 256 vertices then forms all its grains', 162 where
+// the vertices are ordered along the mesh (1.3 times the grains in all), but up
+// to 768 (6 times) where they are not.  Up to 512 blocks (131,072 vertices, two
+// workgroups a CU) the chip has room for that; above, a sample of the blocks has
+// to have at most kWinOwnMost grains each on average.
+constexpr int kWinOwnMost = 256;
+bool win_own_rule(const sevc_state* s, const std::vector<int>& vg, const std::vector<uint8_t>& ven) {
+    const size_t nb = s->V / kBlock, every = std::max<size_t>(1, nb / 64);
+    if (nb <= 512) return true;
+    size_t met = 0, seen = 0;
+    std::vector<int> g;
+    for (size_t b = 0; b < nb; b += every, ++seen) {
+        g.clear();
+        for (size_t v = b * kBlock; v < (b + 1) * kBlock; ++v)
+            if (ven[v]) g.insert(g.end(), vg.begin() + 3 * v, vg.begin() + 3 * v + 3);
+        std::sort(g.begin(), g.end());
+        met += std::unique(g.begin(), g.end()) - g.begin();
+    }
+    return met <= kWinOwnMost * seen;
 }
 
 // Tile table of the one-pass velocity: VT consecutive vertex slots of one
@@ -773,6 +798,7 @@ int sevc_batch_create(const sevc_options* opts, const sevc_mesh* meshes, int32_t
         }
         s->vel_path = 0;
     }
+    s->win.own = win_own_rule(s, vg, ven);
     UP(d.pos, pos.data(), pos.size() * 8); UP(d.vel, vel.data(), vel.size() * 8);
     UP(d.vb, vb.data(), vb.size() * 4); UP(d.vg, vg.data(), vg.size() * 4); UP(d.ven, ven.data(), V);
     UP(d.venergy, venergy.data(), V * 8); UP(d.vparts, vparts.data(), 4 * V * 8);
@@ -1596,13 +1622,16 @@ int win_buffer(sevc_state* s, T** p, size_t* have, size_t n) {
 int win_fixed_buffers(sevc_state* s) {
     auto& w = s->win;
     if (w.dse) return SEVC_OK;               // the last one allocated below
-    const size_t V = s->V, n2 = 2 * V;
+    const size_t V = s->V, G = s->G, n2 = 2 * V, nvb = static_cast<size_t>(s->d.nvb);
     int rc;
     if ((rc = dalloc(s, &w.lamA, n2)) || (rc = dalloc(s, &w.lamB, n2)) || (rc = dalloc(s, &w.acc_mu, V)) ||
         (rc = dalloc(s, &w.acc_s, V)) || (rc = dalloc(s, &w.acc_se, 3 * V)) ||
         (rc = dalloc(s, &w.nbr, V)) || (rc = dalloc(s, &w.vse, 3 * V)) ||
         (s->any_aniso && (rc = dalloc(s, &w.veb, 3 * V)) != SEVC_OK) ||
-        (rc = dalloc(s, &w.wl, 3 * static_cast<size_t>(s->G))) || (rc = dalloc(s, &w.wn, static_cast<size_t>(s->G))) ||
+        (w.own ? (rc = dalloc(s, &w.wb.loc, V)) || (rc = dalloc(s, &w.wb.count, nvb)) ||
+                     (rc = dalloc(s, &w.wb.grain, kWinBlockGrains * nvb)) ||
+                     (rc = dalloc(s, &w.wb.list, 3 * kWinBlockGrains * nvb))
+               : (rc = dalloc(s, &w.wl, 3 * G)) || (rc = dalloc(s, &w.wn, G)) || (rc = dalloc(s, &w.neg, G))) ||
         (rc = dalloc(s, &w.part, 4 * static_cast<size_t>(s->d.nvb))) ||
         (rc = dalloc(s, &w.out, 2 * static_cast<size_t>(s->B))) ||
         (rc = dalloc(s, &w.dse, static_cast<size_t>(s->G))))
@@ -1620,12 +1649,13 @@ void win_run_segment(sevc_state* s, int len, int last) {
     const size_t n2 = 2 * static_cast<size_t>(s->V);
     for (int i = 0; i < len; ++i) {
         const double* X = w.seg + i * n2;
-        uint8_t* neg = w.segN + static_cast<size_t>(i) * s->G;
-        launch(s, "win_area", k_win_area, d.ngb, kBlock, d, X, static_cast<const int4*>(w.wl),
-               static_cast<const int*>(w.wn), neg, i == last ? d.garea : static_cast<double*>(nullptr));
-        launch(s, "win_step", k_win_step, d.nvb, kBlock, d, X, static_cast<const uint8_t*>(neg),
-               static_cast<const int4*>(w.nbr), static_cast<const double*>(w.vse), static_cast<const double*>(w.veb),
-               w.seg + (i + 1) * n2, i == last ? 1 : 0);
+        if (!w.own || i == last)
+            launch(s, "win_area", k_win_area, d.ngb, kBlock, d, X, static_cast<const int4*>(w.wl),
+                   static_cast<const int*>(w.wn), w.neg, i == last ? d.garea : static_cast<double*>(nullptr));
+        launch(s, "win_step", w.own ? k_win_step<true> : k_win_step<false>, d.nvb, kBlock, d, X,
+               static_cast<const uint8_t*>(w.neg), w.wb, static_cast<const int4*>(w.nbr),
+               static_cast<const double*>(w.vse), static_cast<const double*>(w.veb), w.seg + (i + 1) * n2,
+               w.segN + static_cast<size_t>(i) * s->V, i == last ? 1 : 0);
     }
 }
 
@@ -1643,14 +1673,14 @@ int sevc_window_forward(sevc_state* s, int32_t steps, int32_t ckpt_every) {
     int rc;
     if ((rc = win_buffer(s, &w.ck, &w.ck_n, std::max<size_t>(1, nck) * n2)) != SEVC_OK ||
         (rc = win_buffer(s, &w.seg, &w.seg_n, (static_cast<size_t>(K) + 1) * n2)) != SEVC_OK ||
-        (rc = win_buffer(s, &w.segN, &w.segN_n, static_cast<size_t>(K) * s->G)) != SEVC_OK)
+        (rc = win_buffer(s, &w.segN, &w.segN_n, static_cast<size_t>(K) * s->V)) != SEVC_OK)
         return rc;
     if ((rc = win_fixed_buffers(s)) != SEVC_OK) return rc;
     w.ready = false;
     w.seeded = false;
     launch(s, "win_prepare", k_win_prepare, d.neb, kBlock, d);
-    launch(s, "win_table_v", k_win_table_v, d.nvb, kBlock, d, w.nbr, w.vse, w.veb);
-    launch(s, "win_table_g", k_win_table_g, d.ngb, kBlock, d, w.wl, w.wn);
+    launch(s, "win_table_v", k_win_table_v, d.nvb, kBlock, d, w.nbr, w.vse, w.veb, w.wb);
+    if (!w.own) launch(s, "win_table_g", k_win_table_g, d.ngb, kBlock, d, w.wl, w.wn);
     HIPCHK(hipMemcpyAsync(w.seg, d.pos, n2 * 8, hipMemcpyDeviceToDevice, s->stream));
     int last = 0;
     for (int c = 0; c < nck; ++c) {
@@ -1700,7 +1730,7 @@ int sevc_adjoint_window(sevc_state* s, const double* const* dL_dpos, sevc_grads*
         }
         for (int i = len - 1; i >= 0; --i) {
             launch(s, "win_adjoint", k_win_adjoint, d.nvb, kBlock, d, static_cast<const double*>(w.seg + i * n2),
-                   static_cast<const uint8_t*>(w.segN + static_cast<size_t>(i) * s->G),
+                   static_cast<const uint8_t*>(w.segN + static_cast<size_t>(i) * s->V),
                    static_cast<const int4*>(w.nbr), static_cast<const double*>(w.vse),
                    static_cast<const double*>(w.veb), static_cast<const double*>(cur), nxt, w.acc_mu, w.acc_s,
                    w.acc_se);

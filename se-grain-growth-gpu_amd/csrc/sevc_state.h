@@ -126,6 +126,16 @@ struct Dev {
     int free_rows;                        // blocks per kind of one free-slot search round (0: the default)
 };
 
+// The grains of each vertex table block and their lists, for the steps of a
+// topology-fixed window (sevc_adjoint.hip); null without.
+constexpr int kWinBlockGrains = 3 * kBlock;
+struct WinBlocks {
+    int* loc;
+    int* count;
+    int2* grain;
+    int4* list;
+};
+
 // One array of a mesh download (k_pack): n items of `src` go to byte `dst` of
 // the staging buffer.  PACK_RAW copies n 4-byte words, PACK_BYTE n bytes,
 // PACK_ID n ids (off taken from those >= 0); PACK_ROW takes the first `row`

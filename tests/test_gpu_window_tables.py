@@ -55,3 +55,36 @@ def test_window_tables(make, gb_eps, steps, every):
     for a, b in zip((dp, ds, dgb, dmu), orc.adjoint(w)):
         assert np.array_equal(np.asarray(a).view(np.uint64), np.asarray(b).view(np.uint64))
     st.close()
+
+
+@pytest.mark.parametrize("order", ["along the mesh", "shuffled"])
+@pytest.mark.parametrize("n", [300, 70_000])
+def test_window_vertex_order(order, n):
+    """Vertices in no order: a block of 256 has up to 700 grains, and above 512
+    blocks the area signs come from a launch of their own."""
+    pos, rid = sevc.voronoi(n, 6)
+    rng = np.random.default_rng(6)
+    o = sevc.default_options()
+    o.GB_eps, o.n_grains, o.dt = 0.0, n, 1e-4 / np.sqrt(n)
+    o.events, o.do_nucleation, o.velocity_model = 0, 0, sevc.VEL_ANALYTIC
+    mesh = sevc.build_mesh(o, pos, rid, rng.random(n), rng.random(n), n)
+    if order == "shuffled":
+        new = rng.permutation(mesh.nv)           # slot of each vertex
+        for k, width in (("pos", 2), ("v_bnd", 3), ("v_grn", 3), ("v_enabled", 1)):
+            a = mesh[k].reshape(mesh.nv, width)
+            b = a.copy()
+            b[new] = a
+            a[:] = b
+        for k in ("b_vtx", "g_vtx"):
+            a = mesh[k]
+            a[a >= 0] = new[a[a >= 0]]
+    assert sevc.check_mesh(mesh)[0] == 0
+    st, orc = sevc.State(o, mesh), Oracle(o, mesh)
+    st.window_forward(7, 3)
+    assert orc.window_forward(7) == 0
+    assert diff_fields(st.get_mesh(), orc.get_mesh(), ["pos", "vel", "g_area"]) == {}
+    w = rng.standard_normal(2 * mesh.nv)
+    (dp, ds, dgb, dmu), = st.adjoint(w)
+    for a, b in zip((dp, ds, dgb, dmu), orc.adjoint(w)):
+        assert np.array_equal(np.asarray(a).view(np.uint64), np.asarray(b).view(np.uint64))
+    st.close()
