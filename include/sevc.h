@@ -372,7 +372,8 @@ typedef struct sevc_grads {
  * main.cu:124-389): `steps` steps of x <- dom_mod(x + dt*mobility*F(x)),
  * F = -grad E the analytic force, with T1/T2/nucleation off and dt the
  * fixed opts.dt, on every member.  Positions are checkpointed every
- * ckpt_every steps (<= 0: every step is kept, no recomputation later).
+ * ckpt_every steps (<= 0: every step is kept, no recomputation later; a
+ * window of at most 2 GB of positions is kept whole in any case).
  * The state ends at the window's end; the next sevc_step or
  * sevc_set_member_params invalidates the window. */
 int sevc_window_forward(sevc_state* s, int32_t steps, int32_t ckpt_every);

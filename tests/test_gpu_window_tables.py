@@ -57,6 +57,28 @@ def test_window_tables(make, gb_eps, steps, every):
     st.close()
 
 
+def test_window_kept_and_recomputed():
+    """A window past the limit of what is kept whole: its reverse pass, from
+    checkpoints (the last segment a short one), against every step kept."""
+    n, steps = 40_009, 1701                      # 16 + 1 bytes a vertex and step: 2.3 GB
+    pos, rid = sevc.voronoi(n, 5)
+    rng = np.random.default_rng(5)
+    o = sevc.default_options()
+    o.GB_eps, o.n_grains, o.dt = 0.3, n, 1e-4 / np.sqrt(n)
+    o.events, o.do_nucleation, o.velocity_model = 0, 0, sevc.VEL_ANALYTIC
+    mesh = sevc.build_mesh(o, pos, rid, rng.random(n), rng.random(n), n)
+    w = rng.standard_normal(2 * mesh.nv)
+    out = []
+    for every in (0, 100):
+        st = sevc.State(o, mesh)
+        st.window_forward(steps, every)
+        (dp, ds, dgb, dmu), = st.adjoint(w)
+        out.append([st.positions(0), dp, ds, np.array([dgb, dmu])])
+        st.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a.view(np.uint64), b.view(np.uint64))
+
+
 @pytest.mark.parametrize("order", ["along the mesh", "shuffled"])
 @pytest.mark.parametrize("n", [300, 70_000])
 def test_window_vertex_order(order, n):
