@@ -54,6 +54,7 @@ __global__ void k_rate_draw(Dev d);
 __global__ void k_head(Dev d, int what);
 __global__ void k_nucl_insert(Dev d);
 __global__ void k_pack(PackList L, char* out);
+__global__ void k_copy_arrays(CopyList L);
 // kernels of sevc_adjoint.hip
 __global__ void k_win_prepare(Dev d);
 __global__ void k_win_table_v(Dev d, int4* nbr, double* vse, double* veb, WinBlocks wb);
@@ -1424,6 +1425,26 @@ std::vector<std::pair<void*, size_t>> state_arrays(const sevc_state* s) {
             {d.ms, sizeof(MState) * static_cast<size_t>(s->B)}};
 }
 constexpr int kMaxCkpt = 64;
+
+// The state's arrays into a checkpoint's buffer (to_buf) or back.
+int copy_state(sevc_state* s, char* buf, bool to_buf) {
+    const auto arrays = state_arrays(s);
+    CopyList L{};
+    size_t off = 0, blocks = 0;
+    for (const auto& a : arrays) {
+        char* x = static_cast<char*>(a.first);
+        if (a.second > 0) {
+            if (L.n == kCopySegs) return fail(s, SEVC_E_INVALID_ARG, "too many arrays in a checkpoint");
+            L.seg[L.n++] = {to_buf ? x : buf + off, to_buf ? buf + off : x, a.second, static_cast<int>(blocks)};
+        }
+        blocks += (a.second + kCopyChunk - 1) / kCopyChunk;
+        off += (a.second + 255) / 256 * 256;
+    }
+    if (blocks > (size_t(1) << 24) - 1) return fail(s, SEVC_E_INVALID_ARG, "checkpoint too large");
+    launch(s, "copy_state", k_copy_arrays, static_cast<int>(blocks), 256, L);
+    HIPCHK(hipGetLastError());
+    return SEVC_OK;
+}
 }  // namespace
 }  // extern "C++"
 
@@ -1439,11 +1460,8 @@ int sevc_checkpoint(sevc_state* s, int32_t slot) {
         if (hipMalloc(&c.buf, total) != hipSuccess) return fail(s, SEVC_E_NOMEM, "no room for a checkpoint");
         c.bytes = total;
     }
-    size_t off = 0;
-    for (auto& a : arrays) {
-        HIPCHK(hipMemcpyAsync(c.buf + off, a.first, a.second, hipMemcpyDeviceToDevice, s->stream));
-        off += (a.second + 255) / 256 * 256;
-    }
+    int rc;
+    if ((rc = copy_state(s, c.buf, true)) != SEVC_OK) return rc;
     HIPCHK(hipMemcpyAsync(s->ms_host.data(), s->d.ms, sizeof(MState) * s->ms_host.size(), hipMemcpyDeviceToHost,
                           s->stream));
     HIPCHK(hipStreamSynchronize(s->stream));
@@ -1455,11 +1473,8 @@ int sevc_restore(sevc_state* s, int32_t slot) {
     if (!s || slot < 0 || slot >= static_cast<int>(s->ckpts.size()) || !s->ckpts[slot].buf)
         return SEVC_E_INVALID_ARG;
     const sevc_state::Ckpt& c = s->ckpts[slot];
-    size_t off = 0;
-    for (auto& a : state_arrays(s)) {
-        HIPCHK(hipMemcpyAsync(a.first, c.buf + off, a.second, hipMemcpyDeviceToDevice, s->stream));
-        off += (a.second + 255) / 256 * 256;
-    }
+    int rc;
+    if ((rc = copy_state(s, c.buf, false)) != SEVC_OK) return rc;
     // the grains listed for the two-triangle search are not kept: all are listed anew
     HIPCHK(hipMemsetAsync(s->d.cnt + C_TRI, 0, sizeof(int), s->stream));
     HIPCHK(hipStreamSynchronize(s->stream));

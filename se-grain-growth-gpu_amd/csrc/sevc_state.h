@@ -152,4 +152,18 @@ struct PackList {
     int n;
 };
 
+// The arrays of a checkpoint or a restore (k_copy_arrays): n bytes from src to
+// dst, both 16-byte aligned, by the workgroups from `first` on.
+struct CopySeg {
+    const char* src;
+    char* dst;
+    unsigned long long n;
+    int first;
+};
+constexpr int kCopySegs = 48, kCopyChunk = 16384;     // bytes per workgroup
+struct CopyList {
+    CopySeg seg[kCopySegs];
+    int n;
+};
+
 }  // namespace sevc
