@@ -3691,96 +3691,134 @@ __global__ void __launch_bounds__(1024) k_nucl_area_up(Dev d) {
 // nucleation (nucleation2.cu)
 // ---------------------------------------------------------------------
 
-struct NuclGeom {
-    double Apos[2], Bpos[2], Cpos[2];
-    double Dpos[2], Epos[2], Fpos[2];   // positions of D, E, F as read
-    int D, E, F, AD, AE, AF, g1, g2, g3;
-    double dE;
+// What a nucleation reads around its site A: the edges AD, AE, AF (slot order)
+// and their other ends, A's grains, and g1, g2, g3 among them (the first part of
+// generate_grain_for_nucleation, nucleation2.cu:116-212).  Everything is loaded
+// in three rounds (A's own data; its edges' ends; the ends' positions and
+// grains), in place of a chain of ten (the Monte Carlo draw of the 2,000-grain
+// example, 14 us of its step of 69: with them and two lanes, 62 in all).
+struct NuclSite {
+    int vb[3], nb[3], gA[3], g1, g2, g3;
+    int2 e[3];                            // ends of AD, AE, AF
+    double2 pA, pN[3];
+    bool ok;
 };
 
-// generate_grain_for_nucleation, nucleation2.cu:116-212
-// (kEnergy: with dE, which the insertion does not use)
-template <bool kEnergy>
-__device__ __forceinline__ int generate_grain(const Dev& d, const Params& P, int A, double eps, double scaling, int do_scale,
-                              NuclGeom* r) {
-    const double Dm = P.D;
-    r->AD = d.vb[3 * A + 0]; r->AE = d.vb[3 * A + 1]; r->AF = d.vb[3 * A + 2];
-    r->D = other_end(d, r->AD, A);
-    r->E = other_end(d, r->AE, A);
-    r->F = other_end(d, r->AF, A);
+// `beside` loads what else the caller needs of A's edges and grains, in the
+// second round.
+template <class Beside>
+__device__ __forceinline__ NuclSite nucl_site(const Dev& d, int A, Beside beside) {
+    NuclSite t;
+    const double2* X = reinterpret_cast<const double2*>(d.pos);
+    load_triple(d.vb, A, t.vb);
+    load_triple(d.vg, A, t.gA);
+    t.pA = X[A];
+#pragma unroll
+    for (int k = 0; k < 3; k++) t.e[k] = reinterpret_cast<const int2*>(d.bvx)[t.vb[k]];
+    beside(t);
+#pragma unroll
+    for (int k = 0; k < 3; k++) t.nb[k] = t.e[k].x == A ? t.e[k].y : t.e[k].x;
+    int gD[3], gE[3];
+    load_triple(d.vg, t.nb[0], gD);
+    load_triple(d.vg, t.nb[1], gE);
+#pragma unroll
+    for (int k = 0; k < 3; k++) t.pN[k] = X[t.nb[k]];
     int ad0, ad1, ae0, ae1;
-    grains_intersect(d, A, r->D, ad0, ad1);
-    grains_intersect(d, A, r->E, ae0, ae1);
-    if (ad0 == ae0 || ad0 == ae1) { r->g2 = ad0; r->g1 = ad1; }
-    else if (ad1 == ae0 || ad1 == ae1) { r->g2 = ad1; r->g1 = ad0; }
-    else return -1;
-    if (ae0 == r->g2) r->g3 = ae1;
-    else if (ae1 == r->g2) r->g3 = ae0;
-    else return -1;
-    if (r->g1 < 0 || r->g2 < 0 || r->g3 < 0) return -1;
-    const double ax = d.pos[2 * A], ay = d.pos[2 * A + 1], rr = d.nucl_r[A];
-    const int nb[3] = {r->D, r->E, r->F};
-    double* out[3] = {r->Apos, r->Bpos, r->Cpos};
-    r->Dpos[0] = d.pos[2 * nb[0]]; r->Dpos[1] = d.pos[2 * nb[0] + 1];
-    r->Epos[0] = d.pos[2 * nb[1]]; r->Epos[1] = d.pos[2 * nb[1] + 1];
-    r->Fpos[0] = d.pos[2 * nb[2]]; r->Fpos[1] = d.pos[2 * nb[2] + 1];
+    triples_intersect(t.gA, gD, ad0, ad1);
+    triples_intersect(t.gA, gE, ae0, ae1);
+    t.ok = true;
+    t.g1 = t.g2 = t.g3 = -1;
+    if (ad0 == ae0 || ad0 == ae1) { t.g2 = ad0; t.g1 = ad1; }
+    else if (ad1 == ae0 || ad1 == ae1) { t.g2 = ad1; t.g1 = ad0; }
+    else t.ok = false;
+    if (ae0 == t.g2) t.g3 = ae1;
+    else if (ae1 == t.g2) t.g3 = ae0;
+    else t.ok = false;
+    t.ok = t.ok && t.g1 >= 0 && t.g2 >= 0 && t.g3 >= 0;
+    return t;
+}
+
+// The nucleus' corners on AD, AE, AF for the radius rr, shrunk with do_scale.
+struct NuclGeom {
+    double Apos[2], Bpos[2], Cpos[2];
+};
+__device__ __forceinline__ NuclGeom nucl_corners(const NuclSite& t, double rr, int do_scale, double Dm) {
+    NuclGeom r;
+    double* out[3] = {r.Apos, r.Bpos, r.Cpos};
+#pragma unroll
     for (int k = 0; k < 3; k++) {
-        double tx = wrapd(d.pos[2 * nb[k]], ax, Dm);
-        double ty = wrapd(d.pos[2 * nb[k] + 1], ay, Dm);
+        double tx = wrapd(t.pN[k].x, t.pA.x, Dm);
+        double ty = wrapd(t.pN[k].y, t.pA.y, Dm);
         double w = rr / mag(tx, ty);
         if (do_scale) w *= 0.99;
-        double px = w * tx + ax, py = w * ty + ay;
+        double px = w * tx + t.pA.x, py = w * ty + t.pA.y;
         out[k][0] = dom_mod(px, Dm);
         out[k][1] = dom_mod(py, Dm);
     }
-    if (!kEnergy) return 0;
-    double LAB = arclen(r->Apos[0], r->Apos[1], r->Bpos[0], r->Bpos[1], Dm);
-    double LBC = arclen(r->Bpos[0], r->Bpos[1], r->Cpos[0], r->Cpos[1], Dm);
-    double LCA = arclen(r->Cpos[0], r->Cpos[1], r->Apos[0], r->Apos[1], Dm);
-    AreaAcc acc;
-    acc.start(ax, ay); acc.push(r->Cpos[0], r->Cpos[1], Dm); acc.push(r->Apos[0], r->Apos[1], Dm);
-    double A1 = acc.finish();
-    acc.start(ax, ay); acc.push(r->Apos[0], r->Apos[1], Dm); acc.push(r->Bpos[0], r->Bpos[1], Dm);
-    double A2 = acc.finish();
-    acc.start(ax, ay); acc.push(r->Bpos[0], r->Bpos[1], Dm); acc.push(r->Cpos[0], r->Cpos[1], Dm);
-    double A3 = acc.finish();
-    double E0 = 0.0, E1;
-    for (int i = 0; i < 3; i++) {
-        if (do_scale) E0 += 0.99 * rr * d.ben[d.vb[3 * A + i]];
-        else E0 += rr * d.ben[d.vb[3 * A + i]];
-    }
-    E0 += A1 * d.gse[r->g1] + A2 * d.gse[r->g2] + A3 * d.gse[r->g3];
-    const double ori = d.nucl_ori[A];
-    E1 = gb_energy_func(ori - d.gori[r->g1], eps) * scaling * LCA;
-    E1 += gb_energy_func(ori - d.gori[r->g2], eps) * scaling * LAB;
-    E1 += gb_energy_func(ori - d.gori[r->g3], eps) * scaling * LBC;
-    r->dE = E1 - E0;
-    return 0;
+    return r;
 }
 
-// compute_nucleation_factor, nucleation2.cu:239-282, with the random pair
-// Philox(seed; step, local vertex id, stream 1).
-// compute_nucleation_factor (nucleation2.cu) for one alive vertex v of a
 // Monte Carlo member: the nucleus radius and orientation from the vertex's
-// own Philox pair, dE and the factor dE - dE'.  The manager needs it only
-// for the vertex it picks, so it runs there, for that vertex alone.
-__device__ __forceinline__ void nucl_factor_at(const Dev& d, const Params& P, const MState& M, int v) {
-    d.dE[v] = 0;
-    d.nfac[v] = 0;
-    double ALs[3];
-    for (int q = 0; q < 3; q++) ALs[q] = edge_len_from(d, d.vb[3 * v + q], v, P.D);
-    double minAL = ALs[0];
-    for (int q = 0; q < 3; q++) if (minAL > ALs[q]) minAL = ALs[q];
+// own Philox pair, dE and the factor dE - dE' (the same with the shrunk
+// nucleus).  The head needs it only for the vertex it picks, so it runs there,
+// for that vertex alone, by a wave: lane 0 forms dE and lane 1 dE'.
+__device__ __forceinline__ void nucl_factor_at(const Dev& d, const Params& P, const MState& M, int v, double* dE, double* nfac) {
+    double ben[3], se[3], go[3];
+    const NuclSite t = nucl_site(d, v, [&](const NuclSite& t_) {
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            ben[k] = d.ben[t_.vb[k]];
+            se[k] = d.gse[t_.gA[k]];
+            go[k] = d.gori[t_.gA[k]];
+        }
+    });
+    const double Dm = P.D;
+    double minAL = 0.0;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const double al = arclen(t.pA.x, t.pA.y, t.pN[k].x, t.pN[k].y, Dm);
+        if (k == 0 || minAL > al) minAL = al;
+    }
     double u0, u1;
     sevc_uniform2(P.seed, (uint32_t)M.n, (uint32_t)(v - P.voff), kStreamMcSite, 0u, &u0, &u1);
-    d.nucl_r[v] = 0.8 * minAL * u0 + 0.1;
-    d.nucl_ori[v] = 2 * SEVC_PI * u1;
-    NuclGeom g0, g1;
-    double de = 0.0, de_ = 0.0;
-    if (generate_grain<true>(d, P, v, P.gb_eps, P.gb_scaling, 0, &g0) == 0) de = g0.dE;
-    d.dE[v] = de;
-    if (generate_grain<true>(d, P, v, P.gb_eps, P.gb_scaling, 1, &g1) == 0) de_ = g1.dE;
-    d.nfac[v] = de - de_;
+    const double rr = 0.8 * minAL * u0 + 0.1, ori = 2 * SEVC_PI * u1;
+    const int do_scale = (int)threadIdx.x & 1;
+    double de = 0.0;
+    if (t.ok) {
+        const NuclGeom r = nucl_corners(t, rr, do_scale, Dm);
+        const double ax = t.pA.x, ay = t.pA.y;
+        double LAB = arclen(r.Apos[0], r.Apos[1], r.Bpos[0], r.Bpos[1], Dm);
+        double LBC = arclen(r.Bpos[0], r.Bpos[1], r.Cpos[0], r.Cpos[1], Dm);
+        double LCA = arclen(r.Cpos[0], r.Cpos[1], r.Apos[0], r.Apos[1], Dm);
+        AreaAcc acc;
+        acc.start(ax, ay); acc.push(r.Cpos[0], r.Cpos[1], Dm); acc.push(r.Apos[0], r.Apos[1], Dm);
+        double A1 = acc.finish();
+        acc.start(ax, ay); acc.push(r.Apos[0], r.Apos[1], Dm); acc.push(r.Bpos[0], r.Bpos[1], Dm);
+        double A2 = acc.finish();
+        acc.start(ax, ay); acc.push(r.Bpos[0], r.Bpos[1], Dm); acc.push(r.Cpos[0], r.Cpos[1], Dm);
+        double A3 = acc.finish();
+        auto of = [&](const double (&x)[3], int g) { return g == t.gA[0] ? x[0] : (g == t.gA[1] ? x[1] : x[2]); };
+        double E0 = 0.0, E1;
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            if (do_scale) E0 += 0.99 * rr * ben[i];
+            else E0 += rr * ben[i];
+        }
+        E0 += A1 * of(se, t.g1) + A2 * of(se, t.g2) + A3 * of(se, t.g3);
+        const double eps = P.gb_eps, scaling = P.gb_scaling;
+        E1 = gb_energy_func(ori - of(go, t.g1), eps) * scaling * LCA;
+        E1 += gb_energy_func(ori - of(go, t.g2), eps) * scaling * LAB;
+        E1 += gb_energy_func(ori - of(go, t.g3), eps) * scaling * LBC;
+        de = E1 - E0;
+    }
+    *dE = __shfl(de, 0);
+    *nfac = *dE - __shfl(de, 1);
+    if (((int)threadIdx.x & 63) == 0) {
+        d.nucl_r[v] = rr;
+        d.nucl_ori[v] = ori;
+        d.dE[v] = *dE;
+        d.nfac[v] = *nfac;
+    }
 }
 
 // Rate mode: grain g of a nucleating member is a candidate with
@@ -4199,29 +4237,39 @@ __device__ __forceinline__ void insert_event(const Dev& d, int m, int A, int B, 
     auto& sdy = lds.sdy;
     const int lane = (int)threadIdx.x & 63;
     const Params& P = d.prm[m];
-    NuclGeom r;
-    // nucleation2.cu:526 passes (scaling, eps) swapped; only dE is affected
-    if (generate_grain<false>(d, P, A, P.gb_scaling, P.gb_eps, 1, &r) != 0) return;
-    const int gl[3] = {r.g1, r.g2, r.g3};
+    // the site, the grains' lists and the nucleus' data, in three rounds of loads
+    // (nothing writes these entries before they are read)
+    int len[3], row[3][kMaxStride / 64];
+    const double rr = d.nucl_r[A], ori = d.nucl_ori[A];
+    const NuclSite t = nucl_site(d, A, [&](const NuclSite& t_) {
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            const int* L = glist(d, t_.gA[k]);
+            len[k] = d.glen[t_.gA[k]];
+#pragma unroll
+            for (int q = 0; q < kMaxStride / 64; q++) row[k][q] = lane + 64 * q < d.S ? L[lane + 64 * q] : -1;
+        }
+    });
+    if (!t.ok) return;
+    const NuclGeom r = nucl_corners(t, rr, 1, P.D);
+    const int AD = t.vb[0], AE = t.vb[1], AF = t.vb[2];
+    const int gl[3] = {t.g1, t.g2, t.g3};
     int sl[3];
     sl[0] = 0;
     sl[1] = gl[1] == gl[0] ? 0 : 1;
     sl[2] = gl[2] == gl[0] ? 0 : (gl[2] == gl[1] ? sl[1] : 2);
     int n_old[3];
 #pragma unroll
-    for (int t = 0; t < 3; t++) n_old[t] = sl[t] == t ? d.glen[gl[t]] : 0;
+    for (int j = 0; j < 3; j++) {
+        const int k = gl[j] == t.gA[0] ? 0 : (gl[j] == t.gA[1] ? 1 : 2);
+        n_old[j] = sl[j] == j ? (k == 0 ? len[0] : k == 1 ? len[1] : len[2]) : 0;
 #pragma unroll
-    for (int t = 0; t < 3; t++) {
-        if (sl[t] != t) continue;
-        const int* L = glist(d, gl[t]);
-        for (int i = lane; i < n_old[t]; i += 64) Ls[t][i] = L[i];
+        for (int q = 0; q < kMaxStride / 64; q++) {
+            const int i = lane + 64 * q;
+            if (i < n_old[j]) Ls[j][i] = k == 0 ? row[0][q] : (k == 1 ? row[1][q] : row[2][q]);
+        }
     }
-    // what the serial edits below read, loaded with the lists (nothing
-    // writes these entries before they are read)
-    int vgA[3];
-#pragma unroll
-    for (int k = 0; k < 3; k++) vgA[k] = d.vg[3 * A + k];
-    const int ae0 = d.bvx[2 * r.AE], ae1 = d.bvx[2 * r.AE + 1], af0 = d.bvx[2 * r.AF];
+    const int (&vgA)[3] = t.gA;
     if (lane == 0) { n_s[0] = n_old[0]; n_s[1] = n_old[1]; n_s[2] = n_old[2]; }
     wave_sync();
     const int cap = P.cap;
@@ -4265,8 +4313,7 @@ __device__ __forceinline__ void insert_event(const Dev& d, int m, int A, int B, 
         wave_sync();
     };
     ladd(sl[0], C, A);
-    if (ae0 == A) ladd(sl[1], B, ae1);
-    else if (ae1 == A) ladd(sl[1], B, ae0);
+    if (t.e[1].x == A || t.e[1].y == A) ladd(sl[1], B, t.nb[1]);
     ladd(sl[2], C, A);
     ladd(sl[2], B, C);
     lremove(sl[2], A);
@@ -4301,9 +4348,9 @@ __device__ __forceinline__ void insert_event(const Dev& d, int m, int A, int B, 
             d.bcand[b] = 0;
             d.conf[b] = -1;
         }
-        d.vb[3 * A] = AB; d.vb[3 * A + 1] = CA; d.vb[3 * A + 2] = r.AD;
-        d.vb[3 * B] = BC; d.vb[3 * B + 1] = AB; d.vb[3 * B + 2] = r.AE;
-        d.vb[3 * C] = CA; d.vb[3 * C + 1] = BC; d.vb[3 * C + 2] = r.AF;
+        d.vb[3 * A] = AB; d.vb[3 * A + 1] = CA; d.vb[3 * A + 2] = AD;
+        d.vb[3 * B] = BC; d.vb[3 * B + 1] = AB; d.vb[3 * B + 2] = AE;
+        d.vb[3 * C] = CA; d.vb[3 * C + 1] = BC; d.vb[3 * C + 2] = AF;
         // nucleate_grain (geometry.h:596-606); its list is written below
         d.glen[g] = 3;
         d.garea[g] = 0;
@@ -4312,17 +4359,17 @@ __device__ __forceinline__ void insert_event(const Dev& d, int m, int A, int B, 
         d.gcand[g] = 0;
         d.gfix[g] = 0;
         d.gtype[g] = T_NUCLEATED;
-        d.gori[g] = d.nucl_ori[A];
+        d.gori[g] = ori;
         {
-            const int k = vgA[0] == r.g3 ? 0 : (vgA[1] == r.g3 ? 1 : (vgA[2] == r.g3 ? 2 : -1));
+            const int k = vgA[0] == t.g3 ? 0 : (vgA[1] == t.g3 ? 1 : (vgA[2] == t.g3 ? 2 : -1));
             if (k >= 0) d.vg[3 * A + k] = g;
         }
-        d.vg[3 * B] = g; d.vg[3 * B + 1] = r.g2; d.vg[3 * B + 2] = r.g3;
-        d.vg[3 * C] = g; d.vg[3 * C + 1] = r.g3; d.vg[3 * C + 2] = r.g1;
-        if (ae0 == A) d.bvx[2 * r.AE] = B;
-        else if (ae1 == A) d.bvx[2 * r.AE + 1] = B;
-        if (af0 == A) d.bvx[2 * r.AF] = C;
-        else d.bvx[2 * r.AF + 1] = C;
+        d.vg[3 * B] = g; d.vg[3 * B + 1] = t.g2; d.vg[3 * B + 2] = t.g3;
+        d.vg[3 * C] = g; d.vg[3 * C + 1] = t.g3; d.vg[3 * C + 2] = t.g1;
+        if (t.e[1].x == A) d.bvx[2 * AE] = B;
+        else if (t.e[1].y == A) d.bvx[2 * AE + 1] = B;
+        if (t.e[2].x == A) d.bvx[2 * AF] = C;
+        else d.bvx[2 * AF + 1] = C;
         atomicAdd((unsigned long long*)&d.ms[m].nucl, 1ull);
     }
     wave_sync();
@@ -4353,15 +4400,15 @@ __device__ __forceinline__ void insert_event(const Dev& d, int m, int A, int B, 
         // the six edges and their ends' positions after the event: AB, BC,
         // CA between the new vertices, AD at A, AE rewired to B, AF to C
         // (arclen gives the same bits in either end order)
-        const int b = lane == 0 ? AB : lane == 1 ? BC : lane == 2 ? CA : lane == 3 ? r.AD : lane == 4 ? r.AE : r.AF;
+        const int b = lane == 0 ? AB : lane == 1 ? BC : lane == 2 ? CA : lane == 3 ? AD : lane == 4 ? AE : AF;
         // by selection (no pointer into r, which would put it in scratch)
         const bool a0 = lane == 0 || lane == 3, b0 = lane == 1 || lane == 4;
         const double x0 = a0 ? r.Apos[0] : (b0 ? r.Bpos[0] : r.Cpos[0]);
         const double y0 = a0 ? r.Apos[1] : (b0 ? r.Bpos[1] : r.Cpos[1]);
         const double x1 = lane == 0 ? r.Bpos[0] : lane == 1 ? r.Cpos[0] : lane == 2 ? r.Apos[0]
-                        : lane == 3 ? r.Dpos[0] : lane == 4 ? r.Epos[0] : r.Fpos[0];
+                        : lane == 3 ? t.pN[0].x : lane == 4 ? t.pN[1].x : t.pN[2].x;
         const double y1 = lane == 0 ? r.Bpos[1] : lane == 1 ? r.Cpos[1] : lane == 2 ? r.Apos[1]
-                        : lane == 3 ? r.Dpos[1] : lane == 4 ? r.Epos[1] : r.Fpos[1];
+                        : lane == 3 ? t.pN[0].y : lane == 4 ? t.pN[1].y : t.pN[2].y;
         d.blen[b] = arclen(x0, y0, x1, y1, Dm);
         const double e = (P.gb_eps == 0.0) ? 1.0 : boundary_compute_energy(d, b, P.gb_eps);
         d.ben[b] = e * P.gb_scaling;
@@ -4464,15 +4511,17 @@ __global__ void __launch_bounds__(kNuclThreads) k_head(Dev d, int what) {
         int k = (int)(u0 * (double)n_alive);
         if (k >= n_alive) k = n_alive - 1;
         const int A = find_kth(d.vblk, rs, d.bc_v, d.ven, 1, k);
-        if (tid == 0 && A >= 0) {
-            nucl_factor_at(d, P, M, A);
-            d.vnuc[A] = 0;
-            if (d.dE[A] < 0) d.vnuc[A] = 1;
-            else if (d.nfac[A] < 0) {
-                double thr = sevc_exp(-P.mc_k * d.dE[A]);
-                if (u1 < thr) d.vnuc[A] = 1;
+        if (tid < 64 && A >= 0) {
+            double dE, nfac;
+            nucl_factor_at(d, P, M, A, &dE, &nfac);
+            const bool take = dE < 0 || (nfac < 0 && u1 < sevc_exp(-P.mc_k * dE));
+            if (tid == 0) {
+                d.vnuc[A] = take ? 1 : 0;
+                if (take) {
+                    kept[0] = A;
+                    nkeep = 1;
+                }
             }
-            if (d.vnuc[A]) { kept[0] = A; nkeep = 1; }
         }
     } else {
         // this member's candidates (grain, list index), then grain order
