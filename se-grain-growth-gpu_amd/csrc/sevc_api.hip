@@ -480,7 +480,7 @@ void launch_step(sevc_state* s, bool diag) {
     }
     const bool one = s->any_events && !s->any_debug && s->busy == 0;
     if (one) {
-        launch(s, "events", k_events, 1, 1024, d);
+        launch(s, "events", k_events, 1, kEvThreads, d);
     } else if (s->any_events) {
         launch(s, "poll_gather", k_poll_gather, kPollBig / 64, 64, d);
         launch(s, "poll", k_poll, 1, 1024, d);

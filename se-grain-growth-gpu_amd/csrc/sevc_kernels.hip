@@ -3045,7 +3045,7 @@ __global__ void k_flip_serial(Dev d) {
 // workgroup's own L1 and L2.  2,000 grains, three events a step: 25 us where
 // the launches took 63; a batch of 45 events a step 51 us where they took 105;
 // 1M grains, 27 events a step, 68 us where they took 130.  Its time grows with
-// the number of edited grains (64 at a time), so busy states take the launches.
+// the number of edited grains (32 at a time), so busy states take the launches.
 //
 // Up to kEvMax listed edges (one to a lane) a lane keeps its edge's
 // surroundings in registers, and everything the stages exchange goes through
@@ -3058,7 +3058,8 @@ __global__ void k_flip_serial(Dev d) {
 // workgroup it took 28 us at 2,000 grains, 66 for the batch, 82 at 1M; the
 // edit records in LDS (instead of memory) and the early loads are 5 us of it.
 // Longer lists, and steps with a two-triangle candidate, run the launches'
-// stages.
+// stages.  512 threads, so that a lane has the registers it needs (182): with
+// 1024 it had 128 and spilled 119 to scratch memory, 3 to 4 us a step.
 // Sizes: an edge has at most three grains in common with its ends, so at most
 // 3 kEvMax grains are labelled (a lane each); a removal flags three grains and
 // records edits at two vertices, a flip four and two.
@@ -3079,7 +3080,7 @@ struct EvLds {
     unsigned char cf[kEvMax];         // the edge's label
     int nt2, ncon, nfl, nrec, changed, two, nslow;
     int slow[kFlag];                  // grains for fix_wave
-    QuickLds quick[16];
+    QuickLds quick[kEvThreads / 64];
     static constexpr int kSlow = 3;
     union {
         FixLds fix[kSlow];
@@ -3087,7 +3088,7 @@ struct EvLds {
     } room;
 };
 static_assert(sizeof(EvLds) <= kPollLds, "the event stages' tables fit");
-static_assert(EvLds::kT2 <= 1024 && 4 * kEvMax <= EvLds::kFlag && EvLds::kFlag < EvLds::kFH && EvLds::kT2 < EvLds::kTH &&
+static_assert(EvLds::kT2 <= 2 * kEvThreads && kEvMax < kEvThreads && 4 * kEvMax <= EvLds::kFlag && EvLds::kFlag < EvLds::kFH && EvLds::kT2 < EvLds::kTH &&
                   EvLds::kRec < EvLds::kRH && 2 * kEvMax < EvLds::kVH && kEvMax < EvLds::kEH,
               "every list and table holds what a step can put in");
 constexpr int kFree = -1, kMany = -2;
@@ -3185,7 +3186,7 @@ __device__ __forceinline__ void ev_edit(const Dev& d, EvLds& s, bool with_area) 
     QuickLds& q = s.quick[wave];
     const double2* X = reinterpret_cast<const double2*>(d.pos);
     fix_items(
-        d, n, [&](int k) { return s.fl[k]; }, [&](int v) { return record_lds(s, v); }, q, wave, 16,
+        d, n, [&](int k) { return s.fl[k]; }, [&](int v) { return record_lds(s, v); }, q, wave, kEvThreads / 64,
         [&](unsigned long long todo, int g) {
             if ((todo >> lane) & 1ull) s.slow[atomicAdd(&s.nslow, 1)] = g;
         },
@@ -3209,7 +3210,7 @@ __device__ __forceinline__ void ev_edit(const Dev& d, EvLds& s, bool with_area) 
         });
     __syncthreads();
     if (s.nslow > 0) {
-        for (int r = tid; r < s.nrec; r += 1024) {
+        for (int r = tid; r < s.nrec; r += kEvThreads) {
             const int v = s.rv[r];
             for (int j = 0; j < 2; j++) set_mod(d, v, j, (s.rfix[r] >> (8 * j)) & 255, s.rgrn[j][r], s.rvrt[j][r]);
             d.mods[v].prev[1] = s.rprev[r];
@@ -3224,10 +3225,10 @@ __device__ __forceinline__ void ev_edit(const Dev& d, EvLds& s, bool with_area) 
         if (wave < EvLds::kSlow)
             fix_clear_items(d, s.nslow, 0, [&](int k) { return s.slow[k]; }, with_area ? 1 : 0, s.room.clear[wave], wave,
                             EvLds::kSlow);
-        for (int r = tid; r < s.nrec; r += 1024) reset_mods(d, s.rv[r]);
+        for (int r = tid; r < s.nrec; r += kEvThreads) reset_mods(d, s.rv[r]);
     }
-    for (int h = tid; h < EvLds::kFH; h += 1024) s.fk[h] = kFree;
-    for (int h = tid; h < EvLds::kRH; h += 1024) s.rk[h] = kFree;
+    for (int h = tid; h < EvLds::kFH; h += kEvThreads) s.fk[h] = kFree;
+    for (int h = tid; h < EvLds::kRH; h += kEvThreads) s.rk[h] = kFree;
     __syncthreads();
     if (tid == 0) s.nfl = s.nslow = s.nrec = 0;
     __syncthreads();
@@ -3245,11 +3246,11 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, Ev
         id = d.c_id[tid];
         tl = d.c_te[tid];
     }
-    for (int h = tid; h < EvLds::kEH; h += 1024) s.ek[h] = kFree;
-    for (int h = tid; h < EvLds::kVH; h += 1024) { s.vk[h] = kFree; s.vp[h] = kFree; }
-    for (int h = tid; h < EvLds::kTH; h += 1024) s.tk[h] = kFree;
-    for (int h = tid; h < EvLds::kFH; h += 1024) s.fk[h] = kFree;
-    for (int h = tid; h < EvLds::kRH; h += 1024) s.rk[h] = kFree;
+    for (int h = tid; h < EvLds::kEH; h += kEvThreads) s.ek[h] = kFree;
+    for (int h = tid; h < EvLds::kVH; h += kEvThreads) { s.vk[h] = kFree; s.vp[h] = kFree; }
+    for (int h = tid; h < EvLds::kTH; h += kEvThreads) s.tk[h] = kFree;
+    for (int h = tid; h < EvLds::kFH; h += kEvThreads) s.fk[h] = kFree;
+    for (int h = tid; h < EvLds::kRH; h += kEvThreads) s.rk[h] = kFree;
     if (tid == 0) s.nt2 = s.ncon = s.nfl = s.nrec = s.two = s.nslow = 0;
     const int c = id.x, m = id.w;
     int2 ab = make_int2(id.y, id.z);
@@ -3259,7 +3260,7 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, Ev
         bool fresh;
         s.ep[ev_put(s.ek, EvLds::kEH, c, &fresh)] = tid;
     }
-    if (tri_items(d, ntri, 1023 - tid, 1024)) s.two = 1;
+    if (tri_items(d, ntri, kEvThreads - 1 - tid, kEvThreads)) s.two = 1;
     // the ends' edges, grains and positions; the edges' other ends and flags;
     // the lengths of the grains around
     FlipIn fi{};
@@ -3466,11 +3467,10 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, Ev
     const EditLds ed{s};
     if (nt2 > 0) {
         // a candidate with no other one around is removed at once (t2_items)
-        bool go = false;
-        int g = 0, mg = 0;
-        if (tid < nt2) {
-            g = s.t2[tid];
-            mg = member_of_grain(d, g);
+        bool go[2] = {false, false};
+#pragma unroll 1
+        for (int u = 0; tid + u * kEvThreads < nt2; u++) {
+            const int g = s.t2[tid + u * kEvThreads];
             const int* L = glist(d, g);
             int h[9];
 #pragma unroll
@@ -3484,11 +3484,17 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, Ev
                 clash = clash || (x != g && x >= 0 && s.tk[ev_find(s.tk, EvLds::kTH, x)] == x);
             }
             if (clash) s.con[atomicAdd(&s.ncon, 1)] = g;
-            go = !clash;
+            if (u == 0) go[0] = !clash;
+            else go[1] = !clash;
         }
         __syncthreads();
-        if (go) remove_grain(d, g, d.prm[mg].D, slot_base(d, mg), ed);
-        wave_count(d, go, mg, &MState::removals);
+#pragma unroll 1
+        for (int u = 0; u * kEvThreads < nt2; u++) {
+            const bool rm = u == 0 ? go[0] : go[1];
+            const int g = rm ? s.t2[tid + u * kEvThreads] : 0, mg = rm ? member_of_grain(d, g) : 0;
+            if (rm) remove_grain(d, g, d.prm[mg].D, slot_base(d, mg), ed);
+            wave_count(d, rm, mg, &MState::removals);
+        }
         __syncthreads();
         if (s.ncon > 0) {
             if (tid == 0) t2_serial(d, s.con, s.ncon, ed);
@@ -3549,7 +3555,7 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, Ev
     return true;
 }
 
-__global__ void __launch_bounds__(1024) k_events(Dev d) {
+__global__ void __launch_bounds__(kEvThreads) k_events(Dev d) {
     __shared__ __align__(16) unsigned char buf[kPollLds];
     const int tid = (int)threadIdx.x, nt = (int)blockDim.x, wave = tid >> 6;
     const int nc = d.cnt[C_CAND], ntri = n_tri(d);
@@ -3561,7 +3567,6 @@ __global__ void __launch_bounds__(1024) k_events(Dev d) {
         tri_items(d, ntri, nt - 1 - tid, nt);
     }
     // the launches' stages
-    constexpr int kWaves = 16;
     struct Room {
         FixLds fix;
         QuickLds quick;

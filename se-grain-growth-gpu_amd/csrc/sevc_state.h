@@ -23,6 +23,7 @@ constexpr int kPollBig = 16384;      // lists up to this length poll with flags 
 // events run in one workgroup (k_events), a busy one's in a launch per stage.
 // The line is where both cost the same (see k_events).
 constexpr int kEvMax = 192;          // longest candidate list that k_events runs in LDS
+constexpr int kEvThreads = 512;     // workgroup of k_events
 constexpr int kHeadGrains = 8192;    // largest member whose candidates k_head draws itself
 constexpr int kHeadEvents = 8;       // most nucleations a member may expect for k_head to apply them itself
 constexpr int kBusyOver = 320, kBusyUnder = 160;
