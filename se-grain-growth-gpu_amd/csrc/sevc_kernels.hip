@@ -2434,21 +2434,29 @@ __device__ __forceinline__ void two_grain_serial(const Dev& d) {
 __device__ __forceinline__ bool tri_items(const Dev& d, int n, int k0, int stride) {
     bool found = false;
     for (int k = k0; k < n; k += stride) {
+        // (tests after the loads, not between them: each would be a wait)
         const int g = d.l_tri[k], m = member_of_grain(d, g);
-        if (!d.genab[g] || d.glen[g] != 3 || !d.ms[m].active || !d.prm[m].events) continue;
         const int* L = glist(d, g);
-        const int vv[3] = {L[0], L[1], L[2]};
-        int bb[9], gv[9], ini[9], end[9], be[9];
+        const uint8_t on = d.genab[g];
+        const int len = d.glen[g], act = d.ms[m].active, ev = d.prm[m].events;
+        int vv[3] = {L[0], L[min(1, d.S - 1)], L[min(2, d.S - 1)]};
+        const bool go = on && len == 3 && act && ev;
+#pragma unroll
+        for (int q = 0; q < 3; q++) vv[q] = go ? vv[q] : 0;
+        int bb[9], gv[9], gl[9], ini[9], end[9], be[9];
 #pragma unroll
         for (int e = 0; e < 9; e++) {
             bb[e] = d.vb[3 * vv[e / 3] + e % 3];
             gv[e] = d.vg[3 * vv[e / 3] + e % 3];
         }
+        if (!go) continue;
 #pragma unroll
         for (int e = 0; e < 9; e++) {
-            ini[e] = d.bvx[2 * bb[e]];
-            end[e] = d.bvx[2 * bb[e] + 1];
+            const int2 x = reinterpret_cast<const int2*>(d.bvx)[bb[e]];
+            ini[e] = x.x;
+            end[e] = x.y;
             be[e] = d.benab[bb[e]];
+            gl[e] = d.glen[max(gv[e], 0)];
         }
 #pragma unroll
         for (int q = 0; q < 3; q++) {
@@ -2458,16 +2466,18 @@ __device__ __forceinline__ bool tri_items(const Dev& d, int n, int k0, int strid
                 const int e = 3 * q + r;
                 const int oe = (ini[e] == vv[q]) ? end[e] : ini[e];
                 if (oe != vv[qc] || !be[e]) continue;
-                int g0 = -1, g1 = -1;
+                int n0 = -1, n1 = -1;                // lengths of the two grains in common
+                bool have = false;
 #pragma unroll
                 for (int x = 0; x < 3; x++) {
                     const int h = gv[3 * q + x];
                     if (h == gv[3 * qc] || h == gv[3 * qc + 1] || h == gv[3 * qc + 2]) {
-                        if (g0 < 0) g0 = h;
-                        else if (g1 < 0) g1 = h;
+                        if (!have) n0 = gl[3 * q + x];
+                        else if (n1 < 0) n1 = gl[3 * q + x];
+                        have = true;
                     }
                 }
-                if (g1 < 0 || d.glen[g0] != 3 || d.glen[g1] != 3) continue;
+                if (n0 != 3 || n1 != 3) continue;
                 const int s = atomicAdd(&d.cnt[C_TWO], 1);     // rare: two adjacent 3-sided grains
                 if (s < d.E) d.l_two[s] = bb[e];
                 found = true;
@@ -2504,10 +2514,10 @@ __global__ void k_poll_gather(Dev d) {
 // One workgroup per step notes the dt of its labels, for the slots that are
 // labelled at the end of the call (k_label_disabled), and empties the lists
 // that the step has read.
-__device__ __forceinline__ void note_step(const Dev& d) {
-    for (int m = (int)threadIdx.x; m < d.B; m += (int)blockDim.x)
+__device__ __forceinline__ void note_step(const Dev& d, int tid, int nt) {
+    for (int m = tid; m < d.B; m += nt)
         if (d.ms[m].active && d.prm[m].events) d.ms[m].lab_dt = member_dt(d.prm[m], d.ms[m]);
-    if (threadIdx.x == 0) {
+    if (tid == 0) {
         d.cnt[C_NEV] = 0;
         d.cnt[C_NUCL] = 0;
         d.cnt[C_RAN] = 1;
@@ -2528,7 +2538,7 @@ __device__ __forceinline__ void two_stage(const Dev& d) {
 __global__ void __launch_bounds__(1024) k_poll(Dev d) {
     __shared__ __align__(16) unsigned char pbuf[kPollLds];
     const int nc = d.cnt[C_CAND];
-    note_step(d);
+    note_step(d, (int)threadIdx.x, (int)blockDim.x);
     if (nc > 0) poll_list(d, nc, pbuf);
     __syncthreads();
     two_stage(d);
@@ -2878,8 +2888,7 @@ __device__ __forceinline__ FlipIn flip_in(const Dev& d, int A, int B) {
 // orientations), then the reference's sequence of tests and writes runs on
 // local copies in the same order and the writes go out.
 template <class Edit>
-__device__ __forceinline__ void flip(const Dev& d, int bnd, const Params& P, const FlipIn& in, Edit ed) {
-    const double D = P.D;
+__device__ __forceinline__ void flip(const Dev& d, int bnd, double D, double gb_eps, const FlipIn& in, Edit ed) {
     const int A = in.A, B = in.B;
     int vA[3], vB[3], gA[3], gB[3];
 #pragma unroll
@@ -2959,7 +2968,7 @@ __device__ __forceinline__ void flip(const Dev& d, int bnd, const Params& P, con
             auto ori = [&](int g) {
                 return g == gi0 ? oi0 : g == gi1 ? oi1 : g == gn0 ? on0 : g == gn1 ? on1 : d.gori[g];
             };
-            e = gb_energy_func(ori(s0) - ori(s1), P.gb_eps);
+            e = gb_energy_func(ori(s0) - ori(s1), gb_eps);
         }
     }
     d.ben[bnd] = e;
@@ -3007,7 +3016,7 @@ __device__ __forceinline__ void flip_items(const Dev& d, int k0, int stride) {
             d.l_flipc[s] = c;
         } else {
             int m = member_of_edge(d, c);
-            flip(d, c, d.prm[m], fi, EditGlobal{d, 2});
+            flip(d, c, d.prm[m].D, d.prm[m].gb_eps, fi, EditGlobal{d, 2});
         }
         wave_count(d, !clash, member_of_edge(d, c), &MState::flips);
     }
@@ -3027,7 +3036,7 @@ __device__ __forceinline__ void flip_serial(const Dev& d, int* list, int n, Edit
         if (!d.benab[c]) continue;
         int m = member_of_edge(d, c);
         if (!d.ms[m].active) continue;
-        flip(d, c, d.prm[m], flip_in(d, d.bvx[2 * c], d.bvx[2 * c + 1]), ed);
+        flip(d, c, d.prm[m].D, d.prm[m].gb_eps, flip_in(d, d.bvx[2 * c], d.bvx[2 * c + 1]), ed);
         atomicAdd(reinterpret_cast<unsigned long long*>(&d.ms[m].flips), 1ull);
     }
 }
@@ -3053,19 +3062,20 @@ __global__ void k_flip_serial(Dev d) {
 // and the flagged grains and the vertices' edit records are small hash tables,
 // so that no stage waits for an atomic on memory or reads back what another
 // one wrote there.  A dependent load takes 1.3 us (2,000 grains) to 2.6 us (1M)
-// in this kernel, so what a later stage reads is touched early, together with
-// other loads (ev_touch).  With the launches' stages one after the other in one
-// workgroup it took 28 us at 2,000 grains, 66 for the batch, 82 at 1M; the
-// edit records in LDS (instead of memory) and the early loads are 5 us of it.
+// in this kernel, so loads are issued rounds before their use and without
+// branches around them: the barriers wait for LDS only, and a 3-sided grain's
+// surroundings arrive during the polling and the conflict check.  With the
+// launches' stages one after the other in one workgroup it took 28 us at 2,000
+// grains, 66 for the batch, 82 at 1M; the edit records in LDS (instead of memory)
+// are 5 us of the difference, the early loads 3 to 9.
 // Longer lists, and steps with a two-triangle candidate, run the launches'
 // stages.  512 threads, so that a lane has the registers it needs (182): with
 // 1024 it had 128 and spilled 119 to scratch memory, 3 to 4 us a step.
-// Sizes: an edge has at most three grains in common with its ends, so at most
-// 3 kEvMax grains are labelled (a lane each); a removal flags three grains and
+// Sizes: a listed edge is one event at most; a removal flags three grains and
 // records edits at two vertices, a flip four and two.
 struct EvLds {
-    static constexpr int kEH = 1024, kVH = 1024, kTH = 2048, kFH = 4096, kRH = 2048;
-    static constexpr int kT2 = 3 * kEvMax, kFlag = 3 * kT2, kRec = 2 * kT2;
+    static constexpr int kEH = 512, kVH = 1024, kTH = 512, kFH = 2048, kRH = 1024;
+    static constexpr int kFlag = 4 * kEvMax, kRec = 2 * kEvMax;
     int ek[kEH], ep[kEH];             // listed edge -> list position
     int vk[kVH], vp[kVH];             // vertex -> the kept edge at it, kMany if several
     int tk[kTH];                      // labelled grains
@@ -3074,7 +3084,7 @@ struct EvLds {
     short ri[kRH];
     int rv[kRec], rgrn[2][kRec], rvrt[2][kRec], rprev[kRec];
     unsigned short rfix[kRec];
-    int t2[kT2], con[kT2];            // labelled grains, conflicting events
+    int con[kEvMax];                  // conflicting events
     double ct[kEvMax];
     int cid[kEvMax];
     unsigned char cf[kEvMax];         // the edge's label
@@ -3088,8 +3098,8 @@ struct EvLds {
     } room;
 };
 static_assert(sizeof(EvLds) <= kPollLds, "the event stages' tables fit");
-static_assert(EvLds::kT2 <= 2 * kEvThreads && kEvMax < kEvThreads && 4 * kEvMax <= EvLds::kFlag && EvLds::kFlag < EvLds::kFH && EvLds::kT2 < EvLds::kTH &&
-                  EvLds::kRec < EvLds::kRH && 2 * kEvMax < EvLds::kVH && kEvMax < EvLds::kEH,
+static_assert(kEvMax < kEvThreads && EvLds::kFlag < EvLds::kFH && kEvMax < EvLds::kTH && EvLds::kRec < EvLds::kRH &&
+                  2 * kEvMax < EvLds::kVH && kEvMax < EvLds::kEH,
               "every list and table holds what a step can put in");
 constexpr int kFree = -1, kMany = -2;
 
@@ -3236,16 +3246,10 @@ __device__ __forceinline__ void ev_edit(const Dev& d, EvLds& s, bool with_area) 
 
 // The event stages for a list of nc <= kEvMax edges; false (nothing done yet)
 // when a two-triangle candidate was found.
-__device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, EvLds& s) {
+__device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, int4 id, double2 tl, EvLds& s) {
     const int tid = (int)threadIdx.x;
     const bool on = tid < nc;
-    // the edge and its ends
-    int4 id = make_int4(-1, 0, 0, 0);
-    double2 tl = make_double2(0.0, 0.0);
-    if (on) {
-        id = d.c_id[tid];
-        tl = d.c_te[tid];
-    }
+    if (!on) id = make_int4(-1, 0, 0, 0);
     for (int h = tid; h < EvLds::kEH; h += kEvThreads) s.ek[h] = kFree;
     for (int h = tid; h < EvLds::kVH; h += kEvThreads) { s.vk[h] = kFree; s.vp[h] = kFree; }
     for (int h = tid; h < EvLds::kTH; h += kEvThreads) s.tk[h] = kFree;
@@ -3261,40 +3265,65 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, Ev
         s.ep[ev_put(s.ek, EvLds::kEH, c, &fresh)] = tid;
     }
     if (tri_items(d, ntri, kEvThreads - 1 - tid, kEvThreads)) s.two = 1;
-    // the ends' edges, grains and positions; the edges' other ends and flags;
-    // the lengths of the grains around
-    FlipIn fi{};
-    bool cand = false, en6[6], ge[3];
-    int w6[6], gl[3];
-    if (on) {
-        fi = flip_in(d, ab.x, ab.y);
-        cand = is_candidate(te, len, member_dt(d.prm[m], d.ms[m]), d.prm[m].flip_thr);
-    }
+    // Two rounds of loads: the ends' edges, grains and positions and the member's
+    // numbers; then the edges' other ends and flags, the lengths of the grains
+    // around, and what later stages read: the first entries of the grains' lists
+    // and what else a flip of the edge touches.  Every lane loads (slot 0 without
+    // an edge): a branch around a load would end in a wait for it.  The barriers
+    // below wait for LDS only, so the later stages' loads are in flight until
+    // their first use.
+    FlipIn fi = flip_in(d, ab.x, ab.y);
+    const Params& P = d.prm[m];
+    const int adaptive = P.adaptive;
+    const double dt_max = P.dt_max, dt_min = P.dt_min, safety = P.dt_safety, thr = P.flip_thr, D = P.D, gb_eps = P.gb_eps;
+    const unsigned long long tau = d.ms[m].tau_bits;
+    bool en6[6], ge[3];
+    int w6[6], gl[3], touch[9], head[3][3];
+    int2 e6[6];
+    uint8_t f6[6], f3[3];
 #pragma unroll
     for (int j = 0; j < 6; j++) {
-        const int x = j < 3 ? fi.vA[j] : fi.vB[j - 3];
-        const bool other = on && x != c;
-        const int2 e = other ? reinterpret_cast<const int2*>(d.bvx)[x] : make_int2(0, 0);
-        en6[j] = other && d.benab[x] != 0;
-        w6[j] = e.x == (j < 3 ? ab.x : ab.y) ? e.y : e.x;
+        const int x = j < 3 ? fi.vA[j] : fi.vB[j - 3], xs = on && x != c ? x : 0;
+        e6[j] = reinterpret_cast<const int2*>(d.bvx)[xs];
+        f6[j] = d.benab[xs];
     }
 #pragma unroll
     for (int q = 0; q < 3; q++) {
-        gl[q] = on ? d.glen[fi.gA[q]] : 0;
-        ge[q] = on && d.genab[fi.gA[q]] != 0;
+        const int ga = on ? fi.gA[q] : 0, gb = on ? fi.gB[q] : 0;
+        gl[q] = d.glen[ga];
+        f3[q] = d.genab[ga];
+        const int *La = glist(d, ga), *Lb = glist(d, gb);
+        touch[3 * q] = Lb[0];
+        touch[3 * q + 1] = d.glen[gb];
+        touch[3 * q + 2] = reinterpret_cast<const int*>(d.gori)[2 * ga];
+#pragma unroll
+        for (int r = 0; r < 3; r++) head[q][r] = La[min(r, d.S - 1)];
     }
-    if (cand) {
-        // what a flip of the edge, and the edits after it, read
-        const bool ori = d.prm[m].gb_eps != 0.0;
-        int t[12];
+    // member_dt and is_candidate, by selects
+    double dt = safety * __longlong_as_double((long long)tau);
+    dt = dt < dt_min ? dt_min : dt;
+    dt = dt > dt_max ? dt_max : dt;
+    dt = (adaptive == 0) | (tau == 0x7FF0000000000000ull) ? dt_max : dt;
+    const bool cand = on & (te >= 0) & ((te <= dt) | ((thr > 0) & (len > 0) & (len < thr)));
 #pragma unroll
-        for (int q = 0; q < 6; q++) {
-            const int g = q < 3 ? fi.gA[q] : fi.gB[q - 3];
-            t[2 * q] = glist(d, g)[0];
-            t[2 * q + 1] = q < 3 ? (ori ? reinterpret_cast<const int*>(d.gori)[2 * g] : 0) : d.glen[g];
+    for (int j = 0; j < 6; j++) {
+        const int x = j < 3 ? fi.vA[j] : fi.vB[j - 3];
+        en6[j] = on & (x != c) & (f6[j] != 0);
+        w6[j] = e6[j].x == (j < 3 ? ab.x : ab.y) ? e6[j].y : e6[j].x;
+    }
+#pragma unroll
+    for (int q = 0; q < 3; q++) ge[q] = on & (f3[q] != 0);
+    // the 3-sided grain that a candidate's ends have in common, for the T2 labels
+    // below.  An edge with two is a two-triangle candidate in a valid mesh; in
+    // any other it takes the launches' stages too.
+    int q3 = -1;
+#pragma unroll
+    for (int q = 2; q >= 0; q--) {
+        const int g = fi.gA[q];
+        if (cand & (gl[q] == 3) & ge[q] & ((g == fi.gB[0]) | (g == fi.gB[1]) | (g == fi.gB[2]))) {
+            if (q3 >= 0) s.two = 1;
+            q3 = q;
         }
-#pragma unroll
-        for (int q = 0; q < 12; q++) ev_touch(t[q]);
     }
     if (on) {
         s.ct[tid] = te;
@@ -3328,6 +3357,24 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, Ev
         }
     }
 
+    // the 3-sided grain's vertices' edges, grains and, for its removal, positions
+    // and flags, loaded during the polling
+    const int g3 = q3 == 0 ? fi.gA[0] : (q3 == 1 ? fi.gA[1] : fi.gA[2]);
+    int vv[3], bb[9], gv[9], on3[3];
+    double x3[3];
+#pragma unroll
+    for (int r = 0; r < 3; r++) vv[r] = q3 < 0 ? 0 : (q3 == 0 ? head[0][r] : (q3 == 1 ? head[1][r] : head[2][r]));
+#pragma unroll
+    for (int e = 0; e < 9; e++) {
+        bb[e] = d.vb[3 * vv[e / 3] + e % 3];
+        gv[e] = d.vg[3 * vv[e / 3] + e % 3];
+    }
+#pragma unroll
+    for (int e = 0; e < 3; e++) {
+        x3[e] = d.pos[2 * (size_t)vv[e]];
+        on3[e] = d.ven[vv[e]];
+    }
+
     // polling (poll_list's rounds)
     auto votes_self = [&](int e) {
         double min_t = 99999999;
@@ -3351,6 +3398,16 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, Ev
         const int ch = s.changed;
         __syncthreads();
         if (!ch) break;
+    }
+    // the ends and flags of the 3-sided grain's vertices' edges, during the
+    // conflict check (slot 0's edges may be unset where there is no such grain)
+    int2 ends3[9];
+    uint8_t be3[9];
+#pragma unroll
+    for (int e = 0; e < 9; e++) {
+        const int x = q3 < 0 ? 0 : bb[e];
+        ends3[e] = reinterpret_cast<const int2*>(d.bvx)[x];
+        be3[e] = d.benab[x];
     }
     // the conflict check (poll_list's), the kept edge at the far end of a
     // neighbour from the vertex table
@@ -3408,93 +3465,52 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, Ev
     }
     __syncthreads();
 
-    // T2 labels (t2_label_items)
-    if (cand) {
-#pragma unroll 1
-        for (int q = 0; q < 3; q++) {
-            const int g = q == 0 ? fi.gA[0] : (q == 1 ? fi.gA[1] : fi.gA[2]);
-            const int n = q == 0 ? gl[0] : (q == 1 ? gl[1] : gl[2]);
-            const bool e_ = q == 0 ? ge[0] : (q == 1 ? ge[1] : ge[2]);
-            if (n != 3 || !e_ || !(g == fi.gB[0] || g == fi.gB[1] || g == fi.gB[2])) continue;
-            const int* L = glist(d, g);
-            const int vv[3] = {L[0], L[1], L[2]};
-            int bb[9];
-            int2 ends[9];
-            bool be[9];
+    // T2 labels (t2_label_items) and removals: a grain's lane labels it, and
+    // removes it at once if no other labelled one is around (t2_items)
 #pragma unroll
-            for (int e = 0; e < 9; e++) bb[e] = d.vb[3 * vv[e / 3] + e % 3];
-            int gv[9], on3[3];
-            double x3[3];
-            // what the removal reads is loaded with them
+    for (int q = 0; q < 9; q++) ev_touch(touch[q]);
 #pragma unroll
-            for (int e = 0; e < 9; e++) gv[e] = d.vg[3 * vv[e / 3] + e % 3];
+    for (int e = 0; e < 3; e++) { ev_touch((int)__double2loint(x3[e])); ev_touch(on3[e]); }
+    bool mine = false;
+    if (q3 >= 0) {
+        auto in_g = [&](int x) { return x == vv[0] || x == vv[1] || x == vv[2]; };
+        bool hit = false;
+        int ans = 0, first = INT_MAX;
 #pragma unroll
-            for (int e = 0; e < 3; e++) {
-                x3[e] = d.pos[2 * (size_t)vv[e]];
-                on3[e] = d.ven[vv[e]];
+        for (int e = 0; e < 9; e++) {
+            const bool in = in_g(ends3[e].x) && in_g(ends3[e].y) && be3[e];
+            if (!in) continue;
+            const int p = edge_pos(bb[e]), lab = p >= 0 ? s.cf[p] : 0;
+            hit = hit || (lab & 1);
+            if (lab & 2) {
+                ans++;
+                first = min(first, bb[e]);
             }
-#pragma unroll
-            for (int e = 0; e < 9; e++) {
-                ends[e] = reinterpret_cast<const int2*>(d.bvx)[bb[e]];
-                be[e] = d.benab[bb[e]] != 0;
-            }
-#pragma unroll
-            for (int e = 0; e < 9; e++) ev_touch(gv[e]);
-#pragma unroll
-            for (int e = 0; e < 3; e++) { ev_touch((int)__double2loint(x3[e])); ev_touch(on3[e]); }
-            auto in_g = [&](int x) { return x == vv[0] || x == vv[1] || x == vv[2]; };
-            bool hit = false;
-            int ans = 0, first = INT_MAX;
-#pragma unroll
-            for (int e = 0; e < 9; e++) {
-                const bool in = in_g(ends[e].x) && in_g(ends[e].y) && be[e];
-                if (!in) continue;
-                const int p = edge_pos(bb[e]), lab = p >= 0 ? s.cf[p] : 0;
-                hit = hit || (lab & 1);
-                if (lab & 2) {
-                    ans++;
-                    first = min(first, bb[e]);
-                }
-            }
-            if (!(hit || ans / 2 == 3) || first != c) continue;
+        }
+        mine = (hit || ans / 2 == 3) && first == c;
+        if (mine) {
             bool fresh;
-            ev_put(s.tk, EvLds::kTH, g, &fresh);
-            s.t2[atomicAdd(&s.nt2, 1)] = g;
+            ev_put(s.tk, EvLds::kTH, g3, &fresh);
+            s.nt2 = 1;
         }
     }
     __syncthreads();
     const int nt2 = s.nt2;
     const EditLds ed{s};
     if (nt2 > 0) {
-        // a candidate with no other one around is removed at once (t2_items)
-        bool go[2] = {false, false};
-#pragma unroll 1
-        for (int u = 0; tid + u * kEvThreads < nt2; u++) {
-            const int g = s.t2[tid + u * kEvThreads];
-            const int* L = glist(d, g);
-            int h[9];
-#pragma unroll
-            for (int e = 0; e < 9; e++) h[e] = d.vg[3 * L[e / 3] + e % 3];
-            bool clash = false;
+        bool clash = false;
+        if (mine) {
 #pragma unroll 1
             for (int e = 0; e < 9; e++) {
-                int x = h[0];
+                int x = gv[0];
 #pragma unroll
-                for (int r = 1; r < 9; r++) x = e == r ? h[r] : x;
-                clash = clash || (x != g && x >= 0 && s.tk[ev_find(s.tk, EvLds::kTH, x)] == x);
+                for (int r = 1; r < 9; r++) x = e == r ? gv[r] : x;
+                clash = clash || (x != g3 && x >= 0 && s.tk[ev_find(s.tk, EvLds::kTH, x)] == x);
             }
-            if (clash) s.con[atomicAdd(&s.ncon, 1)] = g;
-            if (u == 0) go[0] = !clash;
-            else go[1] = !clash;
+            if (clash) s.con[atomicAdd(&s.ncon, 1)] = g3;
+            else remove_grain(d, g3, D, slot_base(d, m), ed);
         }
-        __syncthreads();
-#pragma unroll 1
-        for (int u = 0; u * kEvThreads < nt2; u++) {
-            const bool rm = u == 0 ? go[0] : go[1];
-            const int g = rm ? s.t2[tid + u * kEvThreads] : 0, mg = rm ? member_of_grain(d, g) : 0;
-            if (rm) remove_grain(d, g, d.prm[mg].D, slot_base(d, mg), ed);
-            wave_count(d, rm, mg, &MState::removals);
-        }
+        wave_count(d, mine && !clash, m, &MState::removals);
         __syncthreads();
         if (s.ncon > 0) {
             if (tid == 0) t2_serial(d, s.con, s.ncon, ed);
@@ -3541,7 +3557,7 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, Ev
             clash = clash || (x != c && flagp(edge_pos(x)));
         }
         if (clash) s.con[atomicAdd(&s.ncon, 1)] = c;
-        else flip(d, c, d.prm[m], fi, ed);
+        else flip(d, c, D, gb_eps, fi, ed);
     }
     wave_count(d, live && !clash, m, &MState::flips);
     __syncthreads();
@@ -3558,11 +3574,20 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, Ev
 __global__ void __launch_bounds__(kEvThreads) k_events(Dev d) {
     __shared__ __align__(16) unsigned char buf[kPollLds];
     const int tid = (int)threadIdx.x, nt = (int)blockDim.x, wave = tid >> 6;
+    // the listed edges with the length of their list (what lies past it is not used)
+    int4 id = make_int4(-1, 0, 0, 0);
+    double2 tl = make_double2(0.0, 0.0);
+    if (tid < kEvMax) {
+        id = d.c_id[tid];
+        tl = d.c_te[tid];
+    }
     const int nc = d.cnt[C_CAND], ntri = n_tri(d);
-    note_step(d);
+    // on lanes that hold no listed edge
+    static_assert(kEvMax <= 192 && kEvThreads > 256, "waves 0 to 2 hold the edges, wave 4 notes the step");
+    if (wave == 4) note_step(d, tid - 256, 64);
     if (nc == 0 && ntri == 0) return;
     if (nc <= kEvMax) {
-        if (events_in_lds(d, nc, ntri, *reinterpret_cast<EvLds*>(buf))) return;
+        if (events_in_lds(d, nc, ntri, id, tl, *reinterpret_cast<EvLds*>(buf))) return;
     } else {
         tri_items(d, ntri, nt - 1 - tid, nt);
     }
