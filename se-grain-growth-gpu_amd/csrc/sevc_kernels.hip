@@ -2077,7 +2077,8 @@ __device__ __forceinline__ void fix_wave(const Dev& d, int g, FixLds& f_) {
 // `grain` gives the items' grains and `record` a vertex's record; `replay`
 // takes a mask of lanes, the first of each group that needs fix_wave, and its
 // grain in those lanes; `after` takes an edited list: each lane's group (its
-// first lane), place, entry and whether it has one, the grain and the length.
+// first lane), place, entry and whether it has one, the grain and the length;
+// `tri` takes the grains left with three vertices (list_tri).
 struct EditRec {
     int g[4], v[4], p[4];
     unsigned fix;
@@ -2092,26 +2093,42 @@ __device__ __forceinline__ EditRec record_global(const Dev& d, int v) {
                    *reinterpret_cast<const unsigned*>(d.mods[v].fix)};
 }
 
-template <class Grain, class Record, class Replay, class After>
+template <class Grain, class Record, class Replay, class After, class Tri>
 __device__ __forceinline__ void fix_items(const Dev& d, int n_items, Grain grain, Record record, QuickLds& f, int w, int nw,
-                                          Replay replay, After after) {
+                                          Replay replay, After after, Tri tri) {
     const int lane = (int)threadIdx.x & 63, l = lane & (kQuick - 1), g0 = lane & ~(kQuick - 1);
     const unsigned below = (1u << l) - 1u;
     // the group's part of a ballot
     auto group = [&](bool x) { return (unsigned)(__ballot(x) >> g0) & 0xFFFFu; };
-    for (int base = 4 * w; base < n_items; base += 4 * nw) {
+    // the next items' loads are issued before the work on the present ones
+    struct Item {
+        int g, n0, v, cap;
+        uint8_t en;
+        bool on;
+    };
+    auto fetch = [&](int base) {
+        Item t;
         const int item = base + (lane >> 4);
-        const bool on = item < n_items;
-        const int g = on ? grain(item) : 0;
+        t.on = item < n_items;
+        t.g = t.on ? grain(item) : 0;
+        const int* L = glist(d, t.g);
+        t.en = d.genab[t.g];
+        t.n0 = d.glen[t.g];
+        t.v = L[min(l, d.S - 1)];
+        t.cap = d.prm[member_of_grain(d, t.g)].cap;
+        return t;
+    };
+    Item next = fetch(4 * w);
+    for (int base = 4 * w; base < n_items; base += 4 * nw) {
+        const Item it = next;
+        next = fetch(base + 4 * nw);
+        const int g = it.g, n0 = it.n0, cap = it.cap, v = l < d.S ? it.v : -1;
         int* L = glist(d, g);
-        const bool en = on && d.genab[g] != 0;
-        const int n0 = d.glen[g], v = l < d.S ? L[l] : -1;
-        const int mem = member_of_grain(d, g);
+        const bool en = it.on && it.en != 0;
         bool slow = en && n0 > kQuick;
         const bool has = en && !slow && l < n0;
         EditRec r = no_edits();
         if (has) r = record(v);
-        const int cap = d.prm[mem].cap;
         int adds = 0, reps = 0, vadd = -1, vrep = -1;
         unsigned rem = 0;
 #pragma unroll
@@ -2186,7 +2203,7 @@ __device__ __forceinline__ void fix_items(const Dev& d, int n_items, Grain grain
             if (l == 0) d.glen[g] = n2;
         }
         after(g0, at, rep ? vrep_src : x, stay && !slow_g, g, en && !slow_g ? n2 : -1);
-        list_tri(d, g, en && !slow_g && l == 0 && n2 == 3);
+        tri(g, en && !slow_g && l == 0 && n2 == 3);
         wave_sync();
         replay(__ballot(en && slow_g && l == 0), g);
     }
@@ -2203,7 +2220,7 @@ __device__ __forceinline__ void fix_stage(const Dev& d, int stage, FixLds& f, Qu
                 wave_sync();
             }
         },
-        [](int, int, int, bool, int, int) {});
+        [](int, int, int, bool, int, int) {}, [&](int g, bool want) { list_tri(d, g, want); });
 }
 
 __global__ void __launch_bounds__(64) k_fix(Dev d, int stage) {
@@ -2431,11 +2448,12 @@ __device__ __forceinline__ void two_grain_serial(const Dev& d) {
 // the set grains_intersect forms from the edge's ends.  An edge that both of
 // its grains list comes twice; the second finds it gone.  (A pass over all
 // grains took 17.5 us at 1M grains, 8 at 2,000.)
-__device__ __forceinline__ bool tri_items(const Dev& d, int n, int k0, int stride) {
+// `first`: the grain at k0, if the caller has it (k0 < n).
+__device__ __forceinline__ bool tri_items(const Dev& d, int n, int k0, int stride, int first = -1) {
     bool found = false;
     for (int k = k0; k < n; k += stride) {
         // (tests after the loads, not between them: each would be a wait)
-        const int g = d.l_tri[k], m = member_of_grain(d, g);
+        const int g = k == k0 && first >= 0 ? first : d.l_tri[k], m = member_of_grain(d, g);
         const int* L = glist(d, g);
         const uint8_t on = d.genab[g];
         const int len = d.glen[g], act = d.ms[m].active, ev = d.prm[m].events;
@@ -2624,6 +2642,7 @@ struct EditGlobal {
     __device__ __forceinline__ void operator()(const int (&g)[N], const bool (&want)[N]) const {
         flag_grains(d, g, want, stage);
     }
+    __device__ __forceinline__ int flip_slot() const { return wave_slot(d.n_flipped, true); }
 };
 
 // remove_grain, topological.h:687-822.  Everything the removal reads is loaded
@@ -2632,26 +2651,51 @@ struct EditGlobal {
 // runs on local copies in the same order -- a later test sees an earlier write
 // exactly as it would in memory -- and the writes go out.
 // The list edits go to `ed`.
+struct RemoveIn {
+    int v[3], vb[9], vg[9];                        // the grain's vertices; their edges and grains
+    double2 p[3];
+    int2 ends[9];                                  // ends of the edges
+    bool on[3], onE[9], onG;                       // flags of the vertices, the edges, the grain
+};
+__device__ __forceinline__ RemoveIn remove_in(const Dev& d, int g) {
+    RemoveIn r;
+    const int* L = glist(d, g);
+#pragma unroll
+    for (int k = 0; k < 3; k++) r.v[k] = L[k];
+#pragma unroll
+    for (int e = 0; e < 9; e++) {
+        r.vb[e] = d.vb[3 * r.v[e / 3] + e % 3];
+        r.vg[e] = d.vg[3 * r.v[e / 3] + e % 3];
+    }
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        r.p[k] = reinterpret_cast<const double2*>(d.pos)[r.v[k]];
+        r.on[k] = d.ven[r.v[k]] != 0;
+    }
+    r.onG = d.genab[g] != 0;
+#pragma unroll
+    for (int e = 0; e < 9; e++) {
+        r.ends[e] = reinterpret_cast<const int2*>(d.bvx)[r.vb[e]];
+        r.onE[e] = d.benab[r.vb[e]] != 0;
+    }
+    return r;
+}
+
 template <class Edit>
-__device__ __forceinline__ void remove_grain(const Dev& d, int g, double D, const SlotBase& S, Edit ed) {
-    const int* Lg = glist(d, g);
-    const int A = Lg[0], B = Lg[1], C = Lg[2];
+__device__ __forceinline__ void remove_grain(const Dev& d, int g, const RemoveIn& in, double D, const SlotBase& S, Edit ed) {
+    const int A = in.v[0], B = in.v[1], C = in.v[2];
     int vA[3], vB[3], vC[3], gA[3], gB[3], gC[3];
-    load_triple(d.vb, A, vA); load_triple(d.vb, B, vB); load_triple(d.vb, C, vC);
-    load_triple(d.vg, A, gA); load_triple(d.vg, B, gB); load_triple(d.vg, C, gC);
-    const double2* X = reinterpret_cast<const double2*>(d.pos);
-    const double2 pA = X[A], pB = X[B], pC = X[C];
-    const bool onB = d.ven[B] != 0, onC = d.ven[C] != 0, onG = d.genab[g] != 0;
     int2 xA[3], xB[3], xC[3];                      // ends of the vertices' edges
     bool onA_[3], onC_[3];                         // flags of A's and C's edges
 #pragma unroll
-    for (int i = 0; i < 3; i++) {
-        xA[i] = reinterpret_cast<const int2*>(d.bvx)[vA[i]];
-        xB[i] = reinterpret_cast<const int2*>(d.bvx)[vB[i]];
-        xC[i] = reinterpret_cast<const int2*>(d.bvx)[vC[i]];
-        onA_[i] = d.benab[vA[i]] != 0;
-        onC_[i] = d.benab[vC[i]] != 0;
+    for (int k = 0; k < 3; k++) {
+        vA[k] = in.vb[k]; vB[k] = in.vb[3 + k]; vC[k] = in.vb[6 + k];
+        gA[k] = in.vg[k]; gB[k] = in.vg[3 + k]; gC[k] = in.vg[6 + k];
+        xA[k] = in.ends[k]; xB[k] = in.ends[3 + k]; xC[k] = in.ends[6 + k];
+        onA_[k] = in.onE[k]; onC_[k] = in.onE[6 + k];
     }
+    const double2 pA = in.p[0], pB = in.p[1], pC = in.p[2];
+    const bool onB = in.on[1], onC = in.on[2], onG = in.onG;
     const double xp0 = pA.x, xp1 = pB.x, xp2 = pC.x, yp0 = pA.y, yp1 = pB.y, yp2 = pC.y;
     double nAB = arclen(xp0, yp0, xp1, yp1, D);
     double nBC = arclen(xp1, yp1, xp2, yp2, D);
@@ -2790,7 +2834,7 @@ __device__ __forceinline__ void t2_items(const Dev& d, int k0, int stride) {
             d.l_t2c[s] = g;
         } else {
             int m = member_of_grain(d, g);
-            remove_grain(d, g, d.prm[m].D, slot_base(d, m), EditGlobal{d, 1});
+            remove_grain(d, g, remove_in(d, g), d.prm[m].D, slot_base(d, m), EditGlobal{d, 1});
         }
         wave_count(d, !clash, member_of_grain(d, g), &MState::removals);
     }
@@ -2810,7 +2854,7 @@ __device__ __forceinline__ void t2_serial(const Dev& d, int* list, int n, Edit e
         if (!d.genab[g]) continue;
         int m = member_of_grain(d, g);
         if (!d.ms[m].active) continue;
-        remove_grain(d, g, d.prm[m].D, slot_base(d, m), ed);
+        remove_grain(d, g, remove_in(d, g), d.prm[m].D, slot_base(d, m), ed);
         atomicAdd(reinterpret_cast<unsigned long long*>(&d.ms[m].removals), 1ull);
     }
 }
@@ -2974,7 +3018,7 @@ __device__ __forceinline__ void flip(const Dev& d, int bnd, double D, double gb_
     d.ben[bnd] = e;
     {
         // rescaled at the next step's start (begin_member) when no full pass runs
-        const int k = wave_slot(d.n_flipped, true);
+        const int k = ed.flip_slot();
         if (k < d.E) d.l_flipped[k] = bnd;
     }
     d.vel[2 * A] = 0; d.vel[2 * A + 1] = 0;
@@ -3088,7 +3132,7 @@ struct EvLds {
     double ct[kEvMax];
     int cid[kEvMax];
     unsigned char cf[kEvMax];         // the edge's label
-    int nt2, ncon, nfl, nrec, changed, two, nslow;
+    int nt2, ncon, nfl, nrec, changed, two, nslow, nflip, ntri;
     int slow[kFlag];                  // grains for fix_wave
     QuickLds quick[kEvThreads / 64];
     static constexpr int kSlow = 3;
@@ -3151,6 +3195,7 @@ struct EditLds {
         s.rfix[r] = (unsigned short)((s.rfix[r] & keep) | ((unsigned)fix << (8 * slot)));
     }
     __device__ __forceinline__ void put_prev(int r, int, int prev) const { s.rprev[r] = prev; }   // of slot 1
+    __device__ __forceinline__ int flip_slot() const { return atomicAdd(&s.nflip, 1); }           // (k_text emptied the list)
     template <int N>
     __device__ __forceinline__ void operator()(const int (&g)[N], const bool (&want)[N]) const {
 #pragma unroll 1
@@ -3196,7 +3241,9 @@ __device__ __forceinline__ void ev_edit(const Dev& d, EvLds& s, bool with_area) 
     QuickLds& q = s.quick[wave];
     const double2* X = reinterpret_cast<const double2*>(d.pos);
     fix_items(
-        d, n, [&](int k) { return s.fl[k]; }, [&](int v) { return record_lds(s, v); }, q, wave, kEvThreads / 64,
+        d, n, [&](int k) { return s.fl[k]; }, [&](int v) { return record_lds(s, v); }, q,
+        (wave + kEvThreads / 128) % (kEvThreads / 64), kEvThreads / 64,   // first the waves that have no event's stores out
+
         [&](unsigned long long todo, int g) {
             if ((todo >> lane) & 1ull) s.slow[atomicAdd(&s.nslow, 1)] = g;
         },
@@ -3217,9 +3264,17 @@ __device__ __forceinline__ void ev_edit(const Dev& d, EvLds& s, bool with_area) 
                 if (k < n2) acc.push_delta(ex, ey);
             }
             if (n2 >= 0 && l == 0) d.garea[g] = n2 > 0 ? acc.finish() : 0.0;
+        },
+        [&](int g, bool want) {
+            // only this workgroup lists grains now, so that the count is kept in LDS
+            if (!want) return;
+            const int k = atomicAdd(&s.ntri, 1);
+            if ((unsigned)k < 6u * (unsigned)d.G) d.l_tri[k] = g;
         });
     __syncthreads();
     if (s.nslow > 0) {
+        if (tid == 0) atomicExch(&d.cnt[C_TRI], s.ntri);
+        __syncthreads();
         for (int r = tid; r < s.nrec; r += kEvThreads) {
             const int v = s.rv[r];
             for (int j = 0; j < 2; j++) set_mod(d, v, j, (s.rfix[r] >> (8 * j)) & 255, s.rgrn[j][r], s.rvrt[j][r]);
@@ -3236,6 +3291,7 @@ __device__ __forceinline__ void ev_edit(const Dev& d, EvLds& s, bool with_area) 
             fix_clear_items(d, s.nslow, 0, [&](int k) { return s.slow[k]; }, with_area ? 1 : 0, s.room.clear[wave], wave,
                             EvLds::kSlow);
         for (int r = tid; r < s.nrec; r += kEvThreads) reset_mods(d, s.rv[r]);
+        if (tid == 0) s.ntri = cnt_now(d, C_TRI);
     }
     for (int h = tid; h < EvLds::kFH; h += kEvThreads) s.fk[h] = kFree;
     for (int h = tid; h < EvLds::kRH; h += kEvThreads) s.rk[h] = kFree;
@@ -3246,7 +3302,7 @@ __device__ __forceinline__ void ev_edit(const Dev& d, EvLds& s, bool with_area) 
 
 // The event stages for a list of nc <= kEvMax edges; false (nothing done yet)
 // when a two-triangle candidate was found.
-__device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, int4 id, double2 tl, EvLds& s) {
+__device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, int4 id, double2 tl, int g_tri, EvLds& s) {
     const int tid = (int)threadIdx.x;
     const bool on = tid < nc;
     if (!on) id = make_int4(-1, 0, 0, 0);
@@ -3255,7 +3311,7 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, in
     for (int h = tid; h < EvLds::kTH; h += kEvThreads) s.tk[h] = kFree;
     for (int h = tid; h < EvLds::kFH; h += kEvThreads) s.fk[h] = kFree;
     for (int h = tid; h < EvLds::kRH; h += kEvThreads) s.rk[h] = kFree;
-    if (tid == 0) s.nt2 = s.ncon = s.nfl = s.nrec = s.two = s.nslow = 0;
+    if (tid == 0) s.nt2 = s.ncon = s.nfl = s.nrec = s.two = s.nslow = s.nflip = s.ntri = 0;
     const int c = id.x, m = id.w;
     int2 ab = make_int2(id.y, id.z);
     const double te = tl.x, len = tl.y;
@@ -3264,7 +3320,7 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, in
         bool fresh;
         s.ep[ev_put(s.ek, EvLds::kEH, c, &fresh)] = tid;
     }
-    if (tri_items(d, ntri, kEvThreads - 1 - tid, kEvThreads)) s.two = 1;
+    if (tri_items(d, ntri, kEvThreads - 1 - tid, kEvThreads, g_tri)) s.two = 1;
     // Two rounds of loads: the ends' edges, grains and positions and the member's
     // numbers; then the edges' other ends and flags, the lengths of the grains
     // around, and what later stages read: the first entries of the grains' lists
@@ -3277,6 +3333,7 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, in
     const int adaptive = P.adaptive;
     const double dt_max = P.dt_max, dt_min = P.dt_min, safety = P.dt_safety, thr = P.flip_thr, D = P.D, gb_eps = P.gb_eps;
     const unsigned long long tau = d.ms[m].tau_bits;
+    const SlotBase slots = slot_base(d, m);
     bool en6[6], ge[3];
     int w6[6], gl[3], touch[9], head[3][3];
     int2 e6[6];
@@ -3332,8 +3389,10 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, in
     }
     __syncthreads();
     if (s.two) return false;
-    if (tid == 0) atomicExch(&d.cnt[C_TRI], 0);         // searched; the edits below list anew
-    if (nc == 0) return true;
+    if (nc == 0) {
+        if (tid == 0) atomicExch(&d.cnt[C_TRI], 0);     // searched
+        return true;
+    }
     auto edge_pos = [&](int x) {
         const int h = ev_find(s.ek, EvLds::kEH, x);
         return s.ek[h] == x ? s.ep[h] : -1;
@@ -3341,27 +3400,28 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, in
     auto flagp = [&](int p) { return p >= 0 && s.cf[p] != 0; };
     // (the first probes of the six searches are read together)
     int ep[6];
-    {
+    auto edge_places = [&](const FlipIn& f, bool want) {
         int hh[6], kk[6];
 #pragma unroll
         for (int j = 0; j < 6; j++) {
-            hh[j] = ev_hash(j < 3 ? fi.vA[j] : fi.vB[j - 3], EvLds::kEH);
+            hh[j] = ev_hash(j < 3 ? f.vA[j] : f.vB[j - 3], EvLds::kEH);
             kk[j] = s.ek[hh[j]];
             ep[j] = s.ep[hh[j]];
         }
 #pragma unroll
         for (int j = 0; j < 6; j++) {
-            const int x = j < 3 ? fi.vA[j] : fi.vB[j - 3];
-            if (!on || kk[j] == kFree) ep[j] = -1;
+            const int x = j < 3 ? f.vA[j] : f.vB[j - 3];
+            if (!want || kk[j] == kFree) ep[j] = -1;
             else if (kk[j] != x) ep[j] = edge_pos(x);
         }
-    }
+    };
+    edge_places(fi, on);
 
     // the 3-sided grain's vertices' edges, grains and, for its removal, positions
     // and flags, loaded during the polling
     const int g3 = q3 == 0 ? fi.gA[0] : (q3 == 1 ? fi.gA[1] : fi.gA[2]);
     int vv[3], bb[9], gv[9], on3[3];
-    double x3[3];
+    double2 p3[3];
 #pragma unroll
     for (int r = 0; r < 3; r++) vv[r] = q3 < 0 ? 0 : (q3 == 0 ? head[0][r] : (q3 == 1 ? head[1][r] : head[2][r]));
 #pragma unroll
@@ -3371,7 +3431,7 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, in
     }
 #pragma unroll
     for (int e = 0; e < 3; e++) {
-        x3[e] = d.pos[2 * (size_t)vv[e]];
+        p3[e] = reinterpret_cast<const double2*>(d.pos)[vv[e]];
         on3[e] = d.ven[vv[e]];
     }
 
@@ -3461,7 +3521,6 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, in
     __syncthreads();                                     // every label read
     if (on) {
         s.cf[tid] = (unsigned char)((keep ? 1 : 0) | (cand ? 2 : 0));
-        d.conf[c] = -1;
     }
     __syncthreads();
 
@@ -3469,9 +3528,7 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, in
     // removes it at once if no other labelled one is around (t2_items)
 #pragma unroll
     for (int q = 0; q < 9; q++) ev_touch(touch[q]);
-#pragma unroll
-    for (int e = 0; e < 3; e++) { ev_touch((int)__double2loint(x3[e])); ev_touch(on3[e]); }
-    bool mine = false;
+    bool mine = false, removed = false;
     if (q3 >= 0) {
         auto in_g = [&](int x) { return x == vv[0] || x == vv[1] || x == vv[2]; };
         bool hit = false;
@@ -3500,17 +3557,36 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, in
     if (nt2 > 0) {
         bool clash = false;
         if (mine) {
-#pragma unroll 1
-            for (int e = 0; e < 9; e++) {
-                int x = gv[0];
+            int kk[9];
 #pragma unroll
-                for (int r = 1; r < 9; r++) x = e == r ? gv[r] : x;
-                clash = clash || (x != g3 && x >= 0 && s.tk[ev_find(s.tk, EvLds::kTH, x)] == x);
+            for (int e = 0; e < 9; e++) kk[e] = s.tk[ev_hash(gv[e], EvLds::kTH)];
+#pragma unroll
+            for (int e = 0; e < 9; e++) {
+                const int x = gv[e];
+                if (x == g3 || x < 0 || kk[e] == kFree) continue;
+                clash = clash || kk[e] == x || s.tk[ev_find(s.tk, EvLds::kTH, x)] == x;
             }
             if (clash) s.con[atomicAdd(&s.ncon, 1)] = g3;
-            else remove_grain(d, g3, D, slot_base(d, m), ed);
+            else {
+                RemoveIn in;
+#pragma unroll
+                for (int k = 0; k < 3; k++) {
+                    in.v[k] = vv[k];
+                    in.p[k] = p3[k];
+                    in.on[k] = on3[k] != 0;
+                }
+#pragma unroll
+                for (int e = 0; e < 9; e++) {
+                    in.vb[e] = bb[e];
+                    in.vg[e] = gv[e];
+                    in.ends[e] = ends3[e];
+                    in.onE[e] = be3[e] != 0;
+                }
+                in.onG = true;
+                remove_grain(d, g3, in, D, slots, ed);
+            }
         }
-        wave_count(d, mine && !clash, m, &MState::removals);
+        removed = mine && !clash;
         __syncthreads();
         if (s.ncon > 0) {
             if (tid == 0) t2_serial(d, s.con, s.ncon, ed);
@@ -3543,51 +3619,55 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, in
         }
         label = !(k < 2 || n0 == 3 || n1 == 3);
     }
-    if (keep) d.bcand[c] = label ? 1 : 0;
     live = live && label;
     if (on) s.cf[tid] = live ? 1 : 0;
     __syncthreads();
+    if (nt2 > 0) edge_places(fi, live);                  // (the edges around may have changed)
     bool clash = false;
     if (live) {
-#pragma unroll 1
-        for (int j = 0; j < 6; j++) {
-            int x = fi.vA[0];
 #pragma unroll
-            for (int r = 1; r < 6; r++) x = j == r ? (r < 3 ? fi.vA[r] : fi.vB[r - 3]) : x;
-            clash = clash || (x != c && flagp(edge_pos(x)));
-        }
+        for (int j = 0; j < 6; j++) clash = clash | ((ep[j] != tid) & (ep[j] >= 0 ? s.cf[max(ep[j], 0)] != 0 : false));
         if (clash) s.con[atomicAdd(&s.ncon, 1)] = c;
         else flip(d, c, D, gb_eps, fi, ed);
     }
-    wave_count(d, live && !clash, m, &MState::flips);
     __syncthreads();
     if (s.ncon > 0) {
         if (tid == 0) flip_serial(d, s.con, s.ncon, ed);
         __syncthreads();
     }
-    if (s.nfl == 0) return true;
     if (tid == 0) d.cnt[C_FIX2] = s.nfl;
-    ev_edit(d, s, false);
+    if (s.nfl > 0) ev_edit(d, s, false);
+    // what no later stage reads goes out last: a load waits for the stores before it
+    if (on) d.conf[c] = -1;
+    if (keep) d.bcand[c] = label ? 1 : 0;
+    wave_count(d, removed, m, &MState::removals);
+    wave_count(d, live && !clash, m, &MState::flips);
+    if (tid == 0) {
+        *d.n_flipped = s.nflip;
+        atomicExch(&d.cnt[C_TRI], s.ntri);              // those searched go, the edits' stay
+    }
     return true;
 }
 
 __global__ void __launch_bounds__(kEvThreads) k_events(Dev d) {
     __shared__ __align__(16) unsigned char buf[kPollLds];
     const int tid = (int)threadIdx.x, nt = (int)blockDim.x, wave = tid >> 6;
-    // the listed edges with the length of their list (what lies past it is not used)
+    // the listed edges, and the grains for the two-triangle search (from the last
+    // lane on), with the lengths of their lists (what lies past them is not used)
     int4 id = make_int4(-1, 0, 0, 0);
     double2 tl = make_double2(0.0, 0.0);
     if (tid < kEvMax) {
         id = d.c_id[tid];
         tl = d.c_te[tid];
     }
+    const int k_tri = kEvThreads - 1 - tid, g_tri = d.l_tri[min((unsigned)k_tri, 6u * (unsigned)d.G - 1u)];
     const int nc = d.cnt[C_CAND], ntri = n_tri(d);
     // on lanes that hold no listed edge
     static_assert(kEvMax <= 192 && kEvThreads > 256, "waves 0 to 2 hold the edges, wave 4 notes the step");
     if (wave == 4) note_step(d, tid - 256, 64);
     if (nc == 0 && ntri == 0) return;
     if (nc <= kEvMax) {
-        if (events_in_lds(d, nc, ntri, id, tl, *reinterpret_cast<EvLds*>(buf))) return;
+        if (events_in_lds(d, nc, ntri, id, tl, g_tri, *reinterpret_cast<EvLds*>(buf))) return;
     } else {
         tri_items(d, ntri, nt - 1 - tid, nt);
     }
