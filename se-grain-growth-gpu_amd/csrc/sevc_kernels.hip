@@ -49,48 +49,41 @@ __device__ __forceinline__ bool rate_nucleates(const Params& P, int n) {
     return (n % gap) == 0;
 }
 
-// Begins a step for member m (one workgroup): loop condition of main.cu:120
-// (time rule), grain rule, nucleation gate main.cu:137-141.
-__device__ __forceinline__ void begin_member(const Dev& d, int m, bool rescale_flipped) {
-    const Params& P = d.prm[m];
-    MState& M = d.ms[m];
-    if (threadIdx.x == 0) {
-        M.tau_bits = 0x7FF0000000000000ull;
-        int nucl_now = 0;
-        const bool runs = !M.done && member_runs(P, M);
-        if (runs) {
-            M.vsteps += M.n_venabled;
-            if (P.events && P.do_nucl) {
-                const int gap = P.gap > 0 ? P.gap : 1;
-                if (P.nucl_mode == SEVC_NUCL_MC) {
-                    if (M.curr_grains <= P.gate_grains) M.allow_nucl = 1;   // main.cu:137-139
-                    nucl_now = ((M.n % gap) == 0 && M.allow_nucl) ? 1 : 0;
-                } else {
-                    nucl_now = rate_nucleates(P, M.n) ? 1 : 0;
-                }
+// Begins a step of a member: loop condition of main.cu:120 (time rule), grain
+// rule, nucleation gate main.cu:137-141.
+__device__ __forceinline__ void begin_state(const Params& P, MState& M) {
+    M.tau_bits = 0x7FF0000000000000ull;
+    int nucl_now = 0;
+    const bool runs = !M.done && member_runs(P, M);
+    if (runs) {
+        M.vsteps += M.n_venabled;
+        if (P.events && P.do_nucl) {
+            const int gap = P.gap > 0 ? P.gap : 1;
+            if (P.nucl_mode == SEVC_NUCL_MC) {
+                if (M.curr_grains <= P.gate_grains) M.allow_nucl = 1;   // main.cu:137-139
+                nucl_now = ((M.n % gap) == 0 && M.allow_nucl) ? 1 : 0;
+            } else {
+                nucl_now = rate_nucleates(P, M.n) ? 1 : 0;
             }
-        } else {
-            M.done = 1;
         }
-        M.nucl_now = nucl_now;
-        M.open = runs ? 1 : 0;
-        M.active = runs ? 1 : 0;
+    } else {
+        M.done = 1;
     }
-    __syncthreads();
-    // flip (topological.h:286) leaves the flipped edge's energy without the
-    // GB_scaling factor until compute_boundary_energies (calculus.h:104-114)
-    // runs at the next step's start.  Steps that skip that pass (GB_eps = 0,
-    // where every other energy is the scale itself) recompute only the
-    // edges flipped since, for the members active in this step (steps that
-    // run k_edge_len_energy recompute every energy there).  k_text empties
-    // the list.
-    const int nf = rescale_flipped && M.active ? min(*d.n_flipped, d.E) : 0;
-    for (int k = (int)threadIdx.x; k < nf; k += (int)blockDim.x) {
-        const int b = d.l_flipped[k];
-        if (member_of_edge(d, b) != m || !d.benab[b]) continue;
-        const double e = (P.gb_eps == 0.0) ? 1.0 : boundary_compute_energy(d, b, P.gb_eps);
-        d.ben[b] = e * P.gb_scaling;
-    }
+    M.nucl_now = nucl_now;
+    M.open = runs ? 1 : 0;
+    M.active = runs ? 1 : 0;
+}
+
+// flip (topological.h:286) leaves the flipped edge's energy without the
+// GB_scaling factor until compute_boundary_energies (calculus.h:104-114) runs at
+// the next step's start.  Steps that skip that pass (GB_eps = 0, where every
+// other energy is the scale itself) recompute only the edges flipped since, for
+// the members active in this step (steps that run k_edge_len_energy recompute
+// every energy there).  k_text empties the list.
+__device__ __forceinline__ void rescale_edge(const Dev& d, const Params& P, int m, int b) {
+    if (member_of_edge(d, b) != m || !d.benab[b]) return;
+    const double e = (P.gb_eps == 0.0) ? 1.0 : boundary_compute_energy(d, b, P.gb_eps);
+    d.ben[b] = e * P.gb_scaling;
 }
 
 // Per table block, for grains, edges and vertices in one launch: the
@@ -130,25 +123,30 @@ __global__ void __launch_bounds__(64 * kCountWaves) k_count_all(Dev d) {
     if (lane == 0) out[lb] = make_int2(r, (bd.e - bd.b) - r);
 }
 
+// The end of a step's lists (one wave): clears their counters and says whether
+// the state is busy.
+__device__ __forceinline__ void end_lists(const Dev& d) {
+    const int lane = (int)threadIdx.x & 63;
+    const int c = lane < C_COUNT ? d.cnt[lane] : 0;
+    const int edited = __builtin_amdgcn_readlane(c, C_FIX1) + __builtin_amdgcn_readlane(c, C_FIX2);
+    const int ran = __builtin_amdgcn_readlane(c, C_RAN);
+    if (lane < C_COUNT) d.cnt[lane] = 0;
+    if (lane == 0 && ran) {
+        const int was = *d.busy, now = edited > kBusyOver ? 1 : (edited < kBusyUnder ? 0 : was);
+        if (now != was) {
+            *d.busy = now;
+            __hip_atomic_store(d.busy_host, now, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
+}
+
 // Sums up member m's last step, if one is open (one workgroup): the per-block
 // partials of the enabled grain and vertex counts, then the step counter,
 // time and stop rules.  Workgroup 0 also clears the step's list counters and
 // says whether the state is busy.
 __device__ __forceinline__ void end_member(const Dev& d, int m) {
     __shared__ int sa[16], sb[16];
-    if (m == 0 && threadIdx.x < 64) {
-        const int c = (int)threadIdx.x < C_COUNT ? d.cnt[threadIdx.x] : 0;
-        const int edited = __builtin_amdgcn_readlane(c, C_FIX1) + __builtin_amdgcn_readlane(c, C_FIX2);
-        const int ran = __builtin_amdgcn_readlane(c, C_RAN);
-        if ((int)threadIdx.x < C_COUNT) d.cnt[threadIdx.x] = 0;
-        if (threadIdx.x == 0 && ran) {
-            const int was = *d.busy, now = edited > kBusyOver ? 1 : (edited < kBusyUnder ? 0 : was);
-            if (now != was) {
-                *d.busy = now;
-                __hip_atomic_store(d.busy_host, now, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            }
-        }
-    }
+    if (m == 0 && threadIdx.x < 64) end_lists(d);
     MState& M = d.ms[m];
     const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wave = tid >> 6, nw = nt >> 6;
     // each lane reads its share of the grain and vertex partials, up to 16
@@ -172,11 +170,7 @@ __device__ __forceinline__ void end_member(const Dev& d, int m) {
 #pragma unroll
         for (int q = 0; q < kBatch; q++) { a += tg[q]; b2 += tv[q]; }
     }
-    // thread 0 may go on to begin the next step, which opens the member: every
-    // wave has to have read the flags before that
-    const bool sum_up = M.active && M.open;
-    __syncthreads();
-    if (!sum_up) return;
+    if (!M.active || !M.open) return;                // the same for the whole workgroup
     a = wave_sum(a);
     b2 = wave_sum(b2);
     if (lane == 0) { sa[wave] = a; sb[wave] = b2; }
@@ -204,11 +198,70 @@ __device__ __forceinline__ void end_member(const Dev& d, int m) {
 // host asks whether all have finished), one workgroup each.
 __global__ void __launch_bounds__(256) k_end(Dev d) { end_member(d, (int)blockIdx.x); }
 
-// The same, and begins the next step: the steps without nucleation, and those
-// whose energies are recomputed before it.
+// Sums up member m's last step and begins the next one (one workgroup): what both
+// read is loaded at once, every thread forms the new loop state from it, and one
+// lane stores it last, so that nothing reads it back or waits for stores in
+// between (2,000 grains: 3.4 us where end and begin one after the other took 5.3).
+struct StepBegin {
+    int active, nucl_now, n;
+};
+__device__ __forceinline__ StepBegin end_begin_member(const Dev& d, int m, bool rescale_flipped) {
+    __shared__ int sa[16], sb[16];
+    const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wave = tid >> 6, nw = nt >> 6;
+    MState v = d.ms[m];
+    const Params P = d.prm[m];
+    const int n_flipped = rescale_flipped ? *d.n_flipped : 0;
+    constexpr int kBatch = 16;
+    const int glo = d.B == 1 ? 0 : d.gblk_first[m], ghi = d.B == 1 ? d.ngb : d.gblk_first[m + 1];
+    const int vlo = d.B == 1 ? 0 : d.vblk_first[m], vhi = d.B == 1 ? d.nvb : d.vblk_first[m + 1];
+    const int ngb = ghi - glo, nvb = vhi - vlo, nmax = max(ngb, nvb);
+    int a = 0, b2 = 0;
+    for (int k0 = tid; k0 < nmax; k0 += kBatch * nt) {
+        int tg[kBatch], tv[kBatch];
+#pragma unroll
+        for (int q = 0; q < kBatch; q++) {
+            const int k = k0 + q * nt;
+            tg[q] = k < ngb ? d.bc_g[glo + k].x : 0;
+            tv[q] = k < nvb ? d.bc_v[vlo + k].x : 0;
+        }
+#pragma unroll
+        for (int q = 0; q < kBatch; q++) { a += tg[q]; b2 += tv[q]; }
+    }
+    a = wave_sum(a);
+    b2 = wave_sum(b2);
+    if (lane == 0) { sa[wave] = a; sb[wave] = b2; }
+    __syncthreads();                                 // (every wave has read the loop state)
+    if (v.active && v.open) {
+        int ra = 0, rb = 0;
+        for (int w = 0; w < nw; w++) { ra += sa[w]; rb += sb[w]; }
+        v.curr_grains = ra;
+        v.n_venabled = rb;
+        v.dt = member_dt(P, v);
+        v.n += 1;
+        v.steps += 1;
+        if (P.adaptive) v.t += v.dt;
+        else v.t = v.n * P.dt_max;
+        if (v.status != 0) v.done = 1;
+        if (v.curr_grains <= P.min_grains && P.min_grains > 0) v.done = 1;
+    }
+    begin_state(P, v);
+    const int nf = v.active ? min(n_flipped, d.E) : 0;
+    for (int k = tid; k < nf; k += nt) rescale_edge(d, P, m, d.l_flipped[k]);
+    if (tid == nt - 64) {
+        // (the event counts and the status are not this kernel's to store)
+        MState& M = d.ms[m];
+        M.n = v.n; M.active = v.active; M.done = v.done; M.curr_grains = v.curr_grains;
+        M.allow_nucl = v.allow_nucl; M.nucl_now = v.nucl_now; M.n_venabled = v.n_venabled; M.open = v.open;
+        M.t = v.t; M.dt = v.dt; M.tau_bits = v.tau_bits; M.vsteps = v.vsteps; M.steps = v.steps;
+    }
+    if (m == 0 && wave == nw - 1) end_lists(d);
+    return StepBegin{v.active, v.nucl_now, v.n};
+}
+
+// The same as a launch: the steps without nucleation, and those whose energies
+// are recomputed before it.
 __global__ void __launch_bounds__(256) k_begin(Dev d, int rescale_flipped) {
-    end_member(d, (int)blockIdx.x);
-    begin_member(d, (int)blockIdx.x, rescale_flipped != 0);
+    end_begin_member(d, (int)blockIdx.x, rescale_flipped != 0);
 }
 
 // ---------------------------------------------------------------------
@@ -1347,7 +1400,7 @@ __global__ void k_text(Dev d) {
     __shared__ int wcnt[kBlock / 64], bbase;
     const int lb_ = xcd_remap((int)blockIdx.x, (int)gridDim.x);
     if (lb_ >= d.neb) return;
-    if (lb_ == 0 && threadIdx.x == 0) *d.n_flipped = 0;   // read by begin_member, filled by the flips
+    if (lb_ == 0 && threadIdx.x == 0) *d.n_flipped = 0;   // read by end_begin_member, filled by the flips
     const Blk bd_ = table_blk(d, d.eblk, lb_);
     const Params& P = d.prm[bd_.m];
     MState& M = d.ms[bd_.m];
@@ -1396,7 +1449,7 @@ __global__ void k_text(Dev d) {
     unsigned long long r = wmin[0];
 #pragma unroll
     for (int w = 1; w < kBlock / 64; w++) r = wmin[w] < r ? wmin[w] : r;
-    // the member's minimum (begin_member set it to +inf): the smallest value
+    // the member's minimum (begin_state set it to +inf): the smallest value
     // whatever the order, so the result equals a serial scan; a block
     // whose minimum is not below the value already there skips the atomic
     const unsigned long long seen = M.tau_bits;
@@ -3017,7 +3070,7 @@ __device__ __forceinline__ void flip(const Dev& d, int bnd, double D, double gb_
     }
     d.ben[bnd] = e;
     {
-        // rescaled at the next step's start (begin_member) when no full pass runs
+        // rescaled at the next step's start (end_begin_member) when no full pass runs
         const int k = ed.flip_slot();
         if (k < d.E) d.l_flipped[k] = bnd;
     }
@@ -3872,7 +3925,7 @@ __device__ __forceinline__ NuclGeom nucl_corners(const NuclSite& t, double rr, i
 // own Philox pair, dE and the factor dE - dE' (the same with the shrunk
 // nucleus).  The head needs it only for the vertex it picks, so it runs there,
 // for that vertex alone, by a wave: lane 0 forms dE and lane 1 dE'.
-__device__ __forceinline__ void nucl_factor_at(const Dev& d, const Params& P, const MState& M, int v, double* dE, double* nfac) {
+__device__ __forceinline__ void nucl_factor_at(const Dev& d, const Params& P, int step, int v, double* dE, double* nfac) {
     double ben[3], se[3], go[3];
     const NuclSite t = nucl_site(d, v, [&](const NuclSite& t_) {
 #pragma unroll
@@ -3890,7 +3943,7 @@ __device__ __forceinline__ void nucl_factor_at(const Dev& d, const Params& P, co
         if (k == 0 || minAL > al) minAL = al;
     }
     double u0, u1;
-    sevc_uniform2(P.seed, (uint32_t)M.n, (uint32_t)(v - P.voff), kStreamMcSite, 0u, &u0, &u1);
+    sevc_uniform2(P.seed, (uint32_t)step, (uint32_t)(v - P.voff), kStreamMcSite, 0u, &u0, &u1);
     const double rr = 0.8 * minAL * u0 + 0.1, ori = 2 * SEVC_PI * u1;
     const int do_scale = (int)threadIdx.x & 1;
     double de = 0.0;
@@ -4281,8 +4334,8 @@ __device__ __forceinline__ int find_kth(const Blk* tbl, const RunScan& rs, const
 }
 
 // The head of a step, one workgroup per member, as `what` asks:
-//  HEAD_BEGIN   sums up the last step and begins this one (end_member,
-//               begin_member; HEAD_RESCALE: with the flipped edges' energies);
+//  HEAD_BEGIN   sums up the last step and begins this one (end_begin_member;
+//               HEAD_RESCALE: with the flipped edges' energies);
 //  HEAD_SELECT  picks the nucleation events of this step and assigns their
 //               free slots:
 //   MC mode (nucleation2.cu:292-443, 33-72, 474): one uniformly chosen alive
@@ -4583,11 +4636,9 @@ __global__ void __launch_bounds__(kNuclThreads) k_head(Dev d, int what) {
     __shared__ int fo_s[kSlotLds];            // the free slots found (grains, boundaries, vertices)
     const int m = blockIdx.x;
     const Params& P = d.prm[m];
-    MState& M = d.ms[m];
-    if (what & HEAD_BEGIN) {
-        end_member(d, m);
-        begin_member(d, m, (what & HEAD_RESCALE) != 0);
-    }
+    StepBegin M;
+    if (what & HEAD_BEGIN) M = end_begin_member(d, m, (what & HEAD_RESCALE) != 0);
+    else M = StepBegin{d.ms[m].active, d.ms[m].nucl_now, d.ms[m].n};
     // a single member's block ranges are the whole tables
     const int gb0 = d.B == 1 ? 0 : d.gblk_first[m], gb1 = d.B == 1 ? d.ngb : d.gblk_first[m + 1];
     const int eb0 = d.B == 1 ? 0 : d.eblk_first[m], eb1 = d.B == 1 ? d.neb : d.eblk_first[m + 1];
@@ -4623,7 +4674,7 @@ __global__ void __launch_bounds__(kNuclThreads) k_head(Dev d, int what) {
         const int A = find_kth(d.vblk, rs, d.bc_v, d.ven, 1, k);
         if (tid < 64 && A >= 0) {
             double dE, nfac;
-            nucl_factor_at(d, P, M, A, &dE, &nfac);
+            nucl_factor_at(d, P, M.n, A, &dE, &nfac);
             const bool take = dE < 0 || (nfac < 0 && u1 < sevc_exp(-P.mc_k * dE));
             if (tid == 0) {
                 d.vnuc[A] = take ? 1 : 0;
