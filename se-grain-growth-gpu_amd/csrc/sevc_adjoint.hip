@@ -37,8 +37,8 @@ __global__ void k_win_prepare(Dev d) {
 //           list has 3 entries or more); kWinOn: an enabled vertex;
 //           kWinSearch: a list neighbour is not the end of one of the
 //           vertex's edges (the steps then search the lists)
-//   vse[3v + j]  stored energy of grain slot j
-//   veb[3v + j]  d gamma_b / d GB_scaling of edge j (null when every member
+//   vse[j V + v]  stored energy of grain slot j
+//   veb[j V + v]  d gamma_b / d GB_scaling of edge j (null when every member
 //           has GB_eps = 0, where it is 1)
 // and the grains' lists in one of two ways.  Where the vertices are ordered
 // along the mesh (win_own_rule), a table block's 256 vertices have about 160
@@ -75,7 +75,7 @@ __global__ void __launch_bounds__(kBlock) k_win_table_v(Dev d, int4* nbr, double
         for (int j = 0; j < 3; j++) {
             const int b = d.vb[3 * v + j];
             w[j] = other_end(d, b, v);
-            if (veb) veb[3 * (size_t)v + j] = (P.gb_eps == 0.0) ? 1.0 : boundary_compute_energy(d, b, P.gb_eps);
+            if (veb) veb[(size_t)j * d.V + v] = (P.gb_eps == 0.0) ? 1.0 : boundary_compute_energy(d, b, P.gb_eps);
         }
 #pragma unroll
         for (int j = 0; j < 3; j++) {
@@ -83,7 +83,7 @@ __global__ void __launch_bounds__(kBlock) k_win_table_v(Dev d, int4* nbr, double
             const int n = d.glen[g];
             const int k = grain_contains_vertex(d, g, v);
             vg[j] = g;
-            vse[3 * (size_t)v + j] = d.gse[g];
+            vse[(size_t)j * d.V + v] = d.gse[g];
             if (k < 0 || n < 3) continue;
             const int* L = glist(d, g);
             const int wp = L[(k + n - 1) % n], wn = L[(k + 1) % n];
@@ -235,8 +235,8 @@ __global__ void __launch_bounds__(kBlock) k_win_step(Dev d, const double* X, con
     uint8_t ng[3];
 #pragma unroll
     for (int j = 0; j < 3; j++) {
-        se[j] = vse[3 * (size_t)iv + j];
-        eb[j] = veb ? veb[3 * (size_t)iv + j] : 1.0;
+        se[j] = vse[(size_t)j * d.V + iv];
+        eb[j] = veb ? veb[(size_t)j * d.V + iv] : 1.0;
     }
     double2 q[3];
     if (kOwn) {
@@ -341,7 +341,7 @@ __global__ void k_win_init(Dev d, double* lam, double* acc_mu, double* acc_s, do
     }
     acc_mu[i] = 0.0;
     acc_s[i] = 0.0;
-    for (int j = 0; j < 3; j++) acc_se[3 * i + j] = 0.0;
+    for (int j = 0; j < 3; j++) acc_se[(size_t)j * d.V + i] = 0.0;
 }
 
 // One reverse step at vertex v, with lambda = dL/dx_{n+1} and the state
@@ -368,9 +368,9 @@ __global__ void __launch_bounds__(kBlock) k_win_adjoint(Dev d, const double* X, 
     double se[3], ebs[3], ase[3];
 #pragma unroll
     for (int j = 0; j < 3; j++) {
-        se[j] = vse[3 * (size_t)v + j];
-        ebs[j] = veb ? veb[3 * (size_t)v + j] : 1.0;
-        ase[j] = acc_se[3 * (size_t)v + j];
+        se[j] = vse[(size_t)j * d.V + v];
+        ebs[j] = veb ? veb[(size_t)j * d.V + v] : 1.0;
+        ase[j] = acc_se[(size_t)j * d.V + v];
     }
     const double am = acc_mu[v], as = acc_s[v];
     if (!(t.w & kWinOn)) {
@@ -431,7 +431,7 @@ __global__ void __launch_bounds__(kBlock) k_win_adjoint(Dev d, const double* X, 
         hgy += c * (la.x - lb.x);
         const double h = sg * 0.5;
         const double tse = -(lx * (h * (dpy + dny)) + ly * (h * (-(dpx + dnx))));
-        acc_se[3 * (size_t)v + j] = ase[j] + dtm * tse;
+        acc_se[(size_t)j * d.V + v] = ase[j] + dtm * tse;
     }
     const double fx = -(ex + gx), fy = -(ey + gy);
     const double hx = hex + hgx, hy = hey + hgy;
@@ -501,7 +501,7 @@ __global__ void k_win_dse(Dev d, const double* acc_se, double* dse) {
             const int v = L[k];
             for (int j = 0; j < 3; j++)
                 if (d.vg[3 * v + j] == i) {
-                    r += acc_se[3 * v + j];
+                    r += acc_se[(size_t)j * d.V + v];
                     break;
                 }
         }
