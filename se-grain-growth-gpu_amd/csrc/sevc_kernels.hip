@@ -1578,7 +1578,7 @@ __device__ __forceinline__ void poll_list(const Dev& d, int nc, unsigned char* p
         // every boundary the rounds and the conflict check look at to its
         // list position (-1: not a listed candidate, whose flag cannot be
         // set since the ends of an enabled edge touch enabled edges only
-        // and k_label lists every enabled candidate).  The rounds and the
+        // and k_text lists every enabled candidate).  The rounds and the
         // check then read LDS only.
         constexpr int kPer = kPollFast / 1024;
         int* cf = reinterpret_cast<int*>(pbuf);
@@ -3148,9 +3148,9 @@ __global__ void k_flip_serial(Dev d) {
 // of launches.  A launch costs 3 to 4.5 us even when its list is empty and
 // starts with cold caches, so that each dependent load of the next stage goes
 // to memory; here the later stages find what the earlier ones read in the
-// workgroup's own L1 and L2.  2,000 grains, three events a step: 25 us where
-// the launches took 63; a batch of 45 events a step 51 us where they took 105;
-// 1M grains, 27 events a step, 68 us where they took 130.  Its time grows with
+// workgroup's own L1 and L2.  2,000 grains, three events a step: 26 us where
+// the launches took 63; a batch of 45 events a step 35 us where they took 105;
+// 1M grains, 27 events a step, 52 us where they took 130.  Its time grows with
 // the number of edited grains (32 at a time), so busy states take the launches.
 //
 // Up to kEvMax listed edges (one to a lane) a lane keeps its edge's
@@ -3161,12 +3161,12 @@ __global__ void k_flip_serial(Dev d) {
 // one wrote there.  A dependent load takes 1.3 us (2,000 grains) to 2.6 us (1M)
 // in this kernel, so loads are issued rounds before their use and without
 // branches around them: the barriers wait for LDS only, and a 3-sided grain's
-// surroundings arrive during the polling and the conflict check.  With the
-// launches' stages one after the other in one workgroup it took 28 us at 2,000
-// grains, 66 for the batch, 82 at 1M; the edit records in LDS (instead of memory)
-// are 5 us of the difference, the early loads 3 to 9.
+// surroundings arrive during the polling and the conflict check.  Loads and
+// stores complete in order, so what no later stage reads is stored at the end.
+// With the launches' stages one after the other in one workgroup it took 28 us at
+// 2,000 grains, 66 for the batch, 82 at 1M.
 // Longer lists, and steps with a two-triangle candidate, run the launches'
-// stages.  512 threads, so that a lane has the registers it needs (182): with
+// stages.  512 threads, so that a lane has the registers it needs (220): with
 // 1024 it had 128 and spilled 119 to scratch memory, 3 to 4 us a step.
 // Sizes: a listed edge is one event at most; a removal flags three grains and
 // records edits at two vertices, a flip four and two.

@@ -21,7 +21,7 @@ constexpr int kPollBig = 16384;      // lists up to this length poll with flags 
 // A step that edits more grains than kBusyOver makes the state busy, one that
 // edits fewer than kBusyUnder makes it calm (member_reduce): a calm state's
 // events run in one workgroup (k_events), a busy one's in a launch per stage.
-// The line is where both cost the same (see k_events).
+// The line is near where both cost the same (see k_events).
 constexpr int kEvMax = 192;          // longest candidate list that k_events runs in LDS
 constexpr int kEvThreads = 512;     // workgroup of k_events
 constexpr int kHeadGrains = 8192;    // largest member whose candidates k_head draws itself
