@@ -4509,6 +4509,7 @@ __device__ __forceinline__ void insert_event(const Dev& d, int m, int A, int B, 
             d.bt[b] = SEVC_MAX_T_EXT;
             set_edge_enabled(d, SB, b, false, true);
             d.bcand[b] = 0;
+            d.blab[b] = 2;          // no slot for k_label_disabled, should the step stop before its labels
             d.conf[b] = -1;
         }
         d.vb[3 * A] = AB; d.vb[3 * A + 1] = CA; d.vb[3 * A + 2] = AD;
