@@ -226,11 +226,27 @@ int fail(sevc_state* s, int code, const std::string& msg) {
             return fail(s, SEVC_E_HIP, std::string(#expr ": ") + hipGetErrorString(e_)); \
     } while (0)
 
+// Device or pinned host memory.  A failure is told to the caller at once, and
+// is not left as the runtime's last error: the launch check of the next call,
+// of any state in this thread, would report it.
+template <typename T>
+hipError_t take_device(T** p, size_t bytes) {
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
+template <typename T>
+hipError_t take_pinned(T** p, size_t bytes) {
+    const hipError_t e = hipHostMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
+
 template <typename T>
 int dalloc(sevc_state* s, T** p, size_t n) {
     void* q = nullptr;
     if (n == 0) n = 1;
-    hipError_t e = hipMalloc(&q, n * sizeof(T));
+    hipError_t e = take_device(&q, n * sizeof(T));
     if (e != hipSuccess) return fail(s, SEVC_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
     s->allocs.push_back(q);
     *p = static_cast<T*>(q);
@@ -693,7 +709,7 @@ int sevc_batch_create(const sevc_options* opts, const sevc_mesh* meshes, int32_t
     d.prm = dprm;
 #undef DA
     if (hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking) != hipSuccess ||
-        hipHostMalloc(&s->busy_h, sizeof(int)) != hipSuccess ||
+        take_pinned(&s->busy_h, sizeof(int)) != hipSuccess ||
         hipEventCreateWithFlags(&s->lag[0], hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&s->lag[1], hipEventDisableTiming) != hipSuccess ||
         hipMemset(d.busy, 0, sizeof(int)) != hipSuccess) {
@@ -1106,7 +1122,7 @@ int stage_room(sevc_state* s, size_t bytes) {
     (void)hipHostFree(s->stage_h);
     s->stage_d = s->stage_h = nullptr;
     s->stage_n = 0;
-    if (hipMalloc(&s->stage_d, bytes) != hipSuccess || hipHostMalloc(&s->stage_h, bytes) != hipSuccess)
+    if (take_device(&s->stage_d, bytes) != hipSuccess || take_pinned(&s->stage_h, bytes) != hipSuccess)
         return fail(s, SEVC_E_NOMEM, "no room for a download");
     s->stage_n = bytes;
     return SEVC_OK;
@@ -1235,8 +1251,8 @@ int sevc_autotune(sevc_state* s, int32_t* tile_grains) {
     // and put back, so the state is left as it was
     double *keep_vel = nullptr, *keep_area = nullptr;
     const size_t nvel = 2 * static_cast<size_t>(s->V), narea = static_cast<size_t>(s->G);
-    if (hipMalloc(&keep_vel, nvel * sizeof(double)) != hipSuccess ||
-        hipMalloc(&keep_area, narea * sizeof(double)) != hipSuccess) {
+    if (take_device(&keep_vel, nvel * sizeof(double)) != hipSuccess ||
+        take_device(&keep_area, narea * sizeof(double)) != hipSuccess) {
         (void)hipFree(keep_vel);
         return fail(s, SEVC_E_NOMEM, "autotune: no room to keep velocities and areas");
     }
@@ -1377,7 +1393,7 @@ int sevc_check_mesh_device(const sevc_mesh* m, int32_t* bad) {
         total += (p.bytes + 255) / 256 * 256;
     }
     char* buf = nullptr;
-    if (hipMalloc(&buf, total) != hipSuccess) return SEVC_E_NOMEM;
+    if (take_device(&buf, total) != hipSuccess) return SEVC_E_NOMEM;
     Params P{};
     P.voff = 0; P.nv = (int)nv; P.eoff = 0; P.ne = (int)ne; P.goff = 0; P.ng = (int)ng;
     P.debug = 1;
@@ -1457,7 +1473,7 @@ int sevc_checkpoint(sevc_state* s, int32_t slot) {
     sevc_state::Ckpt& c = s->ckpts[slot];
     if (!c.buf) {
         HIPCHK(hipStreamSynchronize(s->stream));
-        if (hipMalloc(&c.buf, total) != hipSuccess) return fail(s, SEVC_E_NOMEM, "no room for a checkpoint");
+        if (take_device(&c.buf, total) != hipSuccess) return fail(s, SEVC_E_NOMEM, "no room for a checkpoint");
         c.bytes = total;
     }
     int rc;
@@ -1855,8 +1871,8 @@ extern "C" int sevc_selftest_math(int32_t op, int32_t n, const double* x, const 
     if (n <= 0 || !x || !y || !out) return SEVC_E_INVALID_ARG;
     double *dx = nullptr, *dy = nullptr, *dout = nullptr;
     const size_t bytes = static_cast<size_t>(n) * sizeof(double);
-    if (hipMalloc(&dx, bytes) != hipSuccess || hipMalloc(&dy, bytes) != hipSuccess ||
-        hipMalloc(&dout, bytes) != hipSuccess) {
+    if (take_device(&dx, bytes) != hipSuccess || take_device(&dy, bytes) != hipSuccess ||
+        take_device(&dout, bytes) != hipSuccess) {
         (void)hipFree(dx); (void)hipFree(dy); (void)hipFree(dout);
         return SEVC_E_NOMEM;
     }
