@@ -1718,14 +1718,16 @@ int sevc_window_forward(sevc_state* s, int32_t steps, int32_t ckpt_every) {
     int K = (ckpt_every <= 0 || ckpt_every > steps) ? std::max(steps, 1) : ckpt_every;
     int rc;
     if (win_whole(s, steps)) K = std::max(steps, 1);
+    // from here on the last window's arrays may be given back, and no reverse
+    // pass may read them, also if this call finds no room
+    w.ready = false;
+    w.seeded = false;
     if ((rc = win_buffer(s, &w.seg, &w.seg_n, (static_cast<size_t>(K) + 1) * n2)) != SEVC_OK ||
         (rc = win_buffer(s, &w.segN, &w.segN_n, static_cast<size_t>(K) * V)) != SEVC_OK)
         return rc;
     const int nck = (steps + K - 1) / K;
     if (nck > 1 && (rc = win_buffer(s, &w.ck, &w.ck_n, static_cast<size_t>(nck) * n2)) != SEVC_OK) return rc;
     if ((rc = win_fixed_buffers(s)) != SEVC_OK) return rc;
-    w.ready = false;
-    w.seeded = false;
     launch(s, "win_prepare", k_win_prepare, d.neb, kBlock, d);
     launch(s, "win_table_v", k_win_table_v, d.nvb, kBlock, d, w.nbr, w.vse, w.veb, w.wb);
     if (!w.own) launch(s, "win_table_g", k_win_table_g, d.ngb, kBlock, d, w.wl, w.wn);

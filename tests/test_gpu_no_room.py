@@ -35,3 +35,27 @@ def test_next_call_works(then):
     else:
         getattr(st, then)()
     st.close()
+
+
+def test_no_reverse_pass_over_a_window_that_is_gone():
+    """A window that finds no room gives the last one's arrays back first."""
+    o, mesh = _start()
+    o.events, o.do_nucleation, o.velocity_model = 0, 0, sevc.VEL_ANALYTIC
+    w = np.random.default_rng(2).standard_normal(2 * mesh.nv)
+    st = sevc.State(o, mesh)
+    st.window_forward(5)
+    with pytest.raises(sevc.SevcError) as e:
+        st.window_forward(TOO_LONG)
+    assert e.value.code == sevc.E_NOMEM
+    with pytest.raises(sevc.SevcError) as e:
+        st.adjoint(w)
+    assert e.value.code == sevc.E_STATE
+    st.window_forward(4)
+    got = st.adjoint(w)[0]
+    st.close()
+    st = sevc.State(o, mesh)
+    st.window_forward(5)
+    st.window_forward(4)
+    for a, b in zip(got, st.adjoint(w)[0]):
+        assert np.array_equal(np.asarray(a).view(np.uint64), np.asarray(b).view(np.uint64))
+    st.close()
