@@ -1824,7 +1824,7 @@ int sevc_area_histogram(sevc_state* s, int32_t n_bins, const double* ranges, con
     int rc;
     if ((rc = win_fixed_buffers(s)) != SEVC_OK) return rc;
     const size_t B = s->B, G = s->G, nb = static_cast<size_t>(n_bins);
-    if (!w.hA) {
+    if (!w.hcount) {                         // the last one allocated below
         if ((rc = dalloc(s, &w.hA, G)) || (rc = dalloc(s, &w.hwg, G)) ||
             (rc = dalloc(s, &w.hpart, static_cast<size_t>(d.ngb) * (kMaxHistBins + 1))) ||
             (rc = dalloc(s, &w.hrange, 3 * B)) || (rc = dalloc(s, &w.htarget, B * kMaxHistBins)) ||

@@ -1,0 +1,66 @@
+/* Loaded before libsevc.so with its symbols global, this stands between that
+ * library and the HIP runtime in a test's own process: it notes the calls that
+ * tell which way the library went, and can refuse one allocation. */
+#define _GNU_SOURCE
+#include <dlfcn.h>
+#include <stddef.h>
+#include <stdio.h>
+#include <stdlib.h>
+
+enum { OUT_OF_MEMORY = 2, MOST = 1 << 16 };      /* hipErrorOutOfMemory */
+
+static struct { int kind; void* what; } seen[MOST];
+static int n_seen, refuse;
+
+static void* real(const char* name) {
+    static void* lib;
+    if (!lib) lib = dlopen("libamdhip64.so.7", RTLD_NOW);
+    void* f = lib ? dlsym(lib, name) : NULL;
+    if (!f) {
+        fprintf(stderr, "no %s: %s\n", name, dlerror());
+        abort();
+    }
+    return f;
+}
+
+static void note(int kind, void* what) {
+    if (n_seen < MOST) {
+        seen[n_seen].kind = kind;
+        seen[n_seen++].what = what;
+    }
+}
+
+/* The n-th allocation from now on is refused (0: none). */
+void calls_refuse(int n) { refuse = n; }
+/* Whether the refusal is still to come. */
+int calls_refuse_left(void) { return refuse; }
+/* Forgets the calls so far; the number of calls; the k-th call. */
+void calls_clear(void) { n_seen = 0; }
+int calls_count(void) { return n_seen; }
+int calls_kind(int k) { return seen[k].kind; }
+void* calls_what(int k) { return seen[k].what; }
+
+int hipMalloc(void** p, size_t n) {
+    if (refuse > 0 && --refuse == 0) return OUT_OF_MEMORY;
+    return ((int (*)(void**, size_t))real("hipMalloc"))(p, n);
+}
+
+int hipHostMalloc(void** p, size_t n, unsigned flags) {
+    if (refuse > 0 && --refuse == 0) return OUT_OF_MEMORY;
+    return ((int (*)(void**, size_t, unsigned))real("hipHostMalloc"))(p, n, flags);
+}
+
+int hipGraphLaunch(void* graph, void* stream) {
+    note('G', graph);
+    return ((int (*)(void*, void*))real("hipGraphLaunch"))(graph, stream);
+}
+
+int hipEventRecord(void* event, void* stream) {
+    note('R', event);
+    return ((int (*)(void*, void*))real("hipEventRecord"))(event, stream);
+}
+
+int hipEventSynchronize(void* event) {
+    note('S', event);
+    return ((int (*)(void*))real("hipEventSynchronize"))(event);
+}
