@@ -1104,7 +1104,8 @@ namespace {
 // mesh that fits goes in one round (one launch, one copy: 2,000 grains 0.3 ms
 // where a copy per array took 15.6); of a larger one only the lists held at
 // another stride than the member's are staged, in rounds, and every other
-// array is copied straight to the caller (each copy is then long enough).
+// array is copied straight to the caller (each copy is then long enough).  With
+// no room for the staging every array goes straight, the lists by a strided copy.
 constexpr size_t kStageMax = size_t(32) << 20;
 
 struct Download {
@@ -1116,16 +1117,21 @@ struct Download {
 
 size_t item_bytes(int kind) { return kind == PACK_BYTE ? 1 : 4; }
 
-int stage_room(sevc_state* s, size_t bytes) {
-    if (s->stage_n >= bytes) return SEVC_OK;
+// Whether there is room for `bytes` of staging (device and pinned memory).
+bool stage_room(sevc_state* s, size_t bytes) {
+    if (s->stage_n >= bytes) return true;
     (void)hipFree(s->stage_d);
     (void)hipHostFree(s->stage_h);
     s->stage_d = s->stage_h = nullptr;
     s->stage_n = 0;
-    if (take_device(&s->stage_d, bytes) != hipSuccess || take_pinned(&s->stage_h, bytes) != hipSuccess)
-        return fail(s, SEVC_E_NOMEM, "no room for a download");
+    if (take_device(&s->stage_d, bytes) != hipSuccess) return false;
+    if (take_pinned(&s->stage_h, bytes) != hipSuccess) {
+        (void)hipFree(s->stage_d);
+        s->stage_d = nullptr;
+        return false;
+    }
     s->stage_n = bytes;
-    return SEVC_OK;
+    return true;
 }
 
 // One staged round: every array of `L` into the staging buffer, one copy,
@@ -1184,7 +1190,7 @@ int sevc_get_mesh(sevc_state* s, int32_t m, sevc_mesh* out) {
     size_t total = 0;
     for (const Download& a : all) total += a.dst ? room(a) : 0;
     int rc;
-    if (total <= kStageMax) {
+    if (total <= kStageMax && stage_room(s, total)) {
         PackList L{};
         Download to[kPackSegs];
         size_t at = 0;
@@ -1194,21 +1200,23 @@ int sevc_get_mesh(sevc_state* s, int32_t m, sevc_mesh* out) {
             to[L.n++] = a;
             at += room(a);
         }
-        if ((rc = stage_room(s, total)) != SEVC_OK) return rc;
         return staged_round(s, L, to, total);
     }
     HIPCHK(hipStreamSynchronize(s->stream));
     for (const Download& a : all) {
         if (!a.dst) continue;
-        if (a.kind != PACK_ROW || S == d.S) {
-            HIPCHK(hipMemcpy(a.dst, a.src, a.n * item_bytes(a.kind), hipMemcpyDeviceToHost));
+        if (a.kind != PACK_ROW || S == d.S || !stage_room(s, kStageMax)) {
+            if (a.kind != PACK_ROW || S == d.S)
+                HIPCHK(hipMemcpy(a.dst, a.src, a.n * item_bytes(a.kind), hipMemcpyDeviceToHost));
+            else
+                HIPCHK(hipMemcpy2D(a.dst, 4 * static_cast<size_t>(S), a.src, 4 * static_cast<size_t>(d.S),
+                                   4 * static_cast<size_t>(S), G, hipMemcpyDeviceToHost));
             if (a.kind == PACK_ID || a.kind == PACK_ROW) {
                 int32_t* x = static_cast<int32_t*>(a.dst);
                 for (size_t i = 0; i < a.n; ++i) if (x[i] >= 0) x[i] -= a.off;
             }
             continue;
         }
-        if ((rc = stage_room(s, kStageMax)) != SEVC_OK) return rc;
         const size_t rows = kStageMax / (4 * static_cast<size_t>(S));
         for (size_t r = 0; r < G; r += rows) {
             Download part = a;

@@ -1,6 +1,6 @@
 /* Loaded before libsevc.so with its symbols global, this stands between that
  * library and the HIP runtime in a test's own process: it notes the calls that
- * tell which way the library went, and can refuse one allocation. */
+ * tell which way the library went, and can refuse allocations. */
 #define _GNU_SOURCE
 #include <dlfcn.h>
 #include <stddef.h>
@@ -10,7 +10,7 @@
 enum { OUT_OF_MEMORY = 2, MOST = 1 << 16 };      /* hipErrorOutOfMemory */
 
 static struct { int kind; void* what; } seen[MOST];
-static int n_seen, refuse;
+static int n_seen, refuse, more;
 
 static void* real(const char* name) {
     static void* lib;
@@ -30,10 +30,23 @@ static void note(int kind, void* what) {
     }
 }
 
-/* The n-th allocation from now on is refused (0: none). */
-void calls_refuse(int n) { refuse = n; }
-/* Whether the refusal is still to come. */
+/* The n-th allocation from now on is refused, and the m that follow it. */
+void calls_refuse(int n, int m) {
+    refuse = n;
+    more = m;
+}
+/* Whether a refusal is still to come. */
 int calls_refuse_left(void) { return refuse; }
+
+static int refused(void) {
+    if (refuse == 0 || --refuse > 0) return 0;
+    if (more > 0) {
+        more--;
+        refuse = 1;
+    }
+    return 1;
+}
+
 /* Forgets the calls so far; the number of calls; the k-th call. */
 void calls_clear(void) { n_seen = 0; }
 int calls_count(void) { return n_seen; }
@@ -41,12 +54,12 @@ int calls_kind(int k) { return seen[k].kind; }
 void* calls_what(int k) { return seen[k].what; }
 
 int hipMalloc(void** p, size_t n) {
-    if (refuse > 0 && --refuse == 0) return OUT_OF_MEMORY;
+    if (refused()) return OUT_OF_MEMORY;
     return ((int (*)(void**, size_t))real("hipMalloc"))(p, n);
 }
 
 int hipHostMalloc(void** p, size_t n, unsigned flags) {
-    if (refuse > 0 && --refuse == 0) return OUT_OF_MEMORY;
+    if (refused()) return OUT_OF_MEMORY;
     return ((int (*)(void**, size_t, unsigned))real("hipHostMalloc"))(p, n, flags);
 }
 

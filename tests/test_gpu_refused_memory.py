@@ -36,7 +36,7 @@ want = st.area_histogram(20, ranges, targets, want_grad=True)
 n = 0
 while True:
     st = window()
-    hip.calls_refuse(n + 1)
+    hip.calls_refuse(n + 1, 0)
     if n == 9:
         st.area_histogram(20, ranges, targets)
         assert hip.calls_refuse_left() > 0        # no allocation is left to refuse
@@ -48,3 +48,30 @@ while True:
 print(n)
 """, tmp_path)
     assert out.split() == ["9"]
+
+
+def test_download(tmp_path):
+    """A download needs no room of its own: without the staging (device or
+    pinned memory refused, once or every time), each array goes straight; lists
+    at the member's stride and at another one."""
+    out = _hip_calls.run(START + """
+from sevc._abi import MESH_ARRAYS
+o2 = o.copy()
+o2.max_vrt_per_grn = o.max_vrt_per_grn + 9
+wide = sevc.build_mesh(o2, pos, rid, rng.random(60), rng.random(60), 60)
+for first, more in ((1, 0), (2, 0), (1, 1000), (2, 1000)):
+    for k, m in enumerate((mesh, wide)):
+        st = sevc.State([o, o2], [mesh, wide])
+        hip.calls_refuse(first, more)
+        got = st.get_mesh(k)
+        assert hip.calls_refuse_left() == (more > 0)
+        hip.calls_refuse(0, 0)
+        again = st.get_mesh(k)
+        for name, *_ in MESH_ARRAYS:
+            assert np.array_equal(got[name], again[name]), (first, more, k, name)
+        for name in ("pos", "v_bnd", "v_grn", "b_vtx", "g_vtx", "g_vlen", "g_SE"):
+            assert np.array_equal(got[name], m[name]), (first, more, k, name)
+        st.close()
+print("ok")
+""", tmp_path)
+    assert out.split() == ["ok"]
