@@ -147,6 +147,8 @@ struct sevc_state {
         char* buf = nullptr;
         size_t bytes = 0;
         std::vector<MState> ms;
+        int busy = -1, word = 0;         // sevc_state::busy and the device's word then
+        bool first = false;              // the state is as kept here, and its next step will tell `busy`
     };
     std::vector<Ckpt> ckpts;
     // staging of downloads (sevc_get_mesh): device and pinned host halves,
@@ -978,6 +980,11 @@ static int busy_now(const sevc_state* s) {
     return s->any_events && !s->any_debug ? *static_cast<volatile int*>(s->busy_h) : 0;
 }
 
+// The state is no longer the one of any checkpoint.
+static void other_state(sevc_state* s) {
+    for (auto& c : s->ckpts) c.first = false;
+}
+
 // After the first step of a state: sum it up (which leaves the device's word),
 // wait for it and take its word.  (Left to the next step's begin, the word came
 // too late: 250k grains with thousands of flips ran a first call of 20 steps in
@@ -986,6 +993,15 @@ static int busy_first(sevc_state* s) {
     launch(s, "end", k_end, s->B, 256, s->d);
     HIPCHK(hipStreamSynchronize(s->stream));
     s->busy = busy_now(s);
+    // the checkpoints that hold this state have the word from now on, so that
+    // a step after their restore need not wait for it
+    for (auto& c : s->ckpts) {
+        if (!c.first) continue;
+        HIPCHK(hipMemcpyAsync(c.buf, s->d.busy, sizeof(int), hipMemcpyDeviceToDevice, s->stream));
+        c.busy = s->busy;
+        c.word = *s->busy_h;
+        c.first = false;
+    }
     return SEVC_OK;
 }
 
@@ -1437,7 +1453,8 @@ namespace {
 std::vector<std::pair<void*, size_t>> state_arrays(const sevc_state* s) {
     const Dev& d = s->d;
     const size_t V = s->V, E = s->E, G = s->G, S = s->S;
-    return {{d.pos, 16 * V}, {d.vel, 16 * V}, {d.vb, 12 * V}, {d.vg, 12 * V}, {d.ven, V},
+    // (the busy word first: busy_first)
+    return {{d.busy, 4}, {d.pos, 16 * V}, {d.vel, 16 * V}, {d.vb, 12 * V}, {d.vg, 12 * V}, {d.ven, V},
             {d.venergy, 8 * V}, {d.vparts, 32 * V}, {d.mods, sizeof(ModRec) * V},
             {d.nucl_r, 8 * V}, {d.nucl_ori, 8 * V}, {d.dE, 8 * V}, {d.nfac, 8 * V}, {d.vnuc, V},
             {d.bvx, 8 * E}, {d.ben, 8 * E}, {d.blen, 8 * E}, {d.bt, 8 * E}, {d.benab, E}, {d.bcand, E},
@@ -1490,13 +1507,16 @@ int sevc_checkpoint(sevc_state* s, int32_t slot) {
                           s->stream));
     HIPCHK(hipStreamSynchronize(s->stream));
     c.ms = s->ms_host;
+    c.busy = s->busy < 0 ? -1 : busy_now(s);
+    c.word = *s->busy_h;
+    c.first = c.busy < 0;
     return SEVC_OK;
 }
 
 int sevc_restore(sevc_state* s, int32_t slot) {
     if (!s || slot < 0 || slot >= static_cast<int>(s->ckpts.size()) || !s->ckpts[slot].buf)
         return SEVC_E_INVALID_ARG;
-    const sevc_state::Ckpt& c = s->ckpts[slot];
+    sevc_state::Ckpt& c = s->ckpts[slot];
     int rc;
     if ((rc = copy_state(s, c.buf, false)) != SEVC_OK) return rc;
     // the grains listed for the two-triangle search are not kept: all are listed anew
@@ -1506,6 +1526,11 @@ int sevc_restore(sevc_state* s, int32_t slot) {
     s->ms_prev = c.ms;
     s->ben_dirty = true;
     s->tri_dirty = true;
+    // the events go as they did for the state that comes back, on both sides
+    s->busy = c.busy;
+    *s->busy_h = c.word;
+    other_state(s);
+    c.first = c.busy < 0;
     s->win.ready = false;
     return SEVC_OK;
 }
@@ -1604,6 +1629,7 @@ int sevc_set_member_mesh(sevc_state* s, int32_t m, const sevc_mesh* me) {
     head_rule(s);
     s->ben_dirty = true;          // energies of the restored topology at the next step
     if (s->any_events && !s->any_debug) s->busy = -1;
+    other_state(s);
     s->tri_dirty = true;
     s->win.ready = false;
     drop_graphs(s);

@@ -1,0 +1,85 @@
+"""The route a step's events take, one launch or a launch per stage, follows the
+state: also where another one comes back from a checkpoint.  Either route gives
+the oracle's bits."""
+import numpy as np
+import pytest
+
+import sevc
+from _util import Oracle, diff_fields
+
+pytestmark = pytest.mark.gpu
+
+
+def _start():
+    """1,000 edited grains a step at first, fewer than 60 after 70 steps."""
+    n = 2000
+    pos, rid = sevc.voronoi(n, 5)
+    rng = np.random.default_rng(5)
+    o = sevc.default_options()
+    o.GB_eps, o.n_grains, o.extra_capacity, o.max_vrt_per_grn, o.seed = 0.0, n, 0.3, 64, 5
+    o.adaptive_dt, o.dt, o.do_nucleation, o.flip_threshold = 0, 1e-5, 0, 0.7 / np.sqrt(n)
+    return o, sevc.build_mesh(o, pos, rid, rng.random(n), rng.random(n), n)
+
+
+def _routes(st, k):
+    """The steps of each route among the next k."""
+    st.enable_timing(True)
+    before = st.kernel_times()
+    st.step(k)
+    after = st.kernel_times()
+    st.enable_timing(False)
+    return tuple(after.get(x, (0, 0))[1] - before.get(x, (0, 0))[1] for x in ("events", "poll"))
+
+
+def _same(st, orc):
+    return diff_fields(st.get_mesh(), orc.get_mesh()) == {}
+
+
+def test_restored_state_takes_its_own_route():
+    o, mesh = _start()
+    st = sevc.State(o, mesh)
+    st.checkpoint(0)                             # before any step: not known yet
+    st.step(4)
+    st.checkpoint(1)                             # busy
+    st.step(90)
+    st.checkpoint(2)                             # calm
+    for _ in range(2):
+        assert _routes(st, 4) == (4, 0)
+        st.restore(0)
+        assert _routes(st, 4) == (0, 4)
+        st.restore(2)
+        assert _routes(st, 4) == (4, 0)
+        st.restore(1)
+        assert _routes(st, 4) == (0, 4)
+        st.restore(2)
+    # a checkpoint that never saw its first step, restored after a calm stretch
+    st.close()
+    st = sevc.State(o, mesh)
+    st.checkpoint(3)
+    st.set_mesh(0, mesh)
+    st.step(90)
+    st.restore(3)
+    assert _routes(st, 4) == (0, 4)
+    st.close()
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_same_bits_after_restores(graph):
+    o, mesh = _start()
+    st, orc = sevc.State(o, mesh), Oracle(o, mesh)
+    st.checkpoint(0)
+    st.step(70, graph=graph)
+    st.checkpoint(1)
+    for _ in range(2):
+        st.restore(0)
+        st.step(12, graph=graph)
+        st.restore(1)
+        st.step(12, graph=graph)
+    assert orc.step(82)[0] == 0
+    assert _same(st, orc)
+    st.restore(0)
+    st.step(20, graph=graph)
+    orc = Oracle(o, mesh)
+    assert orc.step(20)[0] == 0
+    assert _same(st, orc)
+    st.close()
