@@ -1023,8 +1023,9 @@ int sevc_step(sevc_state* s, int32_t n_steps, sevc_step_stats* st) {
         s->timing_skip = false;
         if (s->busy < 0 && (rc = busy_first(s)) != SEVC_OK) return rc;
         if ((k + 1) % kLag == 0) {
+            // (the last interval's end; the one before that has been waited for)
             const int w = ((k + 1) / kLag) & 1;
-            if (k >= 2 * kLag) HIPCHK(hipEventSynchronize(s->lag[w]));
+            if (k >= kLag) HIPCHK(hipEventSynchronize(s->lag[w ^ 1]));
             HIPCHK(hipEventRecord(s->lag[w], s->stream));
         }
         if (s->timing && s->pending.size() > 4000) {

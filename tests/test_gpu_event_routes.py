@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 import sevc
+import _hip_calls
 from _util import Oracle, diff_fields
 
 pytestmark = pytest.mark.gpu
@@ -83,3 +84,32 @@ def test_same_bits_after_restores(graph):
     assert orc.step(20)[0] == 0
     assert _same(st, orc)
     st.close()
+
+
+START = """
+n = 2000
+pos, rid = sevc.voronoi(n, 5)
+rng = np.random.default_rng(5)
+o = sevc.default_options()
+o.GB_eps, o.n_grains, o.extra_capacity, o.max_vrt_per_grn, o.seed = 0.0, n, 0.3, 64, 5
+o.adaptive_dt, o.dt, o.do_nucleation, o.flip_threshold = 0, 1e-5, 0, 0.7 / np.sqrt(n)
+mesh = sevc.build_mesh(o, pos, rid, rng.random(n), rng.random(n), n)
+st = sevc.State(o, mesh)
+"""
+
+
+def test_a_call_hears_of_the_device_in_time(tmp_path):
+    """Every 32 steps an event is recorded, and the one before it has been
+    waited for by then: a call is at most 64 steps ahead of the device."""
+    out = _hip_calls.run(START + """
+hip.calls_clear()
+st.step(300)
+made, waited = [], -1
+for kind, event in calls():
+    if kind == "R":
+        print(len(made) - waited, end=" ")
+        made.append(event)
+    if kind == "S":
+        waited = len(made) - 1 - made[::-1].index(event)
+""", tmp_path)
+    assert out.split() == ["1"] * 9
