@@ -116,12 +116,13 @@ struct sevc_state {
     bool any_stop = false;                   // a member with a stop rule (tmax, nmax, leave_percent)
     std::vector<MState> ms_host, ms_prev;
     std::vector<MState> ms_poll;             // members' state read while a call runs (all finished?)
-    // graph replay: gexec holds kGraphSteps steps, gexec1 one step
-    hipGraphExec_t gexec = nullptr;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t gexec1 = nullptr;
-    hipGraph_t graph1 = nullptr;
-    int gbusy = -1;                      // how the captured steps run the events
+    // graph replay: kGraphSteps steps and one step, for a calm state's events
+    // and a busy one's, each captured when first needed
+    struct Steps {
+        hipGraph_t many = nullptr, one = nullptr;
+        hipGraphExec_t run_many = nullptr, run_one = nullptr;
+    };
+    Steps graphs[2];
     // kernel timing
     bool timing = false;
     bool timing_hot_only = false;
@@ -202,12 +203,17 @@ void expect_events(sevc_state* s, int m, const double* SE) {
     if (e > s->ev_rate[m]) s->ev_rate[m] = e;
 }
 
+void drop_steps(sevc_state::Steps& g) {
+    if (g.run_many) (void)hipGraphExecDestroy(g.run_many);
+    if (g.run_one) (void)hipGraphExecDestroy(g.run_one);
+    if (g.many) (void)hipGraphDestroy(g.many);
+    if (g.one) (void)hipGraphDestroy(g.one);
+    g = sevc_state::Steps{};
+}
+
 // Captured steps hold table sizes and parameters: dropped when they change.
 void drop_graphs(sevc_state* s) {
-    if (s->gexec) { (void)hipGraphExecDestroy(s->gexec); s->gexec = nullptr; }
-    if (s->graph) { (void)hipGraphDestroy(s->graph); s->graph = nullptr; }
-    if (s->gexec1) { (void)hipGraphExecDestroy(s->gexec1); s->gexec1 = nullptr; }
-    if (s->graph1) { (void)hipGraphDestroy(s->graph1); s->graph1 = nullptr; }
+    for (auto& g : s->graphs) drop_steps(g);
 }
 
 // A failed sevc_batch_create: the reason goes to sevc_last_error(NULL).
@@ -1006,13 +1012,25 @@ static int busy_first(sevc_state* s) {
 }
 
 // A call is at most 2 kLag steps ahead of the device, so that it hears of a
-// state that turns busy or calm.
+// state that turns busy or calm: every kLag steps the end of the last interval
+// is waited for and this one's is marked.
 constexpr int kLag = 32;
+struct Lead {
+    int at = 0, n = 0;                           // the last mark's step, the marks so far
+};
+static int keep_lead(sevc_state* s, Lead* l, int k) {
+    if (k - l->at < kLag) return SEVC_OK;
+    l->at = k;
+    if (l->n > 0) HIPCHK(hipEventSynchronize(s->lag[(l->n - 1) & 1]));
+    HIPCHK(hipEventRecord(s->lag[l->n++ & 1], s->stream));
+    return SEVC_OK;
+}
 
 int sevc_step(sevc_state* s, int32_t n_steps, sevc_step_stats* st) {
     if (!s || n_steps < 0) return SEVC_E_INVALID_ARG;
     if (n_steps > 0) s->win.ready = false;       // the topology may change
     const int poll = stop_poll(s);
+    Lead lead;
     int rc;
     for (int k = 0; k < n_steps; ++k) {
         bool diag = s->diag_next;
@@ -1022,12 +1040,7 @@ int sevc_step(sevc_state* s, int32_t n_steps, sevc_step_stats* st) {
         launch_step(s, diag);
         s->timing_skip = false;
         if (s->busy < 0 && (rc = busy_first(s)) != SEVC_OK) return rc;
-        if ((k + 1) % kLag == 0) {
-            // (the last interval's end; the one before that has been waited for)
-            const int w = ((k + 1) / kLag) & 1;
-            if (k >= kLag) HIPCHK(hipEventSynchronize(s->lag[w ^ 1]));
-            HIPCHK(hipEventRecord(s->lag[w], s->stream));
-        }
+        if ((rc = keep_lead(s, &lead, k + 1)) != SEVC_OK) return rc;
         if (s->timing && s->pending.size() > 4000) {
             (void)hipStreamSynchronize(s->stream);
             collect_timers(s);
@@ -1041,28 +1054,29 @@ int sevc_step(sevc_state* s, int32_t n_steps, sevc_step_stats* st) {
     return rc;
 }
 
-// Captures kGraphSteps steps and one step as graphs, as the state stands
-// (busy or not).  They hold the steady step; one that must recompute the
-// energies or list the 3-sided grains runs outside them.
-static int capture(sevc_state* s) {
+// Captures kGraphSteps steps and one step as graphs, with the events of a busy
+// state or of a calm one.  They hold the steady step; one that must recompute
+// the energies or list the 3-sided grains runs outside them.
+static int capture(sevc_state* s, int busy) {
     HIPCHK(hipStreamSynchronize(s->stream));
-    drop_graphs(s);
+    sevc_state::Steps& g = s->graphs[busy];
+    drop_steps(g);
     const bool timing = s->timing, dirty = s->ben_dirty, tri = s->tri_dirty;
-    const int busy = s->busy;
+    const int was = s->busy;
     s->timing = s->ben_dirty = s->tri_dirty = false;
-    s->gbusy = s->busy = std::max(busy, 0);
+    s->busy = busy;
     HIPCHK(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
     for (int k = 0; k < kGraphSteps; ++k) launch_step(s, false);
-    HIPCHK(hipStreamEndCapture(s->stream, &s->graph));
-    HIPCHK(hipGraphInstantiate(&s->gexec, s->graph, nullptr, nullptr, 0));
+    HIPCHK(hipStreamEndCapture(s->stream, &g.many));
+    HIPCHK(hipGraphInstantiate(&g.run_many, g.many, nullptr, nullptr, 0));
     HIPCHK(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
     launch_step(s, false);
-    HIPCHK(hipStreamEndCapture(s->stream, &s->graph1));
-    HIPCHK(hipGraphInstantiate(&s->gexec1, s->graph1, nullptr, nullptr, 0));
+    HIPCHK(hipStreamEndCapture(s->stream, &g.one));
+    HIPCHK(hipGraphInstantiate(&g.run_one, g.one, nullptr, nullptr, 0));
     s->ben_dirty = dirty;
     s->tri_dirty = tri;
     s->timing = timing;
-    s->busy = busy;
+    s->busy = was;
     return SEVC_OK;
 }
 
@@ -1071,26 +1085,31 @@ int sevc_step_graph(sevc_state* s, int32_t n_steps, sevc_step_stats* st) {
     if (n_steps > 0) s->win.ready = false;
     int rc;
     const int poll = stop_poll(s);
-    for (int k = 0, next_poll = poll; k < n_steps || !s->gexec;) {
+    Lead lead;
+    for (int k = 0, next_poll = poll;;) {
+        if (s->busy >= 0) s->busy = busy_now(s);
+        const int busy = std::max(s->busy, 0);
+        const sevc_state::Steps& g = s->graphs[busy];
+        if (k >= n_steps && (s->graphs[0].run_one || s->graphs[1].run_one)) break;
         if (k < n_steps && (s->diag_next || s->ben_dirty || s->busy < 0 || (s->tri_dirty && s->any_events))) {
             const bool diag = s->diag_next;
             s->diag_next = false;
             launch_step(s, diag);
             if (s->busy < 0 && (rc = busy_first(s)) != SEVC_OK) return rc;
             k += 1;
-        } else if (!s->gexec || (s->gbusy != s->busy && s->busy >= 0)) {
-            if ((rc = capture(s)) != SEVC_OK) return rc;
+        } else if (!g.run_one) {
+            if ((rc = capture(s, busy)) != SEVC_OK) return rc;
         } else if (n_steps - k >= kGraphSteps) {
-            HIPCHK(hipGraphLaunch(s->gexec, s->stream));
+            HIPCHK(hipGraphLaunch(g.run_many, s->stream));
             k += kGraphSteps;
-        } else if (k < n_steps) {
-            HIPCHK(hipGraphLaunch(s->gexec1, s->stream));
+        } else {
+            HIPCHK(hipGraphLaunch(g.run_one, s->stream));
             k += 1;
         }
+        if ((rc = keep_lead(s, &lead, k)) != SEVC_OK) return rc;
         if (k >= next_poll && k < n_steps) {
             next_poll = k + poll;
             if (all_done(s)) break;
-            s->busy = busy_now(s);               // the stream is idle: the device's word is up to date
         }
     }
     rc = finish_call(s, n_steps > 0);

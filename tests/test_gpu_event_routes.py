@@ -113,3 +113,24 @@ for kind, event in calls():
         waited = len(made) - 1 - made[::-1].index(event)
 """, tmp_path)
     assert out.split() == ["1"] * 9
+
+
+def test_a_call_of_graph_steps_follows_the_state(tmp_path):
+    """A busy state that grows calm within one call changes from one captured
+    run of steps to another, and each is captured once; the oracle's bits."""
+    out = _hip_calls.run(START + """
+from _util import Oracle, diff_fields
+st.checkpoint(0)
+orc = Oracle(o, mesh)
+assert orc.step(257)[0] == 0
+for _ in range(2):
+    st.restore(0)
+    hip.calls_clear()
+    st.step(257, graph=True)
+    runs = [x for kind, x in calls() if kind == "G"]
+    kinds = sorted(set(runs), key=runs.index)
+    print(len(kinds), runs == sorted(runs, key=kinds.index), hash(tuple(kinds)))
+    assert diff_fields(st.get_mesh(), orc.get_mesh()) == {}
+""", tmp_path)
+    a, b = [x.split() for x in out.splitlines()]
+    assert a[:2] == ["2", "True"] and a == b, out
