@@ -4946,9 +4946,10 @@ __global__ void __launch_bounds__(256) k_pack(PackList L, char* out) {
 }
 
 // The arrays of a checkpoint or a restore in one launch, 16 KB to a workgroup,
-// four 16-byte loads in flight a lane.  A copy per array was 38 launches of 2.6 us
-// or more: 40 steps of 60 grains from a restored start 1.51 -> 1.32 ms; at 1M
-// grains it is the bytes that count, and nothing changed.
+// four 16-byte loads in flight a lane (10,000 grains 11.6 us, with the loads one
+// after the other 21.4; 100,000 grains 23 and 32; 1M 251 and 261).  A copy per
+// array was 38 launches of 2.6 us or more: 40 steps of 60 grains from a restored
+// start 1.51 -> 1.32 ms.
 __global__ void __launch_bounds__(256) k_copy_arrays(CopyList L) {
     int k = 0;
     while (k + 1 < L.n && (int)blockIdx.x >= L.seg[k + 1].first) k++;
@@ -4958,19 +4959,20 @@ __global__ void __launch_bounds__(256) k_copy_arrays(CopyList L) {
     const int n = left < kCopyChunk ? (int)left : kCopyChunk, n16 = n >> 4;
     const int4* a = reinterpret_cast<const int4*>(s.src + b0);
     int4* o = reinterpret_cast<int4*>(s.dst + b0);
-    constexpr int kEach = kCopyChunk / 16 / 256;
-    int4 x[kEach];
-#pragma unroll
-    for (int q = 0; q < kEach; q++) {
-        const int i = (int)threadIdx.x + 256 * q;
-        if (i < n16) x[q] = a[i];
+    static_assert(kCopyChunk == 16 * 4 * 256, "four loads a lane");
+    const int i = (int)threadIdx.x;
+    if (n == kCopyChunk) {
+        // (no test between them: a load under one of its own is waited for there,
+        // and an array filled under tests goes through LDS)
+        const int4 x0 = a[i], x1 = a[i + 256], x2 = a[i + 512], x3 = a[i + 768];
+        o[i] = x0;
+        o[i + 256] = x1;
+        o[i + 512] = x2;
+        o[i + 768] = x3;
+        return;
     }
-#pragma unroll
-    for (int q = 0; q < kEach; q++) {
-        const int i = (int)threadIdx.x + 256 * q;
-        if (i < n16) o[i] = x[q];
-    }
-    const int r = 16 * n16 + (int)threadIdx.x;           // at most 15 bytes over
+    for (int k16 = i; k16 < n16; k16 += 256) o[k16] = a[k16];
+    const int r = 16 * n16 + i;                          // at most 15 bytes over
     if (r < n) s.dst[b0 + r] = s.src[b0 + r];
 }
 
