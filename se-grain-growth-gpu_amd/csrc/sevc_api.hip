@@ -7,6 +7,7 @@
 #include <cstdio>
 #include <cstring>
 #include <map>
+#include <numeric>
 #include <string>
 #include <vector>
 
@@ -164,6 +165,7 @@ struct sevc_state {
     struct Window {
         int steps = 0, K = 0, nck = 0, holds = -1;
         bool ready = false, own = true;
+        std::vector<long long> met, seen;  // a sample of each member's table blocks (win_sample)
         double *ck = nullptr, *seg = nullptr;
         uint8_t *segN = nullptr, *neg = nullptr;
         size_t ck_n = 0, seg_n = 0, segN_n = 0;
@@ -387,20 +389,32 @@ int pick_vtile(const sevc_state* s, const std::vector<int>& vg, const std::vecto
 // to 768 (6 times) where they are not.  Up to 512 blocks (131,072 vertices, two
 // workgroups a CU) the chip has room for that; above, a sample of the blocks has
 // to have at most kWinOwnMost grains each on average.
-constexpr int kWinOwnMost = 256;
-bool win_own_rule(const sevc_state* s, const std::vector<int>& vg, const std::vector<uint8_t>& ven) {
-    const size_t nb = s->V / kBlock, every = std::max<size_t>(1, nb / 64);
-    if (nb <= 512) return true;
-    size_t met = 0, seen = 0;
+constexpr int kWinOwnMost = 256, kWinOwnAny = 512;
+
+// Samples the table blocks of member m, whose vertex grains and flags are given.
+void win_sample(sevc_state* s, int m, const int* vg, const uint8_t* ven) {
+    auto& w = s->win;
+    w.met.resize(s->B);
+    w.seen.resize(s->B);
+    w.met[m] = w.seen[m] = 0;
+    if (s->d.nvb <= kWinOwnAny) return;
+    const int every = s->d.nvb / 64 * kBlock;
     std::vector<int> g;
-    for (size_t b = 0; b < nb; b += every, ++seen) {
+    for (int b = 0; b < s->nv[m]; b += every) {
         g.clear();
-        for (size_t v = b * kBlock; v < (b + 1) * kBlock; ++v)
-            if (ven[v]) g.insert(g.end(), vg.begin() + 3 * v, vg.begin() + 3 * v + 3);
+        for (int v = b; v < std::min(b + kBlock, s->nv[m]); ++v)
+            if (ven[v]) g.insert(g.end(), vg + 3 * static_cast<size_t>(v), vg + 3 * static_cast<size_t>(v) + 3);
         std::sort(g.begin(), g.end());
-        met += std::unique(g.begin(), g.end()) - g.begin();
+        w.met[m] += std::unique(g.begin(), g.end()) - g.begin();
+        w.seen[m] += 1;
     }
-    return met <= kWinOwnMost * seen;
+}
+
+void win_own_rule(sevc_state* s) {
+    auto& w = s->win;
+    const long long met = std::accumulate(w.met.begin(), w.met.end(), 0LL);
+    const long long seen = std::accumulate(w.seen.begin(), w.seen.end(), 0LL);
+    w.own = met <= kWinOwnMost * seen;
 }
 
 // Tile table of the one-pass velocity: VT consecutive vertex slots of one
@@ -823,7 +837,9 @@ int sevc_batch_create(const sevc_options* opts, const sevc_mesh* meshes, int32_t
         }
         s->vel_path = 0;
     }
-    s->win.own = win_own_rule(s, vg, ven);
+    for (int m = 0; m < B; ++m)
+        win_sample(s, m, vg.data() + 3 * static_cast<size_t>(s->voff[m]), ven.data() + s->voff[m]);
+    win_own_rule(s);
     UP(d.pos, pos.data(), pos.size() * 8); UP(d.vel, vel.data(), vel.size() * 8);
     UP(d.vb, vb.data(), vb.size() * 4); UP(d.vg, vg.data(), vg.size() * 4); UP(d.ven, ven.data(), V);
     UP(d.venergy, venergy.data(), V * 8); UP(d.vparts, vparts.data(), 4 * V * 8);
@@ -1651,6 +1667,8 @@ int sevc_set_member_mesh(sevc_state* s, int32_t m, const sevc_mesh* me) {
     if (s->any_events && !s->any_debug) s->busy = -1;
     other_state(s);
     s->tri_dirty = true;
+    win_sample(s, m, vg.data(), ven.data());
+    win_own_rule(s);
     s->win.ready = false;
     drop_graphs(s);
     return SEVC_OK;
@@ -1707,19 +1725,31 @@ int win_buffer(sevc_state* s, T** p, size_t* have, size_t n) {
 int win_fixed_buffers(sevc_state* s) {
     auto& w = s->win;
     if (w.dse) return SEVC_OK;               // the last one allocated below
-    const size_t V = s->V, G = s->G, n2 = 2 * V, nvb = static_cast<size_t>(s->d.nvb);
+    const size_t V = s->V, n2 = 2 * V;
     int rc;
     if ((rc = dalloc(s, &w.lamA, n2)) || (rc = dalloc(s, &w.lamB, n2)) || (rc = dalloc(s, &w.acc_mu, V)) ||
         (rc = dalloc(s, &w.acc_s, V)) || (rc = dalloc(s, &w.acc_se, 3 * V)) ||
         (rc = dalloc(s, &w.nbr, V)) || (rc = dalloc(s, &w.vse, 3 * V)) ||
         (s->any_aniso && (rc = dalloc(s, &w.veb, 3 * V)) != SEVC_OK) ||
-        (w.own ? (rc = dalloc(s, &w.wb.loc, V)) || (rc = dalloc(s, &w.wb.count, nvb)) ||
-                     (rc = dalloc(s, &w.wb.grain, kWinBlockGrains * nvb)) ||
-                     (rc = dalloc(s, &w.wb.list, 3 * kWinBlockGrains * nvb))
-               : (rc = dalloc(s, &w.wl, 3 * G)) || (rc = dalloc(s, &w.wn, G)) || (rc = dalloc(s, &w.neg, G))) ||
         (rc = dalloc(s, &w.part, 4 * static_cast<size_t>(s->d.nvb))) ||
         (rc = dalloc(s, &w.out, 2 * static_cast<size_t>(s->B))) ||
         (rc = dalloc(s, &w.dse, static_cast<size_t>(s->G))))
+        return rc;
+    return SEVC_OK;
+}
+
+// The lists of a window's grains, by table block where the steps form the area
+// signs themselves (w.own), else by grain; each kind is kept once it was needed.
+int win_list_buffers(sevc_state* s) {
+    auto& w = s->win;
+    const size_t V = s->V, G = s->G, nvb = static_cast<size_t>(s->d.nvb);
+    int rc;
+    if (w.own && !w.wb.list &&
+        ((rc = dalloc(s, &w.wb.loc, V)) || (rc = dalloc(s, &w.wb.count, nvb)) ||
+         (rc = dalloc(s, &w.wb.grain, kWinBlockGrains * nvb)) || (rc = dalloc(s, &w.wb.list, 3 * kWinBlockGrains * nvb))))
+        return rc;
+    if (!w.own && !w.neg &&
+        ((rc = dalloc(s, &w.wl, 3 * G)) || (rc = dalloc(s, &w.wn, G)) || (rc = dalloc(s, &w.neg, G))))
         return rc;
     return SEVC_OK;
 }
@@ -1748,13 +1778,15 @@ void win_run_segment(sevc_state* s, int len, int last) {
     const Dev& d = s->d;
     auto& w = s->win;
     const size_t n2 = 2 * static_cast<size_t>(s->V);
+    const int4* wl = w.own ? nullptr : w.wl;
+    uint8_t* neg = w.own ? nullptr : w.neg;
     for (int i = 0; i < len; ++i) {
         const double* X = w.seg + i * n2;
         if (!w.own || i == last)
-            launch(s, "win_area", k_win_area, d.ngb, kBlock, d, X, static_cast<const int4*>(w.wl),
-                   static_cast<const int*>(w.wn), w.neg, i == last ? d.garea : static_cast<double*>(nullptr));
+            launch(s, "win_area", k_win_area, d.ngb, kBlock, d, X, wl, static_cast<const int*>(w.wn), neg,
+                   i == last ? d.garea : static_cast<double*>(nullptr));
         launch(s, "win_step", w.own ? k_win_step<true> : k_win_step<false>, d.nvb, kBlock, d, X,
-               static_cast<const uint8_t*>(w.neg), w.wb, static_cast<const int4*>(w.nbr),
+               static_cast<const uint8_t*>(neg), w.wb, static_cast<const int4*>(w.nbr),
                static_cast<const double*>(w.vse), static_cast<const double*>(w.veb), w.seg + (i + 1) * n2,
                w.segN + static_cast<size_t>(i) * s->V, i == last ? 1 : 0);
     }
@@ -1781,9 +1813,10 @@ int sevc_window_forward(sevc_state* s, int32_t steps, int32_t ckpt_every) {
         return rc;
     const int nck = (steps + K - 1) / K;
     if (nck > 1 && (rc = win_buffer(s, &w.ck, &w.ck_n, static_cast<size_t>(nck) * n2)) != SEVC_OK) return rc;
-    if ((rc = win_fixed_buffers(s)) != SEVC_OK) return rc;
+    if ((rc = win_fixed_buffers(s)) != SEVC_OK || (rc = win_list_buffers(s)) != SEVC_OK) return rc;
     launch(s, "win_prepare", k_win_prepare, d.neb, kBlock, d);
-    launch(s, "win_table_v", k_win_table_v, d.nvb, kBlock, d, w.nbr, w.vse, w.veb, w.wb);
+    launch(s, "win_table_v", k_win_table_v, d.nvb, kBlock, d, w.nbr, w.vse, w.veb,
+           w.own ? w.wb : WinBlocks{});
     if (!w.own) launch(s, "win_table_g", k_win_table_g, d.ngb, kBlock, d, w.wl, w.wn);
     HIPCHK(hipMemcpyAsync(w.seg, d.pos, n2 * 8, hipMemcpyDeviceToDevice, s->stream));
     int last = 0;
