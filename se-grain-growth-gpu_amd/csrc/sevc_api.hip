@@ -1705,15 +1705,21 @@ int sevc_set_member_params(sevc_state* s, int32_t m, const double* pos, const do
 
 namespace {
 
+template <typename T>
+void dfree(sevc_state* s, T** p) {
+    if (!*p) return;
+    (void)hipFree(*p);
+    s->allocs.erase(std::find(s->allocs.begin(), s->allocs.end(), static_cast<void*>(*p)));
+    *p = nullptr;
+}
+
 // (Re)allocate a window buffer of at least n values.
 template <typename T>
 int win_buffer(sevc_state* s, T** p, size_t* have, size_t n) {
     if (*p && *have >= n) return SEVC_OK;
     if (*p) {
         (void)hipStreamSynchronize(s->stream);
-        (void)hipFree(*p);
-        s->allocs.erase(std::find(s->allocs.begin(), s->allocs.end(), static_cast<void*>(*p)));
-        *p = nullptr;
+        dfree(s, p);
     }
     *have = 0;
     int rc = dalloc(s, p, n);
@@ -1740,14 +1746,20 @@ int win_fixed_buffers(sevc_state* s) {
 
 // The lists of a window's grains, by table block where the steps form the area
 // signs themselves (w.own), else by grain; each kind is kept once it was needed.
+// Those by table block take 172 bytes a vertex, by grain 27: with no room for the
+// first the state has the second.
 int win_list_buffers(sevc_state* s) {
     auto& w = s->win;
     const size_t V = s->V, G = s->G, nvb = static_cast<size_t>(s->d.nvb);
     int rc;
     if (w.own && !w.wb.list &&
-        ((rc = dalloc(s, &w.wb.loc, V)) || (rc = dalloc(s, &w.wb.count, nvb)) ||
-         (rc = dalloc(s, &w.wb.grain, kWinBlockGrains * nvb)) || (rc = dalloc(s, &w.wb.list, 3 * kWinBlockGrains * nvb))))
-        return rc;
+        (dalloc(s, &w.wb.loc, V) || dalloc(s, &w.wb.count, nvb) || dalloc(s, &w.wb.grain, kWinBlockGrains * nvb) ||
+         dalloc(s, &w.wb.list, 3 * kWinBlockGrains * nvb))) {
+        dfree(s, &w.wb.loc);
+        dfree(s, &w.wb.count);
+        dfree(s, &w.wb.grain);
+        w.own = false;
+    }
     if (!w.own && !w.neg &&
         ((rc = dalloc(s, &w.wl, 3 * G)) || (rc = dalloc(s, &w.wn, G)) || (rc = dalloc(s, &w.neg, G))))
         return rc;

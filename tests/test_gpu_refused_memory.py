@@ -75,3 +75,40 @@ for first, more in ((1, 0), (2, 0), (1, 1000), (2, 1000)):
 print("ok")
 """, tmp_path)
     assert out.split() == ["ok"]
+
+
+def test_window(tmp_path):
+    """Of a window's arrays only the lists by table block (four, the last ones)
+    can be done without."""
+    out = _hip_calls.run(START + """
+def results(st):
+    st.window_forward(3)
+    return [np.concatenate([np.ravel(x) for x in st.adjoint(np.arange(2.0 * mesh.nv))[0]]), st.positions(0),
+            st.get_mesh()["g_area"]]
+
+want = results(sevc.State(o, mesh))
+said = []
+while True:
+    st = sevc.State(o, mesh)
+    hip.calls_refuse(len(said) + 1, 0)
+    try:
+        st.window_forward(3)
+        said.append("done")
+    except sevc.SevcError as e:
+        assert e.code == sevc.E_NOMEM
+        said.append("refused")
+    if hip.calls_refuse_left() > 0:                # more than the call asks for
+        break
+    st = sevc.State(o, mesh)
+    hip.calls_refuse(len(said), 0)
+    try:
+        got = results(st)
+    except sevc.SevcError as e:
+        got = results(st)
+    for a, b in zip(got, want):
+        assert np.array_equal(a.view(np.uint64), b.view(np.uint64)), len(said)
+    st.close()
+print(*said)
+""", tmp_path)
+    said = out.split()
+    assert said[-5:] == ["done"] * 5 and set(said[:-5]) == {"refused"}, out
