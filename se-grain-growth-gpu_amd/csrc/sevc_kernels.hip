@@ -3151,7 +3151,8 @@ __global__ void k_flip_serial(Dev d) {
 // workgroup's own L1 and L2.  2,000 grains, three events a step: 26 us where
 // the launches took 63; a batch of 45 events a step 35 us where they took 105;
 // 1M grains, 27 events a step, 52 us where they took 130.  Its time grows with
-// the number of edited grains (32 at a time), so busy states take the launches.
+// the number of edited grains (32 at a time), so busy states take the launches
+// (kBusyOver: both routes' times).
 //
 // Up to kEvMax listed edges (one to a lane) a lane keeps its edge's
 // surroundings in registers, and everything the stages exchange goes through

@@ -19,14 +19,23 @@ constexpr int kNuclThreads = 1024;   // workgroup of the nucleation manager (one
 constexpr int kPollFast = 2048;      // candidate lists up to this length poll with registers and LDS (two per lane)
 constexpr int kPollBig = 16384;      // lists up to this length poll with flags and t_ext in LDS
 // A step that edits more grains than kBusyOver makes the state busy, one that
-// edits fewer than kBusyUnder makes it calm (member_reduce): a calm state's
-// events run in one workgroup (k_events), a busy one's in a launch per stage.
-// The line is near where both cost the same (see k_events).
+// edits fewer than kBusyUnder makes it calm (end_lists): a calm state's events
+// run in one workgroup (k_events), a busy one's in a launch per stage.  The
+// grains of all members count together, as one workgroup runs them all.  Both
+// routes cost the same at 350 to 500 edited grains, whatever the size and the
+// batch; a step, one workgroup / a launch per stage, in us:
+//     edited grains     160-220   260-300   340-350   380-405   470-505   570-1130
+//     2,000 grains      83 / 98   97 / 106  103 / 108 115 / 108 138 / 111
+//     20,000            80 / 96   97 / 106  101 / 106 107 / 111
+//     250,000                                                   156 / 156 288 / 169
+//     1,000,000        293 / 319 305 / 322            340 / 327 323 / 323 504 / 341
+//     8 of 2,000                  95 / 106  103 / 111 104 / 109 123 / 115 159 / 118
+//     32 of 1,000       90 / 109  98 / 112            127 / 121
 constexpr int kEvMax = 192;          // longest candidate list that k_events runs in LDS
 constexpr int kEvThreads = 512;     // workgroup of k_events
 constexpr int kHeadGrains = 8192;    // largest member whose candidates k_head draws itself
 constexpr int kHeadEvents = 8;       // most nucleations a member may expect for k_head to apply them itself
-constexpr int kBusyOver = 320, kBusyUnder = 160;
+constexpr int kBusyOver = 400, kBusyUnder = 320;
 constexpr int kCountWaves = 4;       // table blocks per workgroup of k_count_all (one wave each)
 
 // What k_head does besides the nucleation's selection.

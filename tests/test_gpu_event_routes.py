@@ -64,6 +64,19 @@ def test_restored_state_takes_its_own_route():
     st.close()
 
 
+def test_route_at_the_line():
+    """Both routes take the same time at 350 to 500 edited grains: the state edits
+    some 600 a step or more up to its 11th step, some 280 to 240 from the 20th to
+    the 24th."""
+    o, mesh = _start()
+    st = sevc.State(o, mesh)
+    st.step(7)
+    assert _routes(st, 4) == (0, 4)
+    st.step(9)
+    assert _routes(st, 4) == (4, 0)
+    st.close()
+
+
 @pytest.mark.parametrize("graph", [False, True])
 def test_same_bits_after_restores(graph):
     o, mesh = _start()
