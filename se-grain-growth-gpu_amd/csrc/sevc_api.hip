@@ -20,8 +20,8 @@ namespace sevc {
 __global__ void k_begin(Dev d, int rescale_flipped);
 __global__ void k_end(Dev d);
 __global__ void k_count_all(Dev d);
-__global__ void k_edge_len_energy(Dev d, int only_nucl);
-__global__ void k_grain_area(Dev d, int only_nucl);
+__global__ void k_edge_len_energy(Dev d);
+__global__ void k_grain_area(Dev d);
 __global__ void k_vertex_energy(Dev d);
 __global__ void k_vel_grain(Dev d, int tuning);
 __global__ void k_vel_vertex(Dev d, int tuning, int listed);
@@ -491,9 +491,9 @@ void launch_step(sevc_state* s, bool diag) {
     if (s->any_rate && !s->head_draw) launch(s, "rate_draw", k_rate_draw, d.ngb, kBlock, d);
     if (all_energies || s->any_analytic || !s->any_nucl) {
         launch(s, "begin", k_begin, s->B, 256, d, all_energies ? 0 : 1);
-        if (all_energies) launch(s, "edge_len_energy", k_edge_len_energy, d.neb, kBlock, d, 0);
+        if (all_energies) launch(s, "edge_len_energy", k_edge_len_energy, d.neb, kBlock, d);
         s->ben_dirty = false;
-        if (diag || s->any_analytic) launch(s, "grain_area", k_grain_area, d.ngb, kBlock, d, 0);
+        if (diag || s->any_analytic) launch(s, "grain_area", k_grain_area, d.ngb, kBlock, d);
         if (diag) launch(s, "vertex_energy", k_vertex_energy, d.nvb, kBlock, d);
         if (s->any_nucl) launch(s, "head", k_head, s->B, kNuclThreads, d, nucl);
     } else {

@@ -270,9 +270,9 @@ __global__ void __launch_bounds__(256) k_begin(Dev d, int rescale_flipped) {
 
 // compute_boundary_arclengths (calculus.h:83-93) fused with
 // compute_boundary_energies (calculus.h:104-114).
-__global__ void k_edge_len_energy(Dev d, int only_nucl) {
+__global__ void k_edge_len_energy(Dev d) {
     TABLE_BLOCK(d.eblk, d.neb)
-    if (!M.active || (only_nucl && !M.nucl_now)) return;
+    if (!M.active) return;
     if (i >= bd_.e || !d.benab[i]) return;
     int a = d.bvx[2 * i], b = d.bvx[2 * i + 1];
     d.blen[i] = arclen(d.pos[2 * a], d.pos[2 * a + 1], d.pos[2 * b], d.pos[2 * b + 1], P.D);
@@ -289,9 +289,9 @@ __device__ __forceinline__ double edge_len_from(const Dev& d, int b, int v, doub
 }
 
 // compute_grain_areas, calculus.h:224-234
-__global__ void k_grain_area(Dev d, int only_nucl) {
+__global__ void k_grain_area(Dev d) {
     TABLE_BLOCK(d.gblk, d.ngb)
-    if (!M.active || (only_nucl && !M.nucl_now)) return;
+    if (!M.active) return;
     if (i >= bd_.e || !d.genab[i]) return;
     d.garea[i] = grain_area(d, i, P.D);
 }
