@@ -372,10 +372,13 @@ typedef struct sevc_grads {
  * main.cu:124-389): `steps` steps of x <- dom_mod(x + dt*mobility*F(x)),
  * F = -grad E the analytic force, with T1/T2/nucleation off and dt the
  * fixed opts.dt, on every member.  Positions are checkpointed every
- * ckpt_every steps (<= 0: every step is kept, no recomputation later; a
- * window of at most 2 GB of positions is kept whole in any case).
- * The state ends at the window's end; the next sevc_step or
- * sevc_set_member_params invalidates the window. */
+ * ckpt_every steps (<= 0: every step is kept, no recomputation later).  A
+ * window whose positions and area signs, 17 bytes a vertex slot and step, take
+ * at most 2 GiB is kept whole too, if an earlier window left the memory for it
+ * or it takes at most an eighth of what is free on the device.
+ * The state ends at the window's end; the next sevc_step,
+ * sevc_set_member_params, sevc_set_member_mesh, sevc_restore or
+ * sevc_window_forward (also one that fails) invalidates the window. */
 int sevc_window_forward(sevc_state* s, int32_t steps, int32_t ckpt_every);
 
 /* Reverse pass over the last window: dL_dpos[m] = dL/dx at the window's

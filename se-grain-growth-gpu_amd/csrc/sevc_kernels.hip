@@ -1497,7 +1497,7 @@ __global__ void k_label_disabled(Dev d) {
 // The boundaries polling and the conflict check look at, for each listed
 // candidate c at position k, mapped to list positions through conf (k_text
 // wrote conf[c] = k; -1 elsewhere), as columns of
-// d.pgat (column f at f * kPollFast):
+// d.pgat (column f at f * kPollBig):
 //   0..5    the boundaries of c's ends a0 (slots 0-2) and a1 (3-5), vb order;
 //   6..23   for slot j = 0..5 and r = 0..2 (column 6 + 3j + r): boundary r
 //           of the far end of the slot's edge x, -1 when x is c, x is
@@ -1690,7 +1690,9 @@ __device__ __forceinline__ void poll_list(const Dev& d, int nc, unsigned char* p
         // to kPollBig candidates in LDS; each candidate's mapped neighbours
         // and bits are read again from k_poll_gather's columns (coalesced,
         // L2-resident) where needed, and the per-candidate results of a
-        // lane are bits of one word (at most 16 candidates per lane).
+        // lane are bits of one word (at most 16 candidates per lane of k_poll's
+        // 1,024 threads, 32 of k_events' 512).
+        static_assert(kPollBig <= 32 * kEvThreads, "a bit of the word for each of a lane's candidates");
         double* ct = reinterpret_cast<double*>(pbuf);
         uint8_t* cf = pbuf + 8 * kPollBig;
         const int* G = d.pgat;
