@@ -1490,7 +1490,8 @@ __global__ void k_text(Dev d) {
 __global__ void k_label_disabled(Dev d) {
     TABLE_BLOCK(d.eblk, d.neb)
     if (i >= bd_.e || !P.events) return;
-    if (d.blab[i] & 2) return;
+    // (a slot enabled since is one of a nucleation that stopped its step: no candidate)
+    if ((d.blab[i] & 2) || d.benab[i]) return;
     d.bcand[i] = is_candidate(d.bt[i], d.blen[i], M.lab_dt, P.flip_thr) ? 1 : 0;
 }
 
@@ -4512,7 +4513,6 @@ __device__ __forceinline__ void insert_event(const Dev& d, int m, int A, int B, 
             d.bt[b] = SEVC_MAX_T_EXT;
             set_edge_enabled(d, SB, b, false, true);
             d.bcand[b] = 0;
-            d.blab[b] = 2;          // no slot for k_label_disabled, should the step stop before its labels
             d.conf[b] = -1;
         }
         d.vb[3 * A] = AB; d.vb[3 * A + 1] = CA; d.vb[3 * A + 2] = AD;
