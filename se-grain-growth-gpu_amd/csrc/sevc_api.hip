@@ -1019,7 +1019,6 @@ static int busy_first(sevc_state* s) {
     // a step after their restore need not wait for it
     for (auto& c : s->ckpts) {
         if (!c.first) continue;
-        HIPCHK(hipMemcpyAsync(c.buf, s->d.busy, sizeof(int), hipMemcpyDeviceToDevice, s->stream));
         c.busy = s->busy;
         c.word = *s->busy_h;
         c.first = false;
@@ -1489,8 +1488,7 @@ namespace {
 std::vector<std::pair<void*, size_t>> state_arrays(const sevc_state* s) {
     const Dev& d = s->d;
     const size_t V = s->V, E = s->E, G = s->G, S = s->S;
-    // (the busy word first: busy_first)
-    return {{d.busy, 4}, {d.pos, 16 * V}, {d.vel, 16 * V}, {d.vb, 12 * V}, {d.vg, 12 * V}, {d.ven, V},
+    return {{d.pos, 16 * V}, {d.vel, 16 * V}, {d.vb, 12 * V}, {d.vg, 12 * V}, {d.ven, V},
             {d.venergy, 8 * V}, {d.vparts, 32 * V}, {d.mods, sizeof(ModRec) * V},
             {d.nucl_r, 8 * V}, {d.nucl_ori, 8 * V}, {d.dE, 8 * V}, {d.nfac, 8 * V}, {d.vnuc, V},
             {d.bvx, 8 * E}, {d.ben, 8 * E}, {d.blen, 8 * E}, {d.bt, 8 * E}, {d.benab, E}, {d.bcand, E},
@@ -1503,10 +1501,13 @@ std::vector<std::pair<void*, size_t>> state_arrays(const sevc_state* s) {
 }
 constexpr int kMaxCkpt = 64;
 
-// The state's arrays into a checkpoint's buffer (to_buf) or back.
-int copy_state(sevc_state* s, char* buf, bool to_buf) {
+// The state's arrays into a checkpoint's buffer (to_buf) or back, then with the
+// device's word on how the events run.
+int copy_state(sevc_state* s, char* buf, bool to_buf, int word) {
     const auto arrays = state_arrays(s);
     CopyList L{};
+    if (!to_buf) L.word = s->d.busy;
+    L.value = word;
     size_t off = 0, blocks = 0;
     for (const auto& a : arrays) {
         char* x = static_cast<char*>(a.first);
@@ -1538,7 +1539,7 @@ int sevc_checkpoint(sevc_state* s, int32_t slot) {
         c.bytes = total;
     }
     int rc;
-    if ((rc = copy_state(s, c.buf, true)) != SEVC_OK) return rc;
+    if ((rc = copy_state(s, c.buf, true, 0)) != SEVC_OK) return rc;
     HIPCHK(hipMemcpyAsync(s->ms_host.data(), s->d.ms, sizeof(MState) * s->ms_host.size(), hipMemcpyDeviceToHost,
                           s->stream));
     HIPCHK(hipStreamSynchronize(s->stream));
@@ -1554,7 +1555,7 @@ int sevc_restore(sevc_state* s, int32_t slot) {
         return SEVC_E_INVALID_ARG;
     sevc_state::Ckpt& c = s->ckpts[slot];
     int rc;
-    if ((rc = copy_state(s, c.buf, false)) != SEVC_OK) return rc;
+    if ((rc = copy_state(s, c.buf, false, c.word)) != SEVC_OK) return rc;
     // the grains listed for the two-triangle search are not kept: all are listed anew
     HIPCHK(hipMemsetAsync(s->d.cnt + C_TRI, 0, sizeof(int), s->stream));
     HIPCHK(hipStreamSynchronize(s->stream));

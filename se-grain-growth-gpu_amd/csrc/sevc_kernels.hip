@@ -4954,6 +4954,7 @@ __global__ void __launch_bounds__(256) k_pack(PackList L, char* out) {
 // array was 38 launches of 2.6 us or more: 40 steps of 60 grains from a restored
 // start 1.51 -> 1.32 ms.
 __global__ void __launch_bounds__(256) k_copy_arrays(CopyList L) {
+    if (L.word && blockIdx.x == 0 && threadIdx.x == 0) *L.word = L.value;
     int k = 0;
     while (k + 1 < L.n && (int)blockIdx.x >= L.seg[k + 1].first) k++;
     const CopySeg s = L.seg[k];

@@ -174,6 +174,8 @@ constexpr int kCopySegs = 48, kCopyChunk = 16384;     // bytes per workgroup
 struct CopyList {
     CopySeg seg[kCopySegs];
     int n;
+    int* word;                           // set to `value` besides (null: none)
+    int value;
 };
 
 }  // namespace sevc
