@@ -196,12 +196,17 @@ void head_rule(sevc_state* s) {
 }
 
 // Events that member m may expect in a step with the stored energies SE (the
-// most so far: earlier ones can come back with a checkpoint).
+// most so far: earlier ones can come back with a checkpoint).  It only says who
+// applies them, so that of a large member a sample will do: the sum over 500,000
+// grains took 250 us of the call that uploads them in 180.
+constexpr int kEventSample = 4096;
 void expect_events(sevc_state* s, int m, const double* SE) {
     const sevc_options& o = s->opts[m];
     if (!(o.events && o.do_nucleation) || o.nucleation_mode != SEVC_NUCL_RATE) return;
     double e = 0.0;
-    for (int g = 0; g < s->ng[m]; ++g) e += std::min(1.0, std::max(0.0, o.nucleation_rate * SE[g]));
+    const int every = std::max(1, s->ng[m] / kEventSample);
+    for (int g = 0; g < s->ng[m]; g += every) e += std::min(1.0, std::max(0.0, o.nucleation_rate * SE[g]));
+    e *= every;
     if (e > s->ev_rate[m]) s->ev_rate[m] = e;
 }
 
