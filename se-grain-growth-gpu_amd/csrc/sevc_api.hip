@@ -20,6 +20,7 @@ namespace sevc {
 __global__ void k_begin(Dev d, int rescale_flipped);
 __global__ void k_end(Dev d);
 __global__ void k_count_all(Dev d);
+__global__ void k_member_clear(Dev d, int m);
 __global__ void k_edge_len_energy(Dev d);
 __global__ void k_grain_area(Dev d);
 __global__ void k_vertex_energy(Dev d);
@@ -1650,11 +1651,6 @@ int sevc_set_member_mesh(sevc_state* s, int32_t m, const sevc_mesh* me) {
     up(d.gse + go, me->g_SE, 8 * static_cast<size_t>(ng));
     up(d.genab + go, genab.data(), static_cast<size_t>(ng));
     up(d.gtype + go, gtype.data(), static_cast<size_t>(ng));
-    ok = ok && hipMemset(d.gfix + go, 0, 4 * static_cast<size_t>(ng)) == hipSuccess &&
-         hipMemset(d.gcand + go, 0, static_cast<size_t>(ng)) == hipSuccess &&
-         hipMemset(d.vnuc + vo, 0, static_cast<size_t>(nv)) == hipSuccess &&
-         hipMemset(d.blab + eo, 2, static_cast<size_t>(ne)) == hipSuccess &&
-         hipMemset(d.cnt + C_TRI, 0, sizeof(int)) == hipSuccess;
     if (!ok) return fail(s, SEVC_E_HIP, "upload of the member's mesh failed");
     // loop state: counts of the new mesh; the step counter and time go on
     MState M;
@@ -1664,6 +1660,9 @@ int sevc_set_member_mesh(sevc_state* s, int32_t m, const sevc_mesh* me) {
     HIPCHK(hipMemcpy(d.ms + m, &M, sizeof(MState), hipMemcpyHostToDevice));
     s->ms_host[static_cast<size_t>(m)].curr_grains = ngr;
     s->ms_host[static_cast<size_t>(m)].n_venabled = nve;
+    const int most = std::max({nv, ne, ng});
+    hipLaunchKernelGGL(k_member_clear, dim3(std::min((most + 255) / 256, 1024)), dim3(256), 0, s->stream, d,
+                       static_cast<int>(m));
     hipLaunchKernelGGL(k_count_all, dim3(count_grid(d)), dim3(64 * kCountWaves), 0, s->stream, d);
     HIPCHK(hipStreamSynchronize(s->stream));
     HIPCHK(hipGetLastError());

@@ -63,6 +63,11 @@ int hipHostMalloc(void** p, size_t n, unsigned flags) {
     return ((int (*)(void**, size_t, unsigned))real("hipHostMalloc"))(p, n, flags);
 }
 
+int hipMemset(void* p, int v, size_t n) {
+    note('M', p);
+    return ((int (*)(void*, int, size_t))real("hipMemset"))(p, v, n);
+}
+
 int hipGraphLaunch(void* graph, void* stream) {
     note('G', graph);
     return ((int (*)(void*, void*))real("hipGraphLaunch"))(graph, stream);
