@@ -112,6 +112,13 @@ struct sevc_state {
     // launch in all; -1: not known yet (the next step is a launch per stage,
     // and its count of edited grains decides)
     int busy = -1;
+    // A mesh that was just made often has many short edges to flip in its first
+    // steps only.  So a new state's word is taken after each of its first steps
+    // until it is calm, kFresh at most: `fresh` is the number of the step to
+    // come (0: past them).  A state restored to where that was not known goes the
+    // same way again: `lead` steps to come are a launch per stage whatever the
+    // word, and do not change it.
+    int fresh = 0, lead = 0;
     int* busy_h = nullptr;                   // pinned, written by the device when it changes
     hipEvent_t lag[2] = {nullptr, nullptr};  // ends of earlier steps of the call (sevc_step)
     bool diag_next = false;
@@ -150,8 +157,9 @@ struct sevc_state {
         char* buf = nullptr;
         size_t bytes = 0;
         std::vector<MState> ms;
-        int busy = -1, word = 0;         // sevc_state::busy and the device's word then
-        bool first = false;              // the state is as kept here, and its next step will tell `busy`
+        int busy = -1, fresh = 0, lead = 0;   // as in sevc_state
+        int word = 0;                    // the device's
+        bool first = false;              // only fresh steps were taken since it was kept or restored
     };
     std::vector<Ckpt> ckpts;
     // staging of downloads (sevc_get_mesh): device and pinned host halves,
@@ -522,7 +530,9 @@ void launch_step(sevc_state* s, bool diag) {
         if (s->tri_dirty) launch(s, "tri_all", k_tri_all, d.ngb, kBlock, d);
         s->tri_dirty = false;
     }
-    const bool one = s->any_events && !s->any_debug && s->busy == 0;
+    d.quiet = s->lead > 0 ? 1 : 0;
+    if (s->lead > 0) s->lead -= 1;
+    const bool one = s->any_events && !s->any_debug && !d.quiet && s->busy == 0;
     if (one) {
         launch(s, "events", k_events, 1, kEvThreads, d);
     } else if (s->any_events) {
@@ -670,6 +680,7 @@ int sevc_batch_create(const sevc_options* opts, const sevc_mesh* meshes, int32_t
     d.poll_fast = kPollFast;
     d.poll_lds = kPollBig;
     d.free_rows = 0;
+    d.quiet = 0;
     int rc = SEVC_OK;
 #define DA(p, n) do { if ((rc = dalloc(s, &(p), (n))) != SEVC_OK) { sevc_destroy(s); return rc; } } while (0)
     DA(d.pos, 2 * V); DA(d.vel, 2 * V); DA(d.vb, 3 * V); DA(d.vg, 3 * V); DA(d.ven, V);
@@ -745,7 +756,8 @@ int sevc_batch_create(const sevc_options* opts, const sevc_mesh* meshes, int32_t
         return SEVC_E_HIP;
     }
     *s->busy_h = 0;
-    s->busy = s->any_events && !s->any_debug ? -1 : 0;
+    s->fresh = s->any_events && !s->any_debug ? 1 : 0;
+    s->busy = -s->fresh;
     d.busy_host = s->busy_h;
 #define UP(dst, src, n) \
     do { if (hipMemcpy((dst), (src), (n), hipMemcpyHostToDevice) != hipSuccess) { sevc_destroy(s); return SEVC_E_HIP; } } while (0)
@@ -1013,20 +1025,29 @@ static void other_state(sevc_state* s) {
     for (auto& c : s->ckpts) c.first = false;
 }
 
-// After the first step of a state: sum it up (which leaves the device's word),
+// After a fresh step of a state: sum it up (which leaves the device's word),
 // wait for it and take its word.  (Left to the next step's begin, the word came
 // too late: 250k grains with thousands of flips ran a first call of 20 steps in
-// one workgroup's event stages, 8.9 ms where it takes 6.)
-static int busy_first(sevc_state* s) {
+// one workgroup's event stages, 8.9 ms where it takes 6.  Taken after the first
+// step alone, 22 members of 2,700 grains, 416 and 283 edits in the first two
+// steps and 100 in the others, ran a first call of 69 steps on the longer route:
+// 11.8 ms, now 9.7.)
+constexpr int kFresh = 4;
+static int take_word(sevc_state* s) {
     launch(s, "end", k_end, s->B, 256, s->d);
     HIPCHK(hipStreamSynchronize(s->stream));
     s->busy = busy_now(s);
-    // the checkpoints that hold this state have the word from now on, so that
-    // a step after their restore need not wait for it
+    const int step = s->fresh;
+    s->fresh = s->busy == 1 && step < kFresh ? step + 1 : 0;
+    if (s->fresh) return SEVC_OK;
+    // the checkpoints that these steps started from have their routes from now
+    // on, so that the steps after a restore need not wait
     for (auto& c : s->ckpts) {
         if (!c.first) continue;
+        c.lead = s->busy == 0 ? step - c.fresh : 0;
         c.busy = s->busy;
         c.word = *s->busy_h;
+        c.fresh = 0;
         c.first = false;
     }
     return SEVC_OK;
@@ -1060,7 +1081,7 @@ int sevc_step(sevc_state* s, int32_t n_steps, sevc_step_stats* st) {
         s->timing_skip = s->timing && (s->timing_steps++ % s->timing_every) != 0;
         launch_step(s, diag);
         s->timing_skip = false;
-        if (s->busy < 0 && (rc = busy_first(s)) != SEVC_OK) return rc;
+        if (s->fresh && (rc = take_word(s)) != SEVC_OK) return rc;
         if ((rc = keep_lead(s, &lead, k + 1)) != SEVC_OK) return rc;
         if (s->timing && s->pending.size() > 4000) {
             (void)hipStreamSynchronize(s->stream);
@@ -1083,7 +1104,8 @@ static int capture(sevc_state* s, int busy) {
     sevc_state::Steps& g = s->graphs[busy];
     drop_steps(g);
     const bool timing = s->timing, dirty = s->ben_dirty, tri = s->tri_dirty;
-    const int was = s->busy;
+    const int was = s->busy, lead = s->lead;
+    s->lead = 0;
     s->timing = s->ben_dirty = s->tri_dirty = false;
     s->busy = busy;
     HIPCHK(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
@@ -1098,6 +1120,7 @@ static int capture(sevc_state* s, int busy) {
     s->tri_dirty = tri;
     s->timing = timing;
     s->busy = was;
+    s->lead = lead;
     return SEVC_OK;
 }
 
@@ -1112,11 +1135,12 @@ int sevc_step_graph(sevc_state* s, int32_t n_steps, sevc_step_stats* st) {
         const int busy = std::max(s->busy, 0);
         const sevc_state::Steps& g = s->graphs[busy];
         if (k >= n_steps && (s->graphs[0].run_one || s->graphs[1].run_one)) break;
-        if (k < n_steps && (s->diag_next || s->ben_dirty || s->busy < 0 || (s->tri_dirty && s->any_events))) {
+        if (k < n_steps && (s->diag_next || s->ben_dirty || s->fresh || s->lead > 0 ||
+                            (s->tri_dirty && s->any_events))) {
             const bool diag = s->diag_next;
             s->diag_next = false;
             launch_step(s, diag);
-            if (s->busy < 0 && (rc = busy_first(s)) != SEVC_OK) return rc;
+            if (s->fresh && (rc = take_word(s)) != SEVC_OK) return rc;
             k += 1;
         } else if (!g.run_one) {
             if ((rc = capture(s, busy)) != SEVC_OK) return rc;
@@ -1551,8 +1575,10 @@ int sevc_checkpoint(sevc_state* s, int32_t slot) {
     HIPCHK(hipStreamSynchronize(s->stream));
     c.ms = s->ms_host;
     c.busy = s->busy < 0 ? -1 : busy_now(s);
+    c.fresh = s->fresh;
+    c.lead = s->lead;
     c.word = *s->busy_h;
-    c.first = c.busy < 0;
+    c.first = c.fresh != 0;
     return SEVC_OK;
 }
 
@@ -1571,9 +1597,11 @@ int sevc_restore(sevc_state* s, int32_t slot) {
     s->tri_dirty = true;
     // the events go as they did for the state that comes back, on both sides
     s->busy = c.busy;
+    s->fresh = c.fresh;
+    s->lead = c.lead;
     *s->busy_h = c.word;
     other_state(s);
-    c.first = c.busy < 0;
+    c.first = c.fresh != 0;
     s->win.ready = false;
     return SEVC_OK;
 }
@@ -1669,7 +1697,9 @@ int sevc_set_member_mesh(sevc_state* s, int32_t m, const sevc_mesh* me) {
     expect_events(s, m, me->g_SE);
     head_rule(s);
     s->ben_dirty = true;          // energies of the restored topology at the next step
-    if (s->any_events && !s->any_debug) s->busy = -1;
+    s->fresh = s->any_events && !s->any_debug ? 1 : 0;
+    s->busy = -s->fresh;
+    s->lead = 0;
     other_state(s);
     s->tri_dirty = true;
     win_sample(s, m, vg.data(), ven.data());

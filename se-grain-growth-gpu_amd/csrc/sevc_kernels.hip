@@ -2611,7 +2611,7 @@ __device__ __forceinline__ void note_step(const Dev& d, int tid, int nt) {
     if (tid == 0) {
         d.cnt[C_NEV] = 0;
         d.cnt[C_NUCL] = 0;
-        d.cnt[C_RAN] = 1;
+        d.cnt[C_RAN] = d.quiet ? 0 : 1;
     }
 }
 

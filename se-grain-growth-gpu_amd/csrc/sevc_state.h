@@ -133,6 +133,7 @@ struct Dev {
     int poll_lds;                         // longest candidate list polled from LDS (<= kPollBig)
     int* busy;                            // 1: many grains edited per step (device copy of *busy_host)
     int* busy_host;                       // the same in pinned host memory, written when it changes
+    int quiet;                            // the step's edits do not change the word
     int free_rows;                        // blocks per kind of one free-slot search round (0: the default)
 };
 

@@ -64,6 +64,67 @@ def test_restored_state_takes_its_own_route():
     st.close()
 
 
+SPIKE = """
+n = 12_000
+pos, rid = sevc.voronoi(n, 5)
+rng = np.random.default_rng(5)
+o = sevc.default_options()
+o.GB_eps, o.n_grains, o.extra_capacity, o.max_vrt_per_grn, o.seed = 0.0, n, 0.3, 64, 5
+o.adaptive_dt, o.dt, o.do_nucleation, o.flip_threshold = 0, 1e-5, 0, 0.3 / np.sqrt(n)
+mesh = sevc.build_mesh(o, pos, rid, rng.random(n), rng.random(n), n)
+st = sevc.State(o, mesh)
+"""
+
+
+def test_a_busy_first_step_alone():
+    """A state that edits some 540 grains in its first step and 230 and fewer in
+    those that follow: a launch per stage for the first two while it is new, for
+    the first one after a restore."""
+    space = {"sevc": sevc, "np": np}
+    exec(SPIKE, space)
+    st = space["st"]
+    st.checkpoint(0)
+    st.step(1)
+    st.checkpoint(1)
+    assert _routes(st, 20) == (19, 1)
+    for _ in range(2):
+        st.restore(0)
+        assert _routes(st, 20) == (19, 1)
+        st.restore(1)
+        assert _routes(st, 20) == (20, 0)
+    st.set_mesh(0, space["mesh"])
+    assert _routes(st, 20) == (18, 2)
+    st.restore(1)
+    st.checkpoint(2)
+    st.restore(0)
+    st.checkpoint(3)
+    st.step(30)
+    st.restore(2)
+    assert _routes(st, 20) == (20, 0)
+    st.restore(3)
+    assert _routes(st, 20) == (19, 1)
+    st.close()
+
+
+def test_a_busy_first_step_alone_by_graphs(tmp_path):
+    """The same with captured steps: one kind of them, and the oracle's bits."""
+    out = _hip_calls.run(SPIKE + """
+from _util import Oracle, diff_fields
+st.checkpoint(0)
+orc = Oracle(o, mesh)
+assert orc.step(17)[0] == 0
+for _ in range(3):
+    st.restore(0)
+    hip.calls_clear()
+    st.step(17, graph=True)
+    runs = [x for kind, x in calls() if kind == "G"]
+    print(len(runs), len(set(runs)), end=" ")
+    assert diff_fields(st.get_mesh(), orc.get_mesh()) == {}
+""", tmp_path)
+    # 15 captured steps after two, then 16 after one
+    assert out.split() == ["8", "2", "2", "1", "2", "1"], out
+
+
 def test_route_at_the_line():
     """Both routes take the same time at 350 to 500 edited grains: the state edits
     some 600 a step or more up to its 11th step, some 280 to 240 from the 20th to
@@ -136,6 +197,7 @@ from _util import Oracle, diff_fields
 st.checkpoint(0)
 orc = Oracle(o, mesh)
 assert orc.step(257)[0] == 0
+st.step(257, graph=True)
 for _ in range(2):
     st.restore(0)
     hip.calls_clear()
