@@ -110,7 +110,7 @@ struct sevc_state {
     bool tri_dirty = true;                   // no grain listed for the two-triangle search yet (upload, restore)
     // how the events run: 1 one launch per stage (a busy state), 0 one
     // launch in all; -1: not known yet (the next step is a launch per stage,
-    // and its count of edited grains decides)
+    // and its count of listed edges decides)
     int busy = -1;
     // A mesh that was just made often has many short edges to flip in its first
     // steps only.  So a new state's word is taken after each of its first steps
@@ -1029,9 +1029,8 @@ static void other_state(sevc_state* s) {
 // wait for it and take its word.  (Left to the next step's begin, the word came
 // too late: 250k grains with thousands of flips ran a first call of 20 steps in
 // one workgroup's event stages, 8.9 ms where it takes 6.  Taken after the first
-// step alone, 22 members of 2,700 grains, 416 and 283 edits in the first two
-// steps and 100 in the others, ran a first call of 69 steps on the longer route:
-// 11.8 ms, now 9.7.)
+// step alone, 22 members of 2,700 grains, busy in the first one or two steps, ran
+// a first call of 69 steps on the longer route: 11.8 ms, now 9.7.)
 constexpr int kFresh = 4;
 static int take_word(sevc_state* s) {
     launch(s, "end", k_end, s->B, 256, s->d);

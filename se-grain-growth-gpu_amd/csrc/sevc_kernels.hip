@@ -145,11 +145,11 @@ __global__ void __launch_bounds__(256) k_member_clear(Dev d, int m) {
 __device__ __forceinline__ void end_lists(const Dev& d) {
     const int lane = (int)threadIdx.x & 63;
     const int c = lane < C_COUNT ? d.cnt[lane] : 0;
-    const int edited = __builtin_amdgcn_readlane(c, C_FIX1) + __builtin_amdgcn_readlane(c, C_FIX2);
+    const int listed = __builtin_amdgcn_readlane(c, C_CAND);
     const int ran = __builtin_amdgcn_readlane(c, C_RAN);
     if (lane < C_COUNT) d.cnt[lane] = 0;
     if (lane == 0 && ran) {
-        const int was = *d.busy, now = edited > kBusyOver ? 1 : (edited < kBusyUnder ? 0 : was);
+        const int was = *d.busy, now = listed > kBusyOver ? 1 : (listed < kBusyUnder ? 0 : was);
         if (now != was) {
             *d.busy = now;
             __hip_atomic_store(d.busy_host, now, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -3170,9 +3170,9 @@ __global__ void k_flip_serial(Dev d) {
 // to memory; here the later stages find what the earlier ones read in the
 // workgroup's own L1 and L2.  2,000 grains, three events a step: 26 us where
 // the launches took 63; a batch of 45 events a step 35 us where they took 105;
-// 1M grains, 27 events a step, 52 us where they took 130.  Its time grows with
-// the number of edited grains (32 at a time), so busy states take the launches
-// (kBusyOver: both routes' times).
+// 1M grains, 27 events a step, 52 us where they took 130.  Past kEvMax listed
+// edges it is the slower way (kBusyOver: both routes' times), so busy states take
+// the launches.
 //
 // Up to kEvMax listed edges (one to a lane) a lane keeps its edge's
 // surroundings in registers, and everything the stages exchange goes through
@@ -3667,7 +3667,6 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, in
             __syncthreads();
             if (tid == 0) s.ncon = 0;
         }
-        if (tid == 0) d.cnt[C_FIX1] = s.nfl;
         ev_edit(d, s, true);
     }
 
@@ -3709,7 +3708,6 @@ __device__ __forceinline__ bool events_in_lds(const Dev& d, int nc, int ntri, in
         if (tid == 0) flip_serial(d, s.con, s.ncon, ed);
         __syncthreads();
     }
-    if (tid == 0) d.cnt[C_FIX2] = s.nfl;
     if (s.nfl > 0) ev_edit(d, s, false);
     // what no later stage reads goes out last: a load waits for the stores before it
     if (on) d.conf[c] = -1;

@@ -18,24 +18,26 @@ constexpr int kMaxHistBins = 64;     // bins of the device area histogram
 constexpr int kNuclThreads = 1024;   // workgroup of the nucleation manager (one per member)
 constexpr int kPollFast = 2048;      // candidate lists up to this length poll with registers and LDS (two per lane)
 constexpr int kPollBig = 16384;      // lists up to this length poll with flags and t_ext in LDS
-// A step that edits more grains than kBusyOver makes the state busy, one that
-// edits fewer than kBusyUnder makes it calm (end_lists): a calm state's events
+// A step that lists more edges than kBusyOver makes the state busy, one that
+// lists fewer than kBusyUnder makes it calm (end_lists): a calm state's events
 // run in one workgroup (k_events), a busy one's in a launch per stage.  The
-// grains of all members count together, as one workgroup runs them all.  Both
-// routes cost the same at 350 to 500 edited grains, whatever the size and the
-// batch; a step, one workgroup / a launch per stage, in us:
-//     edited grains     160-220   260-300   340-350   380-405   470-505   570-1130
-//     2,000 grains      83 / 98   97 / 106  103 / 108 115 / 108 138 / 111
-//     20,000            80 / 96   97 / 106  101 / 106 107 / 111
-//     250,000                                                   156 / 156 288 / 169
-//     1,000,000        293 / 319 305 / 322            340 / 327 323 / 323 504 / 341
-//     8 of 2,000                  95 / 106  103 / 111 104 / 109 123 / 115 159 / 118
-//     32 of 1,000       90 / 109  98 / 112            127 / 121
+// edges of all members count together, as one workgroup runs them all.  The line
+// lies where both cost the same, which is near kEvMax at every size, in batches
+// and for flips, removals and nucleations alike: past it the one workgroup runs
+// the launches' stages.  A step, one workgroup / a launch per stage, in us:
+//     listed edges                      80-95     125-145   153-176   190-205   215-245
+//     2,000 grains, flips              94 / 104  109 / 112 111 / 111 135 / 116 162 / 118
+//     20,000, flips                   101 / 114  121 / 124           170 / 126
+//     250,000, flips                  157 / 173            183 / 176           258 / 183
+//     1,000,000, flips                336 / 354  350 / 362 353 / 357
+//     400,000 to 500,000, nucleations            243 / 266 271 / 264 282 / 268 328 / 285
+//     8 of 2,000, flips                          113 / 116 117 / 115 165 / 119 180 / 125
+//     32 of 2,000, nucleations        157 / 183  177 / 192
 constexpr int kEvMax = 192;          // longest candidate list that k_events runs in LDS
 constexpr int kEvThreads = 512;     // workgroup of k_events
 constexpr int kHeadGrains = 8192;    // largest member whose candidates k_head draws itself
 constexpr int kHeadEvents = 8;       // most nucleations a member may expect for k_head to apply them itself
-constexpr int kBusyOver = 400, kBusyUnder = 320;
+constexpr int kBusyOver = 180, kBusyUnder = 150;
 constexpr int kCountWaves = 4;       // table blocks per workgroup of k_count_all (one wave each)
 
 // What k_head does besides the nucleation's selection.
@@ -131,9 +133,9 @@ struct Dev {
     int* chk_bad;                         // violations per member found by the last check
     int poll_fast;                        // longest candidate list polled from registers (<= kPollFast)
     int poll_lds;                         // longest candidate list polled from LDS (<= kPollBig)
-    int* busy;                            // 1: many grains edited per step (device copy of *busy_host)
+    int* busy;                            // 1: many edges listed per step (device copy of *busy_host)
     int* busy_host;                       // the same in pinned host memory, written when it changes
-    int quiet;                            // the step's edits do not change the word
+    int quiet;                            // the step's list does not change the word
     int free_rows;                        // blocks per kind of one free-slot search round (0: the default)
 };
 

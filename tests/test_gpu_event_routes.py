@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 
 def _start():
-    """1,000 edited grains a step at first, fewer than 60 after 70 steps."""
+    """More than 300 listed edges a step at first, fewer than 30 after 70 steps."""
     n = 2000
     pos, rid = sevc.voronoi(n, 5)
     rng = np.random.default_rng(5)
@@ -65,7 +65,7 @@ def test_restored_state_takes_its_own_route():
 
 
 SPIKE = """
-n = 12_000
+n = 16_000
 pos, rid = sevc.voronoi(n, 5)
 rng = np.random.default_rng(5)
 o = sevc.default_options()
@@ -77,7 +77,7 @@ st = sevc.State(o, mesh)
 
 
 def test_a_busy_first_step_alone():
-    """A state that edits some 540 grains in its first step and 230 and fewer in
+    """A state that flips 170 edges in its first step and a third and fewer in
     those that follow: a launch per stage for the first two while it is new, for
     the first one after a restore."""
     space = {"sevc": sevc, "np": np}
@@ -126,9 +126,8 @@ for _ in range(3):
 
 
 def test_route_at_the_line():
-    """Both routes take the same time at 350 to 500 edited grains: the state edits
-    some 600 a step or more up to its 11th step, some 280 to 240 from the 20th to
-    the 24th."""
+    """Both routes take the same time at some 170 listed edges: the state lists 250
+    a step or more up to its 11th step, 128 and fewer from the 18th."""
     o, mesh = _start()
     st = sevc.State(o, mesh)
     st.step(7)
